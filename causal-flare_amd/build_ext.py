@@ -40,6 +40,9 @@ FILE_FLAGS = {
     "flare_ar_prep.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "flare_ar_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "flare_ar_pc.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "flare_wave_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "flare_wave_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "flare_wave_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

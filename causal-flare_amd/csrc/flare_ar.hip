@@ -13,6 +13,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <initializer_list>
 #include <mutex>
 
 #include "flare_common.h"
@@ -204,6 +205,22 @@ __global__ __launch_bounds__(kNT) void chunk_output_kernel(
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
+// Banks with an instance of flare_wave.h: any M up to 256 (latents past M are masked),
+// equal head dims of 16, 32, 48, 64, 96 or 128, chunks of whole 16-token tiles, and rows
+// that 16-byte accesses reach (the dims make every row a multiple of 16 bytes long, so the
+// base pointers decide).  Everything else stays on the tokenwise kernels, which take 2 to 28
+// times as long on every bank measured here (M 32 to 256, D 32 to 128, 16-bit and fp32).
+static bool wave_shape(int64_t M, int64_t Dk, int64_t Dv) {
+    const int64_t dt = Dv / 16;
+    return Dk == Dv && Dv % 16 == 0 && (dt == 1 || dt == 2 || dt == 3 || dt == 4 || dt == 6 || dt == 8) && M <= 256;
+}
+static bool wave_supported(int64_t M, int64_t Dk, int64_t Dv, int64_t chunk, std::initializer_list<const void*> ptrs) {
+    if (!wave_shape(M, Dk, Dv) || chunk % 16 != 0) return false;
+    for (const void* p : ptrs)
+        if (((uintptr_t)p & 15) != 0) return false;
+    return true;
+}
+
 static int launch_prepare(const void* Q, const void* K, const void* V, int dtype, int64_t B,
                           int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv, float scale,
                           int64_t chunk, float* cmax, float* cden, float* cnum,
@@ -216,9 +233,15 @@ static int launch_prepare(const void* Q, const void* K, const void* V, int dtype
         if (output_pc_enabled() && (M == 128 || M == 256))
             return launch_prepare_pc(Q, K, V, B, N, H, M, Dk, scale, chunk, cmax, cden, cnum, tmask,
                                      dtype == FLARE_F16, stream);
-        if (tmask == nullptr)
+        if (tmask == nullptr && !output_pc_enabled())
             return launch_prepare_mfma(Q, K, V, B, N, H, M, Dk, scale, chunk, cmax, cden, cnum, dtype == FLARE_F16,
                                        stream);
+    }
+    if (power <= 0.0f && (mfma_phase_mask() & 1) && wave_supported(M, Dk, Dv, chunk, {Q, K, V, cnum})) {
+        const WaveArgs a{Q, K, V, nullptr, nullptr, B, N, H, M, Dk, scale, chunk, tmask};
+        return dtype == FLARE_BF16  ? wave::prepare_bf16(a, cmax, cden, cnum, stream)
+               : dtype == FLARE_F16 ? wave::prepare_f16(a, cmax, cden, cnum, stream)
+                                    : wave::prepare_f32(a, cmax, cden, cnum, stream);
     }
     FLARE_REQUIRE(Dv <= 4 * kPrepCols, "chunk_prepare: Dv=%lld exceeds %d", (long long)Dv, 4 * kPrepCols);
     const int64_t NC = (N + chunk - 1) / chunk;
@@ -337,6 +360,13 @@ static int launch_output(const void* Q, const void* K, const void* V, const void
             return scalar(redo);
         }
     }
+    if (power <= 0.0f && (mfma_phase_mask() & 2) && lse_dec == nullptr &&
+        wave_supported(M, Dk, Dv, chunk, {Q, K, V, Qdec, Kdec, pnum, Y})) {
+        const WaveArgs a{Q, K, V, Qdec, Kdec, B, N, H, M, Dk, scale, chunk, tmask};
+        return dtype == FLARE_BF16  ? wave::output_bf16(a, pmax, pden, pnum, Y, out_dtype, stream)
+               : dtype == FLARE_F16 ? wave::output_f16(a, pmax, pden, pnum, Y, out_dtype, stream)
+                                    : wave::output_f32(a, pmax, pden, pnum, Y, out_dtype, stream);
+    }
     return scalar(nullptr);
 }
 
@@ -352,11 +382,7 @@ int launch_prefix_public(float* cmax, float* cden, float* cnum, int64_t BH, int6
     return launch_prefix(cmax, cden, cnum, BH, NC, M, Dv, m0, d0, u0, m_fin, d_fin, u_fin, stream);
 }
 
-int64_t default_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
-    // One round of chunk workgroups over the device: about one (chunk, b, h)
-    // per resident workgroup slot.  Longer chunks mean fewer, cheaper summaries (phase 2
-    // and the summary traffic of phases 1 and 3 shrink with them); each chunk
-    // is a multiple of 64 tokens, between 64 and 8192.
+static int device_cus() {
     static int cus = 0;
     if (cus <= 0) {
         int dev = 0, n = 0;
@@ -366,14 +392,36 @@ int64_t default_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
         else
             cus = 256;
     }
+    return cus;
+}
+
+// One round of chunk workgroups over the device: about one (chunk, b, h) per resident
+// workgroup slot of the producer / consumer kernels.  Longer chunks mean fewer, cheaper
+// summaries (phase 2 and the summary traffic of phases 1 and 3 shrink with them); each chunk
+// is a multiple of 64 tokens, between 64 and 8192.
+static int64_t round_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
     const int64_t BH = B * H;
     // the output kernel fills a compute unit with one workgroup, except for the
     // small banks (M * Dv below 128 x 128), where two share it
     const int64_t per_cu = (M * Dv >= 128 * 128) ? 1 : 2;
-    const int64_t target_chunks = (per_cu * cus + BH - 1) / BH;
+    const int64_t target_chunks = (per_cu * device_cus() + BH - 1) / BH;
     int64_t c = (N + target_chunks - 1) / target_chunks;
     c = ((c + 63) / 64) * 64;
     if (c < 64) c = 64;
+    if (c > 8192) c = 8192;
+    return c;
+}
+
+int64_t default_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
+    if (!wave_shape(M, Dv, Dv) || ((M == 128 || M == 256) && (Dv == 64 || Dv == 128))) return round_chunk(B, N, H, M, Dv);
+    // The wave kernels: about two waves per SIMD over the device (8 a compute unit), each
+    // wave with 64 latents of a narrow bank or 32 of a wider one.
+    const int64_t NW = Dv <= 32 && M > 32 ? (M + 63) / 64 : (M + 31) / 32;
+    const int64_t wgs = B * H * NW;
+    const int64_t target_chunks = (8 * device_cus() + wgs - 1) / wgs;
+    int64_t c = (N + target_chunks - 1) / target_chunks;
+    c = ((c + 31) / 32) * 32;
+    if (c < 32) c = 32;
     if (c > 8192) c = 8192;
     return c;
 }
@@ -641,7 +689,11 @@ int flare_ar_forward_noalloc(const void* Q, const void* K, const void* V, const 
     FLARE_REQUIRE(Q && K && V && Y, "ar_forward_noalloc: null pointer");
     FLARE_REQUIRE(B > 0 && N > 0 && H > 0 && M > 0 && Dk > 0 && Dv > 0,
                   "ar_forward_noalloc: sizes must be positive");
-    if (chunk <= 0) chunk = default_chunk(B, N, H, M, Dv);
+    if (chunk <= 0) {
+        chunk = default_chunk(B, N, H, M, Dv);
+        // the shorter chunks of the wave kernels only where their summaries fit as well
+        if (flare_ar_forward_workspace_size(B, N, H, M, Dv, chunk) > kScratchBytes) chunk = round_chunk(B, N, H, M, Dv);
+    }
     // the separate-decoder workspace when it fits (MFMA path), else the plain one
     size_t bytes = flare_ar_forward_workspace_size(B, N, H, M, Dv, chunk);
     FLARE_REQUIRE(bytes <= kScratchBytes,

@@ -159,3 +159,25 @@ int ar_backward_run(const void* Q, const void* K, const void* V, const void* Qde
                     const void* dY, void* dQ, void* dK, void* dV, void* dQdec, void* dKdec, void* workspace,
                     size_t workspace_bytes, hipStream_t stream, float power);
 }  // namespace flare
+
+namespace flare {
+// The chunked forward on fp32 matrix products (flare_wave.h).
+struct WaveArgs {
+    const void *Q, *K, *V, *Qdec, *Kdec;
+    int64_t B, N, H, M, D;
+    float scale;
+    int64_t chunk;
+    const int32_t* tmask;
+};
+namespace wave {
+int prepare_f32(const WaveArgs& a, float* cmax, float* cden, float* cnum, hipStream_t st);
+int prepare_bf16(const WaveArgs& a, float* cmax, float* cden, float* cnum, hipStream_t st);
+int prepare_f16(const WaveArgs& a, float* cmax, float* cden, float* cnum, hipStream_t st);
+int output_f32(const WaveArgs& a, const float* pmax, const float* pden, const float* pnum, void* Y, int out_dtype,
+               hipStream_t st);
+int output_bf16(const WaveArgs& a, const float* pmax, const float* pden, const float* pnum, void* Y, int out_dtype,
+                hipStream_t st);
+int output_f16(const WaveArgs& a, const float* pmax, const float* pden, const float* pnum, void* Y, int out_dtype,
+               hipStream_t st);
+}  // namespace wave
+}  // namespace flare

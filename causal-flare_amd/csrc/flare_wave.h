@@ -1,0 +1,734 @@
+// flare_wave.h -- chunked causal FLARE forward with wave-private latents and fp32 matrix
+// products (phases 1 and 3; phase 2 is chunk_prefix_kernel).
+//
+// Serves fp32 inputs of every bank and 16-bit inputs of the banks that have no instance of
+// the 16-bit kernels in flare_ar_prep.hip / flare_ar_out.hip: M <= 256, Dk = Dv = 16 DT.
+// Everything the tokenwise kernels (flare_ar.hip) hold in fp32 stays in fp32: the weights
+// E and W, the numerator U and every product of them run on the fp32 MFMA (16x16x4); the
+// scores of 16-bit inputs run on the 16-bit MFMA, whose products are exact.
+//
+// Why waves own latents: a wave holds MT*16 latents over all D value columns, so scores,
+// running max, den, numerator and the in-tile products need no other wave; the waves of a
+// workgroup only add their partial outputs, one barrier per 16-token tile (none when one
+// wave holds the bank).  The operand layouts of v_mfma_f32_16x16x4 then make every product
+// of a tile a register-to-register chain.  With lane = (g, c), g = lane / 16, c = lane % 16:
+//   C of a product        row 4g + i (i = register), column c
+//   A / B of a product    row (column) c, contraction index g; register i of a C tile is
+//                         therefore the operand for contraction indices 4g + i.
+//   scores^T [m][t], U [m][d], G^T [tau][t], y [t][d] are all C tiles; W and E contract over
+//   m straight from the scores' registers, G over tau straight from its own.  Only E of the
+//   U update needs the other orientation; it crosses through a wave-private LDS tile.
+//
+// What bounds it: the fp32 MFMA.  A 64 x 32 bank issues 88 of them a 16-token tile and wave
+// in phase 3 (2,816 cycles of its SIMD's matrix pipe) against about 1,300 cycles of vector
+// instructions.  Measured on MI355X, whole forward, tokenwise kernels -> these:
+//   bf16 B 8, N 4096, H 16, M 64, D 32     4937 -> 174 us (prepare 41, scan 7, output 139)
+//   fp16 B 3, N 1531, H 8, M 96, D 64, cached state and mask   1135 -> 136 us
+//   fp32 B 1, N 256, H 8, M 64, D 32        283 ->  31 us
+// Errors against 64 bits: fp32 outputs 2.5e-7 -> 1.4e-7, 16-bit ones unchanged.
+#pragma once
+
+#include "flare_common.h"
+#include "flare_mfma.h"
+
+namespace flare {
+namespace wave {
+
+using mfma::bf16x8;
+using mfma::f32x4;
+using mfma::kLog2e;
+
+constexpr int TT = 16;              // tokens per tile
+// A latent's max may rise by this much (nats) inside a tile before the tile runs token by
+// token: below it every den and weight of the tile keeps full fp32 precision against the
+// tile's max (e^-60 is far above the fp32 underflow).
+constexpr float kTileJump = 60.0f;
+
+__device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// ---------------------------------------------------------------------------
+// Rows of D contraction elements as an MFMA operand: lane (g, c) holds its share of row c.
+// ---------------------------------------------------------------------------
+template <typename T, int D>
+struct RowOp {   // 16-bit: steps of 32 columns, 8 a lane group; a last step of 16 fills two groups
+    static constexpr int S = (D + 31) / 32;
+    bf16x8 a[S];
+    __device__ __forceinline__ void load(const T* row, int g) {
+        const mfma::bf16* p = reinterpret_cast<const mfma::bf16*>(row);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            if (32 * s + 32 <= D) {
+                a[s] = *reinterpret_cast<const bf16x8*>(p + 32 * s + 8 * g);
+            } else {
+                const bf16x8 x = *reinterpret_cast<const bf16x8*>(p + 32 * s + 8 * (g & 1));
+                a[s] = g < 2 ? x : bf16x8{};
+            }
+        }
+    }
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int s = 0; s < S; ++s) a[s] = bf16x8{};
+    }
+};
+template <int D>
+struct RowOp<float, D> {   // lane group g holds columns [g D/4, (g+1) D/4)
+    f32x4 a[D / 16];
+    __device__ __forceinline__ void load(const float* row, int g) {
+#pragma unroll
+        for (int s = 0; s < D / 16; ++s) a[s] = *reinterpret_cast<const f32x4*>(row + g * (D / 4) + 4 * s);
+    }
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int s = 0; s < D / 16; ++s) a[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+};
+
+// c += x . y^T over D (rows of x become C rows, rows of y C columns)
+template <typename T, int D>
+__device__ __forceinline__ f32x4 dot_rows(const RowOp<T, D>& x, const RowOp<T, D>& y, f32x4 c) {
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int s = 0; s < D / 16; ++s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c = mma4(x.a[s][e], y.a[s][e], c);
+    } else {
+        constexpr bool F16 = __is_same(T, __half);
+#pragma unroll
+        for (int s = 0; s < RowOp<T, D>::S; ++s) c = mfma::mma_in<F16>(x.a[s], y.a[s], c);
+    }
+    return c;
+}
+
+// ---------------------------------------------------------------------------
+// Column tiles of a row of D = 16 DT values.  Which 16 columns make tile dt is free (a
+// product only needs both sides to agree), so lane c takes consecutive columns, in pieces
+// of 8, 4, 2 and 1: loads and stores are as wide as the pieces.
+// ---------------------------------------------------------------------------
+template <int DT>
+__host__ __device__ constexpr int piece_of(int dt) {   // size of the piece that holds tile dt
+    int off = 0;
+    for (int p = 8; p >= 1; p >>= 1)
+        if (DT & p) {
+            if (dt < off + p) return p;
+            off += p;
+        }
+    return 1;
+}
+template <int DT>
+__host__ __device__ constexpr int piece_off(int dt) {  // first tile of that piece
+    int off = 0;
+    for (int p = 8; p >= 1; p >>= 1)
+        if (DT & p) {
+            if (dt < off + p) return off;
+            off += p;
+        }
+    return off;
+}
+// column of tile dt at lane c
+template <int DT>
+__device__ __forceinline__ int col_of(int dt, int c) {
+    return 16 * piece_off<DT>(dt) + c * piece_of<DT>(dt) + (dt - piece_off<DT>(dt));
+}
+
+template <typename T>
+__device__ __forceinline__ float word_f32(unsigned w, bool hi) {
+    if constexpr (__is_same(T, __half)) {
+        return (float)__builtin_bit_cast(mfma::f16, (unsigned short)(hi ? w >> 16 : w & 0xffffu));
+    } else {
+        return __builtin_bit_cast(float, hi ? (w & 0xffff0000u) : (w << 16));
+    }
+}
+
+// One row's columns of lane c, raw (16-bit types stay packed until they are used).
+template <typename T, int DT>
+struct ColRow {
+    static constexpr int W = sizeof(T) == 4 ? DT : (DT + 1) / 2;
+    unsigned w[W];
+    __device__ __forceinline__ void load(const T* row, int c) {
+#pragma unroll
+        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
+            const T* p = row + col_of<DT>(dt, c);
+            const int P = piece_of<DT>(dt);
+            if constexpr (sizeof(T) == 4) {
+                if (P == 8) {
+                    *reinterpret_cast<uint4*>(w + dt) = reinterpret_cast<const uint4*>(p)[0];
+                    *reinterpret_cast<uint4*>(w + dt + 4) = reinterpret_cast<const uint4*>(p)[1];
+                } else if (P == 4) {
+                    *reinterpret_cast<uint4*>(w + dt) = *reinterpret_cast<const uint4*>(p);
+                } else if (P == 2) {
+                    *reinterpret_cast<uint2*>(w + dt) = *reinterpret_cast<const uint2*>(p);
+                } else {
+                    w[dt] = *reinterpret_cast<const unsigned*>(p);
+                }
+            } else {
+                if (P == 8) *reinterpret_cast<uint4*>(w + dt / 2) = *reinterpret_cast<const uint4*>(p);
+                else if (P == 4) *reinterpret_cast<uint2*>(w + dt / 2) = *reinterpret_cast<const uint2*>(p);
+                else if (P == 2) w[dt / 2] = *reinterpret_cast<const unsigned*>(p);
+                else w[dt / 2] = *reinterpret_cast<const unsigned short*>(p);
+            }
+        }
+    }
+    __device__ __forceinline__ float get(int dt) const {
+        if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, w[dt]);
+        else return word_f32<T>(w[dt / 2], dt & 1);
+    }
+};
+
+// x and x of the lane SWAP away (in some order), in every lane.
+template <int SWAP>
+__device__ __forceinline__ void lane_pair(float x, float& a, float& b) {
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    unsigned lo, hi;    // (bit casts need scalars: of a vector's element they read element 0)
+    if constexpr (SWAP == 32) {
+        auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        lo = r[0];
+        hi = r[1];
+    } else {
+        auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        lo = r[0];
+        hi = r[1];
+    }
+    a = __builtin_bit_cast(float, lo);
+    b = __builtin_bit_cast(float, hi);
+}
+// sum / max over the four lane groups (lanes c, c + 16, c + 32, c + 48), in every lane
+__device__ __forceinline__ float group_max(float x) {
+    float a, b;
+    lane_pair<32>(x, a, b);
+    lane_pair<16>(fmaxf(a, b), a, b);
+    return fmaxf(a, b);
+}
+__device__ __forceinline__ float group_sum(float x) {
+    float a, b;
+    lane_pair<32>(x, a, b);
+    lane_pair<16>(a + b, a, b);
+    return a + b;
+}
+
+__device__ __forceinline__ float exp_nat(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
+__device__ __forceinline__ float safe_ref(float m) { return m == kNegInf ? 0.0f : m; }
+
+// Writes by other lanes of the wave to LDS are visible after this (a wave's LDS
+// operations complete in order; the fence keeps the compiler from reordering them).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Registers decide what a wave keeps at hand.  The latents' rows stay in registers unless
+// they are fp32 rows of 96 columns or more (64 registers at D = 128): those are read again
+// each tile, from cache.  The next tile's tokens are fetched ahead up to D = 64; beyond, the
+// second wave of a SIMD covers the latency (fetching ahead spilled 92 to 764 bytes a lane).
+template <typename T, int DT, bool SEP>
+constexpr bool latents_in_regs() { return sizeof(T) == 2 ? (DT <= 6 || !SEP) : (DT <= 3 || (DT == 4 && !SEP)); }
+template <int DT>
+constexpr bool fetch_ahead() { return DT <= 4; }
+
+// ---------------------------------------------------------------------------
+// Phase 1: the summary (max, den, num) of one chunk.  grid = (NC, B*H), one wave per
+// MT*16 latents.  Scores are taken as [tau][m] (C rows = tokens), which is the A operand of
+// U^T += V^T E directly, and U^T keeps a latent in one lane column, so a moved max rescales
+// it with per-lane factors.
+// ---------------------------------------------------------------------------
+template <typename T, int MT, int DT>
+__global__ __launch_bounds__(64 * (16 / MT)) void wave_prepare_kernel(
+    const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, int N, int H, int M, float scale,
+    int chunk, float* __restrict__ cmax, float* __restrict__ cden, float* __restrict__ cnum,
+    const int32_t* __restrict__ tmask) {
+    constexpr int D = 16 * DT;
+    const int ch = blockIdx.x, NC = gridDim.x, bh = blockIdx.y;
+    const int b = bh / H, h = bh % H;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+    const int mb = w * 16 * MT;
+
+    constexpr bool QREG = latents_in_regs<T, DT, false>(), AHEAD = fetch_ahead<DT>();
+    RowOp<T, D> q[QREG ? MT : 1];
+    auto load_q = [&](RowOp<T, D>& r, int mt) {
+        const int m = mb + 16 * mt + c;
+        if (m < M) r.load(Q + ((size_t)h * M + m) * D, g);
+        else r.zero();
+    };
+    if constexpr (QREG) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) load_q(q[mt], mt);
+    }
+    float mx[MT], den[MT];
+    f32x4 u[MT][DT];       // U^T: row 4g + i is the value column col_of(dt, 4g + i), lane c the latent
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        mx[mt] = kNegInf;
+        den[mt] = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) u[mt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+
+    const int t0 = ch * chunk, t1 = min(N, t0 + chunk);
+    const size_t stride = (size_t)H * D;
+    const T* kb = K + ((size_t)b * N * H + h) * D;
+    const T* vb = V + ((size_t)b * N * H + h) * D;
+    RowOp<T, D> kn;
+    ColRow<T, DT> vn[4];
+    auto fetch = [&](int t) {
+        kn.load(kb + (size_t)min(t + c, t1 - 1) * stride, g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vn[i].load(vb + (size_t)min(t + 4 * g + i, t1 - 1) * stride, c);
+    };
+    if constexpr (AHEAD) fetch(t0);
+    for (int t = t0; t < t1; t += TT) {
+        if constexpr (!AHEAD) fetch(t);
+        const RowOp<T, D> k = kn;
+        float v[4][DT];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) v[i][dt] = vn[i].get(dt);
+        if constexpr (AHEAD) {
+            if (t + TT < t1) fetch(t + TT);
+        }
+        bool ok[4] = {true, true, true, true};     // token t + 4g + i takes part
+        const bool part = t + TT > t1 || tmask != nullptr;
+        if (part) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int ti = t + 4 * g + i;
+                ok[i] = ti < t1 && (tmask == nullptr || tmask[(size_t)b * N + ti] != 0);
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) v[i][dt] = ok[i] ? v[i][dt] : 0.0f;
+            }
+        }
+        f32x4 e[MT];
+        float mnew[MT];
+        bool moved = false;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            if constexpr (!QREG) load_q(q[0], mt);
+            f32x4 s = dot_rows<T, D>(k, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+            float top = kNegInf;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[i] = ok[i] ? s[i] * scale : kNegInf;
+                top = fmaxf(top, s[i]);
+            }
+            mnew[mt] = fmaxf(mx[mt], group_max(top));
+            moved |= mnew[mt] != mx[mt];
+            e[mt] = s;
+        }
+        if (__any(moved)) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const float r = mx[mt] == kNegInf ? 0.0f : exp_nat(mx[mt] - mnew[mt]);
+                den[mt] *= r;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) u[mt][dt][i] *= r;
+                mx[mt] = mnew[mt];
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const float ref = safe_ref(mx[mt]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                e[mt][i] = exp_nat(e[mt][i] - ref);
+                den[mt] += e[mt][i];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) u[mt][dt] = mma4(v[i][dt], e[mt][i], u[mt][dt]);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        den[mt] = group_sum(den[mt]);
+        const int m = mb + 16 * mt + c;
+        if (m < M) {
+            const size_t si = ((size_t)bh * NC + ch) * M + m;
+            if (g == 0) {
+                cmax[si] = mx[mt];
+                cden[si] = den[mt];
+            }
+            float* row = cnum + si * D;
+#pragma unroll
+            for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float* p = row + col_of<DT>(dt, 4 * g + i);
+                    const int P = piece_of<DT>(dt);
+                    if (P >= 4) {
+#pragma unroll
+                        for (int j = 0; j < P; j += 4)
+                            *reinterpret_cast<f32x4*>(p + j) = f32x4{u[mt][dt + j][i], u[mt][dt + j + 1][i],
+                                                                     u[mt][dt + j + 2][i], u[mt][dt + j + 3][i]};
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < P; ++j) p[j] = u[mt][dt + j][i];
+                    }
+                }
+        }
+    }
+}
+
+// n consecutive results to Y (out_dtype code), starting at element idx
+template <int P>
+__device__ __forceinline__ void store_cols(void* Y, size_t idx, const float* x, int out_dtype) {
+    if (out_dtype == FLARE_F32) {
+        float* p = reinterpret_cast<float*>(Y) + idx;
+        if constexpr (P >= 4) {
+#pragma unroll
+            for (int j = 0; j < P; j += 4) *reinterpret_cast<f32x4*>(p + j) = f32x4{x[j], x[j + 1], x[j + 2], x[j + 3]};
+        } else {
+#pragma unroll
+            for (int j = 0; j < P; ++j) p[j] = x[j];
+        }
+    } else {
+        unsigned short h[P];
+#pragma unroll
+        for (int j = 0; j < P; ++j)
+            h[j] = out_dtype == FLARE_BF16 ? __builtin_bit_cast(unsigned short, (mfma::bf16)x[j])
+                                           : __builtin_bit_cast(unsigned short, (mfma::f16)x[j]);
+        unsigned short* p = reinterpret_cast<unsigned short*>(Y) + idx;
+        if constexpr (P == 8) {
+            *reinterpret_cast<uint4*>(p) = make_uint4(h[0] | (unsigned)h[1] << 16, h[2] | (unsigned)h[3] << 16,
+                                                      h[4] | (unsigned)h[5] << 16, h[6] | (unsigned)h[7] << 16);
+        } else if constexpr (P == 4) {
+            *reinterpret_cast<uint2*>(p) = make_uint2(h[0] | (unsigned)h[1] << 16, h[2] | (unsigned)h[3] << 16);
+        } else if constexpr (P == 2) {
+            *reinterpret_cast<unsigned*>(p) = h[0] | (unsigned)h[1] << 16;
+        } else {
+            *p = h[0];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Phase 3: replay of one chunk from its exclusive prefix, and the readout.
+// grid = (NC, B*H), one wave per MT*16 latents (NW = blockDim.x / 64 waves).
+//
+// Per 16-token tile and wave, from scores^T [m][t]:
+//   m' = max(m, tile max), E = e^(s - m'), d_t = d + cumulative E along the tokens,
+//   W = p / d_t with p = e^(s_dec - wave max) the decoder weights before their sum,
+//   G^T = E W^T (masked to tau <= t),  y = W U + G V,  U += E^T V.
+// One wave: W takes the softmax sum at once.  Several: each wave writes its y, max and sum
+// to LDS and the workgroup merges them (the token softmax over waves), double-buffered.
+//
+// A tile in which some latent's max rises by more than kTileJump, whose V holds a
+// non-finite value, or whose first token has no finite reference near the tile's max, runs
+// token by token: the same body with every other token masked, 16 times.  Each pass moves
+// the reference exactly to its token, as the tokenwise recurrence does.
+// ---------------------------------------------------------------------------
+template <int MT, int DT>
+__host__ __device__ constexpr int e_pitch() { return 16 * MT + 4; }
+
+template <int MT, int DT>
+inline size_t wave_output_lds(int NW) {
+    return sizeof(float) * ((size_t)NW * TT * e_pitch<MT, DT>() + (NW > 1 ? 2 * (size_t)NW * TT * (16 * DT + 2) : 0));
+}
+
+template <typename T, int MT, int DT, bool SEP>
+__global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
+    const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, const T* __restrict__ Qdec,
+    const T* __restrict__ Kdec, int N, int H, int M, float scale, int chunk, const float* __restrict__ pmax,
+    const float* __restrict__ pden, const float* __restrict__ pnum, void* __restrict__ Y, int out_dtype,
+    const int32_t* __restrict__ tmask) {
+    constexpr int D = 16 * DT;
+    constexpr int EP = e_pitch<MT, DT>();
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    const int ch = blockIdx.x, NC = gridDim.x, bh = blockIdx.y;
+    const int b = bh / H, h = bh % H;
+    const int NW = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+    const int mb = w * 16 * MT;
+    float* etile = smem + w * TT * EP;                 // this wave's E, [tau][m]
+    float* ypart = smem + NW * TT * EP;                // [2][NW][TT][D]
+    float* ystat = ypart + 2 * NW * TT * D;            // [2][NW][2][TT]: max, sum
+
+    constexpr bool QREG = latents_in_regs<T, DT, SEP>(), AHEAD = fetch_ahead<DT>();
+    RowOp<T, D> q[QREG ? MT : 1], kd[SEP && QREG ? MT : 1];
+    auto load_latent = [&](RowOp<T, D>& r, const T* base, int mt) {
+        const int m = mb + 16 * mt + c;
+        if (m < M) r.load(base + ((size_t)h * M + m) * D, g);
+        else r.zero();
+    };
+    if constexpr (QREG) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            load_latent(q[mt], Q, mt);
+            if constexpr (SEP) load_latent(kd[mt], Kdec, mt);
+        }
+    }
+    // latent mb + 16 mt + 4g + i: max, den (the same in the 16 lanes of a row), U row
+    float mx[MT][4], den[MT][4];
+    f32x4 u[MT][DT];
+    const size_t pbase = ((size_t)bh * NC + ch) * M;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = mb + 16 * mt + 4 * g + i;
+            mx[mt][i] = m < M ? pmax[pbase + m] : kNegInf;
+            den[mt][i] = m < M ? pden[pbase + m] : 0.0f;
+            ColRow<float, DT> r;
+            if (m < M) r.load(pnum + (pbase + m) * D, c);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) u[mt][dt][i] = m < M ? r.get(dt) : 0.0f;
+        }
+
+    const int t0 = ch * chunk, t1 = min(N, t0 + chunk);
+    const size_t stride = (size_t)H * D;
+    const T* kb = K + ((size_t)b * N * H + h) * D;
+    const T* vb = V + ((size_t)b * N * H + h) * D;
+    const T* qb = SEP ? Qdec + ((size_t)b * N * H + h) * D : nullptr;
+    RowOp<T, D> kn, qn;
+    ColRow<T, DT> vn[4];
+    auto fetch = [&](int t) {
+        kn.load(kb + (size_t)min(t + c, t1 - 1) * stride, g);
+        if constexpr (SEP) qn.load(qb + (size_t)min(t + c, t1 - 1) * stride, g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vn[i].load(vb + (size_t)min(t + 4 * g + i, t1 - 1) * stride, c);
+    };
+    if constexpr (AHEAD) fetch(t0);
+    int buf = 0;
+    for (int t = t0; t < t1; t += TT) {
+        if constexpr (!AHEAD) fetch(t);
+        // scores^T, then the next tile's loads
+        f32x4 s[MT], p[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            if constexpr (!QREG) load_latent(q[0], Q, mt);
+            s[mt] = dot_rows<T, D>(q[QREG ? mt : 0], kn, f32x4{0.f, 0.f, 0.f, 0.f});
+            if constexpr (SEP) {
+                if constexpr (!QREG) load_latent(kd[0], Kdec, mt);
+                p[mt] = dot_rows<T, D>(kd[QREG ? mt : 0], qn, f32x4{0.f, 0.f, 0.f, 0.f});
+            }
+        }
+        float v[4][DT];
+        float vbad = 0.0f;                             // NaN when a value is not finite
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                v[i][dt] = vn[i].get(dt);
+                vbad = __builtin_fmaf(v[i][dt], 0.0f, vbad);
+            }
+        if constexpr (AHEAD) {
+            if (t + TT < t1) fetch(t + TT);
+        }
+
+        bool live = true;                              // token t + c takes part
+        if (t + TT > t1 || tmask != nullptr)
+            live = t + c < t1 && (tmask == nullptr || tmask[(size_t)b * N + t + c] != 0);
+        const unsigned lmask = (unsigned)(__ballot(live) & 0xffffu);   // the 16 tokens, wave-uniform
+        const int first = lmask ? __builtin_ctz(lmask) : 0;
+
+        float top[MT][4];
+        bool slow = vbad != vbad, bare = false;
+        float wmax = kNegInf;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool in = live && mb + 16 * mt + 4 * g + i < M;
+                s[mt][i] = in ? s[mt][i] * scale : kNegInf;
+                if constexpr (SEP) p[mt][i] = in ? p[mt][i] * scale : kNegInf;
+                else p[mt][i] = s[mt][i];
+                wmax = fmaxf(wmax, p[mt][i]);
+                top[mt][i] = mfma::row_max16(s[mt][i]);
+                if (mb + 16 * mt + 4 * g + i < M) {
+                    slow |= top[mt][i] - mx[mt][i] > kTileJump && mx[mt][i] != kNegInf;
+                    bare |= mx[mt][i] == kNegInf;
+                }
+            }
+        if (__any(bare)) {
+            // no earlier token: the tile's first live token is the lowest reference
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float s0 = __shfl(s[mt][i], (lane & 48) | first, 64);
+                    if (mb + 16 * mt + 4 * g + i < M && mx[mt][i] == kNegInf)
+                        slow |= !(top[mt][i] - s0 <= kTileJump) && top[mt][i] != kNegInf;
+                }
+        }
+        // decoder weights of this wave's latents
+        wmax = group_max(wmax);
+        float psum = 0.0f;
+        {
+            const float ref = safe_ref(wmax);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    p[mt][i] = exp_nat(p[mt][i] - ref);
+                    psum += p[mt][i];
+                }
+        }
+        psum = group_sum(psum);
+        if (NW == 1) {
+            const float inv = psum > 0.0f ? 1.0f / psum : 0.0f;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) p[mt][i] *= inv;
+        }
+        if (lmask != 0xffffu) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) v[i][dt] = (lmask >> (4 * g + i)) & 1 ? v[i][dt] : 0.0f;
+        }
+
+        const bool step = __any(slow);
+        unsigned rest = lmask;                         // tokens still to be taken
+        unsigned rows = ~lmask & 0xffffu;              // output rows of this pass; masked ones come with the first
+        do {
+            // all live tokens at once, or the lowest one left
+            const unsigned take = step ? rest & -rest : rest;
+            rest &= ~take;
+            rows |= take;
+            f32x4 y[DT];
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) y[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const bool on = (take >> c) & 1;
+            f32x4 e[MT], wt[MT];
+            bool moved = false;
+            float mnew[MT][4];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float tm = step ? __shfl(s[mt][i], (lane & 48) | (__builtin_ctz(take | 0x10000u) & 15), 64)
+                                          : top[mt][i];
+                    mnew[mt][i] = take ? fmaxf(mx[mt][i], tm) : mx[mt][i];
+                    moved |= mnew[mt][i] != mx[mt][i];
+                }
+            if (__any(moved)) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float r = mx[mt][i] == mnew[mt][i] ? 1.0f
+                                        : mx[mt][i] == kNegInf   ? 0.0f
+                                                                 : exp_nat(mx[mt][i] - mnew[mt][i]);
+                        den[mt][i] *= r;
+#pragma unroll
+                        for (int dt = 0; dt < DT; ++dt) u[mt][dt][i] *= r;
+                        mx[mt][i] = mnew[mt][i];
+                    }
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float x = exp_nat(s[mt][i] - safe_ref(mx[mt][i]));
+                    e[mt][i] = on ? x : 0.0f;
+                    const float d = den[mt][i] + mfma::row_scan16(e[mt][i]);
+                    const float wv = p[mt][i] * __builtin_amdgcn_rcpf(d > 0.0f ? d : 1.0f);
+                    wt[mt][i] = on ? wv : 0.0f;
+                    den[mt][i] = mfma::row_bcast15(d);
+                }
+                *reinterpret_cast<f32x4*>(etile + c * EP + 16 * mt + 4 * g) = e[mt];
+            }
+            wave_lds_sync();
+            // G^T [tau][t], masked to tau <= t
+            f32x4 ga = {0.f, 0.f, 0.f, 0.f}, gb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                ga = mma4(e[mt][0], wt[mt][0], ga);
+                gb = mma4(e[mt][1], wt[mt][1], gb);
+                ga = mma4(e[mt][2], wt[mt][2], ga);
+                gb = mma4(e[mt][3], wt[mt][3], gb);
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) y[dt] = mma4(wt[mt][i], u[mt][dt][i], y[dt]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float gm = 4 * g + i <= c ? ga[i] + gb[i] : 0.0f;
+                const bool von = !step || ((take >> (4 * g + i)) & 1);
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) y[dt] = mma4(gm, von ? v[i][dt] : 0.0f, y[dt]);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const float ea = etile[(4 * g + i) * EP + 16 * mt + c];
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) u[mt][dt] = mma4(ea, von ? v[i][dt] : 0.0f, u[mt][dt]);
+                }
+            }
+            wave_lds_sync();
+            if (NW == 1) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int ti = t + 4 * g + i;
+                    if (ti >= t1 || !((rows >> (4 * g + i)) & 1)) continue;
+                    const size_t row = (((size_t)b * N + ti) * H + h) * D;
+#pragma unroll
+                    for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
+                        float o[8];
+                        const int P = piece_of<DT>(dt);
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) o[j] = j < P ? y[(dt + j) < DT ? dt + j : 0][i] : 0.0f;
+                        const size_t at = row + col_of<DT>(dt, c);
+                        if (P == 8) store_cols<8>(Y, at, o, out_dtype);
+                        else if (P == 4) store_cols<4>(Y, at, o, out_dtype);
+                        else if (P == 2) store_cols<2>(Y, at, o, out_dtype);
+                        else store_cols<1>(Y, at, o, out_dtype);
+                    }
+                }
+            } else {
+                float* yw = ypart + ((size_t)buf * NW + w) * TT * D;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if ((rows >> (4 * g + i)) & 1) {
+#pragma unroll
+                        for (int dt = 0; dt < DT; ++dt) yw[(4 * g + i) * D + col_of<DT>(dt, c)] = y[dt][i];
+                    }
+            }
+            rows = 0;
+        } while (rest != 0);
+
+        if (NW > 1) {
+            float* sw = ystat + ((size_t)buf * NW + w) * 2 * TT;
+            if (g == 0) {
+                sw[c] = wmax;
+                sw[TT + c] = psum;
+            }
+            __syncthreads();
+            const float* yr = ypart + (size_t)buf * NW * TT * D;
+            const float* sr = ystat + (size_t)buf * NW * 2 * TT;
+            for (int x = threadIdx.x; x < TT * D / 4; x += blockDim.x) {
+                const int ti = x / (D / 4), col = 4 * (x % (D / 4));
+                float mm = kNegInf;
+                for (int k = 0; k < NW; ++k) mm = fmaxf(mm, sr[k * 2 * TT + ti]);
+                const float ref = safe_ref(mm);
+                float sum = 0.0f;
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                for (int k = 0; k < NW; ++k) {
+                    const float f = exp_nat(sr[k * 2 * TT + ti] - ref);
+                    sum += f * sr[k * 2 * TT + TT + ti];
+                    const f32x4 yk = *reinterpret_cast<const f32x4*>(yr + ((size_t)k * TT + ti) * D + col);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[j] += f * yk[j];
+                }
+                const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+                float o[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[j] = acc[j] * inv;
+                if (t + ti < t1) store_cols<4>(Y, (((size_t)b * N + t + ti) * H + h) * D + col, o, out_dtype);
+            }
+            buf ^= 1;
+        }
+    }
+}
+
+}  // namespace wave
+}  // namespace flare

@@ -1,0 +1,113 @@
+"""GPU tests of the wave kernels (csrc/flare_wave.h): the chunked forward on fp32 matrix
+products, for fp32 inputs and for the banks without an instance of the 16-bit kernels.
+
+The oracle is the fp64 tokenwise recurrence.  Bars: fp32 and every state |a - b| <= 1e-5 +
+1e-4 |b| (sums of at most N = 150 fp32 terms of size O(1): N 2^-24 = 9e-6), 16-bit outputs
+one rounding on top (2^-8 bf16, 2^-11 fp16, of |b|)."""
+import numpy as np
+import pytest
+import torch
+
+import flare_oracle as O
+from _util import seeded, to_np
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+ROUND = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def _close(a, b, dtype, what):
+    a, b = to_np(a).astype(np.float64), np.asarray(b, dtype=np.float64)
+    bound = 1e-5 + (1e-4 + ROUND[dtype]) * np.abs(b)
+    worst = float((np.abs(a - b) - bound).max())
+    assert np.isfinite(a).all() and worst <= 0, f"{what}: past the bar by {worst:.3e}"
+
+
+def _prefill(q, k, v, **kw):
+    from causal_flare import flare_autoregressive_prefill_triton
+    put = lambda t: {n: x.to(DEV) for n, x in t.items()} if isinstance(t, dict) else t.to(DEV)
+    kw = {n: put(t) for n, t in kw.items() if t is not None}
+    return flare_autoregressive_prefill_triton(q.to(DEV), k.to(DEV), v.to(DEV), **kw)
+
+
+# one per head dim and latent-tile count; latents and lengths off every tile edge
+SHAPES = [(5, 16, 3), (16, 16, 16), (33, 32, 17), (64, 32, 150), (80, 32, 33), (256, 32, 40), (40, 48, 65),
+          (64, 64, 1), (96, 64, 95), (192, 96, 50), (256, 128, 47)]
+
+
+@pytest.mark.parametrize("M,D,N", SHAPES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("form", ["plain", "state_mask", "separate"])
+def test_wave_prefill(M, D, N, dtype, form):
+    print("CASE wave_prefill", M, D, N, dtype, form, flush=True)
+    if (M, D) == (256, 128) and dtype is not torch.float32:
+        pytest.skip("this bank has a 16-bit kernel")
+    B, H = 2, 2
+    q, k, v = seeded(31 * M + D, B, N, H, M, D, D, dtype, q_std=D ** -0.5)
+    g = torch.Generator().manual_seed(M + D)
+    state = mask = qd = kd = None
+    if form == "state_mask":
+        state = {"m": torch.randn(B, H, M, generator=g), "d": 1.0 + torch.rand(B, H, M, generator=g),
+                 "u": torch.randn(B, H, M, D, generator=g)}
+        mask = (torch.rand(B, N, generator=g) < 0.7).to(torch.int32)
+        mask[0, : min(N, 18)] = 0          # a whole tile of masked tokens, and a masked start
+    if form == "separate":
+        qd = torch.randn(B, N, H, D, generator=g).to(dtype)
+        kd = (torch.randn(H, M, D, generator=g) * D ** -0.5).to(dtype)
+    y, st = _prefill(q, k, v, state=state, attention_mask=mask, Q_dec=qd, K_dec=kd)
+    ref, rst = O.brute_ar_state(q, k, v, state=state, scale=1.0, attention_mask=mask, Q_dec=qd, K_dec=kd)
+    _close(y, ref, dtype, "y")
+    for n in ("m", "d", "u"):
+        _close(st[n], rst[n], torch.float32, n)
+
+
+@pytest.mark.parametrize("M,D,dtype", [(64, 32, torch.bfloat16), (96, 64, torch.float16), (128, 64, torch.float32),
+                                       (40, 16, torch.float32)])
+def test_wave_score_jumps_and_infinite_values(M, D, dtype):
+    """Scores that rise by 90 to 400 nats inside a tile (at the start of the sequence, mid-tile
+    and on a tile's last token) and, apart from them, an infinite value row: the tokens before
+    each keep their exact outputs, as the tokenwise recurrence gives them."""
+    print("CASE wave_jumps", M, D, dtype, flush=True)
+    B, N, H = 1, 70, 2
+    q, k, v = seeded(77 + M, B, N, H, M, D, D, dtype, q_std=D ** -0.5)
+    kj = k.clone()
+    for t, nats, lat in ((3, 90.0, 1), (21, 200.0, 7), (47, 400.0, 12)):
+        for h in range(H):
+            row = q[h, lat].float()
+            kj[0, t, h] = (row * (nats / row.square().sum())).to(dtype)
+    y, st = _prefill(q, kj, v)
+    ref, rst = O.brute_ar_state(q, kj, v, scale=1.0)
+    # a score of 400 nats carries |s| 2^-24 = 2.4e-5 of its fp32 sum into e^s
+    a, b = to_np(y).astype(np.float64), np.asarray(ref)
+    assert np.isfinite(a).all()
+    assert (np.abs(a - b) - (1e-4 + (2e-4 + ROUND[dtype]) * np.abs(b))).max() <= 0
+    vi = v.clone()
+    vi[0, 37, 0, 5] = float("inf")
+    y, _ = _prefill(q, k, vi)
+    clean, _ = _prefill(q, k, v)
+    assert torch.equal(y[0, :32], clean[0, :32]) and torch.equal(y[0, :, 1], clean[0, :, 1])
+    _close(y[0, 32:37, 0], to_np(clean[0, 32:37, 0]), dtype, "tokens of the tile before the infinite one")
+    assert not torch.isfinite(y[0, 37:, 0, 5]).any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_wave_unaligned_inputs(dtype):
+    """Inputs that start off a 16-byte boundary run on the tokenwise kernels, with the same
+    results."""
+    print("CASE wave_unaligned", dtype, flush=True)
+    B, N, H, M, D = 1, 40, 2, 64, 32
+    q, k, v = seeded(5, B, N, H, M, D, D, dtype, q_std=D ** -0.5)
+    y0, _ = _prefill(q, k, v)
+
+    def shifted(t):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+        buf[1:] = t.reshape(-1).to(DEV)
+        return buf[1:].view(t.shape)
+
+    from causal_flare import flare_autoregressive_prefill_triton
+    for which in range(3):
+        args = [t.to(DEV) for t in (q, k, v)]
+        args[which] = shifted((q, k, v)[which])
+        assert args[which].data_ptr() % 16 != 0
+        y, _ = flare_autoregressive_prefill_triton(*args)
+        _close(y, to_np(y0), dtype, f"input {which} unaligned")
