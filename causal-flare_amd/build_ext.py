@@ -43,6 +43,9 @@ FILE_FLAGS = {
     "flare_wave_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "flare_wave_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "flare_wave_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "flare_wave_bwd_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "flare_wave_bwd_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "flare_wave_bwd_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

@@ -210,15 +210,17 @@ __global__ __launch_bounds__(kNT) void chunk_output_kernel(
 // that 16-byte accesses reach (the dims make every row a multiple of 16 bytes long, so the
 // base pointers decide).  Everything else stays on the tokenwise kernels, which take 2 to 28
 // times as long on every bank measured here (M 32 to 256, D 32 to 128, 16-bit and fp32).
-static bool wave_shape(int64_t M, int64_t Dk, int64_t Dv) {
+bool wave_shape(int64_t M, int64_t Dk, int64_t Dv) {
     const int64_t dt = Dv / 16;
     return Dk == Dv && Dv % 16 == 0 && (dt == 1 || dt == 2 || dt == 3 || dt == 4 || dt == 6 || dt == 8) && M <= 256;
 }
-static bool wave_supported(int64_t M, int64_t Dk, int64_t Dv, int64_t chunk, std::initializer_list<const void*> ptrs) {
-    if (!wave_shape(M, Dk, Dv) || chunk % 16 != 0) return false;
+bool wave_aligned(std::initializer_list<const void*> ptrs) {
     for (const void* p : ptrs)
         if (((uintptr_t)p & 15) != 0) return false;
     return true;
+}
+static bool wave_supported(int64_t M, int64_t Dk, int64_t Dv, int64_t chunk, std::initializer_list<const void*> ptrs) {
+    return wave_shape(M, Dk, Dv) && chunk % 16 == 0 && wave_aligned(ptrs);
 }
 
 static int launch_prepare(const void* Q, const void* K, const void* V, int dtype, int64_t B,

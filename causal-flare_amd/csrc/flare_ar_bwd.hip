@@ -1217,7 +1217,27 @@ static int launch_contract(const T* q, const T* k, const T* qd, const T* kd, boo
     int rc;
     constexpr bool kHalf = std::is_same<T, __half>::value;
     constexpr bool k16 = std::is_same<T, __hip_bfloat16>::value || kHalf;
-    if (k16 && bwd_dk_mfma_supported(M, Dk)) {
+    // Where rows can be read 16 bytes at a time: the wave kernels.  Against the 16-bit MFMA
+    // kernels below, dQ 74 -> 33 us and dK 41 -> 43 at bf16 B 4, N 4096, H 16, M 128, D 64, dQ
+    // 162 -> 126 and dK 127 -> 94 at N 16384, H 16, M 256, D 128; against the scalar ones, dQ
+    // 296 -> 10 and dK 89 -> 10 at B 4, N 2011, H 16, M 64, D 32.
+    const bool wave = (mfma_phase_mask() & 3) == 3 && wave_shape(M, Dk, Dk) && M % 16 == 0 && 4 * N * M < (int64_t)1 << 31 &&
+                      wave_aligned({q, k, qd, kd, dK, dQd, DS, AL, C});
+    const wave::ContractPtrs cp{DS, C, AL, gy, cgz};
+    auto rows = [&](const T* r1, const T* r2, void* out) {
+        return kHalf ? wave::rows_f16(cp, r1, r2, B, N, H, M, Dk, scale, out, st)
+               : k16 ? wave::rows_bf16(cp, r1, r2, B, N, H, M, Dk, scale, out, st)
+                     : wave::rows_f32(cp, r1, r2, B, N, H, M, Dk, scale, out, st);
+    };
+    auto cols = [&](const T* r1, const T* r2, float* P) {
+        return kHalf ? wave::cols_f16(cp, r1, r2, B, N, H, M, Dk, P, st)
+               : k16 ? wave::cols_bf16(cp, r1, r2, B, N, H, M, Dk, P, st)
+                     : wave::cols_f32(cp, r1, r2, B, N, H, M, Dk, P, st);
+    };
+    if (wave) {
+        if ((rc = rows(q, dsum || sep_q ? nullptr : kd, dK))) return rc;
+        if (sep_q && (rc = rows(nullptr, kd, dQd))) return rc;
+    } else if (k16 && bwd_dk_mfma_supported(M, Dk)) {
         if ((rc = launch_dk_mfma(q, kd, sep_q, sep_k, B, N, H, M, Dk, scale, DS, AL, C, gy, cgz, dsum, dK, dQd, kHalf, st)))
             return rc;
     } else {
@@ -1226,7 +1246,10 @@ static int launch_contract(const T* q, const T* k, const T* qd, const T* kd, boo
                            cgz, dsum, static_cast<T*>(dK), static_cast<T*>(dQd));
         if ((rc = check_launch("bwd_dk_kernel"))) return rc;
     }
-    if (k16 && bwd_dq_mfma_supported(M, Dk)) {
+    if (wave) {
+        if ((rc = cols(k, dsum || sep_k ? nullptr : qd, P1))) return rc;
+        if (sep_k && (rc = cols(nullptr, qd, P2))) return rc;
+    } else if (k16 && bwd_dq_mfma_supported(M, Dk)) {
         if ((rc = launch_dq_mfma(k, qd, sep_q, sep_k, B, N, H, M, Dk, DS, AL, C, gy, cgz, dsum, P1, P2, kHalf, st))) return rc;
     } else {
         hipLaunchKernelGGL(bwd_dq_kernel<T>, dim3((unsigned)NG, (unsigned)BH, (unsigned)((Dk + 63) / 64)),
@@ -1434,6 +1457,73 @@ bool ar_backward_supported(int64_t M, int64_t Dk, int64_t Dv) {
            Dv >= 16 && Dv <= 512;
 }
 
+// The wave backward's workspace (flare_wave_bwd.h) and its chunk: two waves per SIMD over
+// the device as the forward, whole 64-token steps, and no more memory than the other
+// kernels' workspace takes.
+struct WaveBwdLayout {
+    int64_t chunk, NC;
+    size_t off_pm, off_pd, off_pn, off_xs, off_ys, off_tm, off_td, off_sw, off_gz, off_ds, off_al, off_lse, off_gy, off_p1,
+        off_p2, total;
+    WaveBwdLayout(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, bool sep, int64_t chunk_) : chunk(chunk_) {
+        NC = (N + chunk - 1) / chunk;
+        const size_t BH = (size_t)B * H, NT = (N + 15) / 16;
+        size_t o = 0;
+        auto take = [&](size_t floats) {
+            const size_t at = o;
+            o += ((floats * sizeof(float) + 255) / 256) * 256;
+            return at;
+        };
+        off_pm = take(BH * NC * M);
+        off_pd = take(BH * NC * M);
+        off_pn = take(BH * NC * M * D);
+        off_xs = take(BH * NC * M * D);
+        off_ys = take(BH * NC * M);
+        off_tm = take(BH * NT * M);
+        off_td = take(BH * NT * M);
+        off_sw = take(BH * NT * ((M + 15) / 16));     // at most one wave per 16 latents
+        off_gz = take(BH * N * M);
+        off_ds = take(BH * N * M);
+        off_al = take(sep ? BH * N * M : 0);
+        off_lse = take(BH * N);
+        off_gy = take(BH * N);
+        off_p1 = take(bwd_partial_floats(B, N, H, M, D));
+        off_p2 = take(sep ? bwd_partial_floats(B, N, H, M, D) : 0);
+        total = o;
+    }
+};
+static int64_t wave_bwd_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, bool sep, size_t bytes) {
+    int64_t c = default_chunk(B, N, H, M, D);
+    c = ((c + 63) / 64) * 64;
+    while (c < N && WaveBwdLayout(B, N, H, M, D, sep, c).total > bytes) c *= 2;
+    return c;
+}
+
+static int run_wave_backward(const void* Q, const void* K, const void* V, const void* Qdec, const void* Kdec, int dtype,
+                             int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale, const void* Y,
+                             const void* dY, void* dQ, void* dK, void* dV, void* dQdec, void* dKdec, char* ws,
+                             const WaveBwdLayout& lay, hipStream_t st) {
+    const bool sep = Qdec != nullptr || Kdec != nullptr;
+    auto at = [&](size_t off) { return reinterpret_cast<float*>(ws + off); };
+    float *pm = at(lay.off_pm), *pd = at(lay.off_pd), *pn = at(lay.off_pn);
+    int rc = launch_prepare_public(Q, K, V, dtype, B, N, H, M, D, D, scale, lay.chunk, pm, pd, pn, st);
+    if (rc) return rc;
+    rc = launch_prefix_public(pm, pd, pn, B * H, lay.NC, M, D, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, st);
+    if (rc) return rc;
+    rc = launch_bwd_gy(dY, Y, dtype, B, N, H, D, at(lay.off_gy), st);
+    if (rc) return rc;
+    const wave::BwdPtrs p{Q, K, V, Qdec ? Qdec : K, Kdec ? Kdec : Q, dY, pm, pd, pn, at(lay.off_xs), at(lay.off_ys),
+                          at(lay.off_tm), at(lay.off_td),
+                          reinterpret_cast<int*>(ws + lay.off_sw), at(lay.off_gz), at(lay.off_ds), at(lay.off_al),
+                          at(lay.off_lse), at(lay.off_gy), dV};
+    rc = dtype == FLARE_BF16  ? wave::bwd_bf16(p, sep, B, N, H, M, D, scale, lay.chunk, st)
+         : dtype == FLARE_F16 ? wave::bwd_f16(p, sep, B, N, H, M, D, scale, lay.chunk, st)
+                              : wave::bwd_f32(p, sep, B, N, H, M, D, scale, lay.chunk, st);
+    if (rc) return rc;
+    return launch_bwd_contract(Q, K, Qdec, Kdec, dtype, B, N, H, M, D, scale, at(lay.off_ds), at(lay.off_al),
+                               at(lay.off_gz), at(lay.off_gy), true, !sep, dQ, dK, dQdec, dKdec, at(lay.off_p1),
+                               at(lay.off_p2), st);
+}
+
 size_t ar_backward_workspace(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv) {
     return BwdLayout(B, N, H, M, Dk, Dv).total;
 }
@@ -1448,6 +1538,15 @@ int ar_backward_run(const void* Q, const void* K, const void* V, const void* Qde
                   lay.total);
     FLARE_REQUIRE((((uintptr_t)workspace) & 255) == 0, "flare_ar_backward: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
+    // (the walks reach a (b, h)'s per-token arrays by 31-bit byte offsets)
+    if (power <= 0.0f && mfma_phase_mask() == 3 && wave_shape(M, Dk, Dv) && 4 * N * M < (int64_t)1 << 31 &&
+        wave_aligned({Q, K, V, Qdec, Kdec, Y, dY, dV})) {
+        const bool sep = Qdec != nullptr || Kdec != nullptr;
+        const WaveBwdLayout wl(B, N, H, M, Dk, sep, wave_bwd_chunk(B, N, H, M, Dk, sep, lay.total));
+        if (wl.total <= lay.total)
+            return run_wave_backward(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dk, scale, Y, dY, dQ, dK, dV, dQdec, dKdec,
+                                     ws, wl, st);
+    }
 #define FLARE_BWD(TY)                                                                                          \
     return run_backward<TY>(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dk, Dv, scale, Y, dY, dQ, dK, dV, dQdec, \
                             dKdec, ws, lay, st, power)

@@ -2,6 +2,8 @@
 #pragma once
 #include <stdint.h>
 
+#include <initializer_list>
+
 namespace flare {
 int64_t default_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv);
 }
@@ -179,5 +181,44 @@ int output_bf16(const WaveArgs& a, const float* pmax, const float* pden, const f
                 hipStream_t st);
 int output_f16(const WaveArgs& a, const float* pmax, const float* pden, const float* pnum, void* Y, int out_dtype,
                hipStream_t st);
+
+// The backward (flare_wave_bwd.h).  Q, K, V, dY, dV and the decoder tensors (K and Q where
+// they are shared) in the input type; the rest is workspace.
+struct BwdPtrs {
+    const void *Q, *K, *V, *Qdec, *Kdec, *dY;
+    const float *pmax, *pden, *pnum;     // exclusive chunk prefixes [B*H, NC, M(, D)]
+    float *xsum, *ysum;                  // chunk terms of X, Y, then (after the scan) X, Y past each chunk
+    float *tmax, *tden;                  // [B*H, NT, M]: state at each 16-token tile's start
+    int* stepwise;                       // [B*H, NT, waves]: tiles walked token by token
+    float *gz, *ds, *al;                 // [B*H, N, M]; al only for separate decoder weights
+    const float *lse, *gy;               // [B*H, N]
+    void* dV;
+};
+// Score gradients of the backward's contractions (flare_wave_contract.h): ds, and for da the
+// arrays it is formed from.
+struct ContractPtrs {
+    const float *ds, *c, *al, *gy;
+    bool cgz;
+};
+// out = scale (ds . r1 + da . r2) over the latents, r1 / r2 [H, M, D] or null
+// P = partial sums over 512-token groups of ds^T r1 + da^T r2, r1 / r2 [B, N, H, D] or null
+#define FLARE_WAVE_CONTRACT(SUFFIX)                                                                                  \
+    int rows_##SUFFIX(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, \
+                      int64_t D, float scale, void* out, hipStream_t st);                                             \
+    int cols_##SUFFIX(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, \
+                      int64_t D, float* P, hipStream_t st);
+FLARE_WAVE_CONTRACT(f32)
+FLARE_WAVE_CONTRACT(bf16)
+FLARE_WAVE_CONTRACT(f16)
+#undef FLARE_WAVE_CONTRACT
+int bwd_f32(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale,
+            int64_t chunk, hipStream_t st);
+int bwd_bf16(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale,
+             int64_t chunk, hipStream_t st);
+int bwd_f16(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale,
+            int64_t chunk, hipStream_t st);
 }  // namespace wave
+// whether a bank and its pointers (16-byte aligned rows) have an instance of the wave kernels
+bool wave_shape(int64_t M, int64_t Dk, int64_t Dv);
+bool wave_aligned(std::initializer_list<const void*> ptrs);
 }  // namespace flare

@@ -38,6 +38,15 @@ using mfma::bf16x8;
 using mfma::f32x4;
 using mfma::kLog2e;
 
+// Words as they are loaded: rows of any element type are read and written through these.
+typedef unsigned u32;
+typedef u32 u32_a __attribute__((may_alias));
+typedef u32 u32x2 __attribute__((ext_vector_type(2), may_alias));
+typedef u32 u32x4 __attribute__((ext_vector_type(4), may_alias));
+typedef unsigned short u16_a __attribute__((may_alias));
+typedef float f32x4_a __attribute__((ext_vector_type(4), may_alias));
+typedef mfma::bf16 bf16x8_a __attribute__((ext_vector_type(8), may_alias));
+
 constexpr int TT = 16;              // tokens per tile
 // A latent's max may rise by this much (nats) inside a tile before the tile runs token by
 // token: below it every den and weight of the tile keeps full fp32 precision against the
@@ -60,9 +69,9 @@ struct RowOp {   // 16-bit: steps of 32 columns, 8 a lane group; a last step of 
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             if (32 * s + 32 <= D) {
-                a[s] = *reinterpret_cast<const bf16x8*>(p + 32 * s + 8 * g);
+                a[s] = *reinterpret_cast<const bf16x8_a*>(p + 32 * s + 8 * g);
             } else {
-                const bf16x8 x = *reinterpret_cast<const bf16x8*>(p + 32 * s + 8 * (g & 1));
+                const bf16x8 x = *reinterpret_cast<const bf16x8_a*>(p + 32 * s + 8 * (g & 1));
                 a[s] = g < 2 ? x : bf16x8{};
             }
         }
@@ -77,7 +86,7 @@ struct RowOp<float, D> {   // lane group g holds columns [g D/4, (g+1) D/4)
     f32x4 a[D / 16];
     __device__ __forceinline__ void load(const float* row, int g) {
 #pragma unroll
-        for (int s = 0; s < D / 16; ++s) a[s] = *reinterpret_cast<const f32x4*>(row + g * (D / 4) + 4 * s);
+        for (int s = 0; s < D / 16; ++s) a[s] = *reinterpret_cast<const f32x4_a*>(row + g * (D / 4) + 4 * s);
     }
     __device__ __forceinline__ void zero() {
 #pragma unroll
@@ -104,27 +113,18 @@ __device__ __forceinline__ f32x4 dot_rows(const RowOp<T, D>& x, const RowOp<T, D
 // ---------------------------------------------------------------------------
 // Column tiles of a row of D = 16 DT values.  Which 16 columns make tile dt is free (a
 // product only needs both sides to agree), so lane c takes consecutive columns, in pieces
-// of 8, 4, 2 and 1: loads and stores are as wide as the pieces.
+// of 4, 2 and 1 tiles: loads and stores are as wide as the pieces.
 // ---------------------------------------------------------------------------
+// (closed forms: they fold away for a tile index known after unrolling)
 template <int DT>
-__host__ __device__ constexpr int piece_of(int dt) {   // size of the piece that holds tile dt
-    int off = 0;
-    for (int p = 8; p >= 1; p >>= 1)
-        if (DT & p) {
-            if (dt < off + p) return p;
-            off += p;
-        }
-    return 1;
+__host__ __device__ constexpr int piece_off(int dt) {  // first tile of the piece that holds tile dt
+    constexpr int full = DT / 4 * 4;
+    return dt < full ? (dt & ~3) : (DT - full == 3 && dt - full == 2) ? full + 2 : full;
 }
 template <int DT>
-__host__ __device__ constexpr int piece_off(int dt) {  // first tile of that piece
-    int off = 0;
-    for (int p = 8; p >= 1; p >>= 1)
-        if (DT & p) {
-            if (dt < off + p) return off;
-            off += p;
-        }
-    return off;
+__host__ __device__ constexpr int piece_of(int dt) {   // size of that piece
+    constexpr int full = DT / 4 * 4;
+    return dt < full ? 4 : DT - full == 3 ? (dt - full < 2 ? 2 : 1) : DT - full;
 }
 // column of tile dt at lane c
 template <int DT>
@@ -148,26 +148,26 @@ struct ColRow {
     unsigned w[W];
     __device__ __forceinline__ void load(const T* row, int c) {
 #pragma unroll
-        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
-            const T* p = row + col_of<DT>(dt, c);
-            const int P = piece_of<DT>(dt);
-            if constexpr (sizeof(T) == 4) {
-                if (P == 8) {
-                    *reinterpret_cast<uint4*>(w + dt) = reinterpret_cast<const uint4*>(p)[0];
-                    *reinterpret_cast<uint4*>(w + dt + 4) = reinterpret_cast<const uint4*>(p)[1];
-                } else if (P == 4) {
-                    *reinterpret_cast<uint4*>(w + dt) = *reinterpret_cast<const uint4*>(p);
-                } else if (P == 2) {
-                    *reinterpret_cast<uint2*>(w + dt) = *reinterpret_cast<const uint2*>(p);
-                } else {
-                    w[dt] = *reinterpret_cast<const unsigned*>(p);
-                }
-            } else {
-                if (P == 8) *reinterpret_cast<uint4*>(w + dt / 2) = *reinterpret_cast<const uint4*>(p);
-                else if (P == 4) *reinterpret_cast<uint2*>(w + dt / 2) = *reinterpret_cast<const uint2*>(p);
-                else if (P == 2) w[dt / 2] = *reinterpret_cast<const unsigned*>(p);
-                else w[dt / 2] = *reinterpret_cast<const unsigned short*>(p);
-            }
+        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) load_piece(row, c, dt);
+    }
+    // the columns of the piece that starts at tile dt
+    __device__ __forceinline__ void load_piece(const T* row, int c, int dt) {
+        const T* p = row + col_of<DT>(dt, c);
+        const int P = piece_of<DT>(dt);
+        const int at = sizeof(T) == 4 ? dt : dt / 2, words = sizeof(T) == 4 ? P : P / 2;
+        if (words == 4) {
+            const u32x4 x = *reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (at + j < W) w[at + j] = x[j];
+        } else if (words == 2) {
+            const u32x2 x = *reinterpret_cast<const u32x2*>(p);
+            w[at] = x[0];
+            if (at + 1 < W) w[at + 1] = x[1];
+        } else if (words == 1) {
+            w[at] = *reinterpret_cast<const u32_a*>(p);
+        } else {
+            w[at] = *reinterpret_cast<const u16_a*>(p);
         }
     }
     __device__ __forceinline__ float get(int dt) const {
@@ -361,15 +361,9 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_prepare_kernel(
                 for (int i = 0; i < 4; ++i) {
                     float* p = row + col_of<DT>(dt, 4 * g + i);
                     const int P = piece_of<DT>(dt);
-                    if (P >= 4) {
 #pragma unroll
-                        for (int j = 0; j < P; j += 4)
-                            *reinterpret_cast<f32x4*>(p + j) = f32x4{u[mt][dt + j][i], u[mt][dt + j + 1][i],
-                                                                     u[mt][dt + j + 2][i], u[mt][dt + j + 3][i]};
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < P; ++j) p[j] = u[mt][dt + j][i];
-                    }
+                    for (int j = 0; j < 4; ++j)
+                        if (j < P) p[j] = u[mt][dt + j < DT ? dt + j : 0][i];
                 }
         }
     }
@@ -380,9 +374,8 @@ template <int P>
 __device__ __forceinline__ void store_cols(void* Y, size_t idx, const float* x, int out_dtype) {
     if (out_dtype == FLARE_F32) {
         float* p = reinterpret_cast<float*>(Y) + idx;
-        if constexpr (P >= 4) {
-#pragma unroll
-            for (int j = 0; j < P; j += 4) *reinterpret_cast<f32x4*>(p + j) = f32x4{x[j], x[j + 1], x[j + 2], x[j + 3]};
+        if constexpr (P == 4) {
+            *reinterpret_cast<f32x4_a*>(p) = f32x4{x[0], x[1], x[2], x[3]};
         } else {
 #pragma unroll
             for (int j = 0; j < P; ++j) p[j] = x[j];
@@ -394,13 +387,10 @@ __device__ __forceinline__ void store_cols(void* Y, size_t idx, const float* x, 
             h[j] = out_dtype == FLARE_BF16 ? __builtin_bit_cast(unsigned short, (mfma::bf16)x[j])
                                            : __builtin_bit_cast(unsigned short, (mfma::f16)x[j]);
         unsigned short* p = reinterpret_cast<unsigned short*>(Y) + idx;
-        if constexpr (P == 8) {
-            *reinterpret_cast<uint4*>(p) = make_uint4(h[0] | (unsigned)h[1] << 16, h[2] | (unsigned)h[3] << 16,
-                                                      h[4] | (unsigned)h[5] << 16, h[6] | (unsigned)h[7] << 16);
-        } else if constexpr (P == 4) {
-            *reinterpret_cast<uint2*>(p) = make_uint2(h[0] | (unsigned)h[1] << 16, h[2] | (unsigned)h[3] << 16);
+        if constexpr (P == 4) {
+            *reinterpret_cast<u32x2*>(p) = u32x2{h[0] | (unsigned)h[1] << 16, h[2] | (unsigned)h[3] << 16};
         } else if constexpr (P == 2) {
-            *reinterpret_cast<unsigned*>(p) = h[0] | (unsigned)h[1] << 16;
+            *reinterpret_cast<u32_a*>(p) = h[0] | (unsigned)h[1] << 16;
         } else {
             *p = h[0];
         }
@@ -633,7 +623,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
                     wt[mt][i] = on ? wv : 0.0f;
                     den[mt][i] = mfma::row_bcast15(d);
                 }
-                *reinterpret_cast<f32x4*>(etile + c * EP + 16 * mt + 4 * g) = e[mt];
+                *reinterpret_cast<f32x4_a*>(etile + c * EP + 16 * mt + 4 * g) = e[mt];
             }
             wave_lds_sync();
             // G^T [tau][t], masked to tau <= t
@@ -673,13 +663,12 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
                     const size_t row = (((size_t)b * N + ti) * H + h) * D;
 #pragma unroll
                     for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
-                        float o[8];
+                        float o[4];
                         const int P = piece_of<DT>(dt);
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) o[j] = j < P ? y[(dt + j) < DT ? dt + j : 0][i] : 0.0f;
+                        for (int j = 0; j < 4; ++j) o[j] = j < P ? y[(dt + j) < DT ? dt + j : 0][i] : 0.0f;
                         const size_t at = row + col_of<DT>(dt, c);
-                        if (P == 8) store_cols<8>(Y, at, o, out_dtype);
-                        else if (P == 4) store_cols<4>(Y, at, o, out_dtype);
+                        if (P == 4) store_cols<4>(Y, at, o, out_dtype);
                         else if (P == 2) store_cols<2>(Y, at, o, out_dtype);
                         else store_cols<1>(Y, at, o, out_dtype);
                     }
@@ -715,7 +704,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
                 for (int k = 0; k < NW; ++k) {
                     const float f = exp_nat(sr[k * 2 * TT + ti] - ref);
                     sum += f * sr[k * 2 * TT + TT + ti];
-                    const f32x4 yk = *reinterpret_cast<const f32x4*>(yr + ((size_t)k * TT + ti) * D + col);
+                    const f32x4 yk = *reinterpret_cast<const f32x4_a*>(yr + ((size_t)k * TT + ti) * D + col);
 #pragma unroll
                     for (int j = 0; j < 4; ++j) acc[j] += f * yk[j];
                 }

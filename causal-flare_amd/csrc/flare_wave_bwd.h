@@ -1,0 +1,950 @@
+// flare_wave_bwd.h -- backward of the chunked causal FLARE forward with wave-private latents
+// (equal head dims, M <= 256).  Per (b, h), latent m and token t, with s the encoder score,
+// D_t the running sum of e^s, alpha_t the decoder softmax, g = dY and U_t the running sum of
+// e^s v (z_t = U_t / D_t):
+//   gz_t  = g_t . U_t / D_t                 da_t = alpha_t (gz_t - g_t . y_t)
+//   X_tau = sum_{t >= tau} (alpha_t / D_t) g_t      Y_tau = sum_{t >= tau} (alpha_t / D_t) gz_t
+//   ds_tau = e^{s_tau} (v_tau . X_tau - Y_tau)      dv_tau = sum_m e^{s_tau} X_tau
+// and dQ, dK (dQ_dec, dK_dec) are contractions of ds + da (ds, da).
+//
+// Two walks over the forward's own kind of chunks replace per-token statistics in memory:
+//   wave_gz   forward over a chunk from its exclusive prefix (max, den, U): writes gz, the
+//             (max, den) at each 16-token tile's start, and the chunk's share of X and Y;
+//   wave_ds   backward over a chunk from the X, Y after it (a reverse scan over chunks):
+//             recomputes a tile's weights from the stored (max, den), writes ds and dv.
+// Between them only gz (fp32) travels per token and latent; scores, weights, decoder softmax
+// and running sums are formed again from K, Q and one (max, den) pair per 16 tokens.
+//
+// Layout: the tile's score-like matrices are C tiles with tokens as rows (lane (g, c):
+// tokens 4g + i, latent c), U and X are kept transposed (rows = value columns, lane column =
+// latent).  g . U, v . X, U += , X += and the in-tile sums then need no data movement; only
+// dv (a sum over latents) needs e, w and X the other way round, through wave-private LDS.
+// A latent is one lane column, so its reference max and its moves are per-lane scalars.
+//
+// Products.  fp32 inputs: fp32 MFMA (16x16x4).  16-bit inputs: every fp32 factor enters the
+// 16x16x32 bf16 MFMA as hi + lo, both halves side by side in the contraction index (16
+// tokens or latents hi, the same 16 lo), so that one instruction takes the whole product
+// with a 16-bit factor and two take a product of two fp32 factors.
+//
+// Numerics.  Weights inside a tile are relative to the latents' max after the tile, X and Y
+// to the max of the tile they were last used in (factors <= 1 as the walk goes back).  A tile
+// in which a max rises by more than kTileJump runs token by token with each token's own max.
+#pragma once
+
+#include <type_traits>
+
+#include "flare_internal.h"
+#include "flare_wave.h"
+
+namespace flare {
+namespace wave {
+
+using mfma::bf16x4;
+using mfma::f16x8;
+
+// ---------------------------------------------------------------------------
+// A row of D = 16 DT values, split over the lane groups as the C rows of a transposed state
+// are: lane group g holds value column col_of(dt, 4g + i) for every dt, i.  Within a piece
+// these are 4 P consecutive columns.
+// ---------------------------------------------------------------------------
+template <int DT>
+__host__ __device__ constexpr int list_at(int dt, int i) {    // position of (dt, i) in the lane's list
+    return 4 * piece_off<DT>(dt) + i * piece_of<DT>(dt) + (dt - piece_off<DT>(dt));
+}
+// tile and register of list position e (valid below 4 DT)
+template <int DT>
+__host__ __device__ constexpr int list_dt(int e) {
+    constexpr int full = DT / 4 * 4, rem = DT - full;
+    const int f = e - 4 * full;
+    return f < 0 ? (e / 16) * 4 + (e & 3) : rem == 1 ? full : f < 8 ? full + (f & 1) : full + 2;
+}
+template <int DT>
+__host__ __device__ constexpr int list_i(int e) {
+    constexpr int full = DT / 4 * 4, rem = DT - full;
+    const int f = e - 4 * full;
+    return f < 0 ? (e >> 2) & 3 : rem == 1 ? f : f < 8 ? f >> 1 : f - 8;
+}
+
+template <typename T, int DT>
+struct GroupRow {
+    static constexpr int W = sizeof(T) == 4 ? 4 * DT : 2 * DT;
+    static constexpr int S = (DT + 1) / 2;                    // steps of 8 values (32 over the groups)
+    unsigned w[W];
+    __device__ __forceinline__ void load(const T* row, int g) {
+#pragma unroll
+        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
+            const int P = piece_of<DT>(dt);
+            const T* p = row + 16 * dt + 4 * g * P;
+            // 4 P values
+            const int at = (sizeof(T) == 4 ? 4 : 2) * dt, words = (sizeof(T) == 4 ? 4 : 2) * P;
+            if (words == 2) {
+                const u32x2 x = *reinterpret_cast<const u32x2*>(p);
+                w[at] = x[0];
+                w[at + 1] = x[1];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (4 * j < words) {
+                        const u32x4 x = reinterpret_cast<const u32x4*>(p)[j];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            if (at + 4 * j + k < W) w[at + 4 * j + k] = x[k];
+                    }
+            }
+        }
+    }
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int j = 0; j < W; ++j) w[j] = 0;
+    }
+    __device__ __forceinline__ float at(int e) const {
+        if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, w[e]);
+        else return word_f32<T>(w[e / 2], e & 1);
+    }
+    // eight values as a 16-bit MFMA operand (zeros past the end)
+    __device__ __forceinline__ bf16x8 op8(int s) const {
+        u32x4 r;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[j] = 4 * s + j < W ? w[4 * s + j] : 0u;
+        return __builtin_bit_cast(bf16x8, r);
+    }
+};
+
+// c += x . y^T over the columns
+template <typename T, int DT>
+__device__ __forceinline__ f32x4 dot_groups(const GroupRow<T, DT>& x, const GroupRow<T, DT>& y, f32x4 c) {
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int e = 0; e < 4 * DT; ++e) c = mma4(x.at(e), y.at(e), c);
+    } else {
+        constexpr bool F16 = __is_same(T, __half);
+#pragma unroll
+        for (int s = 0; s < GroupRow<T, DT>::S; ++s) c = mfma::mma_in<F16>(x.op8(s), y.op8(s), c);
+    }
+    return c;
+}
+
+// ---------------------------------------------------------------------------
+// Operands of products over 16 contraction indices 4g + i (tokens or latents of a tile).
+// ---------------------------------------------------------------------------
+struct F4 {          // fp32 products
+    float v[4];
+};
+struct Pair4 {       // fp32 values as bf16 hi + lo
+    bf16x4 h, l;
+};
+struct Exact4 {      // bf16 values
+    bf16x4 x;
+};
+__device__ __forceinline__ bf16x8 cat(bf16x4 a, bf16x4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+
+__device__ __forceinline__ f32x4 mm(const F4& a, const F4& b, f32x4 c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c = mma4(a.v[i], b.v[i], c);
+    return c;
+}
+__device__ __forceinline__ f32x4 mm(const Pair4& a, const Exact4& b, f32x4 c) {
+    return mfma::mma(cat(a.h, a.l), cat(b.x, b.x), c);
+}
+__device__ __forceinline__ f32x4 mm(const Exact4& a, const Pair4& b, f32x4 c) {
+    return mfma::mma(cat(a.x, a.x), cat(b.h, b.l), c);
+}
+__device__ __forceinline__ f32x4 mm(const Pair4& a, const Pair4& b, f32x4 c) {
+    const bf16x8 hl = cat(a.h, a.l);
+    c = mfma::mma(hl, cat(b.h, b.h), c);
+    return mfma::mma(hl, cat(b.l, b.l), c);
+}
+
+template <typename T> struct ProdOf { typedef Pair4 F; };            // type of an fp32 factor
+template <> struct ProdOf<float> { typedef F4 F; };
+template <typename F>
+__device__ __forceinline__ F factor(float x0, float x1, float x2, float x3) {
+    F r;
+    if constexpr (__is_same(F, F4)) {
+        r.v[0] = x0;
+        r.v[1] = x1;
+        r.v[2] = x2;
+        r.v[3] = x3;
+    } else {
+        mfma::split_bf16x4(x0, x1, x2, x3, r.h, r.l);
+    }
+    return r;
+}
+
+// Tokens 4g + i of a 16-token tile, value column col_of(dt, c): the factor of the products
+// over tokens.
+template <typename T, int DT>
+struct TokCols {
+    typedef typename std::conditional<sizeof(T) == 4, F4,
+                                      typename std::conditional<__is_same(T, __half), Pair4, Exact4>::type>::type Op;
+    ColRow<T, DT> r[4];
+    __device__ __forceinline__ Op op(int dt) const {
+        Op o;
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o.v[i] = r[i].get(dt);
+        } else if constexpr (__is_same(T, __half)) {
+            mfma::split_bf16x4(r[0].get(dt), r[1].get(dt), r[2].get(dt), r[3].get(dt), o.h, o.l);
+        } else {
+            const unsigned sel = dt & 1 ? 0x07060302u : 0x05040100u;
+            u32x2 p;
+            p[0] = __builtin_amdgcn_perm(r[1].w[dt / 2], r[0].w[dt / 2], sel);
+            p[1] = __builtin_amdgcn_perm(r[3].w[dt / 2], r[2].w[dt / 2], sel);
+            o.x = __builtin_bit_cast(bf16x4, p);
+        }
+        return o;
+    }
+};
+
+// c += x . u over the columns: rows of x (lane column = row) against a transposed state
+// (rows = columns col_of(dt, 4g + i), lane column = latent); C rows are x's rows.
+template <typename T, int DT>
+__device__ __forceinline__ f32x4 dot_state(const GroupRow<T, DT>& x, const f32x4 (&u)[DT], f32x4 c) {
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c = mma4(x.at(list_at<DT>(dt, i)), u[dt][i], c);
+    } else {
+#pragma unroll
+        for (int s = 0; s < GroupRow<T, DT>::S; ++s) {
+            bf16x4 h[2], l[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                float y[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int e = 8 * s + 4 * q + j;
+                    y[j] = e < 4 * DT ? u[e < 4 * DT ? list_dt<DT>(e) : 0][list_i<DT>(e)] : 0.0f;
+                }
+                mfma::split_bf16x4(y[0], y[1], y[2], y[3], h[q], l[q]);
+            }
+            const bf16x8 uh = cat(h[0], h[1]), ul = cat(l[0], l[1]);
+            if constexpr (__is_same(T, __half)) {
+                const f16x8 xf = __builtin_bit_cast(f16x8, x.op8(s));
+                bf16x8 xh, xl;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) SPLIT2(mfma::bf16, (float)xf[e], xh[e], xl[e]);
+                c = mfma::mma(xh, uh, c);
+                c = mfma::mma(xh, ul, c);
+                c = mfma::mma(xl, uh, c);
+            } else {
+                c = mfma::mma(x.op8(s), uh, c);
+                c = mfma::mma(x.op8(s), ul, c);
+            }
+        }
+    }
+    return c;
+}
+
+// Over the lane groups of a lane column: the sum of x over lower groups, over higher
+// groups, and over all.
+__device__ __forceinline__ void group_scan(float x, int g, float& below, float& above, float& all) {
+    float even, odd, lo, hi;
+    lane_pair<16>(x, even, odd);
+    lane_pair<32>(even + odd, lo, hi);
+    below = (g & 1 ? even : 0.0f) + (g & 2 ? lo : 0.0f);
+    above = (g & 1 ? 0.0f : odd) + (g & 2 ? 0.0f : hi);
+    all = lo + hi;
+}
+// value of register i (wave-uniform) of token j = 4 (j / 4) + i at every lane of its column
+__device__ __forceinline__ float token_value(const float (&x)[4], int j, int c) {
+    const int i = j & 3;
+    const float v = i == 0 ? x[0] : i == 1 ? x[1] : i == 2 ? x[2] : x[3];
+    return __shfl(v, (j >> 2) * 16 + c, 64);
+}
+
+
+// Registers: the latents' rows stay there up to D = 64 (fp32: 32), else they are read again
+// each tile, from cache.
+template <typename T, int DT, bool SEP>
+constexpr bool bwd_latents_in_regs() { return sizeof(T) == 2 ? DT <= 4 : DT <= (SEP ? 2 : 3); }
+
+// Nothing is scheduled across: keeps a stage's operands from being loaded stages early, which
+// is what the registers cannot hold.
+template <int DT>
+__device__ __forceinline__ void stage() {
+    if constexpr (DT > 4) __builtin_amdgcn_sched_barrier(0);
+}
+
+// fp32 array of one (b, h) through a buffer descriptor: loads past its end read 0 and stores
+// there are dropped, so edge tokens and masked latents need no branches (a branch per element
+// split the tile into some 80 blocks that nothing could be scheduled across).
+constexpr unsigned kNowhere = 0x80000000u;                          // byte offset past every array
+struct Floats {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Floats(const float* p, size_t n)
+        : r(__builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(n * sizeof(float)), 0x00020000)) {}
+    __device__ __forceinline__ float load(unsigned byte) const {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, byte, 0, 0));
+    }
+    __device__ __forceinline__ void store(unsigned byte, float x) const {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), r, byte, 0, 0);
+    }
+};
+
+// One tile's token rows (K, V, g and, for separate decoder weights, Q_dec) in LDS, shared by
+// the workgroup's waves: read from memory once, and held in no wave's registers.  Rows are
+// padded by 16 bytes (the operand reads go down 16 rows).  The next tile travels in a few
+// registers a thread while the current one is worked on.
+template <typename T, int DT, bool SEP>
+struct TileRows {
+    static constexpr int D = 16 * DT;
+    // (fp32 rows of 128: the backward walk's LDS has no room for Q_dec, read from cache there)
+    static constexpr bool QD = SEP && !(sizeof(T) == 4 && DT == 8);
+    static constexpr int R = QD ? 4 : 3;
+    static constexpr int CPR = D * (int)sizeof(T) / 16;             // 16-byte pieces a row
+    static constexpr int PITCH = D + 16 / (int)sizeof(T);           // elements
+    static constexpr int CHUNKS = TT * CPR;                         // pieces of one array's tile
+    static constexpr int PF = sizeof(T) == 2 ? 1 : 2;               // pieces of an array a thread can hold
+    static constexpr size_t BYTES = (size_t)R * TT * PITCH * sizeof(T);
+    u32x4 held[R][PF];
+    static __device__ __forceinline__ u32x4 piece(const T* p, int stride, int x, int t, int t1) {
+        return reinterpret_cast<const u32x4*>(p + (size_t)min(t + x / CPR, t1 - 1) * stride)[x % CPR];
+    }
+    static __device__ __forceinline__ void put(T* lds, int x, u32x4 val) {
+        *reinterpret_cast<u32x4*>(lds + (x / CPR) * PITCH + (x % CPR) * (16 / (int)sizeof(T))) = val;
+    }
+    static __device__ __forceinline__ bool holds() { return CHUNKS <= PF * (int)blockDim.x; }
+    __device__ __forceinline__ void fetch(const BwdPtrs& a, size_t tok, int stride, int t, int t1) {
+        if (!holds()) return;
+#pragma unroll
+        for (int n = 0; n < PF; ++n) {
+            const int x = min((int)(threadIdx.x + n * blockDim.x), CHUNKS - 1);
+            held[0][n] = piece((const T*)a.K + tok, stride, x, t, t1);
+            held[1][n] = piece((const T*)a.V + tok, stride, x, t, t1);
+            held[2][n] = piece((const T*)a.dY + tok, stride, x, t, t1);
+            if constexpr (QD) held[3][n] = piece((const T*)a.Qdec + tok, stride, x, t, t1);
+        }
+    }
+    __device__ __forceinline__ void store(T* lds, const BwdPtrs& a, size_t tok, int stride, int t, int t1) {
+        constexpr int A = TT * PITCH;                               // elements of one array's tile
+        if (holds()) {
+#pragma unroll
+            for (int n = 0; n < PF; ++n) {
+                const int x = threadIdx.x + n * blockDim.x;
+                if (x < CHUNKS) {
+#pragma unroll
+                    for (int k = 0; k < R; ++k) put(lds + k * A, x, held[k][n]);
+                }
+            }
+        } else {
+            for (int x = threadIdx.x; x < CHUNKS; x += blockDim.x) {
+                put(lds, x, piece((const T*)a.K + tok, stride, x, t, t1));
+                put(lds + A, x, piece((const T*)a.V + tok, stride, x, t, t1));
+                put(lds + 2 * A, x, piece((const T*)a.dY + tok, stride, x, t, t1));
+                if constexpr (QD) put(lds + 3 * A, x, piece((const T*)a.Qdec + tok, stride, x, t, t1));
+            }
+        }
+    }
+    static __device__ __forceinline__ const T* row(const T* lds, int a, int r) { return lds + (a * TT + r) * PITCH; }
+};
+
+// ---------------------------------------------------------------------------
+// Decoder log-sum-exp of every token.  One wave takes 64 tokens against all latents; the
+// latents' rows come from cache.
+// ---------------------------------------------------------------------------
+constexpr int kLseTiles = 4;
+template <typename T, int DT>
+__global__ __launch_bounds__(256) void wave_lse_kernel(const T* __restrict__ Qd, const T* __restrict__ Kd, int N, int H,
+                                                       int M, float scale, float* __restrict__ lse) {
+    constexpr int D = 16 * DT;
+    const int bh = blockIdx.y, b = bh / H, h = bh % H;
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    const int t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * TT * kLseTiles;
+    if (t0 >= N) return;
+    GroupRow<T, DT> k[kLseTiles];
+    float mx[kLseTiles], sum[kLseTiles];
+#pragma unroll
+    for (int j = 0; j < kLseTiles; ++j) {
+        k[j].load(Qd + (((size_t)b * N + min(t0 + TT * j + c, N - 1)) * H + h) * D, g);
+        mx[j] = kNegInf;
+        sum[j] = 0.0f;
+    }
+    for (int m0 = 0; m0 < M; m0 += 16) {
+        GroupRow<T, DT> q;
+        q.load(Kd + ((size_t)h * M + min(m0 + c, M - 1)) * D, g);
+#pragma unroll
+        for (int j = 0; j < kLseTiles; ++j) {
+            f32x4 s = dot_groups<T, DT>(q, k[j], f32x4{0.f, 0.f, 0.f, 0.f});
+            float top = mx[j];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[i] = m0 + 4 * g + i < M ? s[i] * scale : kNegInf;
+                top = fmaxf(top, s[i]);
+            }
+            const float ref = safe_ref(top);
+            float a = sum[j] * exp_nat(mx[j] - ref);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a += exp_nat(s[i] - ref);
+            sum[j] = a;
+            mx[j] = top;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kLseTiles; ++j) {
+        const float top = group_max(mx[j]), ref = safe_ref(top);
+        const float all = group_sum(sum[j] * exp_nat(mx[j] - ref));
+        const int t = t0 + TT * j + c;
+        if (g == 0 && t < N) lse[(size_t)bh * N + t] = ref + __logf(all);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Forward walk of a chunk: gz, tile states, the chunk's X and Y.  grid (NC, B*H), one wave
+// per MT*16 latents; the waves share a tile's rows and exchange nothing else.
+//
+// j < 0: the whole tile.  j >= 0: the tile is being walked token by token (see kTileJump) and
+// j is the token; the loop then comes back with the same tile.  (As an inner loop over
+// tokens this took 45 to 60 registers more.)
+// ---------------------------------------------------------------------------
+template <typename T, int MT, int DT, bool SEP>
+__global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int N, int H, int M, float scale, int chunk) {
+    constexpr int D = 16 * DT;
+    typedef typename ProdOf<T>::F F;
+    typedef TileRows<T, DT, SEP> Rows;
+    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>();
+    extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
+    const int ch = blockIdx.x, NC = gridDim.x, bh = blockIdx.y;
+    const int b = bh / H, h = bh % H;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, NW = blockDim.x >> 6, g = lane >> 4, c = lane & 15;
+    const int mb = wv * 16 * MT;
+    const int NT = (N + TT - 1) / TT;
+    const int t0 = ch * chunk, t1 = min(N, t0 + chunk);
+    const int stride = H * D;
+    const size_t tok = ((size_t)b * N * H + h) * D;
+    // this (b, h)'s rows of the per-token arrays, reached by 32-bit offsets
+    const Floats gz_out(a.gz + (size_t)bh * N * M, (size_t)N * M), lse_in(a.lse + (size_t)bh * N, N);
+    unsigned lat[MT];                             // byte offset of this lane's latent in a row
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) lat[mt] = mb + 16 * mt + c < M ? 4u * (mb + 16 * mt + c) : kNowhere;
+
+    GroupRow<T, DT> q[QREG ? MT : 1], kd[SEP && QREG ? MT : 1];
+    auto latent_row = [&](GroupRow<T, DT>& r, const void* base, int mt) {
+        // (past the bank: its last row; such a latent has no decoder weight and is never stored)
+        r.load((const T*)base + ((size_t)h * M + min(mb + 16 * mt + c, M - 1)) * D, g);
+    };
+    float mx[MT], den[MT], er[MT], ysum[MT];      // er = e^(max at the chunk's start - mx)
+    f32x4 u[MT][DT], x[MT][DT];
+    const size_t pbase = ((size_t)bh * NC + ch) * M;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int m = mb + 16 * mt + c;
+        const bool in = m < M;
+        if constexpr (QREG) {
+            latent_row(q[mt], a.Q, mt);
+            if constexpr (SEP) latent_row(kd[mt], a.Kdec, mt);
+        }
+        mx[mt] = in ? a.pmax[pbase + m] : kNegInf;
+        den[mt] = in ? a.pden[pbase + m] : 0.0f;
+        er[mt] = mx[mt] == kNegInf ? 0.0f : 1.0f;
+        ysum[mt] = 0.0f;
+        GroupRow<float, DT> r;
+        if (in) r.load(a.pnum + (pbase + m) * D, g);
+        else r.zero();
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) u[mt][dt][i] = r.at(list_at<DT>(dt, i));
+            x[mt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+
+    Rows rows;
+    rows.fetch(a, tok, stride, t0, t1);
+    rows.store((T*)tile_lds, a, tok, stride, t0, t1);
+    __syncthreads();
+    int buf = 0, t = t0, j = -1;
+    while (true) {
+        const T* tl = (const T*)(tile_lds + buf * Rows::BYTES);
+        if (j <= 0 && t + TT < t1) rows.fetch(a, tok, stride, t + TT, t1);
+        float s[MT][4], al[MT][4], top[MT], lse[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lse[i] = lse_in.load(4u * (t + 4 * g + i));
+        bool slow = false;
+        {
+            GroupRow<T, DT> kr;
+            kr.load(Rows::row(tl, 0, c), g);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                if constexpr (!QREG) latent_row(q[0], a.Q, mt);
+                const f32x4 r = dot_groups<T, DT>(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+                top[mt] = kNegInf;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[mt][i] = t + 4 * g + i < t1 ? r[i] * scale : kNegInf;
+                    top[mt] = fmaxf(top[mt], s[mt][i]);
+                }
+                top[mt] = group_max(top[mt]);
+                const float low = mx[mt] == kNegInf ? __shfl(s[mt][0], c, 64) : mx[mt];
+                slow |= !(top[mt] - low <= kTileJump) && mb + 16 * mt + c < M;
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            f32x4 z = {s[mt][0], s[mt][1], s[mt][2], s[mt][3]};
+            if constexpr (SEP) {
+                GroupRow<T, DT> qr;
+                qr.load(Rows::QD ? Rows::row(tl, 3, c) : (const T*)a.Qdec + tok + (size_t)min(t + c, t1 - 1) * stride, g);
+                if constexpr (!QREG) latent_row(kd[0], a.Kdec, mt);
+                z = dot_groups<T, DT>(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                for (int i = 0; i < 4; ++i) z[i] *= scale;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) al[mt][i] = t + 4 * g + i < t1 ? exp_nat(z[i] - lse[i]) : 0.0f;
+        }
+        stage<DT>();
+        // g_t . v_tau as the [t][tau] factor of sums over tau (C rows tau, lane column t)
+        F gvf;
+        GroupRow<T, DT> gr;
+        gr.load(Rows::row(tl, 2, c), g);
+        {
+            GroupRow<T, DT> vr;
+            vr.load(Rows::row(tl, 1, c), g);
+            const f32x4 r = dot_groups<T, DT>(vr, gr, f32x4{0.f, 0.f, 0.f, 0.f});
+            gvf = factor<F>(4 * g <= c ? r[0] : 0.0f, 4 * g + 1 <= c ? r[1] : 0.0f, 4 * g + 2 <= c ? r[2] : 0.0f,
+                            4 * g + 3 <= c ? r[3] : 0.0f);
+        }
+        if (j <= 0) {
+            // a value of g that is not finite: the backward walk keeps it to its own token
+            float bad = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4 * DT; ++e) bad = __builtin_fmaf(gr.at(e), 0.0f, bad);
+            const bool step = __any(slow || bad != bad);
+            if (lane == 0) a.stepwise[((size_t)bh * NT + t / TT) * NW + wv] = step;
+            j = __any(slow) ? 0 : -1;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                if (g == 0 && mb + 16 * mt + c < M) {
+                    const size_t ti = ((size_t)bh * NT + t / TT) * M + mb + 16 * mt + c;
+                    a.tmax[ti] = mx[mt];
+                    a.tden[ti] = den[mt];
+                }
+        }
+        F ef[MT], wf[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            stage<DT>();
+            const float mnew = fmaxf(mx[mt], j >= 0 ? token_value(s[mt], j, c) : top[mt]);
+            if (__any(mnew != mx[mt])) {
+                const float r = mx[mt] == mnew ? 1.0f : mx[mt] == kNegInf ? 0.0f : exp_nat(mx[mt] - mnew);
+                den[mt] *= r;
+                er[mt] *= r;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) u[mt][dt][i] *= r;
+                mx[mt] = mnew;
+            }
+            const float ref = safe_ref(mx[mt]);
+            float e[4], d[4], run = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float ev = exp_nat(s[mt][i] - ref);
+                e[i] = j < 0 || 4 * g + i == j ? ev : 0.0f;
+                run += e[i];
+                d[i] = run;
+            }
+            float below, above, all;
+            group_scan(run, g, below, above, all);
+            ef[mt] = factor<F>(e[0], e[1], e[2], e[3]);
+            f32x4 p = dot_state<T, DT>(gr, u[mt], f32x4{0.f, 0.f, 0.f, 0.f});
+            p = mm(gvf, ef[mt], p);
+            float w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float dv = den[mt] + below + d[i];
+                const float inv = __builtin_amdgcn_rcpf(dv > 0.0f ? dv : 1.0f);
+                const bool on = j < 0 || 4 * g + i == j;
+                const float gz = p[i] * inv;
+                w[i] = on ? al[mt][i] * er[mt] * inv : 0.0f;      // (al is 0 past the sequence)
+                ysum[mt] += w[i] == 0.0f ? 0.0f : w[i] * gz;
+                gz_out.store(on ? 4u * M * (t + 4 * g + i) + lat[mt] : kNowhere, gz);
+            }
+            den[mt] += all;
+            wf[mt] = factor<F>(w[0], w[1], w[2], w[3]);
+        }
+        // U += E^T V, X += W^T g, a piece of value columns at a time
+#pragma unroll
+        for (int d0 = 0; d0 < DT; d0 += piece_of<DT>(d0)) {
+            stage<DT>();
+            TokCols<T, DT> vc, gc;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                vc.r[i].load_piece(Rows::row(tl, 1, 4 * g + i), c, d0);
+                gc.r[i].load_piece(Rows::row(tl, 2, 4 * g + i), c, d0);
+            }
+#pragma unroll
+            for (int dt = d0; dt < d0 + piece_of<DT>(d0); ++dt) {
+                const auto vo = vc.op(dt), go = gc.op(dt);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    u[mt][dt] = mm(vo, ef[mt], u[mt][dt]);
+                    x[mt][dt] = mm(go, wf[mt], x[mt][dt]);
+                }
+            }
+        }
+        if (j >= 0 && ++j < min(TT, t1 - t)) continue;
+        j = -1;
+        t += TT;
+        if (t >= t1) break;
+        buf ^= 1;
+        rows.store((T*)(tile_lds + buf * Rows::BYTES), a, tok, stride, t, t1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        ysum[mt] = group_sum(ysum[mt]);
+        const int m = mb + 16 * mt + c;
+        if (m < M) {
+            if (g == 0) a.ysum[pbase + m] = ysum[mt];
+            float* row = a.xsum + (pbase + m) * D;
+#pragma unroll
+            for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (k < piece_of<DT>(dt)) row[col_of<DT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Reverse scan over chunks: the terms of chunk c (relative to the max at its start) become
+// X, Y after chunk c (relative to the max at its end, the next chunk's start).  One thread
+// per (b*h, latent, value column), and one more column for Y.
+// ---------------------------------------------------------------------------
+static __global__ __launch_bounds__(256) void wave_carry_kernel(float* __restrict__ xsum, float* __restrict__ ysum,
+                                                         const float* __restrict__ pmax, int NC, int M, int D, int rows) {
+    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+    if (gid >= rows * (D + 1)) return;
+    const int row = gid / (D + 1), col = gid % (D + 1);
+    const int bh = row / M, m = row % M;
+    float run = 0.0f, mnext = 0.0f;       // X after chunk ch, relative to mnext = pmax of chunk ch + 1
+    constexpr int BATCH = 8;
+    for (int c1 = NC; c1 > 0; c1 -= BATCH) {
+        float v[BATCH], mm[BATCH];
+#pragma unroll
+        for (int k = 0; k < BATCH; ++k) {
+            const int ch = c1 - 1 - k;
+            const size_t si = ((size_t)bh * NC + max(ch, 0)) * M + m;
+            v[k] = col < D ? xsum[si * D + col] : ysum[si];
+            mm[k] = pmax[si];
+        }
+#pragma unroll
+        for (int k = 0; k < BATCH; ++k) {
+            const int ch = c1 - 1 - k;
+            if (ch < 0) break;
+            const size_t si = ((size_t)bh * NC + ch) * M + m;
+            if (col < D) xsum[si * D + col] = run;
+            else ysum[si] = run;
+            // relative to this chunk's start (a first chunk starts at -inf and has no reader)
+            const float f = ch + 1 < NC && mm[k] != kNegInf ? exp_nat(mm[k] - mnext) : 0.0f;
+            run = v[k] + (f > 0.0f ? run * f : 0.0f);
+            mnext = mm[k];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Backward walk of a chunk: ds and dv.  grid (NC, B*H), one wave per MT*16 latents.  Whether
+// a tile is walked token by token is read from the forward walk's marks, for the whole
+// workgroup alike (its waves add their dv rows at barriers).
+// ---------------------------------------------------------------------------
+template <int MT, int DT>
+__host__ __device__ constexpr int ds_wave_floats() {      // wave-private LDS: X tile, or the e / w tiles, or dv rows
+    const int xt = MT * 16 * (16 * DT + 4), ew = 2 * TT * (16 * MT + 4), dv = TT * 16 * DT;
+    const int a = xt > ew ? xt : ew;
+    return a > dv ? a : dv;
+}
+
+template <typename T, int MT, int DT, bool SEP>
+__global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int N, int H, int M, float scale, int chunk) {
+    constexpr int D = 16 * DT, EP = 16 * MT + 4, XP = D + 4;
+    constexpr int OD = sizeof(T) == 4 ? FLARE_F32 : __is_same(T, __half) ? FLARE_F16 : FLARE_BF16;
+    typedef typename ProdOf<T>::F F;
+    typedef TileRows<T, DT, SEP> Rows;
+    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>();
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    const int ch = blockIdx.x, NC = gridDim.x, bh = blockIdx.y;
+    const int b = bh / H, h = bh % H;
+    const int NW = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+    const int mb = wv * 16 * MT;
+    const int NT = (N + TT - 1) / TT;
+    const int t0 = ch * chunk, t1 = min(N, t0 + chunk);
+    const int stride = H * D;
+    const size_t tok = ((size_t)b * N * H + h) * D;
+    T* tl = reinterpret_cast<T*>(smem + NW * ds_wave_floats<MT, DT>());
+    float* own = smem + wv * ds_wave_floats<MT, DT>();
+    float *etile = own, *wtile = own + TT * EP, *xtile = own, *vtile = own;
+    const size_t per = (size_t)N * M;
+    const Floats gz_in(a.gz + bh * per, per), lse_in(a.lse + (size_t)bh * N, N), gy_in(a.gy + (size_t)bh * N, N);
+    const Floats ds_out(a.ds + bh * per, per), al_out(SEP ? a.al + bh * per : a.ds, SEP ? per : 0);
+    const Floats tmax_in(a.tmax + (size_t)bh * NT * M, (size_t)NT * M), tden_in(a.tden + (size_t)bh * NT * M, (size_t)NT * M);
+    unsigned lat[MT];                             // byte offset of this lane's latent in a row
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) lat[mt] = mb + 16 * mt + c < M ? 4u * (mb + 16 * mt + c) : kNowhere;
+
+    GroupRow<T, DT> q[QREG ? MT : 1], kd[SEP && QREG ? MT : 1];
+    auto latent_row = [&](GroupRow<T, DT>& r, const void* base, int mt) {
+        // (past the bank: its last row; such a latent has no decoder weight and is never stored)
+        r.load((const T*)base + ((size_t)h * M + min(mb + 16 * mt + c, M - 1)) * D, g);
+    };
+    float mref[MT], ysum[MT];
+    f32x4 x[MT][DT];
+    const size_t pbase = ((size_t)bh * NC + ch) * M;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int m = mb + 16 * mt + c;
+        if constexpr (QREG) {
+            latent_row(q[mt], a.Q, mt);
+            if constexpr (SEP) latent_row(kd[mt], a.Kdec, mt);
+        }
+        const bool tail = m < M && ch + 1 < NC;
+        mref[mt] = tail ? a.pmax[pbase + M + m] : 0.0f;
+        ysum[mt] = tail ? a.ysum[pbase + m] : 0.0f;
+        GroupRow<float, DT> r;
+        if (tail) r.load(a.xsum + (pbase + m) * D, g);
+        else r.zero();
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[mt][dt][i] = r.at(list_at<DT>(dt, i));
+    }
+
+    Rows rows;
+    int t = t0 + (t1 - 1 - t0) / TT * TT, j = -1;
+    rows.fetch(a, tok, stride, t, t1);
+    rows.store(tl, a, tok, stride, t, t1);
+    __syncthreads();
+    while (true) {
+        const bool begin = j < 0;
+        if (begin) {
+            if (t > t0) rows.fetch(a, tok, stride, t - TT, t1);
+            const int mark = a.stepwise[((size_t)bh * NT + t / TT) * NW + min(lane, NW - 1)];
+            j = __any(mark) ? min(TT, t1 - t) - 1 : -1;
+        }
+        float s[MT][4], top[MT], m0[MT], d0[MT], gz[MT][4], lse[4], gy[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            lse[i] = lse_in.load(4u * (t + 4 * g + i));
+            gy[i] = SEP ? 0.0f : gy_in.load(4u * (t + 4 * g + i));
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) gz[mt][i] = gz_in.load(4u * M * (t + 4 * g + i) + lat[mt]);
+        }
+        {
+            GroupRow<T, DT> kr;
+            kr.load(Rows::row(tl, 0, c), g);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                m0[mt] = tmax_in.load(4u * M * (t / TT) + lat[mt]);
+                d0[mt] = tden_in.load(4u * M * (t / TT) + lat[mt]);
+                if constexpr (!QREG) latent_row(q[0], a.Q, mt);
+                const f32x4 r = dot_groups<T, DT>(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+                top[mt] = kNegInf;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[mt][i] = t + 4 * g + i < t1 ? r[i] * scale : kNegInf;
+                    top[mt] = fmaxf(top[mt], s[mt][i]);
+                }
+                top[mt] = group_max(top[mt]);
+            }
+        }
+        stage<DT>();
+        // g_t . v_tau as the [tau][t] factor of sums over t (C rows t, lane column tau)
+        GroupRow<T, DT> vr;
+        vr.load(Rows::row(tl, 1, c), g);
+        F gvf;
+        {
+            GroupRow<T, DT> gr;
+            gr.load(Rows::row(tl, 2, c), g);
+            const f32x4 r = dot_groups<T, DT>(gr, vr, f32x4{0.f, 0.f, 0.f, 0.f});
+            gvf = factor<F>(4 * g >= c ? r[0] : 0.0f, 4 * g + 1 >= c ? r[1] : 0.0f, 4 * g + 2 >= c ? r[2] : 0.0f,
+                            4 * g + 3 >= c ? r[3] : 0.0f);
+        }
+        F wf[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            stage<DT>();
+            f32x4 z = {s[mt][0], s[mt][1], s[mt][2], s[mt][3]};
+            if constexpr (SEP) {
+                GroupRow<T, DT> qr;
+                qr.load(Rows::QD ? Rows::row(tl, 3, c) : (const T*)a.Qdec + tok + (size_t)min(t + c, t1 - 1) * stride, g);
+                if constexpr (!QREG) latent_row(kd[0], a.Kdec, mt);
+                z = dot_groups<T, DT>(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                for (int i = 0; i < 4; ++i) z[i] *= scale;
+            }
+            // the max after the tile; token by token, the max and the den at token j
+            float mc = fmaxf(m0[mt], top[mt]), dj = 1.0f;
+            if (j >= 0) {
+                mc = m0[mt];
+                dj = d0[mt];
+                for (int k = 0; k <= j; ++k) {
+                    const float sk = token_value(s[mt], k, c), mn = fmaxf(mc, sk), r = safe_ref(mn);
+                    dj = (mc == kNegInf ? 0.0f : dj * exp_nat(mc - r)) + exp_nat(sk - r);
+                    mc = mn;
+                }
+            }
+            const float ref = safe_ref(mc);
+            if (__any(ref != mref[mt])) {
+                // (the max falls as the walk goes back; the bound keeps a last chunk's zeros zero)
+                const float r = exp_nat(fminf(ref - mref[mt], 1.0f));
+                ysum[mt] *= r;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[mt][dt][i] *= r;
+                mref[mt] = ref;
+            }
+            float e[4], d[4], al[4], w[4], wg[4], run = 0.0f, wrun = 0.0f, below, above, all;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float ev = exp_nat(s[mt][i] - ref);
+                e[i] = j < 0 || 4 * g + i == j ? ev : 0.0f;
+                run += e[i];
+                d[i] = run;
+                al[i] = t + 4 * g + i < t1 && lat[mt] != kNowhere ? exp_nat(z[i] - lse[i]) : 0.0f;
+                if constexpr (SEP) al_out.store(4u * M * (t + 4 * g + i) + lat[mt], al[i]);
+            }
+            group_scan(run, g, below, above, all);
+            const float start = m0[mt] == kNegInf ? 0.0f : d0[mt] * exp_nat(m0[mt] - ref);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float dd = j >= 0 ? dj : start + below + d[i];
+                w[i] = j < 0 || 4 * g + i == j ? al[i] * __builtin_amdgcn_rcpf(dd > 0.0f ? dd : 1.0f) : 0.0f;
+                wg[i] = w[i] == 0.0f ? 0.0f : w[i] * gz[mt][i];
+                wrun += wg[i];
+            }
+            group_scan(wrun, g, below, above, all);
+            wf[mt] = factor<F>(w[0], w[1], w[2], w[3]);
+            f32x4 xz = dot_state<T, DT>(vr, x[mt], f32x4{0.f, 0.f, 0.f, 0.f});
+            xz = mm(gvf, wf[mt], xz);
+            // Y at token 4g + i: later tokens and itself
+            float suffix = ysum[mt] + above;
+#pragma unroll
+            for (int i = 3; i >= 0; --i) {
+                suffix += wg[i];
+                float r = e[i] * (xz[i] - suffix);
+                if constexpr (!SEP) r += al[i] * (gz[mt][i] - gy[i]);
+                ds_out.store(j < 0 || 4 * g + i == j ? 4u * M * (t + 4 * g + i) + lat[mt] : kNowhere, r);
+                etile[(4 * g + i) * EP + 16 * mt + c] = e[i];
+                wtile[(4 * g + i) * EP + 16 * mt + c] = w[i];
+            }
+            ysum[mt] += all;
+        }
+        wave_lds_sync();
+        F ef[MT];
+        f32x4 G = {0.f, 0.f, 0.f, 0.f};       // [t][tau] summed over this wave's latents
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const f32x4 er = *reinterpret_cast<const f32x4_a*>(etile + c * EP + 16 * mt + 4 * g);
+            const f32x4 wr = *reinterpret_cast<const f32x4_a*>(wtile + c * EP + 16 * mt + 4 * g);
+            ef[mt] = factor<F>(er[0], er[1], er[2], er[3]);
+            G = mm(factor<F>(wr[0], wr[1], wr[2], wr[3]), ef[mt], G);
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (k < piece_of<DT>(dt))
+                            xtile[(16 * mt + c) * XP + col_of<DT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
+        wave_lds_sync();
+        const F gf = factor<F>(4 * g >= c ? G[0] : 0.0f, 4 * g + 1 >= c ? G[1] : 0.0f, 4 * g + 2 >= c ? G[2] : 0.0f,
+                               4 * g + 3 >= c ? G[3] : 0.0f);
+        // dv rows and X += W^T g, a piece of value columns at a time
+        f32x4 dv[DT];
+#pragma unroll
+        for (int d1 = 0; d1 < DT; d1 += piece_of<DT>(d1)) {
+            stage<DT>();
+            ColRow<float, DT> xr[MT][4];
+            TokCols<T, DT> gc;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                gc.r[i].load_piece(Rows::row(tl, 2, 4 * g + i), c, d1);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) xr[mt][i].load_piece(xtile + (16 * mt + 4 * g + i) * XP, c, d1);
+            }
+            // token by token: the other tokens' g, which may not be finite, times zero.  (A select
+            // each time and no branch: after a branch around it the compiler reads the product
+            // above too early on the skipped side.)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int k = 0; k < ColRow<T, DT>::W; ++k) gc.r[i].w[k] = j < 0 || 4 * g + i == j ? gc.r[i].w[k] : 0u;
+#pragma unroll
+            for (int dt = d1; dt < d1 + piece_of<DT>(d1); ++dt) {
+                f32x4 r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    r = mm(ef[mt], factor<F>(xr[mt][0].get(dt), xr[mt][1].get(dt), xr[mt][2].get(dt), xr[mt][3].get(dt)), r);
+                const auto go = gc.op(dt);
+                dv[dt] = mm(gf, go, r);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) x[mt][dt] = mm(go, wf[mt], x[mt][dt]);
+            }
+        }
+        // rows of this pass; the tile's last pass brings the next tile in
+        const bool last = j <= 0, more = last && t > t0;
+        if (NW == 1) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int ti = t + 4 * g + i;
+                if (ti >= t1 || !(j < 0 || 4 * g + i == j)) continue;
+                const size_t row = tok + (size_t)ti * stride;
+#pragma unroll
+                for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
+                    float o[4];
+                    const int P = piece_of<DT>(dt);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) o[k] = k < P ? dv[dt + k < DT ? dt + k : 0][i] : 0.0f;
+                    const size_t at = row + col_of<DT>(dt, c);
+                    if (P == 4) store_cols<4>(a.dV, at, o, OD);
+                    else if (P == 2) store_cols<2>(a.dV, at, o, OD);
+                    else store_cols<1>(a.dV, at, o, OD);
+                }
+            }
+            wave_lds_sync();
+            if (more) rows.store(tl, a, tok, stride, t - TT, t1);
+            wave_lds_sync();
+        } else {
+            wave_lds_sync();
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) vtile[(4 * g + i) * D + col_of<DT>(dt, c)] = dv[dt][i];
+            __syncthreads();
+            if (more) rows.store(tl, a, tok, stride, t - TT, t1);      // every wave is done with this tile's rows
+            for (int e = threadIdx.x; e < TT * D / 4; e += blockDim.x) {
+                const int ti = e / (D / 4), col = 4 * (e % (D / 4));
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                for (int k = 0; k < NW; ++k) {
+                    const f32x4 r = *reinterpret_cast<const f32x4_a*>(smem + k * ds_wave_floats<MT, DT>() + ti * D + col);
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) acc[n] += r[n];
+                }
+                const float o[4] = {acc[0], acc[1], acc[2], acc[3]};
+                if (t + ti < t1 && (j < 0 || ti == j)) store_cols<4>(a.dV, tok + (size_t)(t + ti) * stride + col, o, OD);
+            }
+            __syncthreads();
+        }
+        if (!last) {
+            --j;
+            continue;
+        }
+        if (!more) break;
+        j = -1;
+        t -= TT;
+    }
+}
+
+}  // namespace wave
+}  // namespace flare

@@ -1,0 +1,108 @@
+// flare_wave_bwd_launch.h -- instances and launchers of flare_wave_bwd.h for one input type
+// (included by one translation unit per type).
+#pragma once
+
+#include "flare_internal.h"
+#include "flare_wave_bwd.h"
+#include "flare_wave_contract.h"
+
+namespace flare {
+namespace wave {
+
+// Latent tiles per wave.  The walks are bound by the latency of a tile's chain, so waves per
+// SIMD count: 16 latents a wave up to D = 64 fit four of them (D = 64: 293 -> 246 us for the
+// backward walk at B 4, N 4096, H 16, M 128), 32 latents of a narrow bank three.  At D = 128
+// a wave of 16 spills and two waves of 32 are faster (990 against 832 us at N 16384, H 16,
+// M 256).
+template <int DT>
+constexpr int bwd_tiles() { return DT <= 2 || DT > 4 ? 2 : 1; }
+
+template <typename T, int MT, int DT, bool SEP>
+int bwd_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk, hipStream_t st) {
+    constexpr int D = 16 * DT;
+    const int NW = (int)((M + 16 * MT - 1) / (16 * MT));
+    const int64_t NC = (N + chunk - 1) / chunk;
+    const dim3 grid((unsigned)NC, (unsigned)(B * H));
+    const int64_t per = TT * kLseTiles * 4;
+    hipLaunchKernelGGL((wave_lse_kernel<T, DT>), dim3((unsigned)((N + per - 1) / per), (unsigned)(B * H)), dim3(256), 0, st,
+                       (const T*)p.Qdec, (const T*)p.Kdec, (int)N, (int)H, (int)M, scale, (float*)p.lse);
+    typedef TileRows<T, DT, SEP> Rows;
+    hipLaunchKernelGGL((wave_gz_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), 2 * Rows::BYTES, st, p, (int)N, (int)H, (int)M, scale,
+                       (int)chunk);
+    const int64_t cols = B * H * M * (D + 1);
+    hipLaunchKernelGGL(wave_carry_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, st, p.xsum, p.ysum, p.pmax,
+                       (int)NC, (int)M, D, (int)(B * H * M));
+    const size_t lds = sizeof(float) * (size_t)NW * ds_wave_floats<MT, DT>() + Rows::BYTES;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute((const void*)wave_ds_kernel<T, MT, DT, SEP>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            set_error("wave_ds_kernel: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
+            return FLARE_ERR_LAUNCH;
+        }
+    }
+    hipLaunchKernelGGL((wave_ds_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), lds, st, p, (int)N, (int)H, (int)M, scale,
+                       (int)chunk);
+    return check_launch("wave backward kernels");
+}
+
+template <typename T, int DT>
+int bwd_dt(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk,
+           hipStream_t st) {
+    constexpr int MT = bwd_tiles<DT>();
+    return sep ? bwd_at<T, MT, DT, true>(p, B, N, H, M, scale, chunk, st)
+               : bwd_at<T, MT, DT, false>(p, B, N, H, M, scale, chunk, st);
+}
+
+template <typename T, int DT>
+int rows_dt(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, float scale,
+            void* out, hipStream_t st) {
+    const int64_t per = 4 * TT * kRowTiles;
+    hipLaunchKernelGGL((wave_rows_kernel<T, DT>), dim3((unsigned)((N + per - 1) / per), (unsigned)(B * H)), dim3(256), 0, st,
+                       p, (const T*)r1, (const T*)r2, (int)N, (int)H, (int)M, scale, (T*)out);
+    return check_launch("wave_rows_kernel");
+}
+template <typename T, int DT>
+int cols_dt(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, float* P,
+            hipStream_t st) {
+    constexpr int MT = DT <= 4 ? 2 : 1;
+    hipLaunchKernelGGL((wave_cols_kernel<T, MT, DT>),
+                       dim3((unsigned)((N + kBwdGroup - 1) / kBwdGroup), (unsigned)((M + 16 * MT - 1) / (16 * MT)),
+                            (unsigned)(B * H)),
+                       dim3(256), 0, st, p, (const T*)r1, (const T*)r2, (int)N, (int)H, (int)M, P);
+    return check_launch("wave_cols_kernel");
+}
+
+#define FLARE_WAVE_DT_CASES(NAME, ...)                                                       \
+    switch (D / 16) {                                                                        \
+        case 1: return NAME<T, 1>(__VA_ARGS__);                                              \
+        case 2: return NAME<T, 2>(__VA_ARGS__);                                              \
+        case 3: return NAME<T, 3>(__VA_ARGS__);                                              \
+        case 4: return NAME<T, 4>(__VA_ARGS__);                                              \
+        case 6: return NAME<T, 6>(__VA_ARGS__);                                              \
+        case 8: return NAME<T, 8>(__VA_ARGS__);                                              \
+        default: break;                                                                      \
+    }                                                                                        \
+    set_error("wave backward: D=%lld has no instance", (long long)D);                        \
+    return FLARE_ERR_INVALID;
+
+template <typename T>
+int rows_type(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D,
+              float scale, void* out, hipStream_t st) {
+    FLARE_WAVE_DT_CASES(rows_dt, p, r1, r2, B, N, H, M, scale, out, st)
+}
+template <typename T>
+int cols_type(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D,
+              float* P, hipStream_t st) {
+    FLARE_WAVE_DT_CASES(cols_dt, p, r1, r2, B, N, H, M, P, st)
+}
+
+template <typename T>
+int bwd_type(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale,
+             int64_t chunk, hipStream_t st) {
+    FLARE_WAVE_DT_CASES(bwd_dt, p, sep, B, N, H, M, scale, chunk, st)
+}
+
+}  // namespace wave
+}  // namespace flare

@@ -111,3 +111,77 @@ def test_wave_unaligned_inputs(dtype):
         assert args[which].data_ptr() % 16 != 0
         y, _ = flare_autoregressive_prefill_triton(*args)
         _close(y, to_np(y0), dtype, f"input {which} unaligned")
+
+
+def _grads(q, k, v, g, qd=None, kd=None, chunk=None):
+    from causal_flare import flare_autoregressive_triton
+    leaves = {n: t.to(DEV).requires_grad_(True) for n, t in (("q", q), ("k", k), ("v", v), ("qd", qd), ("kd", kd))
+              if t is not None}
+    y = flare_autoregressive_triton(leaves["q"], leaves["k"], leaves["v"], Q_dec=leaves.get("qd"), K_dec=leaves.get("kd"))
+    y.backward(g.to(DEV))
+    return {n: t.grad for n, t in leaves.items()}
+
+
+# the backward's bars (test_gpu_backward.py): fp32 1e-4 of the largest entry, 16-bit the rounding
+# of the results and of the saved output in g.y (2e-2 bf16, an eighth of it fp16).  fp16 adds the
+# products of fp32 factors as bf16 hi + lo, 2^-17 of |g.v| (4 at D = 16: 3e-5 against the floor
+# of 1e-2) where gz - g.y cancels exactly (N = 1, true gradient 0): 2.5e-3 + 3e-3.
+GRAD_BAR = {torch.float32: 1e-4, torch.bfloat16: 2e-2, torch.float16: 5.5e-3}
+
+
+def _check_grads(got, refs, dtype, what):
+    for (n, x), r in zip(got.items(), refs):
+        a, r = to_np(x).astype(np.float64), np.asarray(r)
+        assert np.isfinite(a).all(), f"{what} d{n}: not finite"
+        err = np.abs(a - r).max() / max(np.abs(r).max(), 1e-2)
+        assert err <= GRAD_BAR[dtype], f"{what} d{n}: {err:.3e}"
+
+
+@pytest.mark.parametrize("M,D,N", [(16, 16, 1), (48, 32, 70), (64, 32, 150), (16, 48, 33), (64, 64, 200), (96, 96, 47),
+                                   (128, 64, 135), (192, 128, 129), (256, 128, 80)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sep", ["", "q", "k", "qk"])
+def test_wave_backward(M, D, N, dtype, sep):
+    """Off every tile edge: latents that fill no wave, partial token tiles, several chunks
+    (64 tokens each at these sizes), each decoder-sharing mode."""
+    print("CASE wave_backward", M, D, N, dtype, sep, flush=True)
+    B, H = 2, 2
+    q, k, v = seeded(7 * M + D, B, N, H, M, D, D, dtype)
+    gen = torch.Generator().manual_seed(M)
+    g = torch.randn(B, N, H, D, generator=gen).to(dtype)
+    qd = torch.randn(B, N, H, D, generator=gen).to(dtype) if "q" in sep else None
+    kd = torch.randn(H, M, D, generator=gen).to(dtype) if "k" in sep else None
+    got = _grads(q, k, v, g, qd, kd)
+    refs = O.ar_grads(q, k, v, g, Q_dec=qd, K_dec=kd)
+    refs = list(refs[:3]) + [r for r, t in zip(refs[3:], (qd, kd)) if t is not None]
+    _check_grads(got, refs, dtype, f"M={M} D={D} N={N} sep={sep}")
+
+
+@pytest.mark.parametrize("M,D,dtype", [(64, 32, torch.float32), (128, 64, torch.float32), (128, 64, torch.bfloat16)])
+def test_wave_backward_jumps_and_infinite_gradient(M, D, dtype):
+    """Scores that rise by 90 to 400 nats inside a tile, at the start, mid-tile and on a chunk's
+    last token: those tiles are walked token by token.  An infinite dY entry reaches dV of its
+    own and earlier tokens only."""
+    print("CASE wave_backward_jumps", M, D, dtype, flush=True)
+    B, N, H = 1, 150, 2
+    q, k, v = seeded(13 + M, B, N, H, M, D, D, dtype, q_std=D ** -0.5)
+    k = k * 0.5
+    for t, nats, lat in ((3, 90.0, 1), (63, 200.0, 7), (105, 400.0, 12)):
+        for h in range(H):
+            row = q[h, lat].float()
+            k[0, t, h] = (row * (nats * D ** 0.5 / row.square().sum())).to(dtype)
+    gen = torch.Generator().manual_seed(M)
+    g = torch.randn(B, N, H, D, generator=gen).to(dtype)
+    got = _grads(q, k, v, g)
+    refs = O.ar_grads(q, k, v, g)
+    if dtype is torch.float32:
+        # (16-bit: da cancels where the softmax peaks, from the rounded output; dV has no such term)
+        _check_grads(got, refs[:3], dtype, "jumps")
+    _check_grads({"v": got["v"]}, refs[2:3], dtype, "jumps")
+    q, k, v = seeded(14 + M, B, N, H, M, D, D, dtype)
+    gi = g.clone()
+    gi[0, 37, 0, 5] = float("inf")
+    clean, inf = _grads(q, k, v, g)["v"], _grads(q, k, v, gi)["v"]
+    assert torch.isfinite(inf[0, 38:]).all()
+    _check_grads({"v": inf[0, 38:]}, [to_np(clean[0, 38:])], dtype, "past the infinite entry")
+    assert not torch.isfinite(inf[0, :38, 0, 5]).any()
