@@ -1457,50 +1457,44 @@ bool ar_backward_supported(int64_t M, int64_t Dk, int64_t Dv) {
            Dv >= 16 && Dv <= 512;
 }
 
-// The wave backward's workspace (flare_wave_bwd.h) and its chunk: two waves per SIMD over
-// the device as the forward, whole 64-token steps, and no more memory than the other
-// kernels' workspace takes.
-struct WaveBwdLayout {
-    int64_t chunk, NC;
-    size_t off_pm, off_pd, off_pn, off_xs, off_ys, off_tm, off_td, off_sw, off_gz, off_ds, off_al, off_lse, off_gy, off_p1,
-        off_p2, total;
-    WaveBwdLayout(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, bool sep, int64_t chunk_) : chunk(chunk_) {
-        NC = (N + chunk - 1) / chunk;
-        const size_t BH = (size_t)B * H, NT = (N + 15) / 16;
-        size_t o = 0;
-        auto take = [&](size_t floats) {
-            const size_t at = o;
-            o += ((floats * sizeof(float) + 255) / 256) * 256;
-            return at;
-        };
-        off_pm = take(BH * NC * M);
-        off_pd = take(BH * NC * M);
-        off_pn = take(BH * NC * M * D);
-        off_xs = take(BH * NC * M * D);
-        off_ys = take(BH * NC * M);
-        off_tm = take(BH * NT * M);
-        off_td = take(BH * NT * M);
-        off_sw = take(BH * NT * ((M + 15) / 16));     // at most one wave per 16 latents
-        off_gz = take(BH * N * M);
-        off_ds = take(BH * N * M);
-        off_al = take(sep ? BH * N * M : 0);
-        off_lse = take(BH * N);
-        off_gy = take(BH * N);
-        off_p1 = take(bwd_partial_floats(B, N, H, M, D));
-        off_p2 = take(sep ? bwd_partial_floats(B, N, H, M, D) : 0);
-        total = o;
-    }
-};
+WaveBwdLayout::WaveBwdLayout(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, bool sep, int64_t chunk_, int64_t tiles)
+    : chunk(chunk_), NC((N + chunk_ - 1) / chunk_) {
+    const size_t BH = (size_t)B * H;
+    size_t o = 0;
+    auto take = [&](size_t floats) {
+        const size_t at = o;
+        o += ((floats * sizeof(float) + 255) / 256) * 256;
+        return at;
+    };
+    off_pm = take(BH * NC * M);
+    off_pd = take(BH * NC * M);
+    off_pn = take(BH * NC * M * D);
+    off_xs = take(BH * NC * M * D);
+    off_ys = take(BH * NC * M);
+    off_tm = take(BH * tiles * M);
+    off_td = take(BH * tiles * M);
+    off_sw = take(BH * tiles * ((M + 15) / 16));     // at most one wave per 16 latents
+    off_gz = take(BH * N * M);
+    off_ds = take(BH * N * M);
+    off_al = take(sep ? BH * N * M : 0);
+    off_lse = take(BH * N);
+    off_gy = take(BH * N);
+    off_p1 = take(bwd_partial_floats(B, N, H, M, D));
+    off_p2 = take(sep ? bwd_partial_floats(B, N, H, M, D) : 0);
+    total = o;
+}
+
+// Its chunk: two waves per SIMD over the device as in the forward, whole 64-token steps, and
+// no more memory than the other kernels' workspace takes.
 static int64_t wave_bwd_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, bool sep, size_t bytes) {
     int64_t c = default_chunk(B, N, H, M, D);
     c = ((c + 63) / 64) * 64;
-    while (c < N && WaveBwdLayout(B, N, H, M, D, sep, c).total > bytes) c *= 2;
+    while (c < N && WaveBwdLayout(B, N, H, M, D, sep, c, (N + 15) / 16).total > bytes) c *= 2;
     return c;
 }
 
 static int run_wave_backward(const void* Q, const void* K, const void* V, const void* Qdec, const void* Kdec, int dtype,
-                             int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale, const void* Y,
-                             const void* dY, void* dQ, void* dK, void* dV, void* dQdec, void* dKdec, char* ws,
+                             int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale, const void* Y, const void* dY, void* dQ, void* dK, void* dV, void* dQdec, void* dKdec, char* ws,
                              const WaveBwdLayout& lay, hipStream_t st) {
     const bool sep = Qdec != nullptr || Kdec != nullptr;
     auto at = [&](size_t off) { return reinterpret_cast<float*>(ws + off); };
@@ -1509,8 +1503,8 @@ static int run_wave_backward(const void* Q, const void* K, const void* V, const 
     if (rc) return rc;
     rc = launch_prefix_public(pm, pd, pn, B * H, lay.NC, M, D, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, st);
     if (rc) return rc;
-    rc = launch_bwd_gy(dY, Y, dtype, B, N, H, D, at(lay.off_gy), st);
-    if (rc) return rc;
+    // (fp32: formed in the walk)
+    if (dtype != FLARE_F32 && (rc = launch_bwd_gy(dY, Y, dtype, B, N, H, D, at(lay.off_gy), st))) return rc;
     const wave::BwdPtrs p{Q, K, V, Qdec ? Qdec : K, Kdec ? Kdec : Q, dY, pm, pd, pn, at(lay.off_xs), at(lay.off_ys),
                           at(lay.off_tm), at(lay.off_td),
                           reinterpret_cast<int*>(ws + lay.off_sw), at(lay.off_gz), at(lay.off_ds), at(lay.off_al),
@@ -1540,9 +1534,9 @@ int ar_backward_run(const void* Q, const void* K, const void* V, const void* Qde
     char* ws = static_cast<char*>(workspace);
     // (the walks reach a (b, h)'s per-token arrays by 31-bit byte offsets)
     if (power <= 0.0f && mfma_phase_mask() == 3 && wave_shape(M, Dk, Dv) && 4 * N * M < (int64_t)1 << 31 &&
-        wave_aligned({Q, K, V, Qdec, Kdec, Y, dY, dV})) {
+        wave_aligned({Q, K, V, Qdec, Kdec, dY, dV})) {
         const bool sep = Qdec != nullptr || Kdec != nullptr;
-        const WaveBwdLayout wl(B, N, H, M, Dk, sep, wave_bwd_chunk(B, N, H, M, Dk, sep, lay.total));
+        const WaveBwdLayout wl(B, N, H, M, Dk, sep, wave_bwd_chunk(B, N, H, M, Dk, sep, lay.total), (N + 15) / 16);
         if (wl.total <= lay.total)
             return run_wave_backward(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dk, scale, Y, dY, dQ, dK, dV, dQdec, dKdec,
                                      ws, wl, st);

@@ -155,6 +155,15 @@ int launch_bwd_contract(const void* Q, const void* K, const void* Qdec, const vo
 // The token-causal backward (shapes as ar_backward_supported).  power > 0: the
 // stablemax encoder weight s(a) in place of e^a (the decoder stays a softmax).
 bool ar_backward_supported(int64_t M, int64_t Dk, int64_t Dv);
+// The wave backward's workspace: chunk prefixes and X / Y terms, `tiles` (max, den) rows
+// (16-token tiles, or blocks), gz, ds, alpha for separate decoder weights, and the partial
+// dQ / dK_dec sums.
+struct WaveBwdLayout {
+    int64_t chunk, NC;
+    size_t off_pm, off_pd, off_pn, off_xs, off_ys, off_tm, off_td, off_sw, off_gz, off_ds, off_al, off_lse, off_gy, off_p1,
+        off_p2, total;
+    WaveBwdLayout(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, bool sep, int64_t chunk, int64_t tiles);
+};
 size_t ar_backward_workspace(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv);
 int ar_backward_run(const void* Q, const void* K, const void* V, const void* Qdec, const void* Kdec, int dtype,
                     int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv, float scale, const void* Y,
@@ -191,7 +200,8 @@ struct BwdPtrs {
     float *tmax, *tden;                  // [B*H, NT, M]: state at each 16-token tile's start
     int* stepwise;                       // [B*H, NT, waves]: tiles walked token by token
     float *gz, *ds, *al;                 // [B*H, N, M]; al only for separate decoder weights
-    const float *lse, *gy;               // [B*H, N]
+    const float* lse;                    // [B*H, N]: decoder log-sum-exp
+    float* gy;                           // [B*H, N]: g . y
     void* dV;
 };
 // Score gradients of the backward's contractions (flare_wave_contract.h): ds, and for da the
@@ -202,9 +212,12 @@ struct ContractPtrs {
 };
 // out = scale (ds . r1 + da . r2) over the latents, r1 / r2 [H, M, D] or null
 // P = partial sums over 512-token groups of ds^T r1 + da^T r2, r1 / r2 [B, N, H, D] or null
+// semi: the block-causal layer's backward walks (flare_wave_semi.h; tmax / tden per block)
 #define FLARE_WAVE_CONTRACT(SUFFIX)                                                                                  \
     int rows_##SUFFIX(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, \
                       int64_t D, float scale, void* out, hipStream_t st);                                             \
+    int semi_##SUFFIX(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale,  \
+                      int64_t chunk, int64_t block, hipStream_t st);                                                   \
     int cols_##SUFFIX(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, \
                       int64_t D, float* P, hipStream_t st);
 FLARE_WAVE_CONTRACT(f32)

@@ -609,6 +609,34 @@ static int run_semi_backward(const void* Q, const void* K, const void* V, const 
                                dKd, P1, P2, s);
 }
 
+// The wave kernels (flare_wave_semi.h) for every bank they have an instance of: no M x D state
+// per block in memory.  Chunks are the forward's (two waves per SIMD over the device), rounded
+// up to whole blocks.
+static int run_wave_semi(const void* Q, const void* K, const void* V, const void* Qdec, const void* Kdec, int dtype,
+                         int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale, int64_t block,
+                         const void* Y, const void* dY, void* dQ, void* dK, void* dV, void* dQd, void* dKd, char* ws,
+                         const WaveBwdLayout& lay, hipStream_t st) {
+    const bool sep = Qdec != nullptr || Kdec != nullptr;
+    auto at = [&](size_t off) { return reinterpret_cast<float*>(ws + off); };
+    float *pm = at(lay.off_pm), *pd = at(lay.off_pd), *pn = at(lay.off_pn);
+    int rc = launch_prepare_public(Q, K, V, dtype, B, N, H, M, D, D, scale, lay.chunk, pm, pd, pn, st);
+    if (rc) return rc;
+    rc = launch_prefix_public(pm, pd, pn, B * H, lay.NC, M, D, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, st);
+    if (rc) return rc;
+    // (fp32: formed in the walk)
+    if (dtype != FLARE_F32 && (rc = launch_bwd_gy(dY, Y, dtype, B, N, H, D, at(lay.off_gy), st))) return rc;
+    const wave::BwdPtrs p{Q, K, V, Qdec ? Qdec : K, Kdec ? Kdec : Q, dY, pm, pd, pn, at(lay.off_xs), at(lay.off_ys),
+                          at(lay.off_tm), at(lay.off_td), reinterpret_cast<int*>(ws + lay.off_sw), at(lay.off_gz),
+                          at(lay.off_ds), at(lay.off_al), at(lay.off_lse), at(lay.off_gy), dV};
+    rc = dtype == FLARE_BF16  ? wave::semi_bf16(p, sep, B, N, H, M, D, scale, lay.chunk, block, st)
+         : dtype == FLARE_F16 ? wave::semi_f16(p, sep, B, N, H, M, D, scale, lay.chunk, block, st)
+                              : wave::semi_f32(p, sep, B, N, H, M, D, scale, lay.chunk, block, st);
+    if (rc) return rc;
+    return launch_bwd_contract(Q, K, Qdec, Kdec, dtype, B, N, H, M, D, scale, at(lay.off_ds), at(lay.off_al),
+                               at(lay.off_gz), at(lay.off_gy), true, !sep, dQ, dK, dQd, dKd, at(lay.off_p1),
+                               at(lay.off_p2), st);
+}
+
 }  // namespace flare
 
 using namespace flare;
@@ -648,6 +676,14 @@ int flare_semi_ar_backward(const void* Q, const void* K, const void* V, const vo
     FLARE_REQUIRE((((uintptr_t)workspace) & 255) == 0, "flare_semi_ar_backward: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (mfma_phase_mask() == 3 && wave_shape(M, Dk, Dv) && 4 * N * M < (int64_t)1 << 31 &&
+        wave_aligned({Q, K, V, Qdec, Kdec, dY, dV})) {
+        const int64_t target = default_chunk(B, N, H, M, Dv);
+        const WaveBwdLayout wl(B, N, H, M, Dv, Qdec || Kdec, ((target + block - 1) / block) * block, N / block);
+        if (wl.total <= lay.total)
+            return run_wave_semi(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dv, scale, block, Y, dY, dQ, dK, dV, dQdec, dKdec,
+                                 ws, wl, st);
+    }
 #define FLARE_SEMI_BWD(TY)                                                                                        \
     return run_semi_backward<TY>(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dk, Dv, scale, block, Y, dY, dQ, dK, dV, \
                                  dQdec, dKdec, ws, lay, st)

@@ -14,6 +14,11 @@
 //             recomputes a tile's weights from the stored (max, den), writes ds and dv.
 // Between them only gz (fp32) travels per token and latent; scores, weights, decoder softmax
 // and running sums are formed again from K, Q and one (max, den) pair per 16 tokens.
+// g . y: for fp32 inputs the sum of alpha gz over the latents, from the very gz it is subtracted
+// from (gz - g . y cancels, and the saved output carries its own rounding: with it the fp32
+// gradients of the block-causal layer were up to 1.4 times as far off).  16-bit inputs take it
+// from the saved output, whose rounding their results have anyway (in the walk it cost 30 us
+// against 16 for its own kernel at B 4, N 4096, H 16, M 128, D 64).
 //
 // Layout: the tile's score-like matrices are C tiles with tokens as rows (lane (g, c):
 // tokens 4g + i, latent c), U and X are kept transposed (rows = value columns, lane column =
@@ -29,6 +34,14 @@
 // Numerics.  Weights inside a tile are relative to the latents' max after the tile, X and Y
 // to the max of the tile they were last used in (factors <= 1 as the walk goes back).  A tile
 // in which a max rises by more than kTileJump runs token by token with each token's own max.
+//
+// Bound by the latency of a tile's chain at two to four waves a SIMD (a third to a half of the
+// vector issue slots are used).  Measured, forward and backward, against per-token statistics
+// and one state per 32 tokens in memory (MI355X):
+//   bf16 B 4, N 4096, H 16, M 128, D 64    1521 -> 574 us (wave_gz 130, wave_ds 225 of it)
+//   bf16 N 16384, H 16, M 256, D 128       3774 -> 1600 us (wave_gz 420, wave_ds 680)
+//   bf16 B 4, N 2011, H 16, M 64, D 32     2947 -> 213 us
+//   fp32 B 2, N 1024, H 8, M 64, D 64, decoder weights of its own   1170 -> 208 us
 #pragma once
 
 #include <type_traits>
@@ -114,8 +127,15 @@ struct GroupRow {
 template <typename T, int DT>
 __device__ __forceinline__ f32x4 dot_groups(const GroupRow<T, DT>& x, const GroupRow<T, DT>& y, f32x4 c) {
     if constexpr (sizeof(T) == 4) {
+        // (two sums over halves: fewer roundings in a row, and shorter chains)
+        f32x4 d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int e = 0; e < 4 * DT; ++e) c = mma4(x.at(e), y.at(e), c);
+        for (int e = 0; e < 2 * DT; ++e) {
+            c = mma4(x.at(e), y.at(e), c);
+            d = mma4(x.at(2 * DT + e), y.at(2 * DT + e), d);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[i] += d[i];
     } else {
         constexpr bool F16 = __is_same(T, __half);
 #pragma unroll
@@ -153,6 +173,20 @@ __device__ __forceinline__ f32x4 mm(const Pair4& a, const Pair4& b, f32x4 c) {
     const bf16x8 hl = cat(a.h, a.l);
     c = mfma::mma(hl, cat(b.h, b.h), c);
     return mfma::mma(hl, cat(b.l, b.l), c);
+}
+
+// c += a b for a c that collects many tiles: fp32 products are summed over the tile first, so
+// that c is rounded once a tile and not once a product.
+template <typename A, typename B>
+__device__ __forceinline__ f32x4 collect(const A& a, const B& b, f32x4 c) {
+    if constexpr (__is_same(A, F4)) {
+        const f32x4 r = mm(a, b, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[i] += r[i];
+        return c;
+    } else {
+        return mm(a, b, c);
+    }
 }
 
 template <typename T> struct ProdOf { typedef Pair4 F; };            // type of an fp32 factor
@@ -201,10 +235,15 @@ struct TokCols {
 template <typename T, int DT>
 __device__ __forceinline__ f32x4 dot_state(const GroupRow<T, DT>& x, const f32x4 (&u)[DT], f32x4 c) {
     if constexpr (sizeof(T) == 4) {
+        f32x4 d[3] = {};
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DT; ++dt) {
+            c = mma4(x.at(list_at<DT>(dt, 0)), u[dt][0], c);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) c = mma4(x.at(list_at<DT>(dt, i)), u[dt][i], c);
+            for (int i = 1; i < 4; ++i) d[i - 1] = mma4(x.at(list_at<DT>(dt, i)), u[dt][i], d[i - 1]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[i] = (c[i] + d[0][i]) + (d[1][i] + d[2][i]);
     } else {
 #pragma unroll
         for (int s = 0; s < GroupRow<T, DT>::S; ++s) {
@@ -390,6 +429,26 @@ __global__ __launch_bounds__(256) void wave_lse_kernel(const T* __restrict__ Qd,
     }
 }
 
+template <typename T>
+constexpr bool own_gy() { return sizeof(T) == 4; }
+// g . y of a tile: each wave's sums over its latents meet in LDS at the tile's barrier.
+// sums: [2][waves][16], the half of the tile's row buffer.
+__device__ __forceinline__ void put_gy(float* sums, const float (&v)[4], int wv, int g, int c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float r = mfma::row_sum16(v[i]);
+        if (c == 0) sums[wv * TT + 4 * g + i] = r;
+    }
+}
+__device__ __forceinline__ void store_gy(const float* sums, int NW, float* gy, int t, int t1) {
+    const int i = threadIdx.x;
+    if (i < TT && t + i < t1) {
+        float r = 0.0f;
+        for (int k = 0; k < NW; ++k) r += sums[k * TT + i];
+        gy[t + i] = r;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Forward walk of a chunk: gz, tile states, the chunk's X and Y.  grid (NC, B*H), one wave
 // per MT*16 latents; the waves share a tile's rows and exchange nothing else.
@@ -403,7 +462,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
     constexpr int D = 16 * DT;
     typedef typename ProdOf<T>::F F;
     typedef TileRows<T, DT, SEP> Rows;
-    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>();
+    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>(), OWN_GY = own_gy<T>();
     extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
     const int ch = blockIdx.x, NC = gridDim.x, bh = blockIdx.y;
     const int b = bh / H, h = bh % H;
@@ -455,6 +514,9 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
     rows.store((T*)tile_lds, a, tok, stride, t0, t1);
     __syncthreads();
     int buf = 0, t = t0, j = -1;
+    float* gsum = reinterpret_cast<float*>(tile_lds + 2 * Rows::BYTES);
+    float* gy_out = a.gy + (size_t)bh * N;
+    float gy[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     while (true) {
         const T* tl = (const T*)(tile_lds + buf * Rows::BYTES);
         if (j <= 0 && t + TT < t1) rows.fetch(a, tok, stride, t + TT, t1);
@@ -492,7 +554,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
                 for (int i = 0; i < 4; ++i) z[i] *= scale;
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) al[mt][i] = t + 4 * g + i < t1 ? exp_nat(z[i] - lse[i]) : 0.0f;
+            for (int i = 0; i < 4; ++i) al[mt][i] = t + 4 * g + i < t1 && lat[mt] != kNowhere ? exp_nat(z[i] - lse[i]) : 0.0f;
         }
         stage<DT>();
         // g_t . v_tau as the [t][tau] factor of sums over tau (C rows tau, lane column t)
@@ -560,6 +622,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
                 const float gz = p[i] * inv;
                 w[i] = on ? al[mt][i] * er[mt] * inv : 0.0f;      // (al is 0 past the sequence)
                 ysum[mt] += w[i] == 0.0f ? 0.0f : w[i] * gz;
+                if constexpr (OWN_GY) gy[i] += on && al[mt][i] != 0.0f ? al[mt][i] * gz : 0.0f;
                 gz_out.store(on ? 4u * M * (t + 4 * g + i) + lat[mt] : kNowhere, gz);
             }
             den[mt] += all;
@@ -580,18 +643,24 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
                 const auto vo = vc.op(dt), go = gc.op(dt);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
-                    u[mt][dt] = mm(vo, ef[mt], u[mt][dt]);
-                    x[mt][dt] = mm(go, wf[mt], x[mt][dt]);
+                    u[mt][dt] = collect(vo, ef[mt], u[mt][dt]);
+                    x[mt][dt] = collect(go, wf[mt], x[mt][dt]);
                 }
             }
         }
         if (j >= 0 && ++j < min(TT, t1 - t)) continue;
         j = -1;
+        float* sums = gsum + buf * NW * TT;
+        if constexpr (OWN_GY) {
+            put_gy(sums, gy, wv, g, c);
+            gy[0] = gy[1] = gy[2] = gy[3] = 0.0f;
+        }
         t += TT;
-        if (t >= t1) break;
         buf ^= 1;
-        rows.store((T*)(tile_lds + buf * Rows::BYTES), a, tok, stride, t, t1);
+        if (t < t1) rows.store((T*)(tile_lds + buf * Rows::BYTES), a, tok, stride, t, t1);
         __syncthreads();
+        if constexpr (OWN_GY) store_gy(sums, NW, gy_out, t - TT, t1);
+        if (t >= t1) break;
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -889,7 +958,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
                 const auto go = gc.op(dt);
                 dv[dt] = mm(gf, go, r);
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) x[mt][dt] = mm(go, wf[mt], x[mt][dt]);
+                for (int mt = 0; mt < MT; ++mt) x[mt][dt] = collect(go, wf[mt], x[mt][dt]);
             }
         }
         // rows of this pass; the tile's last pass brings the next tile in

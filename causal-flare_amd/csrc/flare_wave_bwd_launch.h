@@ -5,6 +5,7 @@
 #include "flare_internal.h"
 #include "flare_wave_bwd.h"
 #include "flare_wave_contract.h"
+#include "flare_wave_semi.h"
 
 namespace flare {
 namespace wave {
@@ -17,34 +18,67 @@ namespace wave {
 template <int DT>
 constexpr int bwd_tiles() { return DT <= 2 || DT > 4 ? 2 : 1; }
 
-template <typename T, int MT, int DT, bool SEP>
-int bwd_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk, hipStream_t st) {
-    constexpr int D = 16 * DT;
-    const int NW = (int)((M + 16 * MT - 1) / (16 * MT));
-    const int64_t NC = (N + chunk - 1) / chunk;
-    const dim3 grid((unsigned)NC, (unsigned)(B * H));
+template <typename T, int DT>
+int launch_lse(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float scale, hipStream_t st) {
     const int64_t per = TT * kLseTiles * 4;
     hipLaunchKernelGGL((wave_lse_kernel<T, DT>), dim3((unsigned)((N + per - 1) / per), (unsigned)(B * H)), dim3(256), 0, st,
                        (const T*)p.Qdec, (const T*)p.Kdec, (int)N, (int)H, (int)M, scale, (float*)p.lse);
-    typedef TileRows<T, DT, SEP> Rows;
-    hipLaunchKernelGGL((wave_gz_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), 2 * Rows::BYTES, st, p, (int)N, (int)H, (int)M, scale,
-                       (int)chunk);
-    const int64_t cols = B * H * M * (D + 1);
+    return check_launch("wave_lse_kernel");
+}
+inline int launch_carry(const BwdPtrs& p, int64_t NC, int64_t M, int64_t D, int64_t rows, hipStream_t st) {
+    const int64_t cols = rows * (D + 1);
     hipLaunchKernelGGL(wave_carry_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, st, p.xsum, p.ysum, p.pmax,
-                       (int)NC, (int)M, D, (int)(B * H * M));
+                       (int)NC, (int)M, (int)D, (int)rows);
+    return check_launch("wave_carry_kernel");
+}
+// Dynamic LDS above the default limit of 64 KB.
+inline int allow_lds(const void* kernel, size_t lds, const char* name) {
+    if (lds <= 64 * 1024) return FLARE_OK;
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess) return FLARE_OK;
+    const hipError_t e = hipGetLastError();
+    set_error("%s: %zu bytes of LDS refused: %s", name, lds, hipGetErrorString(e));
+    return FLARE_ERR_LAUNCH;
+}
+
+template <typename T, int MT, int DT, bool SEP>
+int bwd_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk, hipStream_t st) {
+    typedef TileRows<T, DT, SEP> Rows;
+    const int NW = (int)((M + 16 * MT - 1) / (16 * MT));
+    const int64_t NC = (N + chunk - 1) / chunk;
+    const dim3 grid((unsigned)NC, (unsigned)(B * H));
+    int rc = launch_lse<T, DT>(p, B, N, H, M, scale, st);
+    if (rc) return rc;
+    const size_t walk_lds = 2 * Rows::BYTES + 2 * NW * TT * sizeof(float);     // row buffers, g . y sums
+    hipLaunchKernelGGL((wave_gz_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), walk_lds, st, p, (int)N, (int)H, (int)M,
+                       scale, (int)chunk);
+    if ((rc = check_launch("wave_gz_kernel"))) return rc;
+    if ((rc = launch_carry(p, NC, M, 16 * DT, B * H * M, st))) return rc;
     const size_t lds = sizeof(float) * (size_t)NW * ds_wave_floats<MT, DT>() + Rows::BYTES;
-    if (lds > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute((const void*)wave_ds_kernel<T, MT, DT, SEP>,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            set_error("wave_ds_kernel: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
-            return FLARE_ERR_LAUNCH;
-        }
-    }
+    if ((rc = allow_lds((const void*)wave_ds_kernel<T, MT, DT, SEP>, lds, "wave_ds_kernel"))) return rc;
     hipLaunchKernelGGL((wave_ds_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), lds, st, p, (int)N, (int)H, (int)M, scale,
                        (int)chunk);
-    return check_launch("wave backward kernels");
+    return check_launch("wave_ds_kernel");
+}
+
+template <typename T, int MT, int DT, bool SEP>
+int semi_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk, int64_t block,
+            hipStream_t st) {
+    typedef StepRows<T, DT, SEP ? 3 : 2> Rows;
+    const int NW = (int)((M + 16 * MT - 1) / (16 * MT));
+    const int64_t NC = (N + chunk - 1) / chunk;
+    const dim3 grid((unsigned)NC, (unsigned)(B * H));
+    int rc = launch_lse<T, DT>(p, B, N, H, M, scale, st);
+    if (rc) return rc;
+    const size_t walk_lds = 2 * Rows::BYTES + 2 * NW * TT * sizeof(float);
+    hipLaunchKernelGGL((wave_semi_gz_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), walk_lds, st, p, (int)N, (int)H,
+                       (int)M, scale, (int)chunk, (int)block);
+    if ((rc = check_launch("wave_semi_gz_kernel"))) return rc;
+    if ((rc = launch_carry(p, NC, M, 16 * DT, B * H * M, st))) return rc;
+    const size_t lds = sizeof(float) * (size_t)NW * semi_wave_floats<MT, DT>() + Rows::BYTES;
+    if ((rc = allow_lds((const void*)wave_semi_ds_kernel<T, MT, DT, SEP>, lds, "wave_semi_ds_kernel"))) return rc;
+    hipLaunchKernelGGL((wave_semi_ds_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), lds, st, p, (int)N, (int)H, (int)M, scale,
+                       (int)chunk, (int)block);
+    return check_launch("wave_semi_ds_kernel");
 }
 
 template <typename T, int DT>
@@ -53,6 +87,14 @@ int bwd_dt(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t 
     constexpr int MT = bwd_tiles<DT>();
     return sep ? bwd_at<T, MT, DT, true>(p, B, N, H, M, scale, chunk, st)
                : bwd_at<T, MT, DT, false>(p, B, N, H, M, scale, chunk, st);
+}
+
+template <typename T, int DT>
+int semi_dt(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk,
+            int64_t block, hipStream_t st) {
+    constexpr int MT = bwd_tiles<DT>();
+    return sep ? semi_at<T, MT, DT, true>(p, B, N, H, M, scale, chunk, block, st)
+               : semi_at<T, MT, DT, false>(p, B, N, H, M, scale, chunk, block, st);
 }
 
 template <typename T, int DT>
@@ -102,6 +144,12 @@ template <typename T>
 int bwd_type(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale,
              int64_t chunk, hipStream_t st) {
     FLARE_WAVE_DT_CASES(bwd_dt, p, sep, B, N, H, M, scale, chunk, st)
+}
+
+template <typename T>
+int semi_type(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale,
+              int64_t chunk, int64_t block, hipStream_t st) {
+    FLARE_WAVE_DT_CASES(semi_dt, p, sep, B, N, H, M, scale, chunk, block, st)
 }
 
 }  // namespace wave

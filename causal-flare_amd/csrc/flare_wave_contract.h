@@ -86,7 +86,7 @@ __global__ __launch_bounds__(256) void wave_rows_kernel(ContractPtrs p, const T*
             for (int dt = 0; dt < DT; ++dt) {
                 const auto op = q.op(dt);
 #pragma unroll
-                for (int k = 0; k < kRowTiles; ++k) acc[k][dt] = mm(f[k], op, acc[k][dt]);
+                for (int k = 0; k < kRowTiles; ++k) acc[k][dt] = collect(f[k], op, acc[k][dt]);
             }
         }
     }
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void wave_cols_kernel(ContractPtrs p, const T*
             for (int dt = 0; dt < DT; ++dt) {
                 const auto op = k.op(dt);
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) acc[mt][dt] = mm(op, f[mt], acc[mt][dt]);
+                for (int mt = 0; mt < MT; ++mt) acc[mt][dt] = collect(op, f[mt], acc[mt][dt]);
             }
         }
     }
