@@ -219,8 +219,11 @@ bool wave_aligned(std::initializer_list<const void*> ptrs) {
         if (((uintptr_t)p & 15) != 0) return false;
     return true;
 }
-static bool wave_supported(int64_t M, int64_t Dk, int64_t Dv, int64_t chunk, std::initializer_list<const void*> ptrs) {
-    return wave_shape(M, Dk, Dv) && chunk % 16 == 0 && wave_aligned(ptrs);
+// (a chunk's rows are reached by 31-bit byte offsets from its first token)
+static bool wave_supported(int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv, int64_t chunk,
+                           std::initializer_list<const void*> ptrs) {
+    return wave_shape(M, Dk, Dv) && chunk % 16 == 0 && (chunk < N ? chunk : N) * H * Dv * 4 < (int64_t)1 << 31 &&
+           wave_aligned(ptrs);
 }
 
 static int launch_prepare(const void* Q, const void* K, const void* V, int dtype, int64_t B,
@@ -239,7 +242,7 @@ static int launch_prepare(const void* Q, const void* K, const void* V, int dtype
             return launch_prepare_mfma(Q, K, V, B, N, H, M, Dk, scale, chunk, cmax, cden, cnum, dtype == FLARE_F16,
                                        stream);
     }
-    if (power <= 0.0f && (mfma_phase_mask() & 1) && wave_supported(M, Dk, Dv, chunk, {Q, K, V, cnum})) {
+    if (power <= 0.0f && (mfma_phase_mask() & 1) && wave_supported(N, H, M, Dk, Dv, chunk, {Q, K, V, cnum})) {
         const WaveArgs a{Q, K, V, nullptr, nullptr, B, N, H, M, Dk, scale, chunk, tmask};
         return dtype == FLARE_BF16  ? wave::prepare_bf16(a, cmax, cden, cnum, stream)
                : dtype == FLARE_F16 ? wave::prepare_f16(a, cmax, cden, cnum, stream)
@@ -363,7 +366,7 @@ static int launch_output(const void* Q, const void* K, const void* V, const void
         }
     }
     if (power <= 0.0f && (mfma_phase_mask() & 2) && lse_dec == nullptr &&
-        wave_supported(M, Dk, Dv, chunk, {Q, K, V, Qdec, Kdec, pnum, Y})) {
+        wave_supported(N, H, M, Dk, Dv, chunk, {Q, K, V, Qdec, Kdec, pnum, Y})) {
         const WaveArgs a{Q, K, V, Qdec, Kdec, B, N, H, M, Dk, scale, chunk, tmask};
         return dtype == FLARE_BF16  ? wave::output_bf16(a, pmax, pden, pnum, Y, out_dtype, stream)
                : dtype == FLARE_F16 ? wave::output_f16(a, pmax, pden, pnum, Y, out_dtype, stream)

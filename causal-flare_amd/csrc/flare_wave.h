@@ -19,13 +19,14 @@
 //   m straight from the scores' registers, G over tau straight from its own.  Only E of the
 //   U update needs the other orientation; it crosses through a wave-private LDS tile.
 //
-// What bounds it: the fp32 MFMA.  A 64 x 32 bank issues 88 of them a 16-token tile and wave
-// in phase 3 (2,816 cycles of its SIMD's matrix pipe) against about 1,300 cycles of vector
-// instructions.  Measured on MI355X, whole forward, tokenwise kernels -> these:
-//   bf16 B 8, N 4096, H 16, M 64, D 32     4937 -> 174 us (prepare 41, scan 7, output 139)
-//   fp16 B 3, N 1531, H 8, M 96, D 64, cached state and mask   1135 -> 136 us
-//   fp32 B 1, N 256, H 8, M 64, D 32        283 ->  31 us
-// Errors against 64 bits: fp32 outputs 2.5e-7 -> 1.4e-7, 16-bit ones unchanged.
+// What bounds it: the fp32 MFMA and the vector instructions together, which two waves a SIMD
+// hardly overlap.  A 64 x 32 bank issues 88 MFMAs a 16-token tile and wave in phase 3 (2,816
+// cycles of its SIMD's matrix pipe, busy 40% of the kernel) and about 880 vector instructions
+// (52%).  Measured on MI355X, whole forward, tokenwise kernels -> these:
+//   bf16 B 8, N 4096, H 16, M 64, D 32     4937 -> 158 us (prepare 41, scan 7, output 124)
+//   fp16 B 3, N 1531, H 8, M 96, D 64, cached state and mask   1135 -> 124 us
+//   fp32 B 1, N 256, H 8, M 64, D 32        283 ->  30 us
+// Errors against 64 bits: fp32 outputs 2.5e-7 -> 1.1e-7, 16-bit ones unchanged.
 #pragma once
 
 #include "flare_common.h"
@@ -48,6 +49,35 @@ typedef float f32x4_a __attribute__((ext_vector_type(4), may_alias));
 typedef mfma::bf16 bf16x8_a __attribute__((ext_vector_type(8), may_alias));
 
 constexpr int TT = 16;              // tokens per tile
+
+// An array through a buffer descriptor: loads past its end read 0 and stores there are
+// dropped, so edge tokens need no branches and no clamped addresses, and a lane's address is
+// one 32-bit offset.  (A branch per element split the tile into some 130 blocks that nothing
+// could be scheduled across: 144 us for phase 3 of the narrow bank above.)
+constexpr unsigned kNowhere = 0x80000000u;                          // byte offset past every array
+struct Bytes {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Bytes(const void* p, size_t n)
+        : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)n, 0x00020000)) {}
+    __device__ __forceinline__ u32x4 b128(unsigned at) const {
+        return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
+    }
+    __device__ __forceinline__ u32x2 b64(unsigned at) const {
+        return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, at, 0, 0));
+    }
+    __device__ __forceinline__ unsigned b32(unsigned at) const { return __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0); }
+    __device__ __forceinline__ unsigned b16(unsigned at) const {
+        return (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, at, 0, 0);
+    }
+    __device__ __forceinline__ void put128(unsigned at, u32x4 x) const {
+        __builtin_amdgcn_raw_buffer_store_b128(x, r, at, 0, 0);
+    }
+    __device__ __forceinline__ void put64(unsigned at, u32x2 x) const { __builtin_amdgcn_raw_buffer_store_b64(x, r, at, 0, 0); }
+    __device__ __forceinline__ void put32(unsigned at, unsigned x) const { __builtin_amdgcn_raw_buffer_store_b32(x, r, at, 0, 0); }
+    __device__ __forceinline__ void put16(unsigned at, unsigned x) const {
+        __builtin_amdgcn_raw_buffer_store_b16((unsigned short)x, r, at, 0, 0);
+    }
+};
 // A latent's max may rise by this much (nats) inside a tile before the tile runs token by
 // token: below it every den and weight of the tile keeps full fp32 precision against the
 // tile's max (e^-60 is far above the fp32 underflow).
@@ -76,9 +106,18 @@ struct RowOp {   // 16-bit: steps of 32 columns, 8 a lane group; a last step of 
             }
         }
     }
-    __device__ __forceinline__ void zero() {
+    // byte offset of this lane within a row, and the load from it
+    static __device__ __forceinline__ unsigned lane(int g) { return 16 * g; }
+    __device__ __forceinline__ void load(const Bytes& b, unsigned row, int g) {
 #pragma unroll
-        for (int s = 0; s < S; ++s) a[s] = bf16x8{};
+        for (int s = 0; s < S; ++s) {
+            if (32 * s + 32 <= D) {
+                a[s] = __builtin_bit_cast(bf16x8, b.b128(row + 64 * s));
+            } else {
+                // the groups past the row read nowhere: zeros
+                a[s] = __builtin_bit_cast(bf16x8, b.b128(g < 2 ? row + 64 * s : kNowhere));
+            }
+        }
     }
 };
 template <int D>
@@ -88,9 +127,10 @@ struct RowOp<float, D> {   // lane group g holds columns [g D/4, (g+1) D/4)
 #pragma unroll
         for (int s = 0; s < D / 16; ++s) a[s] = *reinterpret_cast<const f32x4_a*>(row + g * (D / 4) + 4 * s);
     }
-    __device__ __forceinline__ void zero() {
+    static __device__ __forceinline__ unsigned lane(int g) { return g * D; }
+    __device__ __forceinline__ void load(const Bytes& b, unsigned row, int) {
 #pragma unroll
-        for (int s = 0; s < D / 16; ++s) a[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < D / 16; ++s) a[s] = __builtin_bit_cast(f32x4, b.b128(row + 16 * s));
     }
 };
 
@@ -170,6 +210,29 @@ struct ColRow {
             w[at] = *reinterpret_cast<const u16_a*>(p);
         }
     }
+    // the same from a buffer: `row` is the row's byte offset
+    __device__ __forceinline__ void load(const Bytes& b, unsigned row, int c) {
+#pragma unroll
+        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
+            const int P = piece_of<DT>(dt), E = (int)sizeof(T);
+            const unsigned at = row + c * (P * E) + 16 * dt * E;
+            const int k = sizeof(T) == 4 ? dt : dt / 2;
+            if (P * E == 16) {
+                const u32x4 x = b.b128(at);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (k + j < W) w[k + j] = x[j];
+            } else if (P * E == 8) {
+                const u32x2 x = b.b64(at);
+                w[k] = x[0];
+                if (k + 1 < W) w[k + 1] = x[1];
+            } else if (P * E == 4) {
+                w[k] = b.b32(at);
+            } else {
+                w[k] = b.b16(at);
+            }
+        }
+    }
     __device__ __forceinline__ float get(int dt) const {
         if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, w[dt]);
         else return word_f32<T>(w[dt / 2], dt & 1);
@@ -209,6 +272,9 @@ __device__ __forceinline__ float group_sum(float x) {
 
 __device__ __forceinline__ float exp_nat(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 __device__ __forceinline__ float safe_ref(float m) { return m == kNegInf ? 0.0f : m; }
+// A reference of -inf (no token yet, every score -inf) counts as this, so that -inf - ref is
+// -inf and not NaN; and a den of 0 (then U is 0 as well) as this.
+constexpr float kLowRef = -1e38f, kTinyDen = 1e-37f;
 
 // Writes by other lanes of the wave to LDS are visible after this (a wave's LDS
 // operations complete in order; the fence keeps the compiler from reordering them).
@@ -226,6 +292,9 @@ template <typename T, int DT, bool SEP>
 constexpr bool latents_in_regs() { return sizeof(T) == 2 ? (DT <= 6 || !SEP) : (DT <= 3 || (DT == 4 && !SEP)); }
 template <int DT>
 constexpr bool fetch_ahead() { return DT <= 4; }
+// Largest workgroup: M <= 256, and waves of 16 latents only up to M = 128 (a workgroup of 16
+// waves would halve their registers).
+__host__ __device__ constexpr int wave_threads(int MT) { return MT == 4 ? 256 : 512; }
 
 // ---------------------------------------------------------------------------
 // Phase 1: the summary (max, den, num) of one chunk.  grid = (NC, B*H), one wave per
@@ -234,7 +303,7 @@ constexpr bool fetch_ahead() { return DT <= 4; }
 // it with per-lane factors.
 // ---------------------------------------------------------------------------
 template <typename T, int MT, int DT>
-__global__ __launch_bounds__(64 * (16 / MT)) void wave_prepare_kernel(
+__global__ __launch_bounds__(wave_threads(MT)) void wave_prepare_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, int N, int H, int M, float scale,
     int chunk, float* __restrict__ cmax, float* __restrict__ cden, float* __restrict__ cnum,
     const int32_t* __restrict__ tmask) {
@@ -246,10 +315,9 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_prepare_kernel(
 
     constexpr bool QREG = latents_in_regs<T, DT, false>(), AHEAD = fetch_ahead<DT>();
     RowOp<T, D> q[QREG ? MT : 1];
-    auto load_q = [&](RowOp<T, D>& r, int mt) {
-        const int m = mb + 16 * mt + c;
-        if (m < M) r.load(Q + ((size_t)h * M + m) * D, g);
-        else r.zero();
+    const Bytes qb(Q + (size_t)h * M * D, (size_t)M * D * sizeof(T));
+    auto load_q = [&](RowOp<T, D>& r, int mt) {                  // past the bank: zeros
+        r.load(qb, (mb + 16 * mt + c) * (D * (int)sizeof(T)) + RowOp<T, D>::lane(g), g);
     };
     if constexpr (QREG) {
 #pragma unroll
@@ -265,36 +333,40 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_prepare_kernel(
         for (int dt = 0; dt < DT; ++dt) u[mt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
+    // the chunk's rows of this head, by byte offset from its first token
     const int t0 = ch * chunk, t1 = min(N, t0 + chunk);
-    const size_t stride = (size_t)H * D;
-    const T* kb = K + ((size_t)b * N * H + h) * D;
-    const T* vb = V + ((size_t)b * N * H + h) * D;
+    const unsigned stride = (unsigned)(H * D) * sizeof(T);
+    const size_t first = (((size_t)b * N + t0) * H + h) * D;
+    const size_t span = (size_t)(t1 - t0 - 1) * stride + D * sizeof(T);
+    const Bytes kb(K + first, span), vb(V + first, span);
+    unsigned krow = c * stride + RowOp<T, D>::lane(g), vrow = 4 * g * stride;
     RowOp<T, D> kn;
     ColRow<T, DT> vn[4];
-    auto fetch = [&](int t) {
-        kn.load(kb + (size_t)min(t + c, t1 - 1) * stride, g);
+    auto fetch = [&]() {                                          // (past the chunk: zeros)
+        kn.load(kb, krow, g);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) vn[i].load(vb + (size_t)min(t + 4 * g + i, t1 - 1) * stride, c);
+        for (int i = 0; i < 4; ++i) vn[i].load(vb, vrow + i * stride, c);
+        krow += TT * stride;
+        vrow += TT * stride;
     };
-    if constexpr (AHEAD) fetch(t0);
+    if constexpr (AHEAD) fetch();
     for (int t = t0; t < t1; t += TT) {
-        if constexpr (!AHEAD) fetch(t);
+        if constexpr (!AHEAD) fetch();
         const RowOp<T, D> k = kn;
         float v[4][DT];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) v[i][dt] = vn[i].get(dt);
-        if constexpr (AHEAD) {
-            if (t + TT < t1) fetch(t + TT);
-        }
-        bool ok[4] = {true, true, true, true};     // token t + 4g + i takes part
-        const bool part = t + TT > t1 || tmask != nullptr;
-        if (part) {
+        if constexpr (AHEAD) fetch();
+        bool ok[4];                                               // token t + 4g + i takes part
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ok[i] = t + 4 * g + i < t1;
+        if (tmask != nullptr) {
+            // (a masked token's value may be anything: it must not meet a weight of zero)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int ti = t + 4 * g + i;
-                ok[i] = ti < t1 && (tmask == nullptr || tmask[(size_t)b * N + ti] != 0);
+                ok[i] = ok[i] && tmask[(size_t)b * N + min(t + 4 * g + i, t1 - 1)] != 0;
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) v[i][dt] = ok[i] ? v[i][dt] : 0.0f;
             }
@@ -397,6 +469,26 @@ __device__ __forceinline__ void store_cols(void* Y, size_t idx, const float* x, 
     }
 }
 
+// the same to a buffer, at byte offset `at`
+__device__ __forceinline__ void put_cols(const Bytes& y, unsigned at, const float (&x)[4], int P, int out_dtype) {
+    if (out_dtype == FLARE_F32) {
+        const u32x4 r = {__builtin_bit_cast(u32, x[0]), __builtin_bit_cast(u32, x[1]), __builtin_bit_cast(u32, x[2]),
+                         __builtin_bit_cast(u32, x[3])};
+        if (P == 4) y.put128(at, r);
+        else if (P == 2) y.put64(at, u32x2{r[0], r[1]});
+        else y.put32(at, r[0]);
+    } else {
+        u32 h[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            h[k] = out_dtype == FLARE_BF16 ? __builtin_bit_cast(unsigned short, (mfma::bf16)x[k])
+                                           : __builtin_bit_cast(unsigned short, (mfma::f16)x[k]);
+        if (P == 4) y.put64(at, u32x2{h[0] | h[1] << 16, h[2] | h[3] << 16});
+        else if (P == 2) y.put32(at, h[0] | h[1] << 16);
+        else y.put16(at, h[0]);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Phase 3: replay of one chunk from its exclusive prefix, and the readout.
 // grid = (NC, B*H), one wave per MT*16 latents (NW = blockDim.x / 64 waves).
@@ -408,10 +500,11 @@ __device__ __forceinline__ void store_cols(void* Y, size_t idx, const float* x, 
 // One wave: W takes the softmax sum at once.  Several: each wave writes its y, max and sum
 // to LDS and the workgroup merges them (the token softmax over waves), double-buffered.
 //
-// A tile in which some latent's max rises by more than kTileJump, whose V holds a
-// non-finite value, or whose first token has no finite reference near the tile's max, runs
-// token by token: the same body with every other token masked, 16 times.  Each pass moves
-// the reference exactly to its token, as the tokenwise recurrence does.
+// j < 0: the whole tile.  A tile in which some latent's max rises by more than kTileJump, whose
+// V holds a non-finite value, or whose first token has no finite reference near the tile's max,
+// is walked token by token (j = the token, the loop comes back with the same tile): the same
+// body with every other token masked, so that the reference moves exactly to each token, as in
+// the tokenwise recurrence.
 // ---------------------------------------------------------------------------
 template <int MT, int DT>
 __host__ __device__ constexpr int e_pitch() { return 16 * MT + 4; }
@@ -422,7 +515,7 @@ inline size_t wave_output_lds(int NW) {
 }
 
 template <typename T, int MT, int DT, bool SEP>
-__global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
+__global__ __launch_bounds__(wave_threads(MT)) void wave_output_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V, const T* __restrict__ Qdec,
     const T* __restrict__ Kdec, int N, int H, int M, float scale, int chunk, const float* __restrict__ pmax,
     const float* __restrict__ pden, const float* __restrict__ pnum, void* __restrict__ Y, int out_dtype,
@@ -441,60 +534,68 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
 
     constexpr bool QREG = latents_in_regs<T, DT, SEP>(), AHEAD = fetch_ahead<DT>();
     RowOp<T, D> q[QREG ? MT : 1], kd[SEP && QREG ? MT : 1];
-    auto load_latent = [&](RowOp<T, D>& r, const T* base, int mt) {
-        const int m = mb + 16 * mt + c;
-        if (m < M) r.load(base + ((size_t)h * M + m) * D, g);
-        else r.zero();
+    const size_t bank = (size_t)M * D;
+    const Bytes qbank(Q + h * bank, bank * sizeof(T)), kbank(SEP ? Kdec + h * bank : Q, SEP ? bank * sizeof(T) : 0);
+    auto load_latent = [&](RowOp<T, D>& r, const Bytes& from, int mt) {          // past the bank: zeros
+        r.load(from, (mb + 16 * mt + c) * (D * (int)sizeof(T)) + RowOp<T, D>::lane(g), g);
     };
     if constexpr (QREG) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            load_latent(q[mt], Q, mt);
-            if constexpr (SEP) load_latent(kd[mt], Kdec, mt);
+            load_latent(q[mt], qbank, mt);
+            if constexpr (SEP) load_latent(kd[mt], kbank, mt);
         }
     }
     // latent mb + 16 mt + 4g + i: max, den (the same in the 16 lanes of a row), U row
     float mx[MT][4], den[MT][4];
     f32x4 u[MT][DT];
-    const size_t pbase = ((size_t)bh * NC + ch) * M;
+    {
+        const size_t pbase = ((size_t)bh * NC + ch) * M;
+        const Bytes pm(pmax + pbase, 4 * (size_t)M), pd(pden + pbase, 4 * (size_t)M), pn(pnum + pbase * D, 4 * bank);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int m = mb + 16 * mt + 4 * g + i;
-            mx[mt][i] = m < M ? pmax[pbase + m] : kNegInf;
-            den[mt][i] = m < M ? pden[pbase + m] : 0.0f;
-            ColRow<float, DT> r;
-            if (m < M) r.load(pnum + (pbase + m) * D, c);
+            for (int i = 0; i < 4; ++i) {
+                const int m = mb + 16 * mt + 4 * g + i;
+                const float x = __builtin_bit_cast(float, pm.b32(4 * m));
+                mx[mt][i] = m < M ? x : kNegInf;
+                den[mt][i] = __builtin_bit_cast(float, pd.b32(4 * m));
+                ColRow<float, DT> r;
+                r.load(pn, m * (4 * D), c);
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) u[mt][dt][i] = m < M ? r.get(dt) : 0.0f;
-        }
+                for (int dt = 0; dt < DT; ++dt) u[mt][dt][i] = r.get(dt);
+            }
+    }
 
+    // the chunk's rows of this head, by byte offset from its first token
     const int t0 = ch * chunk, t1 = min(N, t0 + chunk);
-    const size_t stride = (size_t)H * D;
-    const T* kb = K + ((size_t)b * N * H + h) * D;
-    const T* vb = V + ((size_t)b * N * H + h) * D;
-    const T* qb = SEP ? Qdec + ((size_t)b * N * H + h) * D : nullptr;
+    const unsigned stride = (unsigned)(H * D) * sizeof(T);
+    const size_t first = (((size_t)b * N + t0) * H + h) * D;
+    const size_t span = (size_t)(t1 - t0 - 1) * stride + D * sizeof(T);
+    const Bytes kb(K + first, span), vb(V + first, span), qb(SEP ? Qdec + first : K, SEP ? span : 0);
+    const int osize = out_dtype == FLARE_F32 ? 4 : 2;
+    const unsigned ostride = (unsigned)(H * D) * osize;
+    const Bytes yb((const char*)Y + first * osize, (size_t)(t1 - t0 - 1) * ostride + D * osize);
+    unsigned krow = c * stride + RowOp<T, D>::lane(g), vrow = 4 * g * stride;
     RowOp<T, D> kn, qn;
     ColRow<T, DT> vn[4];
-    auto fetch = [&](int t) {
-        kn.load(kb + (size_t)min(t + c, t1 - 1) * stride, g);
-        if constexpr (SEP) qn.load(qb + (size_t)min(t + c, t1 - 1) * stride, g);
+    auto fetch = [&]() {                                // (past the chunk: zeros)
+        kn.load(kb, krow, g);
+        if constexpr (SEP) qn.load(qb, krow, g);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) vn[i].load(vb + (size_t)min(t + 4 * g + i, t1 - 1) * stride, c);
+        for (int i = 0; i < 4; ++i) vn[i].load(vb, vrow + i * stride, c);
     };
-    if constexpr (AHEAD) fetch(t0);
-    int buf = 0;
-    for (int t = t0; t < t1; t += TT) {
-        if constexpr (!AHEAD) fetch(t);
+    fetch();
+    int buf = 0, t = t0, j = -1;
+    while (true) {
         // scores^T, then the next tile's loads
         f32x4 s[MT], p[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            if constexpr (!QREG) load_latent(q[0], Q, mt);
+            if constexpr (!QREG) load_latent(q[0], qbank, mt);
             s[mt] = dot_rows<T, D>(q[QREG ? mt : 0], kn, f32x4{0.f, 0.f, 0.f, 0.f});
             if constexpr (SEP) {
-                if constexpr (!QREG) load_latent(kd[0], Kdec, mt);
+                if constexpr (!QREG) load_latent(kd[0], kbank, mt);
                 p[mt] = dot_rows<T, D>(kd[QREG ? mt : 0], qn, f32x4{0.f, 0.f, 0.f, 0.f});
             }
         }
@@ -507,50 +608,95 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
                 v[i][dt] = vn[i].get(dt);
                 vbad = __builtin_fmaf(v[i][dt], 0.0f, vbad);
             }
-        if constexpr (AHEAD) {
-            if (t + TT < t1) fetch(t + TT);
-        }
-
-        bool live = true;                              // token t + c takes part
-        if (t + TT > t1 || tmask != nullptr)
-            live = t + c < t1 && (tmask == nullptr || tmask[(size_t)b * N + t + c] != 0);
+        bool live = t + c < t1;                        // token t + c takes part
+        if (tmask != nullptr) live = live && tmask[(size_t)b * N + min(t + c, t1 - 1)] != 0;
         const unsigned lmask = (unsigned)(__ballot(live) & 0xffffu);   // the 16 tokens, wave-uniform
-        const int first = lmask ? __builtin_ctz(lmask) : 0;
-
-        float top[MT][4];
-        bool slow = vbad != vbad, bare = false;
-        float wmax = kNegInf;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const bool in = live && mb + 16 * mt + 4 * g + i < M;
-                s[mt][i] = in ? s[mt][i] * scale : kNegInf;
-                if constexpr (SEP) p[mt][i] = in ? p[mt][i] * scale : kNegInf;
+                s[mt][i] *= scale;
+                if constexpr (SEP) p[mt][i] *= scale;
                 else p[mt][i] = s[mt][i];
-                wmax = fmaxf(wmax, p[mt][i]);
-                top[mt][i] = mfma::row_max16(s[mt][i]);
-                if (mb + 16 * mt + 4 * g + i < M) {
-                    slow |= top[mt][i] - mx[mt][i] > kTileJump && mx[mt][i] != kNegInf;
-                    bare |= mx[mt][i] == kNegInf;
-                }
             }
-        if (__any(bare)) {
-            // no earlier token: the tile's first live token is the lowest reference
+        if (mb + 16 * MT > M) {                        // this wave's share ends past the bank
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float s0 = __shfl(s[mt][i], (lane & 48) | first, 64);
-                    if (mb + 16 * mt + 4 * g + i < M && mx[mt][i] == kNegInf)
-                        slow |= !(top[mt][i] - s0 <= kTileJump) && top[mt][i] != kNegInf;
+                    const bool out = mb + 16 * mt + 4 * g + i >= M;
+                    s[mt][i] = out ? kNegInf : s[mt][i];
+                    p[mt][i] = out ? kNegInf : p[mt][i];
                 }
         }
-        // decoder weights of this wave's latents
+        // the tokens of this pass: the others score -inf and hold no value
+        auto keep = [&](unsigned take) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[mt][i] = (take >> c) & 1 ? s[mt][i] : kNegInf;
+                    p[mt][i] = (take >> c) & 1 ? p[mt][i] : kNegInf;
+                }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) v[i][dt] = (take >> (4 * g + i)) & 1 ? v[i][dt] : 0.0f;
+        };
+        if (j < 0 && __any(vbad != vbad) && lmask != 0) j = __builtin_ctz(lmask);
+        if (j >= 0) keep(1u << j);
+        else if (lmask != 0xffffu) keep(lmask);
+
+        bool moved = false;                            // a score passes its latent's max
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) moved |= s[mt][i] > mx[mt][i];
+        if (__any(moved)) {
+            float top[MT][4], rise = 0.0f;             // rise: the largest move of a reference in the tile
+            const int first = lmask ? __builtin_ctz(lmask) : 0;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    top[mt][i] = mfma::row_max16(s[mt][i]);
+                    // (no earlier token: from the tile's first live one)
+                    const float low = mx[mt][i] == kNegInf ? __shfl(s[mt][i], (lane & 48) | first, 64) : mx[mt][i];
+                    const float up = top[mt][i] == kNegInf ? 0.0f : top[mt][i] - low;
+                    rise = fmaxf(rise, up == up ? up : 2.0f * kTileJump);
+                }
+            if (j < 0 && __any(rise > kTileJump)) {
+                j = first;
+                keep(1u << j);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) top[mt][i] = mfma::row_max16(s[mt][i]);
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float mnew = fmaxf(mx[mt][i], top[mt][i]);
+                    const float r = mx[mt][i] == mnew ? 1.0f : mx[mt][i] == kNegInf ? 0.0f : exp_nat(mx[mt][i] - mnew);
+                    den[mt][i] *= r;
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) u[mt][dt][i] *= r;
+                    mx[mt][i] = mnew;
+                }
+        }
+        // this pass's output rows (masked tokens come with the first one), and the tokens left
+        const unsigned take = j < 0 ? lmask : 1u << j;
+        const unsigned rows = j < 0 ? 0xffffu : j == __builtin_ctz(lmask) ? take | (~lmask & 0xffffu) : take;
+        const unsigned after = j < 0 ? 0u : lmask & ~((2u << j) - 1u);
+
+        // decoder weights of this wave's latents (a masked token's scores are -inf: weights 0)
+        float wmax = kNegInf, psum = 0.0f;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) wmax = fmaxf(fmaxf(wmax, fmaxf(p[mt][0], p[mt][1])), fmaxf(p[mt][2], p[mt][3]));
         wmax = group_max(wmax);
-        float psum = 0.0f;
         {
-            const float ref = safe_ref(wmax);
+            const float ref = fmaxf(wmax, kLowRef);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -560,121 +706,78 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
                 }
         }
         psum = group_sum(psum);
-        if (NW == 1) {
-            const float inv = psum > 0.0f ? 1.0f / psum : 0.0f;
+        const float norm = NW > 1 ? 1.0f : psum > 0.0f ? 1.0f / psum : psum;       // (a NaN stays one)
+        f32x4 e[MT], wt[MT];
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) p[mt][i] *= inv;
+            for (int i = 0; i < 4; ++i) {
+                e[mt][i] = exp_nat(s[mt][i] - fmaxf(mx[mt][i], kLowRef));
+                const float d = den[mt][i] + mfma::row_scan16(e[mt][i]);
+                wt[mt][i] = p[mt][i] * norm * __builtin_amdgcn_rcpf(fmaxf(d, kTinyDen));
+                den[mt][i] = mfma::row_bcast15(d);
+            }
+            *reinterpret_cast<f32x4_a*>(etile + c * EP + 16 * mt + 4 * g) = e[mt];
         }
-        if (lmask != 0xffffu) {
+        wave_lds_sync();
+        // the next tile's rows, once this one has no further pass
+        if (AHEAD && after == 0) {
+            krow += TT * stride;
+            vrow += TT * stride;
+            fetch();
+        }
+        // G^T [tau][t], masked to tau <= t
+        f32x4 ga = {0.f, 0.f, 0.f, 0.f}, gb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            ga = mma4(e[mt][0], wt[mt][0], ga);
+            gb = mma4(e[mt][1], wt[mt][1], gb);
+            ga = mma4(e[mt][2], wt[mt][2], ga);
+            gb = mma4(e[mt][3], wt[mt][3], gb);
+        }
+        f32x4 y[DT];
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) y[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt) v[i][dt] = (lmask >> (4 * g + i)) & 1 ? v[i][dt] : 0.0f;
+                for (int dt = 0; dt < DT; ++dt) y[dt] = mma4(wt[mt][i], u[mt][dt][i], y[dt]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float gm = 4 * g + i <= c ? ga[i] + gb[i] : 0.0f;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) y[dt] = mma4(gm, v[i][dt], y[dt]);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const float ea = etile[(4 * g + i) * EP + 16 * mt + c];
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) u[mt][dt] = mma4(ea, v[i][dt], u[mt][dt]);
+            }
         }
-
-        const bool step = __any(slow);
-        unsigned rest = lmask;                         // tokens still to be taken
-        unsigned rows = ~lmask & 0xffffu;              // output rows of this pass; masked ones come with the first
-        do {
-            // all live tokens at once, or the lowest one left
-            const unsigned take = step ? rest & -rest : rest;
-            rest &= ~take;
-            rows |= take;
-            f32x4 y[DT];
+        wave_lds_sync();
+        if (NW == 1) {
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) y[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-            const bool on = (take >> c) & 1;
-            f32x4 e[MT], wt[MT];
-            bool moved = false;
-            float mnew[MT][4];
+            for (int i = 0; i < 4; ++i) {
+                const unsigned row = (rows >> (4 * g + i)) & 1 ? (unsigned)(t - t0 + 4 * g + i) * ostride : kNowhere;
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+                for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
+                    float o[4];
+                    const int P = piece_of<DT>(dt);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float tm = step ? __shfl(s[mt][i], (lane & 48) | (__builtin_ctz(take | 0x10000u) & 15), 64)
-                                          : top[mt][i];
-                    mnew[mt][i] = take ? fmaxf(mx[mt][i], tm) : mx[mt][i];
-                    moved |= mnew[mt][i] != mx[mt][i];
+                    for (int k = 0; k < 4; ++k) o[k] = k < P ? y[dt + k < DT ? dt + k : 0][i] : 0.0f;
+                    put_cols(yb, row + col_of<DT>(dt, c) * osize, o, P, out_dtype);
                 }
-            if (__any(moved)) {
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float r = mx[mt][i] == mnew[mt][i] ? 1.0f
-                                        : mx[mt][i] == kNegInf   ? 0.0f
-                                                                 : exp_nat(mx[mt][i] - mnew[mt][i]);
-                        den[mt][i] *= r;
-#pragma unroll
-                        for (int dt = 0; dt < DT; ++dt) u[mt][dt][i] *= r;
-                        mx[mt][i] = mnew[mt][i];
-                    }
             }
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float x = exp_nat(s[mt][i] - safe_ref(mx[mt][i]));
-                    e[mt][i] = on ? x : 0.0f;
-                    const float d = den[mt][i] + mfma::row_scan16(e[mt][i]);
-                    const float wv = p[mt][i] * __builtin_amdgcn_rcpf(d > 0.0f ? d : 1.0f);
-                    wt[mt][i] = on ? wv : 0.0f;
-                    den[mt][i] = mfma::row_bcast15(d);
-                }
-                *reinterpret_cast<f32x4_a*>(etile + c * EP + 16 * mt + 4 * g) = e[mt];
-            }
-            wave_lds_sync();
-            // G^T [tau][t], masked to tau <= t
-            f32x4 ga = {0.f, 0.f, 0.f, 0.f}, gb = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                ga = mma4(e[mt][0], wt[mt][0], ga);
-                gb = mma4(e[mt][1], wt[mt][1], gb);
-                ga = mma4(e[mt][2], wt[mt][2], ga);
-                gb = mma4(e[mt][3], wt[mt][3], gb);
-            }
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+        } else {
+            float* yw = ypart + ((size_t)buf * NW + w) * TT * D;
+            if (j < 0) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int dt = 0; dt < DT; ++dt) y[dt] = mma4(wt[mt][i], u[mt][dt][i], y[dt]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float gm = 4 * g + i <= c ? ga[i] + gb[i] : 0.0f;
-                const bool von = !step || ((take >> (4 * g + i)) & 1);
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) y[dt] = mma4(gm, von ? v[i][dt] : 0.0f, y[dt]);
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    const float ea = etile[(4 * g + i) * EP + 16 * mt + c];
-#pragma unroll
-                    for (int dt = 0; dt < DT; ++dt) u[mt][dt] = mma4(ea, von ? v[i][dt] : 0.0f, u[mt][dt]);
-                }
-            }
-            wave_lds_sync();
-            if (NW == 1) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int ti = t + 4 * g + i;
-                    if (ti >= t1 || !((rows >> (4 * g + i)) & 1)) continue;
-                    const size_t row = (((size_t)b * N + ti) * H + h) * D;
-#pragma unroll
-                    for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
-                        float o[4];
-                        const int P = piece_of<DT>(dt);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) o[j] = j < P ? y[(dt + j) < DT ? dt + j : 0][i] : 0.0f;
-                        const size_t at = row + col_of<DT>(dt, c);
-                        if (P == 4) store_cols<4>(Y, at, o, out_dtype);
-                        else if (P == 2) store_cols<2>(Y, at, o, out_dtype);
-                        else store_cols<1>(Y, at, o, out_dtype);
-                    }
-                }
+                    for (int dt = 0; dt < DT; ++dt) yw[(4 * g + i) * D + col_of<DT>(dt, c)] = y[dt][i];
             } else {
-                float* yw = ypart + ((size_t)buf * NW + w) * TT * D;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     if ((rows >> (4 * g + i)) & 1) {
@@ -682,15 +785,20 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
                         for (int dt = 0; dt < DT; ++dt) yw[(4 * g + i) * D + col_of<DT>(dt, c)] = y[dt][i];
                     }
             }
-            rows = 0;
-        } while (rest != 0);
-
+        }
         if (NW > 1) {
             float* sw = ystat + ((size_t)buf * NW + w) * 2 * TT;
-            if (g == 0) {
+            if (g == 0 && ((rows >> c) & 1)) {
                 sw[c] = wmax;
                 sw[TT + c] = psum;
             }
+        }
+        if (after != 0) {                              // this tile's next token
+            j = __builtin_ctz(after);
+            continue;
+        }
+        j = -1;
+        if (NW > 1) {
             __syncthreads();
             const float* yr = ypart + (size_t)buf * NW * TT * D;
             const float* sr = ystat + (size_t)buf * NW * 2 * TT;
@@ -706,15 +814,22 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_output_kernel(
                     sum += f * sr[k * 2 * TT + TT + ti];
                     const f32x4 yk = *reinterpret_cast<const f32x4_a*>(yr + ((size_t)k * TT + ti) * D + col);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[j] += f * yk[j];
+                    for (int n = 0; n < 4; ++n) acc[n] += f * yk[n];
                 }
                 const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
                 float o[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) o[j] = acc[j] * inv;
-                if (t + ti < t1) store_cols<4>(Y, (((size_t)b * N + t + ti) * H + h) * D + col, o, out_dtype);
+                for (int n = 0; n < 4; ++n) o[n] = acc[n] * inv;
+                put_cols(yb, (unsigned)(t - t0 + ti) * ostride + col * osize, o, 4, out_dtype);
             }
             buf ^= 1;
+        }
+        t += TT;
+        if (t >= t1) break;
+        if constexpr (!AHEAD) {
+            krow += TT * stride;
+            vrow += TT * stride;
+            fetch();
         }
     }
 }

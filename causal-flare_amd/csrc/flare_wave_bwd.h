@@ -306,10 +306,7 @@ __device__ __forceinline__ void stage() {
     if constexpr (DT > 4) __builtin_amdgcn_sched_barrier(0);
 }
 
-// fp32 array of one (b, h) through a buffer descriptor: loads past its end read 0 and stores
-// there are dropped, so edge tokens and masked latents need no branches (a branch per element
-// split the tile into some 80 blocks that nothing could be scheduled across).
-constexpr unsigned kNowhere = 0x80000000u;                          // byte offset past every array
+// fp32 array of one (b, h) through a buffer descriptor (see Bytes).
 struct Floats {
     __amdgpu_buffer_rsrc_t r;
     __device__ __forceinline__ Floats(const float* p, size_t n)

@@ -8,11 +8,20 @@
 namespace flare {
 namespace wave {
 
-// Latent tiles per wave.  Narrow banks (D <= 32) take 64 latents in one wave: the numerator
-// is then 32 registers or less, a 64-latent bank needs no second wave and no barrier, and V
-// is read once.  Wider ones keep 32 latents, for occupancy.
+// Latent tiles per wave, the chunk being set: the most that still leave a wave per SIMD (1024),
+// since fewer, larger waves repeat less (V, the y rows, G V); below that, smaller waves for a
+// shorter chain.  Narrow banks (D <= 32) go up to 64 latents, a 64-latent bank then needs no
+// second wave and no barrier; wider ones to 32, for registers.  Phase 3, us, with 64 / 32 / 16
+// latents a wave: bf16 B 8, N 4096, H 16, M 64, D 32 (2048 / 4096 / 8192 waves) 124 / 132 / 145;
+// fp32 B 2, N 1024, H 8, M 64, D 64 in chunks of 128 (256 / 512 waves of 32 / 16) 46 / 36.
+// 16 latents a wave only up to M = 128 (see wave_threads) and D = 64.
 template <int DT>
-constexpr int latent_tiles(int64_t M) { return DT <= 2 && M > 32 ? 4 : 2; }
+int latent_tiles(const WaveArgs& a) {
+    const int64_t wgs = a.B * a.H * ((a.N + a.chunk - 1) / a.chunk);
+    for (int mt = DT <= 2 ? 4 : 2; mt > 1; mt >>= 1)
+        if (wgs * ((a.M + 16 * mt - 1) / (16 * mt)) >= 1024) return mt;
+    return a.M <= 128 && DT <= 4 ? 1 : 2;
+}
 
 template <typename T, int MT, int DT>
 int prepare_at(const WaveArgs& a, float* cmax, float* cden, float* cnum, hipStream_t st) {
@@ -55,15 +64,21 @@ int output_sep(const WaveArgs& a, const float* pmax, const float* pden, const fl
 
 template <typename T, int DT>
 int prepare_dt(const WaveArgs& a, float* cmax, float* cden, float* cnum, hipStream_t st) {
+    const int mt = latent_tiles<DT>(a);
     if constexpr (DT <= 2)
-        if (latent_tiles<DT>(a.M) == 4) return prepare_at<T, 4, DT>(a, cmax, cden, cnum, st);
+        if (mt == 4) return prepare_at<T, 4, DT>(a, cmax, cden, cnum, st);
+    if constexpr (DT <= 4)
+        if (mt == 1) return prepare_at<T, 1, DT>(a, cmax, cden, cnum, st);
     return prepare_at<T, 2, DT>(a, cmax, cden, cnum, st);
 }
 template <typename T, int DT>
 int output_dt(const WaveArgs& a, const float* pmax, const float* pden, const float* pnum, void* Y, int out_dtype,
               hipStream_t st) {
+    const int mt = latent_tiles<DT>(a);
     if constexpr (DT <= 2)
-        if (latent_tiles<DT>(a.M) == 4) return output_sep<T, 4, DT>(a, pmax, pden, pnum, Y, out_dtype, st);
+        if (mt == 4) return output_sep<T, 4, DT>(a, pmax, pden, pnum, Y, out_dtype, st);
+    if constexpr (DT <= 4)
+        if (mt == 1) return output_sep<T, 1, DT>(a, pmax, pden, pnum, Y, out_dtype, st);
     return output_sep<T, 2, DT>(a, pmax, pden, pnum, Y, out_dtype, st);
 }
 
