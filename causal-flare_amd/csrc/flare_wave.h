@@ -24,7 +24,7 @@
 // cycles of its SIMD's matrix pipe, busy 40% of the kernel) and about 880 vector instructions
 // (52%).  Measured on MI355X, whole forward, tokenwise kernels -> these:
 //   bf16 B 8, N 4096, H 16, M 64, D 32     4937 -> 158 us (prepare 41, scan 7, output 124)
-//   fp16 B 3, N 1531, H 8, M 96, D 64, cached state and mask   1135 -> 124 us
+//   fp16 B 3, N 1531, H 8, M 96, D 64, cached state and mask   1135 ->  72 us
 //   fp32 B 1, N 256, H 8, M 64, D 32        283 ->  30 us
 // Errors against 64 bits: fp32 outputs 2.5e-7 -> 1.1e-7, 16-bit ones unchanged.
 #pragma once

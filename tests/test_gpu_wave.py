@@ -211,3 +211,30 @@ def test_wave_semi_backward(M, D, N, block, dtype, sep):
     refs = O.semi_grads(q, k, v, g, block, Q_dec=qd, K_dec=kd)
     refs = list(refs[:3]) + [r for r, t in zip(refs[3:], (qd, kd)) if t is not None]
     _check_grads({n: t.grad for n, t in leaves.items()}, refs, dtype, f"M={M} D={D} N={N} block={block} sep={sep}")
+
+
+@pytest.mark.parametrize("M,D,dtype", [(64, 32, torch.float32), (96, 64, torch.float16), (128, 64, torch.bfloat16),
+                                       (256, 128, torch.bfloat16), (256, 64, torch.float16), (40, 80, torch.float32)])
+@pytest.mark.parametrize("sep", [False, True])
+def test_all_kept_mask_is_no_mask(M, D, dtype, sep):
+    """A mask that keeps every token is not looked for on the host at these sizes: its launches
+    have to give what the unmasked ones do, also where a value row is infinite."""
+    from causal_flare import flare_autoregressive_prefill_triton
+    print("CASE all_kept", M, D, dtype, sep, flush=True)
+    B, N, H = 2, 209, 2
+    q, k, v = seeded(31 + M, B, N, H, M, D, D, dtype, q_std=D ** -0.5)
+    dec = {}
+    if sep:
+        qd, kd, _ = seeded(32 + M, B, N, H, M, D, D, dtype, q_std=D ** -0.5)
+        dec = dict(Q_dec=kd.to(DEV), K_dec=qd.to(DEV))
+    v[1, 150, 0, 3] = float("inf")
+    args = [t.to(DEV) for t in (q, k, v)]
+    y, st = flare_autoregressive_prefill_triton(*args, **dec)
+    for mask in (torch.ones(B, N, dtype=torch.bool), torch.full((B, N), 2, dtype=torch.int64, device=DEV)):
+        ym, sm = flare_autoregressive_prefill_triton(*args, **dec, attention_mask=mask)
+        a, b = to_np(ym).astype(np.float64), to_np(y).astype(np.float64)
+        same = np.isfinite(b)
+        assert np.array_equal(np.isfinite(a), same)
+        _close(torch.from_numpy(a[same]), b[same], dtype, "y")
+        for n in ("m", "d"):
+            _close(sm[n], to_np(st[n]), torch.float32, n)
