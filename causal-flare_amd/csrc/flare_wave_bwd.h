@@ -35,13 +35,17 @@
 // to the max of the tile they were last used in (factors <= 1 as the walk goes back).  A tile
 // in which a max rises by more than kTileJump runs token by token with each token's own max.
 //
-// Bound by the latency of a tile's chain at two to four waves a SIMD (a third to a half of the
-// vector issue slots are used).  Measured, forward and backward, against per-token statistics
-// and one state per 32 tokens in memory (MI355X):
-//   bf16 B 4, N 4096, H 16, M 128, D 64    1521 -> 574 us (wave_gz 130, wave_ds 225 of it)
-//   bf16 N 16384, H 16, M 256, D 128       3774 -> 1600 us (wave_gz 420, wave_ds 680)
-//   bf16 B 4, N 2011, H 16, M 64, D 32     2947 -> 213 us
-//   fp32 B 2, N 1024, H 8, M 64, D 64, decoder weights of its own   1170 -> 208 us
+// Bound by vector issue and the latency of a tile's chain at two to three waves a SIMD (some
+// 60% of the issue slots are used, 12% of the matrix pipe's).  What is read the other way round
+// (V, g, X and the e / w tiles of 16-bit kernels) comes through transposing LDS reads, X, e and w
+// already split into bf16 hi + lo: splitting after the read took a third more instructions
+// (1,691 against 1,114 in the backward walk at D = 128; 677 -> 515 us at N 16384, M 256).
+// Measured, forward and backward, against per-token statistics and one state per 32 tokens in
+// memory (MI355X):
+//   bf16 B 4, N 4096, H 16, M 128, D 64    1521 -> 520 us (wave_gz 121, wave_ds 161 of it)
+//   bf16 N 16384, H 16, M 256, D 128       3774 -> 1403 us (wave_gz 411, wave_ds 515)
+//   bf16 B 4, N 2011, H 16, M 64, D 32     2947 -> 196 us
+//   fp32 B 2, N 1024, H 8, M 64, D 64, decoder weights of its own   1170 -> 207 us
 #pragma once
 
 #include <type_traits>
@@ -56,37 +60,38 @@ using mfma::bf16x4;
 using mfma::f16x8;
 
 // ---------------------------------------------------------------------------
+// Value columns.  Lane c (or C row c) of column tile dt is value column walk_col(dt, c).  fp32
+// kernels keep the pieces of col_of (several tiles' columns side by side, so that a lane reads
+// 16 bytes); 16-bit ones (FLAT) take column 16 dt + c, the order of the transposing LDS reads.
+// ---------------------------------------------------------------------------
+template <int DT, bool FLAT>
+__host__ __device__ constexpr int walk_piece(int dt) { return FLAT ? 1 : piece_of<DT>(dt); }
+// column tiles taken at a time: two where each has a read of its own (four held 16 registers more
+// and spilled at D = 64: 130 against 119 us for the forward walk)
+template <typename T, int DT>
+__host__ __device__ constexpr int step_of(int dt) { return sizeof(T) == 2 ? (dt + 2 <= DT ? 2 : 1) : piece_of<DT>(dt); }
+template <int DT, bool FLAT>
+__device__ __forceinline__ int walk_col(int dt, int c) { return FLAT ? 16 * dt + c : col_of<DT>(dt, c); }
+
+// ---------------------------------------------------------------------------
 // A row of D = 16 DT values, split over the lane groups as the C rows of a transposed state
-// are: lane group g holds value column col_of(dt, 4g + i) for every dt, i.  Within a piece
+// are: lane group g holds value column walk_col(dt, 4g + i) for every dt, i.  Within a piece
 // these are 4 P consecutive columns.
 // ---------------------------------------------------------------------------
-template <int DT>
+template <int DT, bool FLAT>
 __host__ __device__ constexpr int list_at(int dt, int i) {    // position of (dt, i) in the lane's list
-    return 4 * piece_off<DT>(dt) + i * piece_of<DT>(dt) + (dt - piece_off<DT>(dt));
-}
-// tile and register of list position e (valid below 4 DT)
-template <int DT>
-__host__ __device__ constexpr int list_dt(int e) {
-    constexpr int full = DT / 4 * 4, rem = DT - full;
-    const int f = e - 4 * full;
-    return f < 0 ? (e / 16) * 4 + (e & 3) : rem == 1 ? full : f < 8 ? full + (f & 1) : full + 2;
-}
-template <int DT>
-__host__ __device__ constexpr int list_i(int e) {
-    constexpr int full = DT / 4 * 4, rem = DT - full;
-    const int f = e - 4 * full;
-    return f < 0 ? (e >> 2) & 3 : rem == 1 ? f : f < 8 ? f >> 1 : f - 8;
+    return FLAT ? 4 * dt + i : 4 * piece_off<DT>(dt) + i * piece_of<DT>(dt) + (dt - piece_off<DT>(dt));
 }
 
-template <typename T, int DT>
+template <typename T, int DT, bool FLAT = false>
 struct GroupRow {
     static constexpr int W = sizeof(T) == 4 ? 4 * DT : 2 * DT;
     static constexpr int S = (DT + 1) / 2;                    // steps of 8 values (32 over the groups)
     unsigned w[W];
     __device__ __forceinline__ void load(const T* row, int g) {
 #pragma unroll
-        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
-            const int P = piece_of<DT>(dt);
+        for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt)) {
+            const int P = walk_piece<DT, FLAT>(dt);
             const T* p = row + 16 * dt + 4 * g * P;
             // 4 P values
             const int at = (sizeof(T) == 4 ? 4 : 2) * dt, words = (sizeof(T) == 4 ? 4 : 2) * P;
@@ -123,9 +128,13 @@ struct GroupRow {
     }
 };
 
-// c += x . y^T over the columns
+// a row as the products with a transposed state read it
 template <typename T, int DT>
-__device__ __forceinline__ f32x4 dot_groups(const GroupRow<T, DT>& x, const GroupRow<T, DT>& y, f32x4 c) {
+using WalkRow = GroupRow<T, DT, sizeof(T) == 2>;
+
+// c += x . y^T over the columns
+template <typename T, int DT, bool FLAT>
+__device__ __forceinline__ f32x4 dot_groups(const GroupRow<T, DT, FLAT>& x, const GroupRow<T, DT, FLAT>& y, f32x4 c) {
     if constexpr (sizeof(T) == 4) {
         // (two sums over halves: fewer roundings in a row, and shorter chains)
         f32x4 d = {0.f, 0.f, 0.f, 0.f};
@@ -230,50 +239,255 @@ struct TokCols {
     }
 };
 
-// c += x . u over the columns: rows of x (lane column = row) against a transposed state
-// (rows = columns col_of(dt, 4g + i), lane column = latent); C rows are x's rows.
+// the columns of one step (two column tiles) of the product below, u as bf16 hi + lo
 template <typename T, int DT>
-__device__ __forceinline__ f32x4 dot_state(const GroupRow<T, DT>& x, const f32x4 (&u)[DT], f32x4 c) {
+__device__ __forceinline__ f32x4 dot_split(const WalkRow<T, DT>& x, int s, bf16x8 uh, bf16x8 ul, f32x4 c) {
+    if constexpr (__is_same(T, __half)) {
+        const f16x8 xf = __builtin_bit_cast(f16x8, x.op8(s));
+        bf16x8 xh, xl;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) SPLIT2(mfma::bf16, (float)xf[e], xh[e], xl[e]);
+        c = mfma::mma(xh, uh, c);
+        c = mfma::mma(xh, ul, c);
+        return mfma::mma(xl, uh, c);
+    } else {
+        c = mfma::mma(x.op8(s), uh, c);
+        return mfma::mma(x.op8(s), ul, c);
+    }
+}
+
+// c += x . u over the columns: rows of x (lane column = row) against a transposed state
+// (rows = columns walk_col(dt, 4g + i), lane column = latent); C rows are x's rows.
+template <typename T, int DT>
+__device__ __forceinline__ f32x4 dot_state(const WalkRow<T, DT>& x, const f32x4 (&u)[DT], f32x4 c) {
     if constexpr (sizeof(T) == 4) {
         f32x4 d[3] = {};
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-            c = mma4(x.at(list_at<DT>(dt, 0)), u[dt][0], c);
+            c = mma4(x.at(list_at<DT, false>(dt, 0)), u[dt][0], c);
 #pragma unroll
-            for (int i = 1; i < 4; ++i) d[i - 1] = mma4(x.at(list_at<DT>(dt, i)), u[dt][i], d[i - 1]);
+            for (int i = 1; i < 4; ++i) d[i - 1] = mma4(x.at(list_at<DT, false>(dt, i)), u[dt][i], d[i - 1]);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) c[i] = (c[i] + d[0][i]) + (d[1][i] + d[2][i]);
     } else {
 #pragma unroll
         for (int s = 0; s < GroupRow<T, DT>::S; ++s) {
-            bf16x4 h[2], l[2];
+            bf16x4 h[2] = {}, l[2] = {};
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                float y[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int e = 8 * s + 4 * q + j;
-                    y[j] = e < 4 * DT ? u[e < 4 * DT ? list_dt<DT>(e) : 0][list_i<DT>(e)] : 0.0f;
+            for (int q = 0; q < 2; ++q)
+                if (2 * s + q < DT) {
+                    const f32x4& y = u[2 * s + q < DT ? 2 * s + q : 0];
+                    mfma::split_bf16x4(y[0], y[1], y[2], y[3], h[q], l[q]);
                 }
-                mfma::split_bf16x4(y[0], y[1], y[2], y[3], h[q], l[q]);
-            }
-            const bf16x8 uh = cat(h[0], h[1]), ul = cat(l[0], l[1]);
-            if constexpr (__is_same(T, __half)) {
-                const f16x8 xf = __builtin_bit_cast(f16x8, x.op8(s));
-                bf16x8 xh, xl;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) SPLIT2(mfma::bf16, (float)xf[e], xh[e], xl[e]);
-                c = mfma::mma(xh, uh, c);
-                c = mfma::mma(xh, ul, c);
-                c = mfma::mma(xl, uh, c);
-            } else {
-                c = mfma::mma(x.op8(s), uh, c);
-                c = mfma::mma(x.op8(s), ul, c);
-            }
+            c = dot_split<T, DT>(x, s, cat(h[0], h[1]), cat(l[0], l[1]), c);
         }
     }
     return c;
+}
+
+// ---------------------------------------------------------------------------
+// 16-bit values of an LDS tile the other way round: lane (g, c) gets rows 4g + i of column c
+// from a tile whose rows start at `tile`, `pitch` apart (ds_read_b64_tr_b16: lane c of a
+// group points at four columns of row 4g + c / 4).
+// ---------------------------------------------------------------------------
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+__device__ __forceinline__ u32x2 tile_tr(const void* tile, int pitch, int g, int c) {
+    const short* p = (const short*)tile + (4 * g + (c >> 2)) * pitch + 4 * (c & 3);
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
+}
+__device__ __forceinline__ Pair4 pair_tr(const bf16x4* hi, int quads, int pitch, int g, int c) {   // lo: `quads` behind
+    return {__builtin_bit_cast(bf16x4, tile_tr(hi, pitch, g, c)), __builtin_bit_cast(bf16x4, tile_tr(hi + quads, pitch, g, c))};
+}
+
+// Tokens 4g + i of the tile in LDS, value column walk_col(dt, c): the factor of the products
+// over tokens.
+template <typename T, int DT>
+struct TileCols {
+    typedef typename TokCols<T, DT>::Op Op;
+    static constexpr bool FLAT = sizeof(T) == 2;
+    typename std::conditional<FLAT, u32x2[DT], ColRow<T, DT>[4]>::type r;
+    // the column tiles of the piece that starts at tile d0; rows from `tile`, `pitch` apart
+    __device__ __forceinline__ void load_piece(const T* tile, int pitch, int g, int c, int d0) {
+        if constexpr (FLAT) {
+#pragma unroll
+            for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) r[dt] = tile_tr(tile + 16 * dt, pitch, g, c);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[i].load_piece(tile + (4 * g + i) * pitch, c, d0);
+        }
+    }
+    // tokens that are off become zero, whatever they hold
+    __device__ __forceinline__ void keep(const bool (&on)[4], int d0) {
+        if constexpr (FLAT) {
+            const unsigned m0 = (on[0] ? 0xffffu : 0u) | (on[1] ? 0xffff0000u : 0u);
+            const unsigned m1 = (on[2] ? 0xffffu : 0u) | (on[3] ? 0xffff0000u : 0u);
+#pragma unroll
+            for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
+                r[dt][0] &= m0;
+                r[dt][1] &= m1;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int k = d0; k < d0 + step_of<T, DT>(d0); ++k) r[i].w[k] = on[i] ? r[i].w[k] : 0u;
+        }
+    }
+    __device__ __forceinline__ Op op(int dt) const {
+        Op o;
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o.v[i] = r[i].get(dt);
+        } else if constexpr (__is_same(T, __half)) {
+            const unsigned a = r[dt][0], b = r[dt][1];
+            mfma::split_bf16x4(word_f32<T>(a, false), word_f32<T>(a, true), word_f32<T>(b, false), word_f32<T>(b, true),
+                               o.h, o.l);
+        } else {
+            o.x = __builtin_bit_cast(bf16x4, r[dt]);
+        }
+        return o;
+    }
+};
+
+// A transposed state of 16 latents in wave-private LDS, a row a latent: fp32, or (FLAT) bf16
+// hi rows and behind them the lo rows, from where both products over it read their operands.
+template <typename T, int DT>
+struct StateTile {
+    static constexpr bool FLAT = sizeof(T) == 2;
+    static constexpr int D = 16 * DT, PITCH = FLAT ? D + 8 : D + 4;
+    static constexpr int FLOATS = 16 * PITCH;                        // (two 16-bit planes, or one of fp32)
+    static constexpr int QUADS = 16 * PITCH / 4;                     // of one 16-bit plane
+    typedef bf16x4 __attribute__((may_alias)) quad_a;
+    static __device__ __forceinline__ quad_a* quad(float* tile, int g, int c, int dt) {
+        return reinterpret_cast<quad_a*>(tile) + (c * PITCH + 16 * dt + 4 * g) / 4;
+    }
+    static __device__ __forceinline__ void put(float* tile, const f32x4 (&u)[DT], int g, int c) {
+#pragma unroll
+        for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt)) {
+            if constexpr (FLAT) {
+                bf16x4 h, l;
+                mfma::split_bf16x4(u[dt][0], u[dt][1], u[dt][2], u[dt][3], h, l);
+                quad(tile, g, c, dt)[0] = h;
+                quad(tile, g, c, dt)[QUADS] = l;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (k < piece_of<DT>(dt)) tile[c * PITCH + col_of<DT>(dt, 4 * g + i) + k] = u[dt + k < DT ? dt + k : 0][i];
+            }
+        }
+    }
+    // put, and c + x . u
+    static __device__ __forceinline__ f32x4 put_dot(float* tile, const WalkRow<T, DT>& x, const f32x4 (&u)[DT], int g, int cl,
+                                                    f32x4 c) {
+        if constexpr (FLAT) {
+#pragma unroll
+            for (int s = 0; s < GroupRow<T, DT>::S; ++s) {
+                bf16x4 h[2] = {}, l[2] = {};
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int dt = 2 * s + q < DT ? 2 * s + q : 0;
+                    if (2 * s + q < DT) {
+                        mfma::split_bf16x4(u[dt][0], u[dt][1], u[dt][2], u[dt][3], h[q], l[q]);
+                        quad(tile, g, cl, dt)[0] = h[q];
+                        quad(tile, g, cl, dt)[QUADS] = l[q];
+                    }
+                }
+                c = dot_split<T, DT>(x, s, cat(h[0], h[1]), cat(l[0], l[1]), c);
+            }
+            return c;
+        } else {
+            put(tile, u, g, cl);
+            return dot_state<T, DT>(x, u, c);
+        }
+    }
+    // c + x . u for a u that was put before
+    static __device__ __forceinline__ f32x4 dot(float* tile, const WalkRow<T, DT>& x, const f32x4 (&u)[DT], int g, int cl,
+                                                f32x4 c) {
+        if constexpr (FLAT) {
+#pragma unroll
+            for (int s = 0; s < GroupRow<T, DT>::S; ++s) {
+                bf16x4 h[2] = {}, l[2] = {};
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    if (2 * s + q < DT) {
+                        h[q] = quad(tile, g, cl, 2 * s + q)[0];
+                        l[q] = quad(tile, g, cl, 2 * s + q)[QUADS];
+                    }
+                c = dot_split<T, DT>(x, s, cat(h[0], h[1]), cat(l[0], l[1]), c);
+            }
+            return c;
+        } else {
+            return dot_state<T, DT>(x, u, c);
+        }
+    }
+    // latents 4g + i, value column walk_col(dt, c): the factor of the products over latents
+    struct Cols {
+        typename std::conditional<FLAT, Pair4[DT], ColRow<float, DT>[4]>::type r;
+        __device__ __forceinline__ void load_piece(const float* tile, int g, int c, int d0) {
+            if constexpr (FLAT) {
+#pragma unroll
+                for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt)
+                    r[dt] = pair_tr((const bf16x4*)tile + 4 * dt, QUADS, PITCH, g, c);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r[i].load_piece(tile + (4 * g + i) * PITCH, c, d0);
+            }
+        }
+        __device__ __forceinline__ typename ProdOf<T>::F op(int dt) const {
+            if constexpr (FLAT) return r[dt];
+            else return factor<F4>(r[0].get(dt), r[1].get(dt), r[2].get(dt), r[3].get(dt));
+        }
+    };
+};
+
+// A C tile [token 4g + i][latent c] of factors in wave-private LDS, read back as the factor
+// with lane column = token and contraction index = latent.
+template <typename T>
+struct TurnTile {
+    static constexpr bool FLAT = sizeof(T) == 2;
+    static constexpr int PITCH = 20;                                 // fp32 rows a token, 16-bit rows a latent
+    static constexpr int FLOATS = 16 * PITCH;
+    typedef typename ProdOf<T>::F F;
+    typedef bf16x4 __attribute__((may_alias)) quad_a;
+    static __device__ __forceinline__ void put(float* tile, const F& f, int g, int c) {
+        if constexpr (FLAT) {
+            quad_a* q = reinterpret_cast<quad_a*>(tile) + (c * PITCH + 4 * g) / 4;
+            q[0] = f.h;
+            q[16 * PITCH / 4] = f.l;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) tile[(4 * g + i) * PITCH + c] = f.v[i];
+        }
+    }
+    static __device__ __forceinline__ F get(const float* tile, int g, int c) {
+        if constexpr (FLAT) {
+            return pair_tr((const bf16x4*)tile, 16 * PITCH / 4, PITCH, g, c);
+        } else {
+            const f32x4 r = *reinterpret_cast<const f32x4_a*>(tile + c * PITCH + 4 * g);
+            return factor<F>(r[0], r[1], r[2], r[3]);
+        }
+    }
+};
+
+// dv of a tile (rows = value columns, lane column = token) as rows a token
+template <int DT, bool FLAT>
+__device__ __forceinline__ void put_rows(float* rows, int pitch, const f32x4 (&dv)[DT], int g, int c) {
+#pragma unroll
+    for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt)) {
+        if constexpr (FLAT) {
+            *reinterpret_cast<f32x4_a*>(rows + c * pitch + 16 * dt + 4 * g) = dv[dt];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (k < piece_of<DT>(dt)) rows[c * pitch + col_of<DT>(dt, 4 * g + i) + k] = dv[dt + k < DT ? dt + k : 0][i];
+        }
+    }
 }
 
 // Over the lane groups of a lane column: the sum of x over lower groups, over higher
@@ -303,7 +517,7 @@ constexpr bool bwd_latents_in_regs() { return sizeof(T) == 2 ? DT <= 4 : DT <= (
 // is what the registers cannot hold.
 template <int DT>
 __device__ __forceinline__ void stage() {
-    if constexpr (DT > 4) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (DT >= 4) __builtin_amdgcn_sched_barrier(0);
 }
 
 // fp32 array of one (b, h) through a buffer descriptor (see Bytes).
@@ -402,7 +616,7 @@ __global__ __launch_bounds__(256) void wave_lse_kernel(const T* __restrict__ Qd,
         q.load(Kd + ((size_t)h * M + min(m0 + c, M - 1)) * D, g);
 #pragma unroll
         for (int j = 0; j < kLseTiles; ++j) {
-            f32x4 s = dot_groups<T, DT>(q, k[j], f32x4{0.f, 0.f, 0.f, 0.f});
+            f32x4 s = dot_groups(q, k[j], f32x4{0.f, 0.f, 0.f, 0.f});
             float top = mx[j];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -459,7 +673,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
     constexpr int D = 16 * DT;
     typedef typename ProdOf<T>::F F;
     typedef TileRows<T, DT, SEP> Rows;
-    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>(), OWN_GY = own_gy<T>();
+    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>(), OWN_GY = own_gy<T>(), FLAT = sizeof(T) == 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
     const int ch = blockIdx.x, NC = gridDim.x, bh = blockIdx.y;
     const int b = bh / H, h = bh % H;
@@ -495,13 +709,13 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
         den[mt] = in ? a.pden[pbase + m] : 0.0f;
         er[mt] = mx[mt] == kNegInf ? 0.0f : 1.0f;
         ysum[mt] = 0.0f;
-        GroupRow<float, DT> r;
+        GroupRow<float, DT, FLAT> r;
         if (in) r.load(a.pnum + (pbase + m) * D, g);
         else r.zero();
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) u[mt][dt][i] = r.at(list_at<DT>(dt, i));
+            for (int i = 0; i < 4; ++i) u[mt][dt][i] = r.at(list_at<DT, FLAT>(dt, i));
             x[mt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
@@ -527,7 +741,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 if constexpr (!QREG) latent_row(q[0], a.Q, mt);
-                const f32x4 r = dot_groups<T, DT>(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+                const f32x4 r = dot_groups(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
                 top[mt] = kNegInf;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -546,7 +760,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
                 GroupRow<T, DT> qr;
                 qr.load(Rows::QD ? Rows::row(tl, 3, c) : (const T*)a.Qdec + tok + (size_t)min(t + c, t1 - 1) * stride, g);
                 if constexpr (!QREG) latent_row(kd[0], a.Kdec, mt);
-                z = dot_groups<T, DT>(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+                z = dot_groups(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                 for (int i = 0; i < 4; ++i) z[i] *= scale;
             }
@@ -556,20 +770,20 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
         stage<DT>();
         // g_t . v_tau as the [t][tau] factor of sums over tau (C rows tau, lane column t)
         F gvf;
-        GroupRow<T, DT> gr;
+        float bad;
+        WalkRow<T, DT> gr;
         gr.load(Rows::row(tl, 2, c), g);
         {
-            GroupRow<T, DT> vr;
+            WalkRow<T, DT> vr;
             vr.load(Rows::row(tl, 1, c), g);
-            const f32x4 r = dot_groups<T, DT>(vr, gr, f32x4{0.f, 0.f, 0.f, 0.f});
+            const f32x4 r = dot_groups(vr, gr, f32x4{0.f, 0.f, 0.f, 0.f});
+            // a value of g that is not finite shows in its products with v (0 times it is NaN); the
+            // backward walk then keeps it to its own token
+            bad = __builtin_fmaf(r[0], 0.0f, __builtin_fmaf(r[1], 0.0f, __builtin_fmaf(r[2], 0.0f, r[3] * 0.0f)));
             gvf = factor<F>(4 * g <= c ? r[0] : 0.0f, 4 * g + 1 <= c ? r[1] : 0.0f, 4 * g + 2 <= c ? r[2] : 0.0f,
                             4 * g + 3 <= c ? r[3] : 0.0f);
         }
         if (j <= 0) {
-            // a value of g that is not finite: the backward walk keeps it to its own token
-            float bad = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 4 * DT; ++e) bad = __builtin_fmaf(gr.at(e), 0.0f, bad);
             const bool step = __any(slow || bad != bad);
             if (lane == 0) a.stepwise[((size_t)bh * NT + t / TT) * NW + wv] = step;
             j = __any(slow) ? 0 : -1;
@@ -627,16 +841,13 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
         }
         // U += E^T V, X += W^T g, a piece of value columns at a time
 #pragma unroll
-        for (int d0 = 0; d0 < DT; d0 += piece_of<DT>(d0)) {
+        for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
             stage<DT>();
-            TokCols<T, DT> vc, gc;
+            TileCols<T, DT> vc, gc;
+            vc.load_piece(Rows::row(tl, 1, 0), Rows::PITCH, g, c, d0);
+            gc.load_piece(Rows::row(tl, 2, 0), Rows::PITCH, g, c, d0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                vc.r[i].load_piece(Rows::row(tl, 1, 4 * g + i), c, d0);
-                gc.r[i].load_piece(Rows::row(tl, 2, 4 * g + i), c, d0);
-            }
-#pragma unroll
-            for (int dt = d0; dt < d0 + piece_of<DT>(d0); ++dt) {
+            for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
                 const auto vo = vc.op(dt), go = gc.op(dt);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
@@ -667,12 +878,12 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
             if (g == 0) a.ysum[pbase + m] = ysum[mt];
             float* row = a.xsum + (pbase + m) * D;
 #pragma unroll
-            for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
+            for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt))
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
                     for (int k = 0; k < 4; ++k)
-                        if (k < piece_of<DT>(dt)) row[col_of<DT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
+                        if (k < walk_piece<DT, FLAT>(dt)) row[walk_col<DT, FLAT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
         }
     }
 }
@@ -719,16 +930,20 @@ static __global__ __launch_bounds__(256) void wave_carry_kernel(float* __restric
 // a tile is walked token by token is read from the forward walk's marks, for the whole
 // workgroup alike (its waves add their dv rows at barriers).
 // ---------------------------------------------------------------------------
-template <int MT, int DT>
-__host__ __device__ constexpr int ds_wave_floats() {      // wave-private LDS: X tile, or the e / w tiles, or dv rows
-    const int xt = MT * 16 * (16 * DT + 4), ew = 2 * TT * (16 * MT + 4), dv = TT * 16 * DT;
+constexpr int dv_pitch(int DT) { return 16 * DT + 4; }
+template <typename T, int MT, int DT>
+__host__ __device__ constexpr int ds_wave_floats() {      // wave-private LDS: X tiles, or the e / w tiles, or dv rows
+    const int xt = MT * StateTile<T, DT>::FLOATS, ew = 2 * MT * TurnTile<T>::FLOATS, dv = TT * dv_pitch(DT);
     const int a = xt > ew ? xt : ew;
     return a > dv ? a : dv;
 }
 
 template <typename T, int MT, int DT, bool SEP>
 __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int N, int H, int M, float scale, int chunk) {
-    constexpr int D = 16 * DT, EP = 16 * MT + 4, XP = D + 4;
+    constexpr int D = 16 * DT, VP = dv_pitch(DT), WF = ds_wave_floats<T, MT, DT>();
+    constexpr bool FLAT = sizeof(T) == 2;
+    typedef StateTile<T, DT> XTile;
+    typedef TurnTile<T> Turn;
     constexpr int OD = sizeof(T) == 4 ? FLARE_F32 : __is_same(T, __half) ? FLARE_F16 : FLARE_BF16;
     typedef typename ProdOf<T>::F F;
     typedef TileRows<T, DT, SEP> Rows;
@@ -743,9 +958,9 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
     const int t0 = ch * chunk, t1 = min(N, t0 + chunk);
     const int stride = H * D;
     const size_t tok = ((size_t)b * N * H + h) * D;
-    T* tl = reinterpret_cast<T*>(smem + NW * ds_wave_floats<MT, DT>());
-    float* own = smem + wv * ds_wave_floats<MT, DT>();
-    float *etile = own, *wtile = own + TT * EP, *xtile = own, *vtile = own;
+    T* tl = reinterpret_cast<T*>(smem + NW * WF);
+    float* own = smem + wv * WF;
+    float *etile = own, *wtile = own + MT * Turn::FLOATS, *xtile = own, *vtile = own;
     const size_t per = (size_t)N * M;
     const Floats gz_in(a.gz + bh * per, per), lse_in(a.lse + (size_t)bh * N, N), gy_in(a.gy + (size_t)bh * N, N);
     const Floats ds_out(a.ds + bh * per, per), al_out(SEP ? a.al + bh * per : a.ds, SEP ? per : 0);
@@ -772,13 +987,13 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
         const bool tail = m < M && ch + 1 < NC;
         mref[mt] = tail ? a.pmax[pbase + M + m] : 0.0f;
         ysum[mt] = tail ? a.ysum[pbase + m] : 0.0f;
-        GroupRow<float, DT> r;
+        GroupRow<float, DT, FLAT> r;
         if (tail) r.load(a.xsum + (pbase + m) * D, g);
         else r.zero();
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) x[mt][dt][i] = r.at(list_at<DT>(dt, i));
+            for (int i = 0; i < 4; ++i) x[mt][dt][i] = r.at(list_at<DT, FLAT>(dt, i));
     }
 
     Rows rows;
@@ -809,7 +1024,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
                 m0[mt] = tmax_in.load(4u * M * (t / TT) + lat[mt]);
                 d0[mt] = tden_in.load(4u * M * (t / TT) + lat[mt]);
                 if constexpr (!QREG) latent_row(q[0], a.Q, mt);
-                const f32x4 r = dot_groups<T, DT>(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+                const f32x4 r = dot_groups(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
                 top[mt] = kNegInf;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -821,17 +1036,18 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
         }
         stage<DT>();
         // g_t . v_tau as the [tau][t] factor of sums over t (C rows t, lane column tau)
-        GroupRow<T, DT> vr;
+        WalkRow<T, DT> vr;
         vr.load(Rows::row(tl, 1, c), g);
         F gvf;
         {
-            GroupRow<T, DT> gr;
+            WalkRow<T, DT> gr;
             gr.load(Rows::row(tl, 2, c), g);
-            const f32x4 r = dot_groups<T, DT>(gr, vr, f32x4{0.f, 0.f, 0.f, 0.f});
+            const f32x4 r = dot_groups(gr, vr, f32x4{0.f, 0.f, 0.f, 0.f});
             gvf = factor<F>(4 * g >= c ? r[0] : 0.0f, 4 * g + 1 >= c ? r[1] : 0.0f, 4 * g + 2 >= c ? r[2] : 0.0f,
                             4 * g + 3 >= c ? r[3] : 0.0f);
         }
         F wf[MT];
+        float e[MT][4], ysuf[MT][4], dec[MT][4];          // Y at the token; the decoder's part of ds
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             stage<DT>();
@@ -840,7 +1056,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
                 GroupRow<T, DT> qr;
                 qr.load(Rows::QD ? Rows::row(tl, 3, c) : (const T*)a.Qdec + tok + (size_t)min(t + c, t1 - 1) * stride, g);
                 if constexpr (!QREG) latent_row(kd[0], a.Kdec, mt);
-                z = dot_groups<T, DT>(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+                z = dot_groups(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                 for (int i = 0; i < 4; ++i) z[i] *= scale;
             }
@@ -866,12 +1082,12 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
                     for (int i = 0; i < 4; ++i) x[mt][dt][i] *= r;
                 mref[mt] = ref;
             }
-            float e[4], d[4], al[4], w[4], wg[4], run = 0.0f, wrun = 0.0f, below, above, all;
+            float d[4], al[4], w[4], wg[4], run = 0.0f, wrun = 0.0f, below, above, all;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float ev = exp_nat(s[mt][i] - ref);
-                e[i] = j < 0 || 4 * g + i == j ? ev : 0.0f;
-                run += e[i];
+                e[mt][i] = j < 0 || 4 * g + i == j ? ev : 0.0f;
+                run += e[mt][i];
                 d[i] = run;
                 al[i] = t + 4 * g + i < t1 && lat[mt] != kNowhere ? exp_nat(z[i] - lse[i]) : 0.0f;
                 if constexpr (SEP) al_out.store(4u * M * (t + 4 * g + i) + lat[mt], al[i]);
@@ -887,121 +1103,91 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
             }
             group_scan(wrun, g, below, above, all);
             wf[mt] = factor<F>(w[0], w[1], w[2], w[3]);
-            f32x4 xz = dot_state<T, DT>(vr, x[mt], f32x4{0.f, 0.f, 0.f, 0.f});
-            xz = mm(gvf, wf[mt], xz);
             // Y at token 4g + i: later tokens and itself
             float suffix = ysum[mt] + above;
 #pragma unroll
             for (int i = 3; i >= 0; --i) {
                 suffix += wg[i];
-                float r = e[i] * (xz[i] - suffix);
-                if constexpr (!SEP) r += al[i] * (gz[mt][i] - gy[i]);
-                ds_out.store(j < 0 || 4 * g + i == j ? 4u * M * (t + 4 * g + i) + lat[mt] : kNowhere, r);
-                etile[(4 * g + i) * EP + 16 * mt + c] = e[i];
-                wtile[(4 * g + i) * EP + 16 * mt + c] = w[i];
+                ysuf[mt][i] = suffix;
+                dec[mt][i] = SEP ? 0.0f : al[i] * (gz[mt][i] - gy[i]);
             }
             ysum[mt] += all;
+            Turn::put(etile + mt * Turn::FLOATS, factor<F>(e[mt][0], e[mt][1], e[mt][2], e[mt][3]), g, c);
+            Turn::put(wtile + mt * Turn::FLOATS, wf[mt], g, c);
         }
         wave_lds_sync();
         F ef[MT];
         f32x4 G = {0.f, 0.f, 0.f, 0.f};       // [t][tau] summed over this wave's latents
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const f32x4 er = *reinterpret_cast<const f32x4_a*>(etile + c * EP + 16 * mt + 4 * g);
-            const f32x4 wr = *reinterpret_cast<const f32x4_a*>(wtile + c * EP + 16 * mt + 4 * g);
-            ef[mt] = factor<F>(er[0], er[1], er[2], er[3]);
-            G = mm(factor<F>(wr[0], wr[1], wr[2], wr[3]), ef[mt], G);
+            ef[mt] = Turn::get(etile + mt * Turn::FLOATS, g, c);
+            G = mm(Turn::get(wtile + mt * Turn::FLOATS, g, c), ef[mt], G);
         }
         wave_lds_sync();
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt) {
+            stage<DT>();
+            f32x4 xz = XTile::put_dot(xtile + mt * XTile::FLOATS, vr, x[mt], g, c, f32x4{0.f, 0.f, 0.f, 0.f});
+            xz = mm(gvf, wf[mt], xz);
 #pragma unroll
-            for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if (k < piece_of<DT>(dt))
-                            xtile[(16 * mt + c) * XP + col_of<DT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
+            for (int i = 0; i < 4; ++i) {
+                const float r = SEP ? e[mt][i] * (xz[i] - ysuf[mt][i]) : e[mt][i] * (xz[i] - ysuf[mt][i]) + dec[mt][i];
+                ds_out.store(j < 0 || 4 * g + i == j ? 4u * M * (t + 4 * g + i) + lat[mt] : kNowhere, r);
+            }
+        }
         wave_lds_sync();
         const F gf = factor<F>(4 * g >= c ? G[0] : 0.0f, 4 * g + 1 >= c ? G[1] : 0.0f, 4 * g + 2 >= c ? G[2] : 0.0f,
                                4 * g + 3 >= c ? G[3] : 0.0f);
-        // dv rows and X += W^T g, a piece of value columns at a time
+        // dv (rows = value columns, lane column = token) and X += W^T g, a piece of value columns
+        // at a time.  Token by token the other tokens' g, which may not be finite, are taken as
+        // zero.  (A select each time and no branch: after a branch around it the compiler reads
+        // the product above too early on the skipped side.)
+        const bool on[4] = {j < 0 || 4 * g == j, j < 0 || 4 * g + 1 == j, j < 0 || 4 * g + 2 == j, j < 0 || 4 * g + 3 == j};
         f32x4 dv[DT];
 #pragma unroll
-        for (int d1 = 0; d1 < DT; d1 += piece_of<DT>(d1)) {
+        for (int d1 = 0; d1 < DT; d1 += step_of<T, DT>(d1)) {
             stage<DT>();
-            ColRow<float, DT> xr[MT][4];
-            TokCols<T, DT> gc;
+            typename XTile::Cols xc[MT];
+            TileCols<T, DT> gc;
+            gc.load_piece(Rows::row(tl, 2, 0), Rows::PITCH, g, c, d1);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                gc.r[i].load_piece(Rows::row(tl, 2, 4 * g + i), c, d1);
+            for (int mt = 0; mt < MT; ++mt) xc[mt].load_piece(xtile + mt * XTile::FLOATS, g, c, d1);
+            gc.keep(on, d1);
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) xr[mt][i].load_piece(xtile + (16 * mt + 4 * g + i) * XP, c, d1);
-            }
-            // token by token: the other tokens' g, which may not be finite, times zero.  (A select
-            // each time and no branch: after a branch around it the compiler reads the product
-            // above too early on the skipped side.)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int k = 0; k < ColRow<T, DT>::W; ++k) gc.r[i].w[k] = j < 0 || 4 * g + i == j ? gc.r[i].w[k] : 0u;
-#pragma unroll
-            for (int dt = d1; dt < d1 + piece_of<DT>(d1); ++dt) {
+            for (int dt = d1; dt < d1 + step_of<T, DT>(d1); ++dt) {
                 f32x4 r = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    r = mm(ef[mt], factor<F>(xr[mt][0].get(dt), xr[mt][1].get(dt), xr[mt][2].get(dt), xr[mt][3].get(dt)), r);
+                for (int mt = 0; mt < MT; ++mt) r = mm(xc[mt].op(dt), ef[mt], r);
                 const auto go = gc.op(dt);
-                dv[dt] = mm(gf, go, r);
+                dv[dt] = mm(go, gf, r);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) x[mt][dt] = collect(go, wf[mt], x[mt][dt]);
             }
         }
         // rows of this pass; the tile's last pass brings the next tile in
         const bool last = j <= 0, more = last && t > t0;
+        wave_lds_sync();
+        put_rows<DT, FLAT>(vtile, VP, dv, g, c);
         if (NW == 1) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int ti = t + 4 * g + i;
-                if (ti >= t1 || !(j < 0 || 4 * g + i == j)) continue;
-                const size_t row = tok + (size_t)ti * stride;
-#pragma unroll
-                for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
-                    float o[4];
-                    const int P = piece_of<DT>(dt);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) o[k] = k < P ? dv[dt + k < DT ? dt + k : 0][i] : 0.0f;
-                    const size_t at = row + col_of<DT>(dt, c);
-                    if (P == 4) store_cols<4>(a.dV, at, o, OD);
-                    else if (P == 2) store_cols<2>(a.dV, at, o, OD);
-                    else store_cols<1>(a.dV, at, o, OD);
-                }
-            }
             wave_lds_sync();
             if (more) rows.store(tl, a, tok, stride, t - TT, t1);
-            wave_lds_sync();
         } else {
-            wave_lds_sync();
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) vtile[(4 * g + i) * D + col_of<DT>(dt, c)] = dv[dt][i];
             __syncthreads();
             if (more) rows.store(tl, a, tok, stride, t - TT, t1);      // every wave is done with this tile's rows
-            for (int e = threadIdx.x; e < TT * D / 4; e += blockDim.x) {
-                const int ti = e / (D / 4), col = 4 * (e % (D / 4));
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                for (int k = 0; k < NW; ++k) {
-                    const f32x4 r = *reinterpret_cast<const f32x4_a*>(smem + k * ds_wave_floats<MT, DT>() + ti * D + col);
-#pragma unroll
-                    for (int n = 0; n < 4; ++n) acc[n] += r[n];
-                }
-                const float o[4] = {acc[0], acc[1], acc[2], acc[3]};
-                if (t + ti < t1 && (j < 0 || ti == j)) store_cols<4>(a.dV, tok + (size_t)(t + ti) * stride + col, o, OD);
-            }
-            __syncthreads();
         }
+        for (int e = threadIdx.x; e < TT * D / 4; e += blockDim.x) {
+            const int ti = e / (D / 4), col = 4 * (e % (D / 4));
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            for (int k = 0; k < NW; ++k) {
+                const f32x4 r = *reinterpret_cast<const f32x4_a*>(smem + k * WF + ti * VP + col);
+#pragma unroll
+                for (int n = 0; n < 4; ++n) acc[n] += r[n];
+            }
+            const float o[4] = {acc[0], acc[1], acc[2], acc[3]};
+            if (t + ti < t1 && (j < 0 || ti == j)) store_cols<4>(a.dV, tok + (size_t)(t + ti) * stride + col, o, OD);
+        }
+        if (NW == 1) wave_lds_sync();
+        else __syncthreads();
         if (!last) {
             --j;
             continue;

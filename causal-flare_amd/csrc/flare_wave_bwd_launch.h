@@ -10,13 +10,11 @@
 namespace flare {
 namespace wave {
 
-// Latent tiles per wave.  The walks are bound by the latency of a tile's chain, so waves per
-// SIMD count: 16 latents a wave up to D = 64 fit four of them (D = 64: 293 -> 246 us for the
-// backward walk at B 4, N 4096, H 16, M 128), 32 latents of a narrow bank three.  At D = 128
-// a wave of 16 spills and two waves of 32 are faster (990 against 832 us at N 16384, H 16,
-// M 256).
-template <int DT>
-constexpr int bwd_tiles() { return DT <= 2 || DT > 4 ? 2 : 1; }
+// Latent tiles per wave of the walks: 32 latents.  With 16, four waves a SIMD fit up to D = 64,
+// but each tile's rows, g v^T products and sums over latents serve half as many: B 4, N 4096,
+// H 16, M 128, D 64 takes 122 + 228 us so and 121 + 161 us with 32; fp32 B 2, N 1024, H 8, M 64,
+// D 64 takes 43 + 36 and 33 + 30 us.  At D = 128 a wave of 16 spills as well.
+constexpr int kWalkTiles = 2;
 
 template <typename T, int DT>
 int launch_lse(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float scale, hipStream_t st) {
@@ -53,7 +51,7 @@ int bwd_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float s
                        scale, (int)chunk);
     if ((rc = check_launch("wave_gz_kernel"))) return rc;
     if ((rc = launch_carry(p, NC, M, 16 * DT, B * H * M, st))) return rc;
-    const size_t lds = sizeof(float) * (size_t)NW * ds_wave_floats<MT, DT>() + Rows::BYTES;
+    const size_t lds = sizeof(float) * (size_t)NW * ds_wave_floats<T, MT, DT>() + Rows::BYTES;
     if ((rc = allow_lds((const void*)wave_ds_kernel<T, MT, DT, SEP>, lds, "wave_ds_kernel"))) return rc;
     hipLaunchKernelGGL((wave_ds_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), lds, st, p, (int)N, (int)H, (int)M, scale,
                        (int)chunk);
@@ -74,7 +72,7 @@ int semi_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float 
                        (int)M, scale, (int)chunk, (int)block);
     if ((rc = check_launch("wave_semi_gz_kernel"))) return rc;
     if ((rc = launch_carry(p, NC, M, 16 * DT, B * H * M, st))) return rc;
-    const size_t lds = sizeof(float) * (size_t)NW * semi_wave_floats<MT, DT>() + Rows::BYTES;
+    const size_t lds = sizeof(float) * (size_t)NW * semi_wave_floats<T, MT, DT>() + Rows::BYTES;
     if ((rc = allow_lds((const void*)wave_semi_ds_kernel<T, MT, DT, SEP>, lds, "wave_semi_ds_kernel"))) return rc;
     hipLaunchKernelGGL((wave_semi_ds_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), lds, st, p, (int)N, (int)H, (int)M, scale,
                        (int)chunk, (int)block);
@@ -84,7 +82,7 @@ int semi_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float 
 template <typename T, int DT>
 int bwd_dt(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk,
            hipStream_t st) {
-    constexpr int MT = bwd_tiles<DT>();
+    constexpr int MT = kWalkTiles;
     return sep ? bwd_at<T, MT, DT, true>(p, B, N, H, M, scale, chunk, st)
                : bwd_at<T, MT, DT, false>(p, B, N, H, M, scale, chunk, st);
 }
@@ -92,7 +90,7 @@ int bwd_dt(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t 
 template <typename T, int DT>
 int semi_dt(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk,
             int64_t block, hipStream_t st) {
-    constexpr int MT = bwd_tiles<DT>();
+    constexpr int MT = kWalkTiles;
     return sep ? semi_at<T, MT, DT, true>(p, B, N, H, M, scale, chunk, block, st)
                : semi_at<T, MT, DT, false>(p, B, N, H, M, scale, chunk, block, st);
 }

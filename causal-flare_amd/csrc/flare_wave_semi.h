@@ -15,8 +15,8 @@
 //
 // Bound by the latency of a step's chain (load, scores, exponentials, products, barrier) at two
 // to four waves a SIMD.  Measured, forward and backward, against one state per block in memory:
-// bf16 B 2, N 8192, blocks of 64, H 16, M 128, D 64: 1448 -> 524 us (wave_semi_gz 115,
-// wave_semi_ds 180 of it).
+// bf16 B 2, N 8192, blocks of 64, H 16, M 128, D 64: 1448 -> 482 us (wave_semi_gz 101,
+// wave_semi_ds 146 of it).
 #pragma once
 
 #include "flare_wave_bwd.h"
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
     constexpr int D = 16 * DT, R = SEP ? 3 : 2;
     typedef typename ProdOf<T>::F F;
     typedef StepRows<T, DT, R> Rows;
-    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>();
+    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>(), FLAT = sizeof(T) == 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
     const int ch = blockIdx.x, NC = gridDim.x, bh = blockIdx.y;
     const int b = bh / H, h = bh % H;
@@ -116,13 +116,13 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
         er[mt] = mx[mt] == kNegInf ? 0.0f : 1.0f;
         part[mt] = ysum[mt] = 0.0f;
         inv[mt] = 0.0f;
-        GroupRow<float, DT> r;
+        GroupRow<float, DT, FLAT> r;
         if (in) r.load(a.pnum + (pbase + m) * D, g);
         else r.zero();
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) u[mt][dt][i] = r.at(list_at<DT>(dt, i));
+            for (int i = 0; i < 4; ++i) u[mt][dt][i] = r.at(list_at<DT, FLAT>(dt, i));
             x[mt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             if constexpr (!QREG) latent_row(q[0], a.Q, mt);
-            s[mt] = dot_groups<T, DT>(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+            s[mt] = dot_groups(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
             for (int i = 0; i < 4; ++i) s[mt][i] *= scale;
         }
@@ -192,19 +192,18 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
                 }
             }
 #pragma unroll
-            for (int d0 = 0; d0 < DT; d0 += piece_of<DT>(d0)) {
-                TokCols<T, DT> vc;
+            for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
+                TileCols<T, DT> vc;
+                vc.load_piece(Rows::row(tl, 1, 0), Rows::PITCH, g, c, d0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) vc.r[i].load_piece(Rows::row(tl, 1, 4 * g + i), c, d0);
-#pragma unroll
-                for (int dt = d0; dt < d0 + piece_of<DT>(d0); ++dt) {
+                for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
                     const auto vo = vc.op(dt);
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) u[mt][dt] = collect(vo, f[mt], u[mt][dt]);
                 }
             }
         } else {
-            GroupRow<T, DT> gr;
+            WalkRow<T, DT> gr;
             gr.load(Rows::row(tl, 1, c), g);
             float lse[4], gy[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -216,7 +215,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
                     GroupRow<T, DT> qr;
                     qr.load(Rows::row(tl, R - 1, c), g);
                     if constexpr (!QREG) latent_row(kd[0], a.Kdec, mt);
-                    z = dot_groups<T, DT>(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+                    z = dot_groups(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                     for (int i = 0; i < 4; ++i) z[i] *= scale;
                 }
@@ -235,12 +234,11 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
             }
             if constexpr (own_gy<T>()) put_gy(gsum + buf * NW * TT, gy, wv, g, c);
 #pragma unroll
-            for (int d0 = 0; d0 < DT; d0 += piece_of<DT>(d0)) {
-                TokCols<T, DT> gc;
+            for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
+                TileCols<T, DT> gc;
+                gc.load_piece(Rows::row(tl, 1, 0), Rows::PITCH, g, c, d0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) gc.r[i].load_piece(Rows::row(tl, 1, 4 * g + i), c, d0);
-#pragma unroll
-                for (int dt = d0; dt < d0 + piece_of<DT>(d0); ++dt) {
+                for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
                     const auto go = gc.op(dt);
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) x[mt][dt] = collect(go, f[mt], x[mt][dt]);
@@ -263,12 +261,12 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
             if (g == 0) a.ysum[pbase + m] = ysum[mt];
             float* row = a.xsum + (pbase + m) * D;
 #pragma unroll
-            for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
+            for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt))
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
                     for (int k = 0; k < 4; ++k)
-                        if (k < piece_of<DT>(dt)) row[col_of<DT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
+                        if (k < walk_piece<DT, FLAT>(dt)) row[walk_col<DT, FLAT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
         }
     }
 }
@@ -278,21 +276,22 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
 // ---------------------------------------------------------------------------
 template <int DT>
 __host__ __device__ constexpr bool semi_x_stays() { return DT <= 4; }
-template <int MT, int DT>
+template <typename T, int MT, int DT>
 __host__ __device__ constexpr int semi_wave_floats() {
-    const int xt = MT * 16 * (16 * DT + 4), dv = TT * 16 * DT;
+    const int xt = MT * StateTile<T, DT>::FLOATS, dv = TT * dv_pitch(DT);
     return semi_x_stays<DT>() ? xt + dv : (xt > dv ? xt : dv);
 }
 
 template <typename T, int MT, int DT, bool SEP>
 __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a, int N, int H, int M, float scale,
                                                                       int chunk, int block) {
-    constexpr int D = 16 * DT, XP = D + 4, R = SEP ? 3 : 2, WF = semi_wave_floats<MT, DT>();
+    constexpr int D = 16 * DT, VP = dv_pitch(DT), R = SEP ? 3 : 2, WF = semi_wave_floats<T, MT, DT>();
+    typedef StateTile<T, DT> XTile;
     constexpr bool STAYS = semi_x_stays<DT>();
     constexpr int OD = sizeof(T) == 4 ? FLARE_F32 : __is_same(T, __half) ? FLARE_F16 : FLARE_BF16;
     typedef typename ProdOf<T>::F F;
     typedef StepRows<T, DT, R> Rows;
-    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>();
+    constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>(), FLAT = sizeof(T) == 2;
     extern __shared__ __attribute__((aligned(16))) float smem[];
     const int ch = blockIdx.x, NC = gridDim.x, bh = blockIdx.y;
     const int b = bh / H, h = bh % H;
@@ -304,8 +303,8 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
     const int stride = H * D;
     const size_t tok = ((size_t)b * N * H + h) * D;
     const T *kb = (const T*)a.K + tok, *vb = (const T*)a.V + tok, *gb = (const T*)a.dY + tok, *qb = (const T*)a.Qdec + tok;
-    float *xtile = smem + wv * WF, *vtile = xtile + (STAYS ? MT * 16 * XP : 0);
-    const int voff = STAYS ? MT * 16 * XP : 0;
+    constexpr int voff = STAYS ? MT * XTile::FLOATS : 0;
+    float *xtile = smem + wv * WF, *vtile = xtile + voff;
     T* tl = reinterpret_cast<T*>(smem + NW * WF);
     const size_t per = (size_t)N * M;
     const Floats gz_in(a.gz + bh * per, per), lse_in(a.lse + (size_t)bh * N, N), gy_in(a.gy + (size_t)bh * N, N);
@@ -332,27 +331,14 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
         mref[mt] = tail ? a.pmax[pbase + M + m] : 0.0f;
         ysum[mt] = tail ? a.ysum[pbase + m] : 0.0f;
         part[mt] = inv[mt] = 0.0f;
-        GroupRow<float, DT> r;
+        GroupRow<float, DT, FLAT> r;
         if (tail) r.load(a.xsum + (pbase + m) * D, g);
         else r.zero();
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) x[mt][dt][i] = r.at(list_at<DT>(dt, i));
+            for (int i = 0; i < 4; ++i) x[mt][dt][i] = r.at(list_at<DT, FLAT>(dt, i));
     }
-
-    auto write_x = [&]() {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if (k < piece_of<DT>(dt))
-                            xtile[(16 * mt + c) * XP + col_of<DT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
-    };
 
     Rows rows;
     int t = t1 - TT, pass = 0;
@@ -403,10 +389,10 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
                     GroupRow<T, DT> qr;
                     qr.load(Rows::row(tl, R - 1, c), g);
                     if constexpr (!QREG) latent_row(kd[0], a.Kdec, mt);
-                    z = dot_groups<T, DT>(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+                    z = dot_groups(qr, kd[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
                 } else {
                     if constexpr (!QREG) latent_row(q[0], a.Q, mt);
-                    z = dot_groups<T, DT>(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
+                    z = dot_groups(kr, q[QREG ? mt : 0], f32x4{0.f, 0.f, 0.f, 0.f});
                 }
                 float w[4];
 #pragma unroll
@@ -419,12 +405,11 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
                 wf[mt] = factor<F>(w[0], w[1], w[2], w[3]);
             }
 #pragma unroll
-            for (int d0 = 0; d0 < DT; d0 += piece_of<DT>(d0)) {
-                TokCols<T, DT> gc;
+            for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
+                TileCols<T, DT> gc;
+                gc.load_piece(Rows::row(tl, 1, 0), Rows::PITCH, g, c, d0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) gc.r[i].load_piece(Rows::row(tl, 1, 4 * g + i), c, d0);
-#pragma unroll
-                for (int dt = d0; dt < d0 + piece_of<DT>(d0); ++dt) {
+                for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
                     const auto go = gc.op(dt);
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) x[mt][dt] = collect(go, wf[mt], x[mt][dt]);
@@ -435,24 +420,25 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
                 for (int mt = 0; mt < MT; ++mt) {
                     ysum[mt] += group_sum(part[mt]);
                     part[mt] = 0.0f;
+                    if constexpr (STAYS) XTile::put(xtile + mt * XTile::FLOATS, x[mt], g, c);
                 }
-                if constexpr (STAYS) write_x();
             }
             __syncthreads();
             if (more) rows.store(tl, kb, np ? vb : gb, np ? vb : qb, stride, nt);
             __syncthreads();
         } else {
-            GroupRow<T, DT> vr;
+            WalkRow<T, DT> vr;
             vr.load(Rows::row(tl, 1, c), g);
-            if constexpr (!STAYS) write_x();
             F ef[MT];
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 if constexpr (!QREG) latent_row(q[0], a.Q, mt);
                 const GroupRow<T, DT>& qm = q[QREG ? mt : 0];
-                const f32x4 s = dot_groups<T, DT>(kr, qm, f32x4{0.f, 0.f, 0.f, 0.f});       // [tau][m]
-                const f32x4 st = dot_groups<T, DT>(qm, kr, f32x4{0.f, 0.f, 0.f, 0.f});      // [m][tau]
-                const f32x4 xz = dot_state<T, DT>(vr, x[mt], f32x4{0.f, 0.f, 0.f, 0.f});
+                const f32x4 s = dot_groups(kr, qm, f32x4{0.f, 0.f, 0.f, 0.f});       // [tau][m]
+                const f32x4 st = dot_groups(qm, kr, f32x4{0.f, 0.f, 0.f, 0.f});      // [m][tau]
+                const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+                const f32x4 xz = STAYS ? XTile::dot(xtile + mt * XTile::FLOATS, vr, x[mt], g, c, zero)
+                                       : XTile::put_dot(xtile + mt * XTile::FLOATS, vr, x[mt], g, c, zero);
                 float et[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -466,33 +452,26 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
             wave_lds_sync();
             f32x4 dv[DT];
 #pragma unroll
-            for (int d1 = 0; d1 < DT; d1 += piece_of<DT>(d1)) {
-                ColRow<float, DT> xr[MT][4];
+            for (int d1 = 0; d1 < DT; d1 += step_of<T, DT>(d1)) {
+                typename XTile::Cols xc[MT];
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int mt = 0; mt < MT; ++mt) xc[mt].load_piece(xtile + mt * XTile::FLOATS, g, c, d1);
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) xr[mt][i].load_piece(xtile + (16 * mt + 4 * g + i) * XP, c, d1);
-#pragma unroll
-                for (int dt = d1; dt < d1 + piece_of<DT>(d1); ++dt) {
+                for (int dt = d1; dt < d1 + step_of<T, DT>(d1); ++dt) {
                     dv[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        dv[dt] = mm(ef[mt], factor<F>(xr[mt][0].get(dt), xr[mt][1].get(dt), xr[mt][2].get(dt), xr[mt][3].get(dt)),
-                                    dv[dt]);
+                    for (int mt = 0; mt < MT; ++mt) dv[dt] = mm(xc[mt].op(dt), ef[mt], dv[dt]);
                 }
             }
             wave_lds_sync();
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) vtile[(4 * g + i) * D + col_of<DT>(dt, c)] = dv[dt][i];
+            put_rows<DT, FLAT>(vtile, VP, dv, g, c);
             __syncthreads();
             if (more) rows.store(tl, kb, np ? vb : gb, np ? vb : qb, stride, nt);     // every wave is done with this tile
             for (int e = threadIdx.x; e < TT * D / 4; e += blockDim.x) {
                 const int ti = e / (D / 4), col = 4 * (e % (D / 4));
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
                 for (int k = 0; k < NW; ++k) {
-                    const f32x4 r = *reinterpret_cast<const f32x4_a*>(smem + k * WF + voff + ti * D + col);
+                    const f32x4 r = *reinterpret_cast<const f32x4_a*>(smem + k * WF + voff + ti * VP + col);
 #pragma unroll
                     for (int n = 0; n < 4; ++n) acc[n] += r[n];
                 }
