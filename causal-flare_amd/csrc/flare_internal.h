@@ -181,6 +181,10 @@ struct WaveArgs {
     const int32_t* tmask;
 };
 namespace wave {
+// readout of the block-causal forward from block states z (flare_wave_semi.h; Qdec and Kdec given)
+int semi_output_f32(const WaveArgs& a, int64_t block, const float* z, void* Y, int out_dtype, float* lse, hipStream_t st);
+int semi_output_bf16(const WaveArgs& a, int64_t block, const float* z, void* Y, int out_dtype, float* lse, hipStream_t st);
+int semi_output_f16(const WaveArgs& a, int64_t block, const float* z, void* Y, int out_dtype, float* lse, hipStream_t st);
 int prepare_f32(const WaveArgs& a, float* cmax, float* cden, float* cnum, hipStream_t st);
 int prepare_bf16(const WaveArgs& a, float* cmax, float* cden, float* cnum, hipStream_t st);
 int prepare_f16(const WaveArgs& a, float* cmax, float* cden, float* cnum, hipStream_t st);

@@ -19,5 +19,8 @@ int cols_f16(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, i
              float* P, hipStream_t st) {
     return cols_type<__half>(p, r1, r2, B, N, H, M, D, P, st);
 }
+int semi_output_f16(const WaveArgs& a, int64_t block, const float* z, void* Y, int out_dtype, float* lse, hipStream_t st) {
+    return semi_output_type<__half>(a, block, z, Y, out_dtype, lse, st);
+}
 }  // namespace wave
 }  // namespace flare

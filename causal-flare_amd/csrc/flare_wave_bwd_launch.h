@@ -96,6 +96,21 @@ int semi_dt(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t
 }
 
 template <typename T, int DT>
+int semi_output_dt(const WaveArgs& a, int64_t block, const float* z, void* Y, int out_dtype, float* lse, hipStream_t st) {
+    // (two tiles a wave share a block's z rows; blocks that are an odd number of tiles take one)
+    const bool two = block % 32 == 0;
+    const int64_t per = 4 * TT * (two ? 2 : 1);
+    const dim3 grid((unsigned)((a.N + per - 1) / per), (unsigned)(a.B * a.H));
+    if (two)
+        hipLaunchKernelGGL((wave_semi_output_kernel<T, DT, 2>), grid, dim3(256), 0, st, (const T*)a.Qdec, (const T*)a.Kdec, z,
+                           (int)a.N, (int)a.H, (int)a.M, a.scale, (int)block, Y, out_dtype, lse);
+    else
+        hipLaunchKernelGGL((wave_semi_output_kernel<T, DT, 1>), grid, dim3(256), 0, st, (const T*)a.Qdec, (const T*)a.Kdec, z,
+                           (int)a.N, (int)a.H, (int)a.M, a.scale, (int)block, Y, out_dtype, lse);
+    return check_launch("wave_semi_output_kernel");
+}
+
+template <typename T, int DT>
 int rows_dt(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, float scale,
             void* out, hipStream_t st) {
     const int64_t per = 4 * TT * kRowTiles;
@@ -148,6 +163,12 @@ template <typename T>
 int semi_type(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale,
               int64_t chunk, int64_t block, hipStream_t st) {
     FLARE_WAVE_DT_CASES(semi_dt, p, sep, B, N, H, M, scale, chunk, block, st)
+}
+
+template <typename T>
+int semi_output_type(const WaveArgs& a, int64_t block, const float* z, void* Y, int out_dtype, float* lse, hipStream_t st) {
+    const int64_t D = a.D;
+    FLARE_WAVE_DT_CASES(semi_output_dt, a, block, z, Y, out_dtype, lse, st)
 }
 
 }  // namespace wave

@@ -70,6 +70,103 @@ struct StepRows {
 };
 
 // ---------------------------------------------------------------------------
+// Readout of the block-causal forward from the blocks' states z = U / den in memory
+// ([B*H][N/block][M][D], fp32): y = sum over latents of the decoder's weight times z.  A wave
+// takes NTK tiles of 16 tokens of one block against all latents, twice: their log-sum-exp, then
+// the weights, whose C tiles are the factor of the fp32 products with z as they are.  Bound by
+// the latency of z's and the latents' rows from cache (a block's z serves its few waves).
+// Measured: forward and backward of bf16 B 4, N 640, blocks of 32, H 16, M 192, D 64 take 307 us,
+// 3,578 with the readout as scalar products in LDS.
+// ---------------------------------------------------------------------------
+template <typename T, int DT, int NTK>
+__global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restrict__ Qd, const T* __restrict__ Kd,
+                                                               const float* __restrict__ z, int N, int H, int M, float scale,
+                                                               int block, void* __restrict__ Y, int out_dtype,
+                                                               float* __restrict__ lse_out) {
+    constexpr int D = 16 * DT;
+    const int bh = blockIdx.y, b = bh / H, h = bh % H;
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    const int t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * TT * NTK;
+    if (t0 >= N) return;                          // (N and block are multiples of 16 NTK)
+    const float* zb = z + ((size_t)bh * (N / block) + t0 / block) * M * D;
+    GroupRow<T, DT> k[NTK];
+    float mx[NTK], sum[NTK], lse[NTK];
+#pragma unroll
+    for (int j = 0; j < NTK; ++j) {
+        k[j].load(Qd + (((size_t)b * N + t0 + TT * j + c) * H + h) * D, g);
+        mx[j] = kNegInf;
+        sum[j] = 0.0f;
+    }
+    auto scores = [&](int m0, f32x4 (&s)[NTK]) {
+        GroupRow<T, DT> q;
+        q.load(Kd + ((size_t)h * M + min(m0 + c, M - 1)) * D, g);
+#pragma unroll
+        for (int j = 0; j < NTK; ++j) {
+            s[j] = dot_groups(q, k[j], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[j][i] = m0 + 4 * g + i < M ? s[j][i] * scale : kNegInf;
+        }
+    };
+    for (int m0 = 0; m0 < M; m0 += 16) {
+        f32x4 s[NTK];
+        scores(m0, s);
+#pragma unroll
+        for (int j = 0; j < NTK; ++j) {
+            const float top = fmaxf(mx[j], fmaxf(fmaxf(s[j][0], s[j][1]), fmaxf(s[j][2], s[j][3])));
+            const float ref = safe_ref(top);
+            float a = sum[j] * exp_nat(mx[j] - ref);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a += exp_nat(s[j][i] - ref);
+            sum[j] = a;
+            mx[j] = top;
+        }
+    }
+    f32x4 y[NTK][DT];
+#pragma unroll
+    for (int j = 0; j < NTK; ++j) {
+        const float top = group_max(mx[j]), ref = safe_ref(top);
+        lse[j] = ref + __logf(group_sum(sum[j] * exp_nat(mx[j] - ref)));
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) y[j][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int m0 = 0; m0 < M; m0 += 16) {
+        ColRow<float, DT> r[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i].load(zb + (size_t)min(m0 + 4 * g + i, M - 1) * D, c);
+        f32x4 s[NTK];
+        scores(m0, s);
+#pragma unroll
+        for (int j = 0; j < NTK; ++j) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[j][i] = exp_nat(s[j][i] - lse[j]);      // 0 past the bank
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[j][dt] = mma4(r[i].get(dt), s[j][i], y[j][dt]);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NTK; ++j) {
+        const int t = t0 + TT * j + c;
+        const size_t row = (((size_t)b * N + t) * H + h) * D;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float o[4];
+                const int P = piece_of<DT>(dt);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = e < P ? y[j][dt + e < DT ? dt + e : 0][i] : 0.0f;
+                const size_t at = row + col_of<DT>(dt, 4 * g + i);
+                if (P == 4) store_cols<4>(Y, at, o, out_dtype);
+                else if (P == 2) store_cols<2>(Y, at, o, out_dtype);
+                else store_cols<1>(Y, at, o, out_dtype);
+            }
+        if (lse_out != nullptr && g == 0) lse_out[(size_t)bh * N + t] = lse[j];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Forward walk: grid (NC, B*H), one wave per MT*16 latents.  chunk and N are multiples of
 // block, block a multiple of 16.
 // ---------------------------------------------------------------------------

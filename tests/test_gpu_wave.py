@@ -238,3 +238,32 @@ def test_all_kept_mask_is_no_mask(M, D, dtype, sep):
         _close(torch.from_numpy(a[same]), b[same], dtype, "y")
         for n in ("m", "d"):
             _close(sm[n], to_np(st[n]), torch.float32, n)
+
+
+@pytest.mark.parametrize("M,D,N,block", [(1, 16, 16, 16), (40, 32, 96, 32), (96, 48, 144, 48), (192, 64, 64, 64),
+                                         (100, 96, 160, 32), (256, 96, 96, 96), (17, 128, 128, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sep", [False, True])
+def test_wave_semi_forward(M, D, N, block, dtype, sep):
+    """The block-causal readout: one and several blocks, one and two token tiles a wave, a last
+    workgroup with idle waves, latents that fill no tile, both decoder modes; then inputs off a
+    16-byte boundary, which run on the kernel without matrix products."""
+    from causal_flare import flare_semi_autoregressive_trition
+    print("CASE wave_semi_forward", M, D, N, block, dtype, sep, flush=True)
+    B, H = 2, 3
+    q, k, v = seeded(7 * M + D, B, N, H, M, D, D, dtype, q_std=D ** -0.5)
+    gen = torch.Generator().manual_seed(M)
+    qd = torch.randn(B, N, H, D, generator=gen).to(dtype) if sep else None
+    kd = (torch.randn(H, M, D, generator=gen) * D ** -0.5).to(dtype) if sep else None
+    ref = np.asarray(O.brute_semi_ar(q, k, v, block, scale=1.0, Q_dec=qd, K_dec=kd))
+    put = lambda t: None if t is None else t.to(DEV)
+
+    def shifted(t):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+        buf[1:] = t.reshape(-1).to(DEV)
+        return buf[1:].view(t.shape)
+
+    for args in ((put(q), put(k)), (put(q), shifted(k))):
+        y, _ = flare_semi_autoregressive_trition(*args, put(v), block_size=block, chunk_size=16, scale=1.0,
+                                                 Q_dec=put(qd), K_dec=put(kd))
+        _close(y, ref, dtype, f"y M={M} D={D} N={N} block={block} sep={sep}")
