@@ -121,19 +121,36 @@ __global__ __launch_bounds__(kNT) void chunk_prepare_kernel(
 // kernel free of cross-thread traffic).  Chunks are loaded kScanBatch at a time
 // before their serial merges run, so one memory latency covers kScanBatch
 // merges.
+//
+// A row's threads all read (max, den) summaries that one of them overwrites, so a row must
+// not leave its wave, whose loads of a batch come before its stores: a wave takes
+// 64 / (Dv/4) whole rows and the lanes left over (16 of 64 at Dv = 96, 4 at 48) do nothing.
+// STATS = false, for rows longer than a wave (Dv > 256), leaves (max, den) alone;
+// chunk_prefix_stats_kernel overwrites them in a launch of its own.
 // ---------------------------------------------------------------------------
 constexpr int kScanBatch = 16;   // chunk summaries loaded before the first merge (config 3 has 16 chunks)
 
+template <bool STATS>
 __global__ __launch_bounds__(256) void chunk_prefix_kernel(
     float* __restrict__ cmax, float* __restrict__ cden, float* __restrict__ cnum, int NC, int M,
     int Dv, int rows, const float* __restrict__ m0, const float* __restrict__ d0,
     const float* __restrict__ u0, float* __restrict__ m_fin, float* __restrict__ d_fin,
     float* __restrict__ u_fin) {
     const int D4 = Dv >> 2;
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= rows * D4) return;
-    const int row = gid / D4, j = gid % D4;    // row = bh * M + m, value columns 4j .. 4j+3
-    const int bh = row / M, m = row % M;
+    int64_t row;                                // row = bh * M + m, value columns 4j .. 4j+3
+    int j;
+    if constexpr (STATS) {
+        const int lane = threadIdx.x & 63, per = 64 / D4;
+        if (lane >= per * D4) return;
+        row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * per + lane / D4;
+        j = lane % D4;
+    } else {
+        const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+        row = gid / D4;
+        j = (int)(gid % D4);
+    }
+    if (row >= rows) return;
+    const int bh = (int)(row / M), m = (int)(row % M);
     float mc = m0 ? m0[row] : kNegInf;
     float dc = d0 ? d0[row] : 0.0f;
     float4 uc = u0 ? reinterpret_cast<const float4*>(u0)[(size_t)row * D4 + j] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -150,11 +167,12 @@ __global__ __launch_bounds__(256) void chunk_prefix_kernel(
             bd[i] = in ? cden[si] : 0.0f;
             bu[i] = in ? num4[si * D4 + j] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
+        if constexpr (STATS) __builtin_amdgcn_wave_barrier();     // no store of this batch before its loads
 #pragma unroll
         for (int i = 0; i < kScanBatch; ++i) {
             if (c0 + i >= NC) break;
             const size_t si = base + (size_t)(c0 + i) * M;
-            if (j == 0) {
+            if (STATS && j == 0) {
                 cmax[si] = mc;
                 cden[si] = dc;
             }
@@ -169,11 +187,34 @@ __global__ __launch_bounds__(256) void chunk_prefix_kernel(
         }
     }
     if (m_fin) {
-        if (j == 0) {
+        if (STATS && j == 0) {
             m_fin[row] = mc;
             d_fin[row] = dc;
         }
         reinterpret_cast<float4*>(u_fin)[(size_t)row * D4 + j] = uc;
+    }
+}
+
+// The (max, den) part of the scan for rows longer than a wave: one thread per row.
+__global__ __launch_bounds__(256) void chunk_prefix_stats_kernel(float* __restrict__ cmax, float* __restrict__ cden, int NC,
+                                                                 int M, int rows, const float* __restrict__ m0,
+                                                                 const float* __restrict__ d0, float* __restrict__ m_fin,
+                                                                 float* __restrict__ d_fin) {
+    const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (row >= rows) return;
+    float mc = m0 ? m0[row] : kNegInf, dc = d0 ? d0[row] : 0.0f;
+    for (int c = 0; c < NC; ++c) {
+        const size_t si = ((size_t)(row / M) * NC + c) * M + row % M;
+        const float bm = cmax[si], bd = cden[si];
+        cmax[si] = mc;
+        cden[si] = dc;
+        const MergeScales ms = merge_scales(mc, bm);
+        dc = dc * ms.sa + bd * ms.sb;
+        mc = ms.m_new;
+    }
+    if (m_fin) {
+        m_fin[row] = mc;
+        d_fin[row] = dc;
     }
 }
 
@@ -273,10 +314,19 @@ static int launch_prefix(float* cmax, float* cden, float* cnum, int64_t BH, int6
     FLARE_REQUIRE((m0 && d0 && u0) || (!m0 && !d0 && !u0), "chunk_prefix: give all of m0/d0/u0 or none");
     FLARE_REQUIRE((m_fin && d_fin && u_fin) || (!m_fin && !d_fin && !u_fin),
                   "chunk_prefix: give all of m_fin/d_fin/u_fin or none");
-    const int64_t threads = BH * M * (Dv / 4);
-    hipLaunchKernelGGL(chunk_prefix_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, cmax,
-                       cden, cnum, (int)NC, (int)M, (int)Dv, (int)(BH * M), m0, d0, u0, m_fin, d_fin, u_fin);
-    return check_launch("chunk_prefix_kernel");
+    const int64_t rows = BH * M;
+    if (Dv <= 256) {
+        const int64_t per = 4 * (64 / (Dv / 4));      // whole rows of a workgroup's four waves
+        hipLaunchKernelGGL(chunk_prefix_kernel<true>, dim3((unsigned)((rows + per - 1) / per)), dim3(256), 0, stream, cmax,
+                           cden, cnum, (int)NC, (int)M, (int)Dv, (int)rows, m0, d0, u0, m_fin, d_fin, u_fin);
+        return check_launch("chunk_prefix_kernel");
+    }
+    hipLaunchKernelGGL(chunk_prefix_kernel<false>, dim3((unsigned)((rows * (Dv / 4) + 255) / 256)), dim3(256), 0, stream,
+                       cmax, cden, cnum, (int)NC, (int)M, (int)Dv, (int)rows, m0, d0, u0, m_fin, d_fin, u_fin);
+    if (const int rc = check_launch("chunk_prefix_kernel")) return rc;
+    hipLaunchKernelGGL(chunk_prefix_stats_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, stream, cmax, cden,
+                       (int)NC, (int)M, (int)rows, m0, d0, m_fin, d_fin);
+    return check_launch("chunk_prefix_stats_kernel");
 }
 
 static int launch_output(const void* Q, const void* K, const void* V, const void* Qdec,
@@ -499,7 +549,7 @@ int flare_forward_kernel_resources(int dtype, int64_t M, int64_t Dk, int64_t Dv,
     const bool f16in = dtype == FLARE_F16;
     const bool tile_shape = Dk == Dv && (M == 128 || M == 256) && (Dk == 64 || Dk == 128);
     if (phase == 1) {
-        FLARE_REQUIRE(hipFuncGetAttributes(&attr, (const void*)chunk_prefix_kernel) == hipSuccess,
+        FLARE_REQUIRE(hipFuncGetAttributes(&attr, (const void*)chunk_prefix_kernel<true>) == hipSuccess,
                       "kernel_resources: hipFuncGetAttributes failed");
         threads = 256;
     } else if (phase == 0) {

@@ -93,3 +93,48 @@ def test_chunk_prefix_scan(dtype):
         mn = np.maximum(m, mx[:, c])
         a, b = np.exp(m - mn), np.exp(mx[:, c] - mn)
         d, u, m = d * a + den[:, c] * b, u * a[..., None] + num[:, c] * b[..., None], mn
+
+
+@pytest.mark.parametrize("BH,M,D,NC", [(90, 256, 96, 20), (90, 256, 48, 37), (7, 33, 16, 17), (3, 80, 100, 18),
+                                       (5, 64, 320, 19), (2, 48, 512, 33), (90, 256, 128, 17)])
+@pytest.mark.parametrize("state", [False, True])
+def test_chunk_prefix_many_rows(BH, M, D, NC, state):
+    """Every row's exclusive scan over more chunks than are loaded at once, with more rows than
+    are resident, at row lengths that do not divide a wave's 64 threads (D/4 = 24, 12, 25) and
+    rows longer than a wave (80, 128): a row's (max, den) is overwritten in place while its
+    threads read it, so none may read a prefix for a summary.  Bar: a merge rounds twice and
+    takes an exponential of at most 12 in size, 16 * 2^-24 of the sums of magnitudes, NC times."""
+    from causal_flare import _lib
+    _case("chunk_prefix_many_rows", BH, M, D, NC, state)
+    g = torch.Generator(device=DEV).manual_seed(D + NC)
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV)
+    cmax, cden, cnum = rnd(BH, NC, M), 1.0 + rnd(BH, NC, M).abs(), rnd(BH, NC, M, D)
+    m0, d0, u0 = (rnd(BH, M), 1.0 + rnd(BH, M).abs(), rnd(BH, M, D)) if state else (None, None, None)
+    fin = [torch.empty((BH, M), device=DEV), torch.empty((BH, M), device=DEV), torch.empty((BH, M, D), device=DEV)]
+    pm, pd, pn = cmax.clone(), cden.clone(), cnum.clone()
+    P = _lib.ptr
+    rc = _lib.lib().flare_chunk_prefix(P(pm), P(pd), P(pn), BH, NC, M, D, P(m0), P(d0), P(u0), *map(P, fin),
+                                       _lib.stream_of(pm.device))
+    _lib.check(rc, "flare_chunk_prefix")
+    bar = NC * 16 * 2.0 ** -24
+    if state:
+        m, d, u, a = m0.clone(), d0.double(), u0.double(), u0.double().abs()
+    else:
+        m = torch.full((BH, M), -float("inf"), device=DEV)
+        d, u = torch.zeros((BH, M), device=DEV).double(), torch.zeros((BH, M, D), device=DEV).double()
+        a = u.clone()
+
+    def check(got, what):
+        assert torch.equal(got[0], m), what
+        assert bool(((got[1].double() - d).abs() <= bar * d).all()), what
+        assert bool(((got[2].double() - u).abs() <= bar * a).all()), what
+
+    for c in range(NC):
+        check((pm[:, c], pd[:, c], pn[:, c]), f"prefix {c}")
+        mn = torch.maximum(m, cmax[:, c])
+        sa, sb = torch.exp(m.double() - mn.double()), torch.exp(cmax[:, c].double() - mn.double())
+        d = d * sa + cden[:, c].double() * sb
+        u = u * sa[..., None] + cnum[:, c].double() * sb[..., None]
+        a = a * sa[..., None] + cnum[:, c].double().abs() * sb[..., None]
+        m = mn
+    check(fin, "final state")
