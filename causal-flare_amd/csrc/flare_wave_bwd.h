@@ -894,11 +894,11 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
 // per (b*h, latent, value column), and one more column for Y.
 // ---------------------------------------------------------------------------
 static __global__ __launch_bounds__(256) void wave_carry_kernel(float* __restrict__ xsum, float* __restrict__ ysum,
-                                                         const float* __restrict__ pmax, int NC, int M, int D, int rows) {
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+                                                         const float* __restrict__ pmax, int NC, int M, int D, int64_t rows) {
+    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;      // (65,535 (b, h) of 256 x 129 pass 2^31)
     if (gid >= rows * (D + 1)) return;
-    const int row = gid / (D + 1), col = gid % (D + 1);
-    const int bh = row / M, m = row % M;
+    const int64_t row = gid / (D + 1);
+    const int col = (int)(gid % (D + 1)), bh = (int)(row / M), m = (int)(row % M);
     float run = 0.0f, mnext = 0.0f;       // X after chunk ch, relative to mnext = pmax of chunk ch + 1
     constexpr int BATCH = 8;
     for (int c1 = NC; c1 > 0; c1 -= BATCH) {

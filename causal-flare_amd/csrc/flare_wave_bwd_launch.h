@@ -26,7 +26,7 @@ int launch_lse(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, flo
 inline int launch_carry(const BwdPtrs& p, int64_t NC, int64_t M, int64_t D, int64_t rows, hipStream_t st) {
     const int64_t cols = rows * (D + 1);
     hipLaunchKernelGGL(wave_carry_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, st, p.xsum, p.ysum, p.pmax,
-                       (int)NC, (int)M, (int)D, (int)rows);
+                       (int)NC, (int)M, (int)D, rows);
     return check_launch("wave_carry_kernel");
 }
 // Dynamic LDS above the default limit of 64 KB.

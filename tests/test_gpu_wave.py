@@ -267,3 +267,23 @@ def test_wave_semi_forward(M, D, N, block, dtype, sep):
         y, _ = flare_semi_autoregressive_trition(*args, put(v), block_size=block, chunk_size=16, scale=1.0,
                                                  Q_dec=put(qd), K_dec=put(kd))
         _close(y, ref, dtype, f"y M={M} D={D} N={N} block={block} sep={sep}")
+
+
+def test_wave_backward_most_heads():
+    """The most (sequence, head) pairs a grid holds, of a 256 x 128 bank: more than 2^31 sums of
+    the scan over chunks.  The last sequences' gradients are those of the same sequences alone."""
+    from causal_flare import flare_autoregressive_triton
+    print("CASE wave_backward_most_heads", flush=True)
+    B, N, H, M, D = 8131, 1, 8, 256, 128             # 65,048 pairs
+    assert B * H * M * (D + 1) > 2 ** 31 and B * H < 65536
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    rnd = lambda *s: torch.randn(s, generator=gen, device=DEV, dtype=torch.bfloat16)
+    q, k, v, g = rnd(H, M, D), rnd(B, N, H, D), rnd(B, N, H, D), rnd(B, N, H, D)
+
+    def grads(rows):
+        kk, vv = k[rows].clone().requires_grad_(True), v[rows].clone().requires_grad_(True)
+        return torch.autograd.grad(flare_autoregressive_triton(q, kk, vv), (kk, vv), g[rows])
+
+    for whole, alone in zip(grads(slice(None)), grads(slice(B - 3, B))):
+        assert torch.equal(whole[-3:], alone)
+    torch.cuda.empty_cache()                         # (some 40 GB of workspace)
