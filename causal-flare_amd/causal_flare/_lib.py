@@ -32,6 +32,7 @@ HEADER_FUNCTIONS = (
     "flare_forward_kernel_resources",
     "flare_ar_backward_workspace_size",
     "flare_ar_backward",
+    "flare_backward_walks",
     "flare_decode_step",
     "flare_semi_ar_workspace_size",
     "flare_semi_ar_workspace_size_sep",
@@ -92,6 +93,8 @@ def _declare(lib):
     lib.flare_ar_backward_workspace_size.argtypes = [_i64] * 6
     lib.flare_ar_backward.restype = _i
     lib.flare_ar_backward.argtypes = ([_vp] * 5 + [_i] + [_i64] * 6 + [_f] + [_vp] * 7 + [_vp, _sz, _vp])
+    lib.flare_backward_walks.restype = _i
+    lib.flare_backward_walks.argtypes = [_i64] * 4
     lib.flare_decode_step.restype = _i
     lib.flare_decode_step.argtypes = [_vp] * 6 + [_i] + [_i64] * 5 + [_f] + [_vp] * 3 + [_vp, _i, _vp]
     lib.flare_semi_ar_workspace_size.restype = _sz

@@ -1221,7 +1221,7 @@ static int launch_contract(const T* q, const T* k, const T* qd, const T* kd, boo
     // kernels below, dQ 74 -> 33 us and dK 41 -> 43 at bf16 B 4, N 4096, H 16, M 128, D 64, dQ
     // 162 -> 126 and dK 127 -> 94 at N 16384, H 16, M 256, D 128; against the scalar ones, dQ
     // 296 -> 10 and dK 89 -> 10 at B 4, N 2011, H 16, M 64, D 32.
-    const bool wave = (mfma_phase_mask() & 3) == 3 && wave_shape(M, Dk, Dk) && M % 16 == 0 && 4 * N * M < (int64_t)1 << 31 &&
+    const bool wave = (mfma_phase_mask() & 3) == 3 && wave_shape(M, Dk, Dk) && M % 16 == 0 && wave_reach(N, M) &&
                       wave_aligned({q, k, qd, kd, dK, dQd, DS, AL, C});
     const wave::ContractPtrs cp{DS, C, AL, gy, cgz};
     auto rows = [&](const T* r1, const T* r2, void* out) {
@@ -1532,9 +1532,7 @@ int ar_backward_run(const void* Q, const void* K, const void* V, const void* Qde
                   lay.total);
     FLARE_REQUIRE((((uintptr_t)workspace) & 255) == 0, "flare_ar_backward: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
-    // (the walks reach a (b, h)'s per-token arrays by 31-bit byte offsets)
-    if (power <= 0.0f && mfma_phase_mask() == 3 && wave_shape(M, Dk, Dv) && 4 * N * M < (int64_t)1 << 31 &&
-        wave_aligned({Q, K, V, Qdec, Kdec, dY, dV})) {
+    if (power <= 0.0f && flare_backward_walks(N, M, Dk, Dv) && wave_aligned({Q, K, V, Qdec, Kdec, dY, dV})) {
         const bool sep = Qdec != nullptr || Kdec != nullptr;
         const WaveBwdLayout wl(B, N, H, M, Dk, sep, wave_bwd_chunk(B, N, H, M, Dk, sep, lay.total), (N + 15) / 16);
         if (wl.total <= lay.total)
@@ -1555,6 +1553,10 @@ int ar_backward_run(const void* Q, const void* K, const void* V, const void* Qde
 using namespace flare;
 
 extern "C" {
+
+int flare_backward_walks(int64_t N, int64_t M, int64_t Dk, int64_t Dv) {
+    return mfma_phase_mask() == 3 && ar_backward_supported(M, Dk, Dv) && wave_shape(M, Dk, Dv) && wave_reach(N, M);
+}
 
 size_t flare_ar_backward_workspace_size(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv) {
     return ar_backward_workspace(B, N, H, M, Dk, Dv);

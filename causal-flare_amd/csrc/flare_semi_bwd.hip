@@ -676,8 +676,7 @@ int flare_semi_ar_backward(const void* Q, const void* K, const void* V, const vo
     FLARE_REQUIRE((((uintptr_t)workspace) & 255) == 0, "flare_semi_ar_backward: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (mfma_phase_mask() == 3 && wave_shape(M, Dk, Dv) && 4 * N * M < (int64_t)1 << 31 &&
-        wave_aligned({Q, K, V, Qdec, Kdec, dY, dV})) {
+    if (flare_backward_walks(N, M, Dk, Dv) && wave_aligned({Q, K, V, Qdec, Kdec, dY, dV})) {
         const int64_t target = default_chunk(B, N, H, M, Dv);
         const WaveBwdLayout wl(B, N, H, M, Dv, Qdec || Kdec, ((target + block - 1) / block) * block, N / block);
         if (wl.total <= lay.total)

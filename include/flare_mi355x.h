@@ -190,6 +190,10 @@ int flare_forward_kernel_resources(int dtype, int64_t M, int64_t Dk, int64_t Dv,
  */
 size_t flare_ar_backward_workspace_size(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dk,
                                         int64_t Dv);
+/* 1 when flare_ar_backward and flare_semi_ar_backward run calls of this shape, with
+ * 16-byte aligned tensors, as walks over chunks (csrc/flare_wave_bwd.h,
+ * flare_wave_semi.h); 0 when they keep per-token statistics in memory. */
+int flare_backward_walks(int64_t N, int64_t M, int64_t Dk, int64_t Dv);
 int flare_ar_backward(const void* Q, const void* K, const void* V, const void* Qdec,
                       const void* Kdec, int dtype, int64_t B, int64_t N, int64_t H, int64_t M,
                       int64_t Dk, int64_t Dv, float scale, const void* Y, const void* dY, void* dQ,

@@ -234,3 +234,24 @@ def test_stablemax_validation():
     # N = 0 needs no kernel
     y = smx(q, k[:, :0], v[:, :0])
     assert y.shape == (1, 0, 2, 16) and y.dtype == v.dtype
+
+
+@pytest.mark.parametrize("M", [16, 48, 112, 176, 240, 32, 128, 256])
+def test_backward_walk_offsets_fit_32_bits(M):
+    """The backward walks reach a (b, h)'s [N, M] fp32 arrays by 32-bit byte offsets that go on to
+    the end of the last 16-token tile and, for latents past the bank, carry 2^31: no length that
+    they take may pass 2^31 within the arrays' tiles (2^32 with the mark, where it would come out
+    as one of the first rows), and every shorter length is taken."""
+    lib = _lib.lib()
+    limit = 2 ** 31 // (4 * M)                       # rows within 2^31 bytes
+    taken = 0
+    for N in range(limit - 40, limit + 40):
+        rows = -(-N // 16) * 16
+        last = 4 * M * (rows - 1) + 4 * (M - 1)      # the largest offset within the bank
+        past = 4 * M * (rows - 1) + 2 ** 31          # a latent past the bank, same row
+        if lib.flare_backward_walks(N, M, 64, 64):
+            taken += 1
+            assert last < 2 ** 31 and past < 2 ** 32, (M, N)
+        else:
+            assert 4 * M * rows >= 2 ** 31, (M, N)
+    assert 0 < taken < 80
