@@ -13,6 +13,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
 #include <initializer_list>
 #include <mutex>
 
@@ -253,7 +254,8 @@ __global__ __launch_bounds__(kNT) void chunk_output_kernel(
 // times as long on every bank measured here (M 32 to 256, D 32 to 128, 16-bit and fp32).
 bool wave_shape(int64_t M, int64_t Dk, int64_t Dv) {
     const int64_t dt = Dv / 16;
-    return Dk == Dv && Dv % 16 == 0 && (dt == 1 || dt == 2 || dt == 3 || dt == 4 || dt == 6 || dt == 8) && M <= 256;
+    return Dk == Dv && Dv % 16 == 0 && (dt == 1 || dt == 2 || dt == 3 || dt == 4 || dt == 6 || dt == 8) && M >= 1 &&
+           M <= 256;
 }
 bool wave_aligned(std::initializer_list<const void*> ptrs) {
     for (const void* p : ptrs)
@@ -455,7 +457,7 @@ static int device_cus() {
 // summaries (phase 2 and the summary traffic of phases 1 and 3 shrink with them); each chunk
 // is a multiple of 64 tokens, between 64 and 8192.
 static int64_t round_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
-    const int64_t BH = B * H;
+    const int64_t BH = std::max<int64_t>(B * H, 1);      // (sizes are checked by the call that follows)
     // the output kernel fills a compute unit with one workgroup, except for the
     // small banks (M * Dv below 128 x 128), where two share it
     const int64_t per_cu = (M * Dv >= 128 * 128) ? 1 : 2;
@@ -472,7 +474,7 @@ int64_t default_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
     // The wave kernels: about two waves per SIMD over the device (8 a compute unit), each
     // wave with 64 latents of a narrow bank or 32 of a wider one.
     const int64_t NW = Dv <= 32 && M > 32 ? (M + 63) / 64 : (M + 31) / 32;
-    const int64_t wgs = B * H * NW;
+    const int64_t wgs = std::max<int64_t>(B * H, 1) * NW;
     const int64_t target_chunks = (8 * device_cus() + wgs - 1) / wgs;
     int64_t c = (N + target_chunks - 1) / target_chunks;
     c = ((c + 31) / 32) * 32;

@@ -240,6 +240,6 @@ bool wave_shape(int64_t M, int64_t Dk, int64_t Dv);
 // Whether the backward's wave kernels reach a (b, h)'s [N, M] fp32 arrays: byte offsets of 31
 // bits for every row of the last 16-token tile, also those past N, since the offset of a latent
 // past the bank (2^31, see kNowhere) is added to them and must not wrap.
-inline bool wave_reach(int64_t N, int64_t M) { return 4 * ((N + 15) / 16 * 16) * M < (int64_t)1 << 31; }
+inline bool wave_reach(int64_t N, int64_t M) { return N > 0 && 4 * ((N + 15) / 16 * 16) * M < (int64_t)1 << 31; }
 bool wave_aligned(std::initializer_list<const void*> ptrs);
 }  // namespace flare

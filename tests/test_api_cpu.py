@@ -255,3 +255,19 @@ def test_backward_walk_offsets_fit_32_bits(M):
         else:
             assert 4 * M * rows >= 2 ** 31, (M, N)
     assert 0 < taken < 80
+
+
+@pytest.mark.parametrize("B,H,M", [(1, 2, 0), (0, 2, 64), (1, 0, 64), (1, 2, -1)])
+@pytest.mark.parametrize("D", [32, 64, 80])
+def test_chunk_policy_of_empty_problems(B, H, M, D):
+    """The chunk length of an empty problem is a number (it is asked for before the call that
+    refuses the sizes), and so are the workspace sizes."""
+    lib = _lib.lib()
+    assert lib.flare_ar_default_chunk(B, 64, H, M, D) > 0
+    lib.flare_ar_forward_workspace_size(B, 64, H, M, D, 0)
+    lib.flare_ar_backward_workspace_size(B, 64, H, M, D, D)
+    lib.flare_semi_ar_backward_workspace_size(B, 64, H, M, D, D, 16)
+    p = ctypes.c_void_p(256)
+    rc = lib.flare_ar_forward(p, p, p, None, None, 0, B, 64, H, M, D, D, 1.0, 0, None, None, None, None, None, None, p, 0,
+                              p, 1 << 30, None)
+    assert rc == -1 and b"positive" in lib.flare_last_error()
