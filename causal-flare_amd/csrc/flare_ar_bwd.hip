@@ -39,6 +39,7 @@
 //   bwd_reduce   sum of the partials over (b, group)
 #include <stdio.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "flare_common.h"
@@ -1484,17 +1485,20 @@ WaveBwdLayout::WaveBwdLayout(int64_t B, int64_t N, int64_t H, int64_t M, int64_t
     total = o;
 }
 
-// Its chunk: two waves per SIMD over the device as in the forward, whole 64-token steps, and
-// no more memory than the other kernels' workspace takes.
-static int64_t wave_bwd_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, bool sep, size_t bytes) {
+// The token-causal walks' layout.  Chunk: two waves per SIMD over the device as in the forward,
+// whole 64-token steps, and longer while that takes more memory than the other kernels would.
+static WaveBwdLayout wave_bwd_layout(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, bool sep) {
+    const size_t bytes = BwdLayout(B, N, H, M, D, D).total;
+    const int64_t tiles = (N + 15) / 16;
     int64_t c = default_chunk(B, N, H, M, D);
     c = ((c + 63) / 64) * 64;
-    while (c < N && WaveBwdLayout(B, N, H, M, D, sep, c, (N + 15) / 16).total > bytes) c *= 2;
-    return c;
+    while (c < N && WaveBwdLayout(B, N, H, M, D, sep, c, tiles).total > bytes) c *= 2;
+    return WaveBwdLayout(B, N, H, M, D, sep, c, tiles);
 }
 
 static int run_wave_backward(const void* Q, const void* K, const void* V, const void* Qdec, const void* Kdec, int dtype,
-                             int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale, const void* Y, const void* dY, void* dQ, void* dK, void* dV, void* dQdec, void* dKdec, char* ws,
+                             int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale, const void* Y,
+                             const void* dY, void* dQ, void* dK, void* dV, void* dQdec, void* dKdec, char* ws,
                              const WaveBwdLayout& lay, hipStream_t st) {
     const bool sep = Qdec != nullptr || Kdec != nullptr;
     auto at = [&](size_t off) { return reinterpret_cast<float*>(ws + off); };
@@ -1519,26 +1523,28 @@ static int run_wave_backward(const void* Q, const void* K, const void* V, const 
 }
 
 size_t ar_backward_workspace(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv) {
-    return BwdLayout(B, N, H, M, Dk, Dv).total;
+    // enough for either route: which one is taken depends on the tensors' alignment too
+    size_t bytes = BwdLayout(B, N, H, M, Dk, Dv).total;
+    if (flare_backward_walks(N, M, Dk, Dv))
+        for (const bool sep : {false, true}) bytes = std::max(bytes, wave_bwd_layout(B, N, H, M, Dk, sep).total);
+    return bytes;
 }
 
 int ar_backward_run(const void* Q, const void* K, const void* V, const void* Qdec, const void* Kdec, int dtype,
                     int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv, float scale, const void* Y,
                     const void* dY, void* dQ, void* dK, void* dV, void* dQdec, void* dKdec, void* workspace,
                     size_t workspace_bytes, hipStream_t st, float power) {
-    const BwdLayout lay(B, N, H, M, Dk, Dv);
-    FLARE_REQUIRE(workspace && workspace_bytes >= lay.total,
-                  "flare_ar_backward: workspace of %zu bytes is smaller than the %zu required", workspace_bytes,
-                  lay.total);
+    const size_t need = ar_backward_workspace(B, N, H, M, Dk, Dv);
+    FLARE_REQUIRE(workspace && workspace_bytes >= need,
+                  "flare_ar_backward: workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
     FLARE_REQUIRE((((uintptr_t)workspace) & 255) == 0, "flare_ar_backward: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
     if (power <= 0.0f && flare_backward_walks(N, M, Dk, Dv) && wave_aligned({Q, K, V, Qdec, Kdec, dY, dV})) {
-        const bool sep = Qdec != nullptr || Kdec != nullptr;
-        const WaveBwdLayout wl(B, N, H, M, Dk, sep, wave_bwd_chunk(B, N, H, M, Dk, sep, lay.total), (N + 15) / 16);
-        if (wl.total <= lay.total)
-            return run_wave_backward(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dk, scale, Y, dY, dQ, dK, dV, dQdec, dKdec,
-                                     ws, wl, st);
+        const WaveBwdLayout lay = wave_bwd_layout(B, N, H, M, Dk, Qdec != nullptr || Kdec != nullptr);
+        return run_wave_backward(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dk, scale, Y, dY, dQ, dK, dV, dQdec, dKdec, ws,
+                                 lay, st);
     }
+    const BwdLayout lay(B, N, H, M, Dk, Dv);
 #define FLARE_BWD(TY)                                                                                          \
     return run_backward<TY>(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dk, Dv, scale, Y, dY, dQ, dK, dV, dQdec, \
                             dKdec, ws, lay, st, power)

@@ -26,6 +26,7 @@
 //   then gy and the dQ / dK contractions (flare_ar_bwd.hip)
 #include <stdio.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "flare_common.h"
@@ -609,9 +610,15 @@ static int run_semi_backward(const void* Q, const void* K, const void* V, const 
                                dKd, P1, P2, s);
 }
 
+// The block-causal walks' layout.  Chunks are the forward's (two waves per SIMD over the device),
+// rounded up to whole blocks.
+static WaveBwdLayout wave_semi_layout(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, bool sep, int64_t block) {
+    const int64_t target = default_chunk(B, N, H, M, D);
+    return WaveBwdLayout(B, N, H, M, D, sep, ((target + block - 1) / block) * block, N / block);
+}
+
 // The wave kernels (flare_wave_semi.h) for every bank they have an instance of: no M x D state
-// per block in memory.  Chunks are the forward's (two waves per SIMD over the device), rounded
-// up to whole blocks.
+// per block in memory.
 static int run_wave_semi(const void* Q, const void* K, const void* V, const void* Qdec, const void* Kdec, int dtype,
                          int64_t B, int64_t N, int64_t H, int64_t M, int64_t D, float scale, int64_t block,
                          const void* Y, const void* dY, void* dQ, void* dK, void* dV, void* dQd, void* dKd, char* ws,
@@ -646,7 +653,11 @@ extern "C" {
 size_t flare_semi_ar_backward_workspace_size(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv,
                                              int64_t block) {
     if (block <= 0) return 0;
-    return SemiBwdLayout(B, N, H, M, Dk, Dv, block).total;
+    // enough for either route: which one is taken depends on the tensors' alignment too
+    size_t bytes = SemiBwdLayout(B, N, H, M, Dk, Dv, block).total;
+    if (flare_backward_walks(N, M, Dk, Dv))
+        for (const bool sep : {false, true}) bytes = std::max(bytes, wave_semi_layout(B, N, H, M, Dv, sep, block).total);
+    return bytes;
 }
 
 int flare_semi_ar_backward(const void* Q, const void* K, const void* V, const void* Qdec, const void* Kdec,
@@ -669,20 +680,18 @@ int flare_semi_ar_backward(const void* Q, const void* K, const void* V, const vo
                   "flare_semi_ar_backward: D_value=%lld must be a multiple of 16 in [16, 512]", (long long)Dv);
     FLARE_REQUIRE(!Qdec || dQdec, "flare_semi_ar_backward: Qdec given without dQdec");
     FLARE_REQUIRE(!Kdec || dKdec, "flare_semi_ar_backward: Kdec given without dKdec");
-    const SemiBwdLayout lay(B, N, H, M, Dk, Dv, block);
-    FLARE_REQUIRE(workspace && workspace_bytes >= lay.total,
-                  "flare_semi_ar_backward: workspace of %zu bytes is smaller than the %zu required", workspace_bytes,
-                  lay.total);
+    const size_t need = flare_semi_ar_backward_workspace_size(B, N, H, M, Dk, Dv, block);
+    FLARE_REQUIRE(workspace && workspace_bytes >= need,
+                  "flare_semi_ar_backward: workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
     FLARE_REQUIRE((((uintptr_t)workspace) & 255) == 0, "flare_semi_ar_backward: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (flare_backward_walks(N, M, Dk, Dv) && wave_aligned({Q, K, V, Qdec, Kdec, dY, dV})) {
-        const int64_t target = default_chunk(B, N, H, M, Dv);
-        const WaveBwdLayout wl(B, N, H, M, Dv, Qdec || Kdec, ((target + block - 1) / block) * block, N / block);
-        if (wl.total <= lay.total)
-            return run_wave_semi(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dv, scale, block, Y, dY, dQ, dK, dV, dQdec, dKdec,
-                                 ws, wl, st);
+        const WaveBwdLayout lay = wave_semi_layout(B, N, H, M, Dv, Qdec || Kdec, block);
+        return run_wave_semi(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dv, scale, block, Y, dY, dQ, dK, dV, dQdec, dKdec, ws,
+                             lay, st);
     }
+    const SemiBwdLayout lay(B, N, H, M, Dk, Dv, block);
 #define FLARE_SEMI_BWD(TY)                                                                                        \
     return run_semi_backward<TY>(Q, K, V, Qdec, Kdec, dtype, B, N, H, M, Dk, Dv, scale, block, Y, dY, dQ, dK, dV, \
                                  dQdec, dKdec, ws, lay, st)

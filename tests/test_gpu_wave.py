@@ -287,3 +287,28 @@ def test_wave_backward_most_heads():
     for whole, alone in zip(grads(slice(None)), grads(slice(B - 3, B))):
         assert torch.equal(whole[-3:], alone)
     torch.cuda.empty_cache()                         # (some 40 GB of workspace)
+
+
+@pytest.mark.parametrize("B,N,H,M,D,block", [(3, 1920, 16, 96, 32, 128), (1, 960, 8, 64, 32, 64), (2, 6336, 4, 64, 128, 64),
+                                             (1, 16, 1, 16, 16, 16)])
+@pytest.mark.parametrize("layer", ["token", "block"])
+def test_backward_of_own_decoder_weights_walks(B, N, H, M, D, block, layer):
+    """Decoder weights of their own, chunks of one block: the sizes asked for hold the walks'
+    arrays, and the walks are what runs."""
+    from torch.profiler import ProfilerActivity, profile
+    from causal_flare import flare_autoregressive_triton, flare_semi_autoregressive_trition
+    print("CASE backward_route", B, N, H, M, D, block, layer, flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(M)
+    rnd = lambda *s: torch.randn(s, generator=gen, device=DEV, dtype=torch.bfloat16).requires_grad_(True)
+    q, k, v, qd, kd = rnd(H, M, D), rnd(B, N, H, D), rnd(B, N, H, D), rnd(B, N, H, D), rnd(H, M, D)
+    if layer == "token":
+        y = flare_autoregressive_triton(q, k, v, Q_dec=qd, K_dec=kd)
+    else:
+        y, _ = flare_semi_autoregressive_trition(q, k, v, block_size=block, chunk_size=16, Q_dec=qd, K_dec=kd)
+    g = torch.ones_like(y)
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        torch.autograd.grad(y, (q, k, v, qd, kd), g)
+        torch.cuda.synchronize()
+    names = " ".join(e.key for e in prof.key_averages())
+    walk = "wave_ds_kernel" if layer == "token" else "wave_semi_ds_kernel"
+    assert walk in names and "wave_rows_kernel" in names and "wave_cols_kernel" in names, names
