@@ -27,9 +27,14 @@
 // A latent is one lane column, so its reference max and its moves are per-lane scalars.
 //
 // Products.  fp32 inputs: fp32 MFMA (16x16x4).  16-bit inputs: every fp32 factor enters the
-// 16x16x32 bf16 MFMA as hi + lo, both halves side by side in the contraction index (16
-// tokens or latents hi, the same 16 lo), so that one instruction takes the whole product
-// with a 16-bit factor and two take a product of two fp32 factors.
+// bf16 MFMA as a sum of P bf16 parts, each the nearest to what the parts before it leave; two
+// parts lie side by side in the contraction index of the 16x16x32 instruction (16 tokens or
+// latents of the first, the same 16 of the second).  P = 3 holds all 24 bits, P = 2 is within
+// 2^-18.  Two parts serve the banks whose states always met the matrix units as two parts (M
+// 128 and 256, D 64 and 128), three the banks whose kernels were all fp32 (three_parts).  Share
+// of dV entries that are not the rounded 64-bit value, against those kernels, fp16, N 1531: M 64,
+// D 32 0.16 -> 0.13% (0.7% with two parts), M 128, D 64 0.73 -> 0.57% (1.1% with two of which
+// the first is cut off and not rounded); dK of separate decoder weights at M 64, D 32 1.75 -> 0.18%.
 //
 // Numerics.  Weights inside a tile are relative to the latents' max after the tile, X and Y
 // to the max of the tile they were last used in (factors <= 1 as the walk goes back).  A tile
@@ -58,6 +63,7 @@ namespace wave {
 
 using mfma::bf16x4;
 using mfma::f16x8;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------
 // Value columns.  Lane c (or C row c) of column tile dt is value column walk_col(dt, c).  fp32
@@ -159,8 +165,9 @@ __device__ __forceinline__ f32x4 dot_groups(const GroupRow<T, DT, FLAT>& x, cons
 struct F4 {          // fp32 products
     float v[4];
 };
-struct Pair4 {       // fp32 values as bf16 hi + lo
-    bf16x4 h, l;
+template <int P>
+struct Split4 {      // fp32 values as P bf16 parts
+    bf16x4 p[P];
 };
 struct Exact4 {      // bf16 values
     bf16x4 x;
@@ -172,16 +179,32 @@ __device__ __forceinline__ f32x4 mm(const F4& a, const F4& b, f32x4 c) {
     for (int i = 0; i < 4; ++i) c = mma4(a.v[i], b.v[i], c);
     return c;
 }
-__device__ __forceinline__ f32x4 mm(const Pair4& a, const Exact4& b, f32x4 c) {
-    return mfma::mma(cat(a.h, a.l), cat(b.x, b.x), c);
+// A third part goes with zeros into the same instruction.  (The 16x16x16 one has room for just
+// that part, but its sum must not continue one of 16x16x32: nothing waits for the longer
+// instruction there, and sums came out without some of its terms.)
+__device__ __forceinline__ bf16x8 third(bf16x4 x) { return cat(x, bf16x4{}); }
+template <int P>
+__device__ __forceinline__ f32x4 mm(const Split4<P>& a, const Exact4& b, f32x4 c) {
+    c = mfma::mma(cat(a.p[0], a.p[1]), cat(b.x, b.x), c);
+    if constexpr (P == 3) c = mfma::mma(third(a.p[2]), cat(b.x, b.x), c);
+    return c;
 }
-__device__ __forceinline__ f32x4 mm(const Exact4& a, const Pair4& b, f32x4 c) {
-    return mfma::mma(cat(a.x, a.x), cat(b.h, b.l), c);
+template <int P>
+__device__ __forceinline__ f32x4 mm(const Exact4& a, const Split4<P>& b, f32x4 c) {
+    c = mfma::mma(cat(a.x, a.x), cat(b.p[0], b.p[1]), c);
+    if constexpr (P == 3) c = mfma::mma(cat(a.x, a.x), third(b.p[2]), c);
+    return c;
 }
-__device__ __forceinline__ f32x4 mm(const Pair4& a, const Pair4& b, f32x4 c) {
-    const bf16x8 hl = cat(a.h, a.l);
-    c = mfma::mma(hl, cat(b.h, b.h), c);
-    return mfma::mma(hl, cat(b.l, b.l), c);
+// (without the parts' products below 2^-26 of the whole)
+template <int P, int R>
+__device__ __forceinline__ f32x4 mm(const Split4<P>& a, const Split4<R>& b, f32x4 c) {
+    const bf16x8 two = cat(a.p[0], a.p[1]);
+    c = mfma::mma(two, cat(b.p[0], b.p[0]), c);
+    c = mfma::mma(two, cat(b.p[1], b.p[1]), c);
+    if constexpr (P == 3 && R == 3) c = mfma::mma(cat(a.p[0], a.p[2]), cat(b.p[2], b.p[0]), c);
+    else if constexpr (P == 3) c = mfma::mma(third(a.p[2]), cat(b.p[0], b.p[0]), c);
+    else if constexpr (R == 3) c = mfma::mma(cat(a.p[0], a.p[0]), third(b.p[2]), c);
+    return c;
 }
 
 // c += a b for a c that collects many tiles: fp32 products are summed over the tile first, so
@@ -198,8 +221,23 @@ __device__ __forceinline__ f32x4 collect(const A& a, const B& b, f32x4 c) {
     }
 }
 
-template <typename T> struct ProdOf { typedef Pair4 F; };            // type of an fp32 factor
-template <> struct ProdOf<float> { typedef F4 F; };
+// nearest parts: what is left after two is within 2^-18 of x, after three within 2^-27
+template <int P>
+__device__ __forceinline__ Split4<P> split4(f32x4 x) {
+    Split4<P> r;
+#pragma unroll
+    for (int n = 0; n < P; ++n) {
+        r.p[n] = __builtin_convertvector(x, bf16x4);
+        const u32x2 b = __builtin_bit_cast(u32x2, r.p[n]);
+        if (n + 1 < P)
+            x = f32x4{x[0] - __builtin_bit_cast(float, b[0] << 16), x[1] - __builtin_bit_cast(float, b[0] & 0xffff0000u),
+                      x[2] - __builtin_bit_cast(float, b[1] << 16), x[3] - __builtin_bit_cast(float, b[1] & 0xffff0000u)};
+    }
+    return r;
+}
+// P: bf16 parts of an fp32 factor of 16-bit kernels
+template <typename T, int P> struct ProdOf { typedef Split4<P> F; };     // type of an fp32 factor
+template <int P> struct ProdOf<float, P> { typedef F4 F; };
 template <typename F>
 __device__ __forceinline__ F factor(float x0, float x1, float x2, float x3) {
     F r;
@@ -209,7 +247,7 @@ __device__ __forceinline__ F factor(float x0, float x1, float x2, float x3) {
         r.v[2] = x2;
         r.v[3] = x3;
     } else {
-        mfma::split_bf16x4(x0, x1, x2, x3, r.h, r.l);
+        r = split4<sizeof(F) / sizeof(bf16x4)>(f32x4{x0, x1, x2, x3});
     }
     return r;
 }
@@ -219,7 +257,7 @@ __device__ __forceinline__ F factor(float x0, float x1, float x2, float x3) {
 template <typename T, int DT>
 struct TokCols {
     typedef typename std::conditional<sizeof(T) == 4, F4,
-                                      typename std::conditional<__is_same(T, __half), Pair4, Exact4>::type>::type Op;
+                                      typename std::conditional<__is_same(T, __half), Split4<2>, Exact4>::type>::type Op;
     ColRow<T, DT> r[4];
     __device__ __forceinline__ Op op(int dt) const {
         Op o;
@@ -227,7 +265,7 @@ struct TokCols {
 #pragma unroll
             for (int i = 0; i < 4; ++i) o.v[i] = r[i].get(dt);
         } else if constexpr (__is_same(T, __half)) {
-            mfma::split_bf16x4(r[0].get(dt), r[1].get(dt), r[2].get(dt), r[3].get(dt), o.h, o.l);
+            o = split4<2>(f32x4{r[0].get(dt), r[1].get(dt), r[2].get(dt), r[3].get(dt)});     // (exact: 11 bits)
         } else {
             const unsigned sel = dt & 1 ? 0x07060302u : 0x05040100u;
             u32x2 p;
@@ -239,26 +277,43 @@ struct TokCols {
     }
 };
 
-// the columns of one step (two column tiles) of the product below, u as bf16 hi + lo
-template <typename T, int DT>
-__device__ __forceinline__ f32x4 dot_split(const WalkRow<T, DT>& x, int s, bf16x8 uh, bf16x8 ul, f32x4 c) {
+// the columns of one step (two column tiles) of the product below, u as P bf16 parts
+template <typename T, int DT, int P>
+__device__ __forceinline__ f32x4 dot_split(const WalkRow<T, DT>& x, int s, const bf16x8 (&u)[P], f32x4 c) {
     if constexpr (__is_same(T, __half)) {
         const f16x8 xf = __builtin_bit_cast(f16x8, x.op8(s));
         bf16x8 xh, xl;
 #pragma unroll
         for (int e = 0; e < 8; ++e) SPLIT2(mfma::bf16, (float)xf[e], xh[e], xl[e]);
-        c = mfma::mma(xh, uh, c);
-        c = mfma::mma(xh, ul, c);
-        return mfma::mma(xl, uh, c);
+#pragma unroll
+        for (int n = 0; n < P; ++n) {
+            c = mfma::mma(xh, u[n], c);
+            if (n + 1 < P) c = mfma::mma(xl, u[n], c);
+        }
     } else {
-        c = mfma::mma(x.op8(s), uh, c);
-        return mfma::mma(x.op8(s), ul, c);
+#pragma unroll
+        for (int n = 0; n < P; ++n) c = mfma::mma(x.op8(s), u[n], c);
     }
+    return c;
+}
+// column tiles 2s and 2s + 1 of a transposed state as the parts above (zeros past the end)
+template <int DT, int P>
+__device__ __forceinline__ void split_step(const f32x4 (&u)[DT], int s, Split4<P> (&x)[2]) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        if (2 * s + q < DT) x[q] = split4<P>(u[2 * s + q < DT ? 2 * s + q : 0]);
+        else x[q] = Split4<P>{};
+    }
+}
+template <int P>
+__device__ __forceinline__ void cat_step(const Split4<P> (&x)[2], bf16x8 (&r)[P]) {
+#pragma unroll
+    for (int n = 0; n < P; ++n) r[n] = cat(x[0].p[n], x[1].p[n]);
 }
 
 // c += x . u over the columns: rows of x (lane column = row) against a transposed state
 // (rows = columns walk_col(dt, 4g + i), lane column = latent); C rows are x's rows.
-template <typename T, int DT>
+template <typename T, int DT, int P>
 __device__ __forceinline__ f32x4 dot_state(const WalkRow<T, DT>& x, const f32x4 (&u)[DT], f32x4 c) {
     if constexpr (sizeof(T) == 4) {
         f32x4 d[3] = {};
@@ -273,14 +328,11 @@ __device__ __forceinline__ f32x4 dot_state(const WalkRow<T, DT>& x, const f32x4 
     } else {
 #pragma unroll
         for (int s = 0; s < GroupRow<T, DT>::S; ++s) {
-            bf16x4 h[2] = {}, l[2] = {};
-#pragma unroll
-            for (int q = 0; q < 2; ++q)
-                if (2 * s + q < DT) {
-                    const f32x4& y = u[2 * s + q < DT ? 2 * s + q : 0];
-                    mfma::split_bf16x4(y[0], y[1], y[2], y[3], h[q], l[q]);
-                }
-            c = dot_split<T, DT>(x, s, cat(h[0], h[1]), cat(l[0], l[1]), c);
+            Split4<P> y[2];
+            bf16x8 parts[P];
+            split_step<DT, P>(u, s, y);
+            cat_step(y, parts);
+            c = dot_split<T, DT, P>(x, s, parts, c);
         }
     }
     return c;
@@ -291,14 +343,17 @@ __device__ __forceinline__ f32x4 dot_state(const WalkRow<T, DT>& x, const f32x4 
 // from a tile whose rows start at `tile`, `pitch` apart (ds_read_b64_tr_b16: lane c of a
 // group points at four columns of row 4g + c / 4).
 // ---------------------------------------------------------------------------
-typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 __device__ __forceinline__ u32x2 tile_tr(const void* tile, int pitch, int g, int c) {
     const short* p = (const short*)tile + (4 * g + (c >> 2)) * pitch + 4 * (c & 3);
     return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
 }
-__device__ __forceinline__ Pair4 pair_tr(const bf16x4* hi, int quads, int pitch, int g, int c) {   // lo: `quads` behind
-    return {__builtin_bit_cast(bf16x4, tile_tr(hi, pitch, g, c)), __builtin_bit_cast(bf16x4, tile_tr(hi + quads, pitch, g, c))};
+template <int P>
+__device__ __forceinline__ Split4<P> split_tr(const bf16x4* first, int quads, int pitch, int g, int c) {   // parts `quads` apart
+    Split4<P> r;
+#pragma unroll
+    for (int n = 0; n < P; ++n) r.p[n] = __builtin_bit_cast(bf16x4, tile_tr(first + n * quads, pitch, g, c));
+    return r;
 }
 
 // Tokens 4g + i of the tile in LDS, value column walk_col(dt, c): the factor of the products
@@ -342,8 +397,7 @@ struct TileCols {
             for (int i = 0; i < 4; ++i) o.v[i] = r[i].get(dt);
         } else if constexpr (__is_same(T, __half)) {
             const unsigned a = r[dt][0], b = r[dt][1];
-            mfma::split_bf16x4(word_f32<T>(a, false), word_f32<T>(a, true), word_f32<T>(b, false), word_f32<T>(b, true),
-                               o.h, o.l);
+            o = split4<2>(f32x4{word_f32<T>(a, false), word_f32<T>(a, true), word_f32<T>(b, false), word_f32<T>(b, true)});
         } else {
             o.x = __builtin_bit_cast(bf16x4, r[dt]);
         }
@@ -351,26 +405,28 @@ struct TileCols {
     }
 };
 
-// A transposed state of 16 latents in wave-private LDS, a row a latent: fp32, or (FLAT) bf16
-// hi rows and behind them the lo rows, from where both products over it read their operands.
-template <typename T, int DT>
+// A transposed state of 16 latents in wave-private LDS, a row a latent: fp32, or (FLAT) the rows
+// of the first bf16 part and behind them those of the others, from where both products over it
+// read their operands.
+template <typename T, int DT, int P>
 struct StateTile {
     static constexpr bool FLAT = sizeof(T) == 2;
     static constexpr int D = 16 * DT, PITCH = FLAT ? D + 8 : D + 4;
-    static constexpr int FLOATS = 16 * PITCH;                        // (two 16-bit planes, or one of fp32)
-    static constexpr int QUADS = 16 * PITCH / 4;                     // of one 16-bit plane
+    static constexpr int FLOATS = FLAT ? 8 * PITCH * P : 16 * PITCH;
+    static constexpr int QUADS = 16 * PITCH / 4;                     // of one part
     typedef bf16x4 __attribute__((may_alias)) quad_a;
     static __device__ __forceinline__ quad_a* quad(float* tile, int g, int c, int dt) {
         return reinterpret_cast<quad_a*>(tile) + (c * PITCH + 16 * dt + 4 * g) / 4;
+    }
+    static __device__ __forceinline__ void put_parts(float* tile, const Split4<P>& x, int g, int c, int dt) {
+#pragma unroll
+        for (int n = 0; n < P; ++n) quad(tile, g, c, dt)[n * QUADS] = x.p[n];
     }
     static __device__ __forceinline__ void put(float* tile, const f32x4 (&u)[DT], int g, int c) {
 #pragma unroll
         for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt)) {
             if constexpr (FLAT) {
-                bf16x4 h, l;
-                mfma::split_bf16x4(u[dt][0], u[dt][1], u[dt][2], u[dt][3], h, l);
-                quad(tile, g, c, dt)[0] = h;
-                quad(tile, g, c, dt)[QUADS] = l;
+                put_parts(tile, split4<P>(u[dt]), g, c, dt);
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -386,22 +442,19 @@ struct StateTile {
         if constexpr (FLAT) {
 #pragma unroll
             for (int s = 0; s < GroupRow<T, DT>::S; ++s) {
-                bf16x4 h[2] = {}, l[2] = {};
+                Split4<P> y[2];
+                bf16x8 parts[P];
+                split_step<DT, P>(u, s, y);
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const int dt = 2 * s + q < DT ? 2 * s + q : 0;
-                    if (2 * s + q < DT) {
-                        mfma::split_bf16x4(u[dt][0], u[dt][1], u[dt][2], u[dt][3], h[q], l[q]);
-                        quad(tile, g, cl, dt)[0] = h[q];
-                        quad(tile, g, cl, dt)[QUADS] = l[q];
-                    }
-                }
-                c = dot_split<T, DT>(x, s, cat(h[0], h[1]), cat(l[0], l[1]), c);
+                for (int q = 0; q < 2; ++q)
+                    if (2 * s + q < DT) put_parts(tile, y[q], g, cl, 2 * s + q);
+                cat_step(y, parts);
+                c = dot_split<T, DT, P>(x, s, parts, c);
             }
             return c;
         } else {
             put(tile, u, g, cl);
-            return dot_state<T, DT>(x, u, c);
+            return dot_state<T, DT, P>(x, u, c);
         }
     }
     // c + x . u for a u that was put before
@@ -410,54 +463,70 @@ struct StateTile {
         if constexpr (FLAT) {
 #pragma unroll
             for (int s = 0; s < GroupRow<T, DT>::S; ++s) {
-                bf16x4 h[2] = {}, l[2] = {};
+                Split4<P> y[2] = {};
+                bf16x8 parts[P];
 #pragma unroll
                 for (int q = 0; q < 2; ++q)
                     if (2 * s + q < DT) {
-                        h[q] = quad(tile, g, cl, 2 * s + q)[0];
-                        l[q] = quad(tile, g, cl, 2 * s + q)[QUADS];
+#pragma unroll
+                        for (int n = 0; n < P; ++n) y[q].p[n] = quad(tile, g, cl, 2 * s + q)[n * QUADS];
                     }
-                c = dot_split<T, DT>(x, s, cat(h[0], h[1]), cat(l[0], l[1]), c);
+                cat_step(y, parts);
+                c = dot_split<T, DT, P>(x, s, parts, c);
             }
             return c;
         } else {
-            return dot_state<T, DT>(x, u, c);
+            return dot_state<T, DT, P>(x, u, c);
         }
     }
     // latents 4g + i, value column walk_col(dt, c): the factor of the products over latents
     struct Cols {
-        typename std::conditional<FLAT, Pair4[DT], ColRow<float, DT>[4]>::type r;
+        typename std::conditional<FLAT, Split4<P>[DT], ColRow<float, DT>[4]>::type r;
         __device__ __forceinline__ void load_piece(const float* tile, int g, int c, int d0) {
             if constexpr (FLAT) {
 #pragma unroll
                 for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt)
-                    r[dt] = pair_tr((const bf16x4*)tile + 4 * dt, QUADS, PITCH, g, c);
+                    r[dt] = split_tr<P>((const bf16x4*)tile + 4 * dt, QUADS, PITCH, g, c);
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) r[i].load_piece(tile + (4 * g + i) * PITCH, c, d0);
             }
         }
-        __device__ __forceinline__ typename ProdOf<T>::F op(int dt) const {
+        __device__ __forceinline__ typename ProdOf<T, P>::F op(int dt) const {
             if constexpr (FLAT) return r[dt];
             else return factor<F4>(r[0].get(dt), r[1].get(dt), r[2].get(dt), r[3].get(dt));
         }
     };
 };
 
+// dv += X^T . e for the 16 latents whose state is in `tile` (dv starts at the first of them)
+template <typename Tile, typename T, int DT, typename F>
+__device__ __forceinline__ void add_state_product(f32x4 (&dv)[DT], const float* tile, const F& e, bool first, int g, int c) {
+#pragma unroll
+    for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
+        typename Tile::Cols xc;
+        xc.load_piece(tile, g, c, d0);
+#pragma unroll
+        for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt)
+            dv[dt] = mm(xc.op(dt), e, first ? f32x4{0.f, 0.f, 0.f, 0.f} : dv[dt]);
+    }
+}
+
 // A C tile [token 4g + i][latent c] of factors in wave-private LDS, read back as the factor
 // with lane column = token and contraction index = latent.
-template <typename T>
+template <typename T, int P>
 struct TurnTile {
     static constexpr bool FLAT = sizeof(T) == 2;
     static constexpr int PITCH = 20;                                 // fp32 rows a token, 16-bit rows a latent
-    static constexpr int FLOATS = 16 * PITCH;
-    typedef typename ProdOf<T>::F F;
+    static constexpr int QUADS = 16 * PITCH / 4;                     // of one part
+    static constexpr int FLOATS = FLAT ? 8 * PITCH * P : 16 * PITCH;
+    typedef typename ProdOf<T, P>::F F;
     typedef bf16x4 __attribute__((may_alias)) quad_a;
     static __device__ __forceinline__ void put(float* tile, const F& f, int g, int c) {
         if constexpr (FLAT) {
             quad_a* q = reinterpret_cast<quad_a*>(tile) + (c * PITCH + 4 * g) / 4;
-            q[0] = f.h;
-            q[16 * PITCH / 4] = f.l;
+#pragma unroll
+            for (int n = 0; n < P; ++n) q[n * QUADS] = f.p[n];
         } else {
 #pragma unroll
             for (int i = 0; i < 4; ++i) tile[(4 * g + i) * PITCH + c] = f.v[i];
@@ -465,7 +534,7 @@ struct TurnTile {
     }
     static __device__ __forceinline__ F get(const float* tile, int g, int c) {
         if constexpr (FLAT) {
-            return pair_tr((const bf16x4*)tile, 16 * PITCH / 4, PITCH, g, c);
+            return split_tr<P>((const bf16x4*)tile, QUADS, PITCH, g, c);
         } else {
             const f32x4 r = *reinterpret_cast<const f32x4_a*>(tile + c * PITCH + 4 * g);
             return factor<F>(r[0], r[1], r[2], r[3]);
@@ -668,10 +737,10 @@ __device__ __forceinline__ void store_gy(const float* sums, int NW, float* gy, i
 // j is the token; the loop then comes back with the same tile.  (As an inner loop over
 // tokens this took 45 to 60 registers more.)
 // ---------------------------------------------------------------------------
-template <typename T, int MT, int DT, bool SEP>
+template <typename T, int MT, int DT, bool SEP, int P>
 __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int N, int H, int M, float scale, int chunk) {
     constexpr int D = 16 * DT;
-    typedef typename ProdOf<T>::F F;
+    typedef typename ProdOf<T, P>::F F;
     typedef TileRows<T, DT, SEP> Rows;
     constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>(), OWN_GY = own_gy<T>(), FLAT = sizeof(T) == 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
@@ -822,7 +891,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
             float below, above, all;
             group_scan(run, g, below, above, all);
             ef[mt] = factor<F>(e[0], e[1], e[2], e[3]);
-            f32x4 p = dot_state<T, DT>(gr, u[mt], f32x4{0.f, 0.f, 0.f, 0.f});
+            f32x4 p = dot_state<T, DT, P>(gr, u[mt], f32x4{0.f, 0.f, 0.f, 0.f});
             p = mm(gvf, ef[mt], p);
             float w[4];
 #pragma unroll
@@ -931,21 +1000,26 @@ static __global__ __launch_bounds__(256) void wave_carry_kernel(float* __restric
 // workgroup alike (its waves add their dv rows at barriers).
 // ---------------------------------------------------------------------------
 constexpr int dv_pitch(int DT) { return 16 * DT + 4; }
-template <typename T, int MT, int DT>
+// X tiles a wave has in LDS at a time: three parts of 96 or 128 columns leave room for one (eight
+// waves of two took 160 and 209 KB)
+template <typename T, int DT, int P>
+__host__ __device__ constexpr bool one_x_tile() { return sizeof(T) == 2 && P == 3 && DT > 4; }
+template <typename T, int MT, int DT, int P>
 __host__ __device__ constexpr int ds_wave_floats() {      // wave-private LDS: X tiles, or the e / w tiles, or dv rows
-    const int xt = MT * StateTile<T, DT>::FLOATS, ew = 2 * MT * TurnTile<T>::FLOATS, dv = TT * dv_pitch(DT);
+    const int xt = (one_x_tile<T, DT, P>() ? 1 : MT) * StateTile<T, DT, P>::FLOATS;
+    const int ew = 2 * MT * TurnTile<T, P>::FLOATS, dv = TT * dv_pitch(DT);
     const int a = xt > ew ? xt : ew;
     return a > dv ? a : dv;
 }
 
-template <typename T, int MT, int DT, bool SEP>
+template <typename T, int MT, int DT, bool SEP, int P>
 __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int N, int H, int M, float scale, int chunk) {
-    constexpr int D = 16 * DT, VP = dv_pitch(DT), WF = ds_wave_floats<T, MT, DT>();
-    constexpr bool FLAT = sizeof(T) == 2;
-    typedef StateTile<T, DT> XTile;
-    typedef TurnTile<T> Turn;
+    constexpr int D = 16 * DT, VP = dv_pitch(DT), WF = ds_wave_floats<T, MT, DT, P>();
+    constexpr bool FLAT = sizeof(T) == 2, ONE = one_x_tile<T, DT, P>();
+    typedef StateTile<T, DT, P> XTile;
+    typedef TurnTile<T, P> Turn;
     constexpr int OD = sizeof(T) == 4 ? FLARE_F32 : __is_same(T, __half) ? FLARE_F16 : FLARE_BF16;
-    typedef typename ProdOf<T>::F F;
+    typedef typename ProdOf<T, P>::F F;
     typedef TileRows<T, DT, SEP> Rows;
     constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>();
     extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -1124,40 +1198,51 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
             G = mm(Turn::get(wtile + mt * Turn::FLOATS, g, c), ef[mt], G);
         }
         wave_lds_sync();
+        f32x4 dv[DT];                         // rows = value columns, lane column = token
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             stage<DT>();
-            f32x4 xz = XTile::put_dot(xtile + mt * XTile::FLOATS, vr, x[mt], g, c, f32x4{0.f, 0.f, 0.f, 0.f});
+            float* xt = xtile + (ONE ? 0 : mt * XTile::FLOATS);
+            f32x4 xz = XTile::put_dot(xt, vr, x[mt], g, c, f32x4{0.f, 0.f, 0.f, 0.f});
             xz = mm(gvf, wf[mt], xz);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float r = SEP ? e[mt][i] * (xz[i] - ysuf[mt][i]) : e[mt][i] * (xz[i] - ysuf[mt][i]) + dec[mt][i];
                 ds_out.store(j < 0 || 4 * g + i == j ? 4u * M * (t + 4 * g + i) + lat[mt] : kNowhere, r);
             }
+            if constexpr (ONE) {
+                wave_lds_sync();
+                add_state_product<XTile, T, DT>(dv, xt, ef[mt], mt == 0, g, c);
+                wave_lds_sync();
+            }
         }
         wave_lds_sync();
         const F gf = factor<F>(4 * g >= c ? G[0] : 0.0f, 4 * g + 1 >= c ? G[1] : 0.0f, 4 * g + 2 >= c ? G[2] : 0.0f,
                                4 * g + 3 >= c ? G[3] : 0.0f);
-        // dv (rows = value columns, lane column = token) and X += W^T g, a piece of value columns
-        // at a time.  Token by token the other tokens' g, which may not be finite, are taken as
+        // dv and X += W^T g, a piece of value columns at a time.  Token by token the other tokens' g, which may not be finite, are taken as
         // zero.  (A select each time and no branch: after a branch around it the compiler reads
         // the product above too early on the skipped side.)
         const bool on[4] = {j < 0 || 4 * g == j, j < 0 || 4 * g + 1 == j, j < 0 || 4 * g + 2 == j, j < 0 || 4 * g + 3 == j};
-        f32x4 dv[DT];
 #pragma unroll
         for (int d1 = 0; d1 < DT; d1 += step_of<T, DT>(d1)) {
             stage<DT>();
-            typename XTile::Cols xc[MT];
+            typename XTile::Cols xc[ONE ? 1 : MT];
             TileCols<T, DT> gc;
             gc.load_piece(Rows::row(tl, 2, 0), Rows::PITCH, g, c, d1);
+            if constexpr (!ONE) {
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) xc[mt].load_piece(xtile + mt * XTile::FLOATS, g, c, d1);
+                for (int mt = 0; mt < MT; ++mt) xc[mt].load_piece(xtile + mt * XTile::FLOATS, g, c, d1);
+            }
             gc.keep(on, d1);
 #pragma unroll
             for (int dt = d1; dt < d1 + step_of<T, DT>(d1); ++dt) {
                 f32x4 r = {0.f, 0.f, 0.f, 0.f};
+                if constexpr (ONE) {
+                    r = dv[dt];
+                } else {
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) r = mm(xc[mt].op(dt), ef[mt], r);
+                    for (int mt = 0; mt < MT; ++mt) r = mm(xc[mt].op(dt), ef[mt], r);
+                }
                 const auto go = gc.op(dt);
                 dv[dt] = mm(go, gf, r);
 #pragma unroll

@@ -16,6 +16,24 @@ namespace wave {
 // D 64 takes 43 + 36 and 33 + 30 us.  At D = 128 a wave of 16 spills as well.
 constexpr int kWalkTiles = 2;
 
+// bf16 parts of the fp32 factors (flare_wave_bwd.h): two for the banks whose kernels hold states
+// and score gradients as bf16 hi + lo (the 16-bit kernels in flare_ar_bwd.hip and
+// flare_bwd_mfma.hip: M 128 and 256, D 64 and 128), three for the others, which were fp32
+// throughout.  Three take 437 us where two take 400 (bf16 B 2, N 2048, H 8, M 192, D 128), 305
+// and 295 (B 4, M 96, D 64, decoder weights of their own), 230 and 214 (B 4, N 2011, H 16, M 64,
+// D 32); of a 256 x 128 bank's X tiles three parts of both would not fit the LDS.
+template <typename T, int DT>
+bool three_parts(int64_t M) { return sizeof(T) == 2 && !((DT == 4 || DT == 8) && (M == 128 || M == 256)); }
+// CALL(P) with the bank's parts (no instance of two where there is no such bank)
+#define FLARE_WAVE_PARTS(CALL)                                     \
+    if constexpr (sizeof(T) == 2 && DT != 4 && DT != 8) {          \
+        return CALL(3);                                            \
+    } else {                                                       \
+        if constexpr (sizeof(T) == 2)                              \
+            if (three_parts<T, DT>(M)) return CALL(3);             \
+        return CALL(2);                                            \
+    }
+
 template <typename T, int DT>
 int launch_lse(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float scale, hipStream_t st) {
     const int64_t per = TT * kLseTiles * 4;
@@ -38,7 +56,7 @@ inline int allow_lds(const void* kernel, size_t lds, const char* name) {
     return FLARE_ERR_LAUNCH;
 }
 
-template <typename T, int MT, int DT, bool SEP>
+template <typename T, int MT, int DT, bool SEP, int P>
 int bwd_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk, hipStream_t st) {
     typedef TileRows<T, DT, SEP> Rows;
     const int NW = (int)((M + 16 * MT - 1) / (16 * MT));
@@ -47,18 +65,18 @@ int bwd_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float s
     int rc = launch_lse<T, DT>(p, B, N, H, M, scale, st);
     if (rc) return rc;
     const size_t walk_lds = 2 * Rows::BYTES + 2 * NW * TT * sizeof(float);     // row buffers, g . y sums
-    hipLaunchKernelGGL((wave_gz_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), walk_lds, st, p, (int)N, (int)H, (int)M,
+    hipLaunchKernelGGL((wave_gz_kernel<T, MT, DT, SEP, P>), grid, dim3(64 * NW), walk_lds, st, p, (int)N, (int)H, (int)M,
                        scale, (int)chunk);
     if ((rc = check_launch("wave_gz_kernel"))) return rc;
     if ((rc = launch_carry(p, NC, M, 16 * DT, B * H * M, st))) return rc;
-    const size_t lds = sizeof(float) * (size_t)NW * ds_wave_floats<T, MT, DT>() + Rows::BYTES;
-    if ((rc = allow_lds((const void*)wave_ds_kernel<T, MT, DT, SEP>, lds, "wave_ds_kernel"))) return rc;
-    hipLaunchKernelGGL((wave_ds_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), lds, st, p, (int)N, (int)H, (int)M, scale,
+    const size_t lds = sizeof(float) * (size_t)NW * ds_wave_floats<T, MT, DT, P>() + Rows::BYTES;
+    if ((rc = allow_lds((const void*)wave_ds_kernel<T, MT, DT, SEP, P>, lds, "wave_ds_kernel"))) return rc;
+    hipLaunchKernelGGL((wave_ds_kernel<T, MT, DT, SEP, P>), grid, dim3(64 * NW), lds, st, p, (int)N, (int)H, (int)M, scale,
                        (int)chunk);
     return check_launch("wave_ds_kernel");
 }
 
-template <typename T, int MT, int DT, bool SEP>
+template <typename T, int MT, int DT, bool SEP, int P>
 int semi_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk, int64_t block,
             hipStream_t st) {
     typedef StepRows<T, DT, SEP ? 3 : 2> Rows;
@@ -68,13 +86,13 @@ int semi_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float 
     int rc = launch_lse<T, DT>(p, B, N, H, M, scale, st);
     if (rc) return rc;
     const size_t walk_lds = 2 * Rows::BYTES + 2 * NW * TT * sizeof(float);
-    hipLaunchKernelGGL((wave_semi_gz_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), walk_lds, st, p, (int)N, (int)H,
+    hipLaunchKernelGGL((wave_semi_gz_kernel<T, MT, DT, SEP, P>), grid, dim3(64 * NW), walk_lds, st, p, (int)N, (int)H,
                        (int)M, scale, (int)chunk, (int)block);
     if ((rc = check_launch("wave_semi_gz_kernel"))) return rc;
     if ((rc = launch_carry(p, NC, M, 16 * DT, B * H * M, st))) return rc;
-    const size_t lds = sizeof(float) * (size_t)NW * semi_wave_floats<T, MT, DT>() + Rows::BYTES;
-    if ((rc = allow_lds((const void*)wave_semi_ds_kernel<T, MT, DT, SEP>, lds, "wave_semi_ds_kernel"))) return rc;
-    hipLaunchKernelGGL((wave_semi_ds_kernel<T, MT, DT, SEP>), grid, dim3(64 * NW), lds, st, p, (int)N, (int)H, (int)M, scale,
+    const size_t lds = sizeof(float) * (size_t)NW * semi_wave_floats<T, MT, DT, P>() + Rows::BYTES;
+    if ((rc = allow_lds((const void*)wave_semi_ds_kernel<T, MT, DT, SEP, P>, lds, "wave_semi_ds_kernel"))) return rc;
+    hipLaunchKernelGGL((wave_semi_ds_kernel<T, MT, DT, SEP, P>), grid, dim3(64 * NW), lds, st, p, (int)N, (int)H, (int)M, scale,
                        (int)chunk, (int)block);
     return check_launch("wave_semi_ds_kernel");
 }
@@ -82,17 +100,21 @@ int semi_at(const BwdPtrs& p, int64_t B, int64_t N, int64_t H, int64_t M, float 
 template <typename T, int DT>
 int bwd_dt(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk,
            hipStream_t st) {
-    constexpr int MT = kWalkTiles;
-    return sep ? bwd_at<T, MT, DT, true>(p, B, N, H, M, scale, chunk, st)
-               : bwd_at<T, MT, DT, false>(p, B, N, H, M, scale, chunk, st);
+#define FLARE_CALL(P)                                                               \
+    (sep ? bwd_at<T, kWalkTiles, DT, true, P>(p, B, N, H, M, scale, chunk, st)      \
+         : bwd_at<T, kWalkTiles, DT, false, P>(p, B, N, H, M, scale, chunk, st))
+    FLARE_WAVE_PARTS(FLARE_CALL)
+#undef FLARE_CALL
 }
 
 template <typename T, int DT>
 int semi_dt(const BwdPtrs& p, bool sep, int64_t B, int64_t N, int64_t H, int64_t M, float scale, int64_t chunk,
             int64_t block, hipStream_t st) {
-    constexpr int MT = kWalkTiles;
-    return sep ? semi_at<T, MT, DT, true>(p, B, N, H, M, scale, chunk, block, st)
-               : semi_at<T, MT, DT, false>(p, B, N, H, M, scale, chunk, block, st);
+#define FLARE_CALL(P)                                                                      \
+    (sep ? semi_at<T, kWalkTiles, DT, true, P>(p, B, N, H, M, scale, chunk, block, st)     \
+         : semi_at<T, kWalkTiles, DT, false, P>(p, B, N, H, M, scale, chunk, block, st))
+    FLARE_WAVE_PARTS(FLARE_CALL)
+#undef FLARE_CALL
 }
 
 template <typename T, int DT>
@@ -110,23 +132,37 @@ int semi_output_dt(const WaveArgs& a, int64_t block, const float* z, void* Y, in
     return check_launch("wave_semi_output_kernel");
 }
 
-template <typename T, int DT>
-int rows_dt(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, float scale,
+template <typename T, int DT, int P>
+int rows_at(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, float scale,
             void* out, hipStream_t st) {
     const int64_t per = 4 * TT * kRowTiles;
-    hipLaunchKernelGGL((wave_rows_kernel<T, DT>), dim3((unsigned)((N + per - 1) / per), (unsigned)(B * H)), dim3(256), 0, st,
+    hipLaunchKernelGGL((wave_rows_kernel<T, DT, P>), dim3((unsigned)((N + per - 1) / per), (unsigned)(B * H)), dim3(256), 0, st,
                        p, (const T*)r1, (const T*)r2, (int)N, (int)H, (int)M, scale, (T*)out);
     return check_launch("wave_rows_kernel");
 }
-template <typename T, int DT>
-int cols_dt(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, float* P,
+template <typename T, int DT, int P>
+int cols_at(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, float* partial,
             hipStream_t st) {
     constexpr int MT = DT <= 4 ? 2 : 1;
-    hipLaunchKernelGGL((wave_cols_kernel<T, MT, DT>),
+    hipLaunchKernelGGL((wave_cols_kernel<T, MT, DT, P>),
                        dim3((unsigned)((N + kBwdGroup - 1) / kBwdGroup), (unsigned)((M + 16 * MT - 1) / (16 * MT)),
                             (unsigned)(B * H)),
-                       dim3(256), 0, st, p, (const T*)r1, (const T*)r2, (int)N, (int)H, (int)M, P);
+                       dim3(256), 0, st, p, (const T*)r1, (const T*)r2, (int)N, (int)H, (int)M, partial);
     return check_launch("wave_cols_kernel");
+}
+template <typename T, int DT>
+int rows_dt(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, float scale,
+            void* out, hipStream_t st) {
+#define FLARE_CALL(P) (rows_at<T, DT, P>(p, r1, r2, B, N, H, M, scale, out, st))
+    FLARE_WAVE_PARTS(FLARE_CALL)
+#undef FLARE_CALL
+}
+template <typename T, int DT>
+int cols_dt(const ContractPtrs& p, const void* r1, const void* r2, int64_t B, int64_t N, int64_t H, int64_t M, float* partial,
+            hipStream_t st) {
+#define FLARE_CALL(P) (cols_at<T, DT, P>(p, r1, r2, B, N, H, M, partial, st))
+    FLARE_WAVE_PARTS(FLARE_CALL)
+#undef FLARE_CALL
 }
 
 #define FLARE_WAVE_DT_CASES(NAME, ...)                                                       \

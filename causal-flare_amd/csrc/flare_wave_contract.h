@@ -1,6 +1,6 @@
 // flare_wave_contract.h -- the backward's contractions of the score gradients with the token
-// and latent rows, on the products of flare_wave_bwd.h (fp32 MFMA for fp32 inputs, bf16 hi +
-// lo for 16-bit ones):
+// and latent rows, on the products of flare_wave_bwd.h (fp32 MFMA for fp32 inputs, bf16
+// parts for 16-bit ones):
 //   rows   out[t][d] = scale sum_m G[t][m] R[m][d]            (dK, dQ_dec)
 //   cols   P[group][m][d] = sum_{t in group} G[t][m] R[t][d]  (dQ, dK_dec, before the sum
 //                                                              over groups and sequences)
@@ -49,12 +49,12 @@ __device__ __forceinline__ GradSrc grad_src(const ContractPtrs& p, bool own, int
 // grid (ceil(N / 128), B*H), four waves of 32 tokens.  r1 / r2: rows [H, M, D] that ds / da
 // contract with (either may be null).
 constexpr int kRowTiles = 2;
-template <typename T, int DT>
+template <typename T, int DT, int P>
 __global__ __launch_bounds__(256) void wave_rows_kernel(ContractPtrs p, const T* __restrict__ r1, const T* __restrict__ r2,
                                                         int N, int H, int M, float scale, T* __restrict__ out) {
     constexpr int D = 16 * DT;
     constexpr int OD = sizeof(T) == 4 ? FLARE_F32 : __is_same(T, __half) ? FLARE_F16 : FLARE_BF16;
-    typedef typename ProdOf<T>::F F;
+    typedef typename ProdOf<T, P>::F F;
     const int bh = blockIdx.y, b = bh / H, h = bh % H;
     const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
     const int t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * TT * kRowTiles;
@@ -100,23 +100,23 @@ __global__ __launch_bounds__(256) void wave_rows_kernel(ContractPtrs p, const T*
 #pragma unroll
             for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
                 float o[4];
-                const int P = piece_of<DT>(dt);
+                const int cols = piece_of<DT>(dt);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = e < P ? scale * acc[k][dt + e < DT ? dt + e : 0][i] : 0.0f;
+                for (int e = 0; e < 4; ++e) o[e] = e < cols ? scale * acc[k][dt + e < DT ? dt + e : 0][i] : 0.0f;
                 const size_t at = row + col_of<DT>(dt, c);
-                if (P == 4) store_cols<4>(out, at, o, OD);
-                else if (P == 2) store_cols<2>(out, at, o, OD);
+                if (cols == 4) store_cols<4>(out, at, o, OD);
+                else if (cols == 2) store_cols<2>(out, at, o, OD);
                 else store_cols<1>(out, at, o, OD);
             }
         }
 }
 
 // grid (groups, ceil(M / (16 MT)), B*H), four waves.  r1 / r2: rows [B, N, H, D].
-template <typename T, int MT, int DT>
+template <typename T, int MT, int DT, int P>
 __global__ __launch_bounds__(256) void wave_cols_kernel(ContractPtrs p, const T* __restrict__ r1, const T* __restrict__ r2,
-                                                        int N, int H, int M, float* __restrict__ P) {
+                                                        int N, int H, int M, float* __restrict__ partial) {
     constexpr int D = 16 * DT, PITCH = D + 4;
-    typedef typename ProdOf<T>::F F;
+    typedef typename ProdOf<T, P>::F F;
     __shared__ __attribute__((aligned(16))) float part[4][16 * MT][PITCH];
     const int bh = blockIdx.z, b = bh / H, h = bh % H;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void wave_cols_kernel(ContractPtrs p, const T*
     for (int x = threadIdx.x; x < 16 * MT * D; x += 256) {
         const int m = x / D, d = x % D;
         if (mb + m < M)
-            P[(((size_t)bh * gridDim.x + blockIdx.x) * M + mb + m) * D + d] =
+            partial[(((size_t)bh * gridDim.x + blockIdx.x) * M + mb + m) * D + d] =
                 (part[0][m][d] + part[1][m][d]) + (part[2][m][d] + part[3][m][d]);
     }
 }

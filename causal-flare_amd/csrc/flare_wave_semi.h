@@ -170,11 +170,11 @@ __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restri
 // Forward walk: grid (NC, B*H), one wave per MT*16 latents.  chunk and N are multiples of
 // block, block a multiple of 16.
 // ---------------------------------------------------------------------------
-template <typename T, int MT, int DT, bool SEP>
+template <typename T, int MT, int DT, bool SEP, int P>
 __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a, int N, int H, int M, float scale,
                                                                       int chunk, int block) {
     constexpr int D = 16 * DT, R = SEP ? 3 : 2;
-    typedef typename ProdOf<T>::F F;
+    typedef typename ProdOf<T, P>::F F;
     typedef StepRows<T, DT, R> Rows;
     constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>(), FLAT = sizeof(T) == 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
 #pragma unroll
                     for (int i = 0; i < 4; ++i) z[i] *= scale;
                 }
-                const f32x4 p = dot_state<T, DT>(gr, u[mt], f32x4{0.f, 0.f, 0.f, 0.f});
+                const f32x4 p = dot_state<T, DT, P>(gr, u[mt], f32x4{0.f, 0.f, 0.f, 0.f});
                 float w[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -373,20 +373,20 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
 // ---------------------------------------------------------------------------
 template <int DT>
 __host__ __device__ constexpr bool semi_x_stays() { return DT <= 4; }
-template <typename T, int MT, int DT>
+template <typename T, int MT, int DT, int P>
 __host__ __device__ constexpr int semi_wave_floats() {
-    const int xt = MT * StateTile<T, DT>::FLOATS, dv = TT * dv_pitch(DT);
+    const int xt = (one_x_tile<T, DT, P>() ? 1 : MT) * StateTile<T, DT, P>::FLOATS, dv = TT * dv_pitch(DT);
     return semi_x_stays<DT>() ? xt + dv : (xt > dv ? xt : dv);
 }
 
-template <typename T, int MT, int DT, bool SEP>
+template <typename T, int MT, int DT, bool SEP, int P>
 __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a, int N, int H, int M, float scale,
                                                                       int chunk, int block) {
-    constexpr int D = 16 * DT, VP = dv_pitch(DT), R = SEP ? 3 : 2, WF = semi_wave_floats<T, MT, DT>();
-    typedef StateTile<T, DT> XTile;
-    constexpr bool STAYS = semi_x_stays<DT>();
+    constexpr int D = 16 * DT, VP = dv_pitch(DT), R = SEP ? 3 : 2, WF = semi_wave_floats<T, MT, DT, P>();
+    typedef StateTile<T, DT, P> XTile;
+    constexpr bool STAYS = semi_x_stays<DT>(), ONE = one_x_tile<T, DT, P>();
     constexpr int OD = sizeof(T) == 4 ? FLARE_F32 : __is_same(T, __half) ? FLARE_F16 : FLARE_BF16;
-    typedef typename ProdOf<T>::F F;
+    typedef typename ProdOf<T, P>::F F;
     typedef StepRows<T, DT, R> Rows;
     constexpr bool QREG = bwd_latents_in_regs<T, DT, SEP>(), FLAT = sizeof(T) == 2;
     extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -527,6 +527,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
             WalkRow<T, DT> vr;
             vr.load(Rows::row(tl, 1, c), g);
             F ef[MT];
+            f32x4 dv[DT];
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 if constexpr (!QREG) latent_row(q[0], a.Q, mt);
@@ -534,8 +535,8 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
                 const f32x4 s = dot_groups(kr, qm, f32x4{0.f, 0.f, 0.f, 0.f});       // [tau][m]
                 const f32x4 st = dot_groups(qm, kr, f32x4{0.f, 0.f, 0.f, 0.f});      // [m][tau]
                 const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-                const f32x4 xz = STAYS ? XTile::dot(xtile + mt * XTile::FLOATS, vr, x[mt], g, c, zero)
-                                       : XTile::put_dot(xtile + mt * XTile::FLOATS, vr, x[mt], g, c, zero);
+                float* xt = xtile + (ONE ? 0 : mt * XTile::FLOATS);
+                const f32x4 xz = STAYS ? XTile::dot(xt, vr, x[mt], g, c, zero) : XTile::put_dot(xt, vr, x[mt], g, c, zero);
                 float et[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -545,19 +546,25 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
                     et[i] = mb + 16 * mt + 4 * g + i < M ? exp_nat(st[i] * scale - mrow[mt][i]) : 0.0f;
                 }
                 ef[mt] = factor<F>(et[0], et[1], et[2], et[3]);
+                if constexpr (ONE) {
+                    wave_lds_sync();
+                    add_state_product<XTile, T, DT>(dv, xt, ef[mt], mt == 0, g, c);
+                    wave_lds_sync();
+                }
             }
-            wave_lds_sync();
-            f32x4 dv[DT];
+            if constexpr (!ONE) {
+                wave_lds_sync();
 #pragma unroll
-            for (int d1 = 0; d1 < DT; d1 += step_of<T, DT>(d1)) {
-                typename XTile::Cols xc[MT];
+                for (int d1 = 0; d1 < DT; d1 += step_of<T, DT>(d1)) {
+                    typename XTile::Cols xc[MT];
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) xc[mt].load_piece(xtile + mt * XTile::FLOATS, g, c, d1);
+                    for (int mt = 0; mt < MT; ++mt) xc[mt].load_piece(xtile + mt * XTile::FLOATS, g, c, d1);
 #pragma unroll
-                for (int dt = d1; dt < d1 + step_of<T, DT>(d1); ++dt) {
-                    dv[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    for (int dt = d1; dt < d1 + step_of<T, DT>(d1); ++dt) {
+                        dv[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) dv[dt] = mm(xc[mt].op(dt), ef[mt], dv[dt]);
+                        for (int mt = 0; mt < MT; ++mt) dv[dt] = mm(xc[mt].op(dt), ef[mt], dv[dt]);
+                    }
                 }
             }
             wave_lds_sync();
