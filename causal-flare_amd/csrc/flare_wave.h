@@ -166,6 +166,14 @@ __host__ __device__ constexpr int piece_of(int dt) {   // size of that piece
     constexpr int full = DT / 4 * 4;
     return dt < full ? 4 : DT - full == 3 ? (dt - full < 2 ? 2 : 1) : DT - full;
 }
+// The pieces by number: a loop that steps by piece_of does not unroll for DT = 3 and 6, and the
+// register arrays that its body indexes then lie in memory (up to 592 bytes a lane; a training
+// step of fp32 B 1, N 2048, H 8, M 128, D 96 took 329 us so and takes 256, block-causal in blocks of
+// 64 408 and 271, fp16 B 2, M 256, D 96 428 and 387).
+template <int DT>
+__host__ __device__ constexpr int pieces() { return DT / 4 + (DT % 4 == 0 ? 0 : DT % 4 == 3 ? 2 : 1); }
+template <int DT>
+__host__ __device__ constexpr int piece_start(int p) { return p <= DT / 4 ? 4 * p : DT / 4 * 4 + 2; }
 // column of tile dt at lane c
 template <int DT>
 __device__ __forceinline__ int col_of(int dt, int c) {
@@ -188,7 +196,7 @@ struct ColRow {
     unsigned w[W];
     __device__ __forceinline__ void load(const T* row, int c) {
 #pragma unroll
-        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) load_piece(row, c, dt);
+        for (int pc = 0, dt = 0; pc < pieces<DT>(); dt = piece_start<DT>(++pc)) load_piece(row, c, dt);
     }
     // the columns of the piece that starts at tile dt
     __device__ __forceinline__ void load_piece(const T* row, int c, int dt) {
@@ -213,7 +221,7 @@ struct ColRow {
     // the same from a buffer: `row` is the row's byte offset
     __device__ __forceinline__ void load(const Bytes& b, unsigned row, int c) {
 #pragma unroll
-        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
+        for (int pc = 0, dt = 0; pc < pieces<DT>(); dt = piece_start<DT>(++pc)) {
             const int P = piece_of<DT>(dt), E = (int)sizeof(T);
             const unsigned at = row + c * (P * E) + 16 * dt * E;
             const int k = sizeof(T) == 4 ? dt : dt / 2;
@@ -288,6 +296,8 @@ __device__ __forceinline__ void wave_lds_sync() {
 // they are fp32 rows of 96 columns or more (64 registers at D = 128): those are read again
 // each tile, from cache.  The next tile's tokens are fetched ahead up to D = 64; beyond, the
 // second wave of a SIMD covers the latency (fetching ahead spilled 92 to 764 bytes a lane).
+// Without it wave_output still spills 216 bytes in fp32 at D = 128 with decoder weights of its own
+// (16 with shared ones), and 12 to 56 in fp16 at D 96 and 128.
 template <typename T, int DT, bool SEP>
 constexpr bool latents_in_regs() { return sizeof(T) == 2 ? (DT <= 6 || !SEP) : (DT <= 3 || (DT == 4 && !SEP)); }
 template <int DT>
@@ -428,7 +438,7 @@ __global__ __launch_bounds__(wave_threads(MT)) void wave_prepare_kernel(
             }
             float* row = cnum + si * D;
 #pragma unroll
-            for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
+            for (int pc = 0, dt = 0; pc < pieces<DT>(); dt = piece_start<DT>(++pc))
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     float* p = row + col_of<DT>(dt, 4 * g + i);
@@ -762,7 +772,7 @@ __global__ __launch_bounds__(wave_threads(MT)) void wave_output_kernel(
             for (int i = 0; i < 4; ++i) {
                 const unsigned row = (rows >> (4 * g + i)) & 1 ? (unsigned)(t - t0 + 4 * g + i) * ostride : kNowhere;
 #pragma unroll
-                for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
+                for (int pc = 0, dt = 0; pc < pieces<DT>(); dt = piece_start<DT>(++pc)) {
                     float o[4];
                     const int P = piece_of<DT>(dt);
 #pragma unroll

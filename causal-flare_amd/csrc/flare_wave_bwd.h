@@ -76,6 +76,17 @@ __host__ __device__ constexpr int walk_piece(int dt) { return FLAT ? 1 : piece_o
 // and spilled at D = 64: 130 against 119 us for the forward walk)
 template <typename T, int DT>
 __host__ __device__ constexpr int step_of(int dt) { return sizeof(T) == 2 ? (dt + 2 <= DT ? 2 : 1) : piece_of<DT>(dt); }
+// these by number, and the most tiles a step has (see pieces: loops over them have to unroll)
+template <int DT, bool FLAT>
+__host__ __device__ constexpr int walk_pieces() { return FLAT ? DT : pieces<DT>(); }
+template <int DT, bool FLAT>
+__host__ __device__ constexpr int walk_start(int p) { return FLAT ? p : piece_start<DT>(p); }
+template <typename T, int DT>
+__host__ __device__ constexpr int steps() { return sizeof(T) == 2 ? (DT + 1) / 2 : pieces<DT>(); }
+template <typename T, int DT>
+__host__ __device__ constexpr int step_start(int s) { return sizeof(T) == 2 ? 2 * s : piece_start<DT>(s); }
+template <typename T>
+__host__ __device__ constexpr int step_most() { return sizeof(T) == 2 ? 2 : 4; }
 template <int DT, bool FLAT>
 __device__ __forceinline__ int walk_col(int dt, int c) { return FLAT ? 16 * dt + c : col_of<DT>(dt, c); }
 
@@ -96,7 +107,7 @@ struct GroupRow {
     unsigned w[W];
     __device__ __forceinline__ void load(const T* row, int g) {
 #pragma unroll
-        for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt)) {
+        for (int pc = 0, dt = 0; pc < walk_pieces<DT, FLAT>(); dt = walk_start<DT, FLAT>(++pc)) {
             const int P = walk_piece<DT, FLAT>(dt);
             const T* p = row + 16 * dt + 4 * g * P;
             // 4 P values
@@ -367,7 +378,8 @@ struct TileCols {
     __device__ __forceinline__ void load_piece(const T* tile, int pitch, int g, int c, int d0) {
         if constexpr (FLAT) {
 #pragma unroll
-            for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) r[dt] = tile_tr(tile + 16 * dt, pitch, g, c);
+            for (int dt = d0; dt < d0 + step_most<T>(); ++dt)
+                if (dt < d0 + step_of<T, DT>(d0)) r[dt] = tile_tr(tile + 16 * dt, pitch, g, c);
         } else {
 #pragma unroll
             for (int i = 0; i < 4; ++i) r[i].load_piece(tile + (4 * g + i) * pitch, c, d0);
@@ -379,7 +391,8 @@ struct TileCols {
             const unsigned m0 = (on[0] ? 0xffffu : 0u) | (on[1] ? 0xffff0000u : 0u);
             const unsigned m1 = (on[2] ? 0xffffu : 0u) | (on[3] ? 0xffff0000u : 0u);
 #pragma unroll
-            for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
+            for (int dt = d0; dt < d0 + step_most<T>(); ++dt) {
+                if (dt >= d0 + step_of<T, DT>(d0)) continue;
                 r[dt][0] &= m0;
                 r[dt][1] &= m1;
             }
@@ -387,7 +400,8 @@ struct TileCols {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int k = d0; k < d0 + step_of<T, DT>(d0); ++k) r[i].w[k] = on[i] ? r[i].w[k] : 0u;
+                for (int k = d0; k < d0 + step_most<T>(); ++k)
+                    if (k < d0 + step_of<T, DT>(d0)) r[i].w[k] = on[i] ? r[i].w[k] : 0u;
         }
     }
     __device__ __forceinline__ Op op(int dt) const {
@@ -424,7 +438,7 @@ struct StateTile {
     }
     static __device__ __forceinline__ void put(float* tile, const f32x4 (&u)[DT], int g, int c) {
 #pragma unroll
-        for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt)) {
+        for (int pc = 0, dt = 0; pc < walk_pieces<DT, FLAT>(); dt = walk_start<DT, FLAT>(++pc)) {
             if constexpr (FLAT) {
                 put_parts(tile, split4<P>(u[dt]), g, c, dt);
             } else {
@@ -485,8 +499,9 @@ struct StateTile {
         __device__ __forceinline__ void load_piece(const float* tile, int g, int c, int d0) {
             if constexpr (FLAT) {
 #pragma unroll
-                for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt)
-                    r[dt] = split_tr<P>((const bf16x4*)tile + 4 * dt, QUADS, PITCH, g, c);
+                for (int dt = d0; dt < d0 + step_most<T>(); ++dt)
+                    if (dt < d0 + step_of<T, DT>(d0))
+                        r[dt] = split_tr<P>((const bf16x4*)tile + 4 * dt, QUADS, PITCH, g, c);
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) r[i].load_piece(tile + (4 * g + i) * PITCH, c, d0);
@@ -503,12 +518,13 @@ struct StateTile {
 template <typename Tile, typename T, int DT, typename F>
 __device__ __forceinline__ void add_state_product(f32x4 (&dv)[DT], const float* tile, const F& e, bool first, int g, int c) {
 #pragma unroll
-    for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
+    for (int st = 0, d0 = 0; st < steps<T, DT>(); d0 = step_start<T, DT>(++st)) {
         typename Tile::Cols xc;
         xc.load_piece(tile, g, c, d0);
 #pragma unroll
-        for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt)
-            dv[dt] = mm(xc.op(dt), e, first ? f32x4{0.f, 0.f, 0.f, 0.f} : dv[dt]);
+        for (int dt = d0; dt < d0 + step_most<T>(); ++dt)
+            if (dt < d0 + step_of<T, DT>(d0))
+                dv[dt] = mm(xc.op(dt), e, first ? f32x4{0.f, 0.f, 0.f, 0.f} : dv[dt]);
     }
 }
 
@@ -546,7 +562,7 @@ struct TurnTile {
 template <int DT, bool FLAT>
 __device__ __forceinline__ void put_rows(float* rows, int pitch, const f32x4 (&dv)[DT], int g, int c) {
 #pragma unroll
-    for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt)) {
+    for (int pc = 0, dt = 0; pc < walk_pieces<DT, FLAT>(); dt = walk_start<DT, FLAT>(++pc)) {
         if constexpr (FLAT) {
             *reinterpret_cast<f32x4_a*>(rows + c * pitch + 16 * dt + 4 * g) = dv[dt];
         } else {
@@ -578,7 +594,10 @@ __device__ __forceinline__ float token_value(const float (&x)[4], int j, int c) 
 
 
 // Registers: the latents' rows stay there up to D = 64 (fp32: 32), else they are read again
-// each tile, from cache.
+// each tile, from cache.  Wide states spill all the same, and the spilled values come back once a
+// tile: at D = 128 wave_gz 548 bytes a lane in fp32 (584 with decoder weights of its own; D = 96
+// 216 and 300), 24 to 140 with three parts and at most 112 with two; wave_ds 120 in fp32, 88 to
+// 184 with three parts; wave_semi_gz 48 (268) in fp32 and 20 to 112 in 16 bits.
 template <typename T, int DT, bool SEP>
 constexpr bool bwd_latents_in_regs() { return sizeof(T) == 2 ? DT <= 4 : DT <= (SEP ? 2 : 3); }
 
@@ -910,13 +929,14 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
         }
         // U += E^T V, X += W^T g, a piece of value columns at a time
 #pragma unroll
-        for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
+        for (int st = 0, d0 = 0; st < steps<T, DT>(); d0 = step_start<T, DT>(++st)) {
             stage<DT>();
             TileCols<T, DT> vc, gc;
             vc.load_piece(Rows::row(tl, 1, 0), Rows::PITCH, g, c, d0);
             gc.load_piece(Rows::row(tl, 2, 0), Rows::PITCH, g, c, d0);
 #pragma unroll
-            for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
+            for (int dt = d0; dt < d0 + step_most<T>(); ++dt) {
+                if (dt >= d0 + step_of<T, DT>(d0)) continue;
                 const auto vo = vc.op(dt), go = gc.op(dt);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
@@ -947,7 +967,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
             if (g == 0) a.ysum[pbase + m] = ysum[mt];
             float* row = a.xsum + (pbase + m) * D;
 #pragma unroll
-            for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt))
+            for (int pc = 0, dt = 0; pc < walk_pieces<DT, FLAT>(); dt = walk_start<DT, FLAT>(++pc))
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1224,7 +1244,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
         // the product above too early on the skipped side.)
         const bool on[4] = {j < 0 || 4 * g == j, j < 0 || 4 * g + 1 == j, j < 0 || 4 * g + 2 == j, j < 0 || 4 * g + 3 == j};
 #pragma unroll
-        for (int d1 = 0; d1 < DT; d1 += step_of<T, DT>(d1)) {
+        for (int st = 0, d1 = 0; st < steps<T, DT>(); d1 = step_start<T, DT>(++st)) {
             stage<DT>();
             typename XTile::Cols xc[ONE ? 1 : MT];
             TileCols<T, DT> gc;
@@ -1235,7 +1255,8 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
             }
             gc.keep(on, d1);
 #pragma unroll
-            for (int dt = d1; dt < d1 + step_of<T, DT>(d1); ++dt) {
+            for (int dt = d1; dt < d1 + step_most<T>(); ++dt) {
+                if (dt >= d1 + step_of<T, DT>(d1)) continue;
                 f32x4 r = {0.f, 0.f, 0.f, 0.f};
                 if constexpr (ONE) {
                     r = dv[dt];

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void wave_rows_kernel(ContractPtrs p, const T*
             if (t >= N) continue;
             const size_t row = (((size_t)b * N + t) * H + h) * D;
 #pragma unroll
-            for (int dt = 0; dt < DT; dt += piece_of<DT>(dt)) {
+            for (int pc = 0, dt = 0; pc < pieces<DT>(); dt = piece_start<DT>(++pc)) {
                 float o[4];
                 const int cols = piece_of<DT>(dt);
 #pragma unroll
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(256) void wave_cols_kernel(ContractPtrs p, const T*
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
+        for (int pc = 0, dt = 0; pc < pieces<DT>(); dt = piece_start<DT>(++pc))
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll

@@ -150,7 +150,7 @@ __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restri
         const int t = t0 + TT * j + c;
         const size_t row = (((size_t)b * N + t) * H + h) * D;
 #pragma unroll
-        for (int dt = 0; dt < DT; dt += piece_of<DT>(dt))
+        for (int pc = 0, dt = 0; pc < pieces<DT>(); dt = piece_start<DT>(++pc))
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 float o[4];
@@ -289,11 +289,12 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
                 }
             }
 #pragma unroll
-            for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
+            for (int st = 0, d0 = 0; st < steps<T, DT>(); d0 = step_start<T, DT>(++st)) {
                 TileCols<T, DT> vc;
                 vc.load_piece(Rows::row(tl, 1, 0), Rows::PITCH, g, c, d0);
 #pragma unroll
-                for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
+                for (int dt = d0; dt < d0 + step_most<T>(); ++dt) {
+                    if (dt >= d0 + step_of<T, DT>(d0)) continue;
                     const auto vo = vc.op(dt);
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) u[mt][dt] = collect(vo, f[mt], u[mt][dt]);
@@ -331,11 +332,12 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
             }
             if constexpr (own_gy<T>()) put_gy(gsum + buf * NW * TT, gy, wv, g, c);
 #pragma unroll
-            for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
+            for (int st = 0, d0 = 0; st < steps<T, DT>(); d0 = step_start<T, DT>(++st)) {
                 TileCols<T, DT> gc;
                 gc.load_piece(Rows::row(tl, 1, 0), Rows::PITCH, g, c, d0);
 #pragma unroll
-                for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
+                for (int dt = d0; dt < d0 + step_most<T>(); ++dt) {
+                    if (dt >= d0 + step_of<T, DT>(d0)) continue;
                     const auto go = gc.op(dt);
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) x[mt][dt] = collect(go, f[mt], x[mt][dt]);
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
             if (g == 0) a.ysum[pbase + m] = ysum[mt];
             float* row = a.xsum + (pbase + m) * D;
 #pragma unroll
-            for (int dt = 0; dt < DT; dt += walk_piece<DT, FLAT>(dt))
+            for (int pc = 0, dt = 0; pc < walk_pieces<DT, FLAT>(); dt = walk_start<DT, FLAT>(++pc))
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -502,11 +504,12 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
                 wf[mt] = factor<F>(w[0], w[1], w[2], w[3]);
             }
 #pragma unroll
-            for (int d0 = 0; d0 < DT; d0 += step_of<T, DT>(d0)) {
+            for (int st = 0, d0 = 0; st < steps<T, DT>(); d0 = step_start<T, DT>(++st)) {
                 TileCols<T, DT> gc;
                 gc.load_piece(Rows::row(tl, 1, 0), Rows::PITCH, g, c, d0);
 #pragma unroll
-                for (int dt = d0; dt < d0 + step_of<T, DT>(d0); ++dt) {
+                for (int dt = d0; dt < d0 + step_most<T>(); ++dt) {
+                    if (dt >= d0 + step_of<T, DT>(d0)) continue;
                     const auto go = gc.op(dt);
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) x[mt][dt] = collect(go, wf[mt], x[mt][dt]);
@@ -555,12 +558,13 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
             if constexpr (!ONE) {
                 wave_lds_sync();
 #pragma unroll
-                for (int d1 = 0; d1 < DT; d1 += step_of<T, DT>(d1)) {
+                for (int st = 0, d1 = 0; st < steps<T, DT>(); d1 = step_start<T, DT>(++st)) {
                     typename XTile::Cols xc[MT];
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) xc[mt].load_piece(xtile + mt * XTile::FLOATS, g, c, d1);
 #pragma unroll
-                    for (int dt = d1; dt < d1 + step_of<T, DT>(d1); ++dt) {
+                    for (int dt = d1; dt < d1 + step_most<T>(); ++dt) {
+                        if (dt >= d1 + step_of<T, DT>(d1)) continue;
                         dv[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                         for (int mt = 0; mt < MT; ++mt) dv[dt] = mm(xc[mt].op(dt), ef[mt], dv[dt]);
