@@ -593,11 +593,112 @@ __device__ __forceinline__ float token_value(const float (&x)[4], int j, int c) 
 }
 
 
+// ---------------------------------------------------------------------------
+// Value columns in which dY is not finite at this token or a later one.  Such a column of X, and of
+// dV from there back, is that infinity (NaN for both signs), which products do not give by
+// themselves: an infinity times the parts of a weight, or times the weight 0 of a latent past the
+// bank, is NaN.  Bit 4 dt + i stands for column walk_col(dt, 4g + i).  The backward walks keep the
+// bits in LDS, two words a lane group for the whole workgroup (a training step of N 16384, H 16, M
+// 256, D 128 takes 1420 us, 1409 without any of this and 1446 with the bits in registers).
+// ---------------------------------------------------------------------------
+template <typename T, int DT>
+struct WildCols {
+    static constexpr bool FLAT = sizeof(T) == 2;
+    unsigned pos = 0, neg = 0;
+    __device__ __forceinline__ void take(float v, int dt, int i) {
+        const unsigned bit = 1u << (4 * dt + i);
+        pos |= !(v <= 3.4e38f) ? bit : 0u;          // (NaN: both)
+        neg |= !(v >= -3.4e38f) ? bit : 0u;
+    }
+    __device__ __forceinline__ void take_row(const T* row, int g) {
+        for (int dt = 0; dt < DT; ++dt)
+            for (int i = 0; i < 4; ++i) {
+                const T v = row[walk_col<DT, FLAT>(dt, 4 * g + i)];
+                if constexpr (sizeof(T) == 4) take(v, dt, i);
+                else take(word_f32<T>(__builtin_bit_cast(unsigned short, v), false), dt, i);
+            }
+    }
+    __device__ __forceinline__ bool any() const { return __any((pos | neg) != 0); }
+    __device__ __forceinline__ bool has(int dt, int i) const { return ((pos | neg) >> (4 * dt + i)) & 1; }
+    __device__ __forceinline__ float value(int dt, int i) const {
+        const unsigned n = 4 * dt + i;
+        const float inf = __builtin_inff();
+        return (pos >> n) & (neg >> n) & 1 ? __builtin_nanf("") : (pos >> n) & 1 ? inf : -inf;
+    }
+    // a column is wild whichever lane shows it
+    __device__ __forceinline__ void add_to(unsigned* bits, int g) const {
+        if (pos != 0) __hip_atomic_fetch_or(bits + 2 * g, pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (neg != 0) __hip_atomic_fetch_or(bits + 2 * g + 1, neg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ void read(const unsigned* bits, int g) {
+        pos = bits[2 * g];
+        neg = bits[2 * g + 1];
+    }
+};
+// NaN where a value of a state is not finite
+template <int DT>
+__device__ __forceinline__ float state_probe(const f32x4 (&x)[DT]) {
+    float r = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r = __builtin_fmaf(x[dt][i], 0.0f, r);
+    return r;
+}
+// a chunk's terms of X: wild columns as they are to be
+template <typename T, int MT, int DT>
+__device__ __forceinline__ void set_wild(f32x4 (&x)[MT][DT], const T* rows, int stride, int t0, int t1, int g) {
+    float probe = 0.0f;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) probe += state_probe(x[mt]);
+    if (!__any(probe != probe)) return;
+    WildCols<T, DT> wild;
+    for (int t = t0; t < t1; ++t) wild.take_row(rows + (size_t)t * stride, g);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[mt][dt][i] = wild.has(dt, i) ? wild.value(dt, i) : x[mt][dt][i];
+}
+// whether X after a chunk has wild columns, which go to `bits`
+template <typename T, int MT, int DT>
+__device__ __forceinline__ bool find_wild(const f32x4 (&x)[MT][DT], unsigned* bits, int g) {
+    float probe = 0.0f;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) probe += state_probe(x[mt]);
+    if (!__any(probe != probe)) return false;
+    WildCols<T, DT> wild;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wild.take(x[mt][dt][i], dt, i);
+    wild.add_to(bits, g);
+    return true;
+}
+// a tile's dv rows in this wave's LDS: their wild columns
+template <typename T, int DT>
+__device__ __forceinline__ bool put_wild(float* rows, int pitch, const unsigned* bits, int g, int c) {
+    wave_lds_sync();
+    WildCols<T, DT> wild;
+    wild.read(bits, g);
+    if (!wild.any()) return false;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (wild.has(dt, i)) rows[c * pitch + walk_col<DT, sizeof(T) == 2>(dt, 4 * g + i)] = wild.value(dt, i);
+    return true;
+}
+
 // Registers: the latents' rows stay there up to D = 64 (fp32: 32), else they are read again
 // each tile, from cache.  Wide states spill all the same, and the spilled values come back once a
-// tile: at D = 128 wave_gz 548 bytes a lane in fp32 (584 with decoder weights of its own; D = 96
-// 216 and 300), 24 to 140 with three parts and at most 112 with two; wave_ds 120 in fp32, 88 to
-// 184 with three parts; wave_semi_gz 48 (268) in fp32 and 20 to 112 in 16 bits.
+// tile.  Bytes a lane at D = 128: wave_gz 564 in fp32 (592 with decoder weights of its own; 220 and
+// 300 at D = 96), 28 to 144 with three parts, at most 112 with two; wave_ds up to 140 in fp32, 104
+// to 192 with three parts, 8 to 40 with two; wave_semi_gz 48 (280) in fp32, 20 to 108 in 16 bits;
+// wave_semi_ds 124 in fp32, at most 64 in fp16.
 template <typename T, int DT, bool SEP>
 constexpr bool bwd_latents_in_regs() { return sizeof(T) == 2 ? DT <= 4 : DT <= (SEP ? 2 : 3); }
 
@@ -866,7 +967,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
             vr.load(Rows::row(tl, 1, c), g);
             const f32x4 r = dot_groups(vr, gr, f32x4{0.f, 0.f, 0.f, 0.f});
             // a value of g that is not finite shows in its products with v (0 times it is NaN); the
-            // backward walk then keeps it to its own token
+            // backward walk then keeps it to its own token (see WildCols)
             bad = __builtin_fmaf(r[0], 0.0f, __builtin_fmaf(r[1], 0.0f, __builtin_fmaf(r[2], 0.0f, r[3] * 0.0f)));
             gvf = factor<F>(4 * g <= c ? r[0] : 0.0f, 4 * g + 1 <= c ? r[1] : 0.0f, 4 * g + 2 <= c ? r[2] : 0.0f,
                             4 * g + 3 <= c ? r[3] : 0.0f);
@@ -959,6 +1060,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
         if constexpr (OWN_GY) store_gy(sums, NW, gy_out, t - TT, t1);
         if (t >= t1) break;
     }
+    set_wild<T, MT, DT>(x, (const T*)a.dY + tok, stride, t0, t1, g);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         ysum[mt] = group_sum(ysum[mt]);
@@ -1090,11 +1192,15 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
             for (int i = 0; i < 4; ++i) x[mt][dt][i] = r.at(list_at<DT, FLAT>(dt, i));
     }
 
+    __shared__ unsigned wild_bits[8];
+    if (threadIdx.x < 8) wild_bits[threadIdx.x] = 0;
+
     Rows rows;
     int t = t0 + (t1 - 1 - t0) / TT * TT, j = -1;
     rows.fetch(a, tok, stride, t, t1);
     rows.store(tl, a, tok, stride, t, t1);
     __syncthreads();
+    bool some_wild = find_wild<T, MT, DT>(x, wild_bits, g);
     while (true) {
         const bool begin = j < 0;
         if (begin) {
@@ -1274,6 +1380,15 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
         const bool last = j <= 0, more = last && t > t0;
         wave_lds_sync();
         put_rows<DT, FLAT>(vtile, VP, dv, g, c);
+        if (j >= 0 || some_wild) {
+            // (a token whose g is not finite is walked by itself)
+            if (j >= 0) {
+                WildCols<T, DT> wild;
+                wild.take_row(Rows::row(tl, 2, j), g);
+                wild.add_to(wild_bits, g);
+            }
+            some_wild = put_wild<T, DT>(vtile, VP, wild_bits, g, c);
+        }
         if (NW == 1) {
             wave_lds_sync();
             if (more) rows.store(tl, a, tok, stride, t - TT, t1);

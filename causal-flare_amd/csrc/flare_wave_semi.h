@@ -352,6 +352,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
         t = nt;
         pass = np;
     }
+    set_wild<T, MT, DT>(x, gb, stride, t0, t1, g);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         ysum[mt] = group_sum(ysum[mt]);
@@ -439,11 +440,15 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
             for (int i = 0; i < 4; ++i) x[mt][dt][i] = r.at(list_at<DT, FLAT>(dt, i));
     }
 
+    __shared__ unsigned wild_bits[8];
+    if (threadIdx.x < 8) wild_bits[threadIdx.x] = 0;
+
     Rows rows;
     int t = t1 - TT, pass = 0;
     rows.fetch(kb, gb, qb, stride, t);
     rows.store(tl, kb, gb, qb, stride, t);
     __syncthreads();
+    bool some_wild = find_wild<T, MT, DT>(x, wild_bits, g);
     while (true) {
         const bool begin = (t + TT) % block == 0, end = t % block == 0;     // first / last tile of a pass
         const int np = end ? pass ^ 1 : pass;
@@ -522,6 +527,13 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
                     part[mt] = 0.0f;
                     if constexpr (STAYS) XTile::put(xtile + mt * XTile::FLOATS, x[mt], g, c);
                 }
+                const float probe = state_probe(x[0]);
+                if (__any(probe != probe)) {          // (t is the block's first token)
+                    WildCols<T, DT> wild;
+                    for (int k = 0; k < block; ++k) wild.take_row(gb + (size_t)(t + k) * stride, g);
+                    wild.add_to(wild_bits, g);
+                    some_wild = true;
+                }
             }
             __syncthreads();
             if (more) rows.store(tl, kb, np ? vb : gb, np ? vb : qb, stride, nt);
@@ -573,6 +585,7 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_ds_kernel(BwdPtrs a,
             }
             wave_lds_sync();
             put_rows<DT, FLAT>(vtile, VP, dv, g, c);
+            if (some_wild) put_wild<T, DT>(vtile, VP, wild_bits, g, c);
             __syncthreads();
             if (more) rows.store(tl, kb, np ? vb : gb, np ? vb : qb, stride, nt);     // every wave is done with this tile
             for (int e = threadIdx.x; e < TT * D / 4; e += blockDim.x) {

@@ -340,3 +340,44 @@ def test_backward_of_own_decoder_weights_walks(B, N, H, M, D, block, layer):
     names = " ".join(e.key for e in prof.key_averages())
     walk = "wave_ds_kernel" if layer == "token" else "wave_semi_ds_kernel"
     assert walk in names and "wave_rows_kernel" in names and "wave_cols_kernel" in names, names
+
+
+@pytest.mark.parametrize("M,D,dtype", [(64, 32, torch.bfloat16), (48, 48, torch.float16), (128, 64, torch.bfloat16),
+                                       (80, 128, torch.float16), (256, 128, torch.bfloat16), (48, 32, torch.float32),
+                                       (64, 96, torch.float32)])
+@pytest.mark.parametrize("block", [0, 48])
+def test_wave_backward_infinite_gradients(M, D, dtype, block):
+    """Infinite dY entries make dV of their column infinite, with their sign, in their own and all
+    earlier tokens (of the block-causal layer: blocks); both signs give NaN.  Other columns are as
+    without them."""
+    from causal_flare import flare_semi_autoregressive_trition
+    print("CASE wave_infinite_gradients", M, D, dtype, block, flush=True)
+    B, N, H = 1, 240, 2
+    q, k, v = seeded(9 * M + D, B, N, H, M, D, D, dtype)
+    g = torch.randn(B, N, H, D, generator=torch.Generator().manual_seed(M)).to(dtype)
+
+    def dv(g):
+        leaves = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+        if block:
+            y, _ = flare_semi_autoregressive_trition(*leaves, block_size=block, chunk_size=16)
+        else:
+            from causal_flare import flare_autoregressive_triton
+            y = flare_autoregressive_triton(*leaves)
+        y.backward(g.to(DEV))
+        return leaves[2].grad.float().cpu()
+
+    inf = float("inf")
+    entries = [(37, 0, 5, inf), (150, 0, 5, inf), (201, 0, D - 1, -inf), (3, 0, D - 1, inf), (239, 1, 0, -inf)]
+    gi = g.clone()
+    want = dv(g)
+    wild = torch.zeros(N, H, D, dtype=torch.bool)
+    for t, h, d, x in entries:
+        gi[0, t, h, d] = x
+        last = (t // block + 1) * block if block else t + 1
+        new = torch.where(wild[:last, h, d], want[0, :last, h, d] + x, torch.full((last,), x))     # (inf - inf: NaN)
+        want[0, :last, h, d] = new
+        wild[:last, h, d] = True
+    got = dv(gi)
+    odd = wild[None]
+    assert torch.equal(torch.nan_to_num(got[odd], nan=7.0), torch.nan_to_num(want[odd], nan=7.0))
+    _check_grads({"v": got[~odd]}, [want[~odd].double().numpy()], dtype, "other columns")
