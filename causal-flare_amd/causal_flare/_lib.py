@@ -26,6 +26,7 @@ HEADER_FUNCTIONS = (
     "flare_ar_forward",
     "flare_ar_forward_masked",
     "flare_ar_default_chunk",
+    "flare_ar_tokenwise_chunk",
     "flare_stablemax_forward",
     "flare_stablemax_backward_workspace_size",
     "flare_stablemax_backward",
@@ -73,8 +74,9 @@ def _declare(lib):
     lib.flare_ar_forward_workspace_size.argtypes = [_i64] * 6
     lib.flare_ar_forward_workspace_size_sep.restype = _sz
     lib.flare_ar_forward_workspace_size_sep.argtypes = [_i64] * 6
-    lib.flare_ar_default_chunk.restype = _i64
-    lib.flare_ar_default_chunk.argtypes = [_i64] * 5
+    for fn in (lib.flare_ar_default_chunk, lib.flare_ar_tokenwise_chunk):
+        fn.restype = _i64
+        fn.argtypes = [_i64] * 5
     lib.flare_stablemax_forward.restype = _i
     lib.flare_stablemax_forward.argtypes = [_vp] * 5 + [_i] + [_i64] * 6 + [_f, _i64, _f, _vp, _i, _vp, _sz, _vp]
     lib.flare_stablemax_backward_workspace_size.restype = _sz

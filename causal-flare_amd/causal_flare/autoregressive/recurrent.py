@@ -93,7 +93,7 @@ class RecurrentFLARE(autograd.Function):
         if T == 0:
             Y = torch.empty((B, 0, H, D), device=K.device, dtype=Q.dtype)
         else:
-            _, chunk = _resolve_chunk_size(None, B, T, H, M, D)
+            _, chunk = _resolve_chunk_size(None, B, T, H, M, D, D)
             qd, kd = (None, None) if shared else _decoder_args(Q, K, Q_dec_r, K_dec_r, sep_q, sep_k)
             Y, _ = run_chunked_forward(Q, K, V, qd, kd, scale=scale, chunk=chunk, out_dtype=Q.dtype)
         ctx.scale = scale

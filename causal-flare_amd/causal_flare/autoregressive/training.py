@@ -34,13 +34,16 @@ from .._common import (
 from .._reference_utils import resolve_flare_causal_decode_inputs
 
 
-def _resolve_chunk_size(chunk_size, B, N, H, M, Dv, validate_only=False) -> tuple[int, int]:
+def _resolve_chunk_size(chunk_size, B, N, H, M, Dk, Dv, validate_only=False) -> tuple[int, int]:
     """(validated chunk_size, kernel chunk length).
 
     The reference's default chunk is 64 (training.py:328-337) and must be a
     multiple of 16 (:344).  Chunk length only changes fp32 rounding, so when
     neither ``chunk_size`` nor FLARE_CHUNK_SIZE is given the library's own
-    policy (about one chunk workgroup per compute unit) is used.
+    policy is used: one round of chunk workgroups over the device for the banks
+    of the 16-bit kernels, two waves a SIMD for the other banks, and for calls
+    on the tokenwise kernels (Dk != Dv) whichever of the two leaves fewer tokens
+    in line.
     """
     explicit = chunk_size
     if explicit is None:
@@ -51,7 +54,9 @@ def _resolve_chunk_size(chunk_size, B, N, H, M, Dv, validate_only=False) -> tupl
     if validate_only:
         return requested, requested
     if explicit is None:
-        return requested, int(_lib.lib().flare_ar_default_chunk(B, N, H, M, Dv))
+        lib = _lib.lib()
+        policy = lib.flare_ar_default_chunk if Dk == Dv else lib.flare_ar_tokenwise_chunk
+        return requested, int(policy(B, N, H, M, Dv))
     return requested, requested
 
 
@@ -207,7 +212,7 @@ class AutoRegressiveFLARE(autograd.Function):
         assert M % 16 == 0, f"M must be divisible by 16. Got M={M}."
         assert D_score % 16 == 0, f"score_head_dim must be divisible by 16. Got score_head_dim={D_score}."
         assert D_value % 16 == 0, f"value_head_dim must be divisible by 16. Got value_head_dim={D_value}."
-        _resolve_chunk_size(chunk_size, B, N, H, M, D_value, validate_only=True)
+        _resolve_chunk_size(chunk_size, B, N, H, M, D_score, D_value, validate_only=True)
         _require_gpu("flare_autoregressive_triton", Q, K, V, Q_dec, K_dec)
         # Output in the compute dtype of K (training.py:322-324, 724-727).
         out_dtype = K.dtype if K.dtype in (torch.bfloat16, torch.float16) else torch.float32
@@ -216,7 +221,7 @@ class AutoRegressiveFLARE(autograd.Function):
         if N == 0:
             Y = torch.empty((B, 0, H, D_value), device=K.device, dtype=out_dtype)
         else:
-            _, chunk = _resolve_chunk_size(chunk_size, B, N, H, M, D_value)
+            _, chunk = _resolve_chunk_size(chunk_size, B, N, H, M, D_score, D_value)
             qd, kd = (None, None) if shared else _decoder_args(Q, K, Q_dec_r, K_dec_r, sep_q, sep_k)
             Y, _ = run_chunked_forward(
                 Q, K, V, qd, kd, scale=scale, chunk=chunk, out_dtype=out_dtype,

@@ -7,9 +7,12 @@
 //                            inference.py:753-814)
 //   3. chunk_output_kernel   tokenwise replay from the chunk prefix and the
 //                            latent softmax readout                 (:1106-1392)
-// All arithmetic is fp32 on CUDA-core-equivalent VALU lanes; inputs may be
-// fp32, bf16 or fp16.  These kernels serve every dtype and shape; the bf16/fp16
-// MFMA kernels in flare_ar_mfma.hip take over the shapes they support.
+// All arithmetic of the kernels here is fp32 on VALU lanes; inputs may be fp32, bf16 or
+// fp16, of any shape.  Phases 1 and 3 go to the matrix products where a bank has an
+// instance: bf16 / fp16 of M 128 and 256, D 64 and 128 to flare_ar_pc.hip and
+// flare_ar_mfma.hip, other banks and fp32 to flare_wave.h (wave_supported below).  What is
+// left for the kernels here: Dk != Dv, other head dims, M > 256, tensors off 16 bytes, chunks
+// off 16 tokens, and the stablemax encoder of those banks.  Phase 2 serves them all.
 #include <stdarg.h>
 #include <stdio.h>
 
@@ -469,8 +472,11 @@ static int64_t round_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t D
     return c;
 }
 
+static bool wave_chunks(int64_t M, int64_t Dv) {
+    return wave_shape(M, Dv, Dv) && !((M == 128 || M == 256) && (Dv == 64 || Dv == 128));
+}
 int64_t default_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
-    if (!wave_shape(M, Dv, Dv) || ((M == 128 || M == 256) && (Dv == 64 || Dv == 128))) return round_chunk(B, N, H, M, Dv);
+    if (!wave_chunks(M, Dv)) return round_chunk(B, N, H, M, Dv);
     // The wave kernels: about two waves per SIMD over the device (8 a compute unit), each
     // wave with 64 latents of a narrow bank or 32 of a wider one.
     const int64_t NW = Dv <= 32 && M > 32 ? (M + 63) / 64 : (M + 31) / 32;
@@ -481,6 +487,35 @@ int64_t default_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
     if (c < 32) c = 32;
     if (c > 8192) c = 8192;
     return c;
+}
+
+// The chunk of calls on the tokenwise kernels whatever the bank (Dk != Dv, the stablemax
+// encoder): of the two policies above the one with fewer tokens in line on the busiest slot, and
+// of equals the shorter, whose last round is the fuller, up to the 128 chunks that the scan takes
+// without adding to the whole.  us, round_chunk / the other (chosen):
+//   Dk 64, Dv 32, B 1, N 256, H 8, M 64              377 / 202 (32 tokens)
+//   Dk 16, Dv 32, B 8, N 4096, H 16, M 64           4162 / 3643 (256)
+//   Dk 32, Dv 64, B 1, N 8192, H 16, M 96           2051 / 2213 (256: 192 leaves a third of a round)
+//   Dk 64, Dv 32, B 1, N 16384, H 4, M 32            776 / 814 (128: 32 tokens are 512 chunks)
+int64_t tokenwise_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
+    const int64_t a = round_chunk(B, N, H, M, Dv);
+    if (!wave_chunks(M, Dv)) return a;
+    const int64_t b = default_chunk(B, N, H, M, Dv), slots = (M * Dv >= 128 * 128 ? 1 : 2) * device_cus();
+    auto in_line = [&](int64_t c) { return (std::max<int64_t>(B * H, 1) * ((N + c - 1) / c) + slots - 1) / slots * c; };
+    const bool shorter = b < a && (N + b - 1) / b <= 128;
+    return in_line(b) < in_line(a) || (in_line(b) == in_line(a) && shorter) ? b : a;
+}
+
+// The chunk of a call that names none; a workspace sized for default_chunk alone stays enough.
+static int64_t call_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dk, int64_t Dv, float power, size_t workspace) {
+    const int64_t c = default_chunk(B, N, H, M, Dv);
+    if (Dk == Dv && power <= 0.0f) return c;
+    const int64_t t = tokenwise_chunk(B, N, H, M, Dv);
+    return flare_ar_forward_workspace_size(B, N, H, M, Dv, t) <= workspace ? t : c;
+}
+// ... and the one to size its workspace for
+static int64_t most_chunks(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
+    return std::min(default_chunk(B, N, H, M, Dv), tokenwise_chunk(B, N, H, M, Dv));
 }
 
 }  // namespace flare
@@ -539,6 +574,10 @@ int flare_chunk_output(const void* Q, const void* K, const void* V, const void* 
     return rc;
 }
 
+int64_t flare_ar_tokenwise_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
+    return tokenwise_chunk(B, N, H, M, Dv);
+}
+
 int64_t flare_ar_default_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv) {
     return default_chunk(B, N, H, M, Dv);
 }
@@ -589,13 +628,13 @@ static size_t summary_bytes(int64_t B, int64_t N, int64_t H, int64_t M, int64_t 
 
 size_t flare_ar_forward_workspace_size(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv,
                                        int64_t chunk) {
-    if (chunk <= 0) chunk = default_chunk(B, N, H, M, Dv);
+    if (chunk <= 0) chunk = most_chunks(B, N, H, M, Dv);
     return summary_bytes(B, N, H, M, Dv, chunk);
 }
 
 size_t flare_ar_forward_workspace_size_sep(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv,
                                            int64_t chunk) {
-    if (chunk <= 0) chunk = default_chunk(B, N, H, M, Dv);
+    if (chunk <= 0) chunk = most_chunks(B, N, H, M, Dv);
     return summary_bytes(B, N, H, M, Dv, chunk) + align256((size_t)B * H * N * M * 2);
 }
 
@@ -617,7 +656,7 @@ int flare_stablemax_forward(const void* Q, const void* K, const void* V, const v
     FLARE_REQUIRE(B > 0 && N > 0 && H > 0 && M > 0 && Dk > 0 && Dv > 0,
                   "stablemax_forward: sizes must be positive");
     FLARE_REQUIRE(power > 0.0f && power < 1e30f, "stablemax_forward: power must be positive and finite");
-    if (chunk <= 0) chunk = default_chunk(B, N, H, M, Dv);
+    if (chunk <= 0) chunk = call_chunk(B, N, H, M, Dk, Dv, power, workspace_bytes);
     const size_t need = flare_ar_forward_workspace_size(B, N, H, M, Dv, chunk);
     if (!workspace || workspace_bytes < need) {
         set_error("stablemax_forward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
@@ -653,7 +692,7 @@ int flare_ar_forward_masked(const void* Q, const void* K, const void* V, const v
                             size_t workspace_bytes, void* stream) {
     FLARE_REQUIRE(Q && K && V && Y, "ar_forward: null pointer");
     FLARE_REQUIRE(B > 0 && N > 0 && H > 0 && M > 0 && Dk > 0 && Dv > 0, "ar_forward: sizes must be positive");
-    if (chunk <= 0) chunk = default_chunk(B, N, H, M, Dv);
+    if (chunk <= 0) chunk = call_chunk(B, N, H, M, Dk, Dv, 0.0f, workspace_bytes);
     const size_t need = flare_ar_forward_workspace_size(B, N, H, M, Dv, chunk);
     if (!workspace || workspace_bytes < need) {
         set_error("ar_forward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
@@ -747,7 +786,7 @@ int flare_ar_forward_noalloc(const void* Q, const void* K, const void* V, const 
     FLARE_REQUIRE(B > 0 && N > 0 && H > 0 && M > 0 && Dk > 0 && Dv > 0,
                   "ar_forward_noalloc: sizes must be positive");
     if (chunk <= 0) {
-        chunk = default_chunk(B, N, H, M, Dv);
+        chunk = call_chunk(B, N, H, M, Dk, Dv, 0.0f, kScratchBytes);
         // the shorter chunks of the wave kernels only where their summaries fit as well
         if (flare_ar_forward_workspace_size(B, N, H, M, Dv, chunk) > kScratchBytes) chunk = round_chunk(B, N, H, M, Dv);
     }

@@ -162,8 +162,10 @@ int flare_stablemax_backward(const void* Q, const void* K, const void* V, const 
                              void* dV, void* dQdec, void* dKdec, void* workspace, size_t workspace_bytes,
                              void* stream);
 
-/* The chunk length flare_ar_forward uses when called with chunk <= 0. */
+/* The chunk length flare_ar_forward uses when called with chunk <= 0 and Dk == Dv; and the one
+ * for Dk != Dv or the stablemax encoder (where the given workspace holds it). */
 int64_t flare_ar_default_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv);
+int64_t flare_ar_tokenwise_chunk(int64_t B, int64_t N, int64_t H, int64_t M, int64_t Dv);
 
 /*
  * Resources of a forward kernel this library launches for the given call

@@ -271,3 +271,20 @@ def test_chunk_policy_of_empty_problems(B, H, M, D):
     rc = lib.flare_ar_forward(p, p, p, None, None, 0, B, 64, H, M, D, D, 1.0, 0, None, None, None, None, None, None, p, 0,
                               p, 1 << 30, None)
     assert rc == -1 and b"positive" in lib.flare_last_error()
+
+
+@pytest.mark.parametrize("B,N,H,M,Dv,want", [(1, 256, 8, 64, 32, 32), (8, 4096, 16, 64, 32, 256), (1, 8192, 16, 96, 64, 256),
+                                             (1, 16384, 4, 32, 32, 128), (1, 8192, 16, 192, 64, 256), (2, 1531, 8, 192, 128, 96),
+                                             (1, 65536, 16, 256, 128, 4096), (2, 500, 3, 40, 80, 64)])
+def test_chunk_policy_of_tokenwise_calls(B, N, H, M, Dv, want):
+    """Calls that stay on the tokenwise kernels (Dk != Dv, stablemax) take the wave kernels' shorter
+    chunks only where their last round of workgroups is no emptier, and a workspace sized for a call
+    that names no chunk holds either kind's."""
+    lib = _lib.lib()
+    tokenwise, default = (f(B, N, H, M, Dv) for f in (lib.flare_ar_tokenwise_chunk, lib.flare_ar_default_chunk))
+    assert tokenwise == want
+    for size in (lib.flare_ar_forward_workspace_size, lib.flare_ar_forward_workspace_size_sep):
+        assert size(B, N, H, M, Dv, 0) >= max(size(B, N, H, M, Dv, c) for c in (tokenwise, default))
+    from causal_flare.autoregressive.training import _resolve_chunk_size
+    assert _resolve_chunk_size(None, B, N, H, M, Dv, Dv)[1] == default
+    assert _resolve_chunk_size(None, B, N, H, M, Dv + 16, Dv)[1] == tokenwise
