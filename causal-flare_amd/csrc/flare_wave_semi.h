@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restri
     const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
     const int t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * TT * NTK;
     if (t0 >= N) return;                          // (N and block are multiples of 16 NTK)
-    const float* zb = z + ((size_t)bh * (N / block) + t0 / block) * M * D;
+    const Bytes zb(z + ((size_t)bh * (N / block) + t0 / block) * M * D, (size_t)M * D * sizeof(float));
     GroupRow<T, DT> k[NTK];
     float mx[NTK], sum[NTK], lse[NTK];
 #pragma unroll
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restri
     for (int m0 = 0; m0 < M; m0 += 16) {
         ColRow<float, DT> r[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[i].load(zb + (size_t)min(m0 + 4 * g + i, M - 1) * D, c);
+        for (int i = 0; i < 4; ++i) r[i].load(zb, (m0 + 4 * g + i) * (4 * D), c);     // past the bank: zeros
         f32x4 s[NTK];
         scores(m0, s);
 #pragma unroll

@@ -381,3 +381,20 @@ def test_wave_backward_infinite_gradients(M, D, dtype, block):
     odd = wild[None]
     assert torch.equal(torch.nan_to_num(got[odd], nan=7.0), torch.nan_to_num(want[odd], nan=7.0))
     _check_grads({"v": got[~odd]}, [want[~odd].double().numpy()], dtype, "other columns")
+
+
+@pytest.mark.parametrize("M,D", [(40, 32), (17, 64), (64, 48)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_wave_semi_forward_infinite_value(M, D, dtype):
+    """An infinite value is infinite in y of its column from its block on, also for a bank that ends
+    inside a tile of latents; everything else is as without it."""
+    from causal_flare import flare_semi_autoregressive_trition
+    print("CASE wave_semi_infinite_value", M, D, dtype, flush=True)
+    B, N, H, block = 1, 192, 2, 48
+    q, k, v = (t.to(DEV) for t in seeded(11 * M + D, B, N, H, M, D, D, dtype, q_std=D ** -0.5))
+    vi = v.clone()
+    vi[0, 100, 1, 7] = float("-inf")
+    y, yi = (flare_semi_autoregressive_trition(q, k, x, block_size=block, chunk_size=16, scale=1.0)[0] for x in (v, vi))
+    assert torch.isneginf(yi[0, 96:, 1, 7]).all()
+    yi[0, 96:, 1, 7] = y[0, 96:, 1, 7]
+    assert torch.equal(yi, y)
