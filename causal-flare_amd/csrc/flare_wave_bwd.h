@@ -813,10 +813,10 @@ __global__ __launch_bounds__(256) void wave_lse_kernel(const T* __restrict__ Qd,
                 top = fmaxf(top, s[i]);
             }
             const float ref = safe_ref(top);
-            float a = sum[j] * exp_nat(mx[j] - ref);
+            float e[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a += exp_nat(s[i] - ref);
-            sum[j] = a;
+            for (int i = 0; i < 4; ++i) e[i] = exp_nat(s[i] - ref);
+            sum[j] = sum[j] * exp_nat(mx[j] - ref) + ((e[0] + e[1]) + (e[2] + e[3]));      // (one rounding of the sum)
             mx[j] = top;
         }
     }

@@ -72,8 +72,10 @@ struct StepRows {
 // ---------------------------------------------------------------------------
 // Readout of the block-causal forward from the blocks' states z = U / den in memory
 // ([B*H][N/block][M][D], fp32): y = sum over latents of the decoder's weight times z.  A wave
-// takes NTK tiles of 16 tokens of one block against all latents, twice: their log-sum-exp, then
-// the weights, whose C tiles are the factor of the fp32 products with z as they are.  Bound by
+// takes NTK tiles of 16 tokens of one block against all latents, twice: the largest score, then the
+// weights relative to it and their sum, the weights' C tiles being the factor of the fp32 products
+// with z as they are.  (A running log-sum-exp and weights taken from it: lse up to 3.5% and y 60%
+// further from 64 bits in fp32, in the same time.)  Bound by
 // the latency of z's and the latents' rows from cache (a block's z serves its few waves).
 // Measured: forward and backward of bf16 B 4, N 640, blocks of 32, H 16, M 192, D 64 take 307 us,
 // 3,578 with the readout as scalar products in LDS.
@@ -90,11 +92,11 @@ __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restri
     if (t0 >= N) return;                          // (N and block are multiples of 16 NTK)
     const Bytes zb(z + ((size_t)bh * (N / block) + t0 / block) * M * D, (size_t)M * D * sizeof(float));
     GroupRow<T, DT> k[NTK];
-    float mx[NTK], sum[NTK], lse[NTK];
+    float ref[NTK], sum[NTK];
 #pragma unroll
     for (int j = 0; j < NTK; ++j) {
         k[j].load(Qd + (((size_t)b * N + t0 + TT * j + c) * H + h) * D, g);
-        mx[j] = kNegInf;
+        ref[j] = kNegInf;
         sum[j] = 0.0f;
     }
     auto scores = [&](int m0, f32x4 (&s)[NTK]) {
@@ -111,21 +113,12 @@ __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restri
         f32x4 s[NTK];
         scores(m0, s);
 #pragma unroll
-        for (int j = 0; j < NTK; ++j) {
-            const float top = fmaxf(mx[j], fmaxf(fmaxf(s[j][0], s[j][1]), fmaxf(s[j][2], s[j][3])));
-            const float ref = safe_ref(top);
-            float a = sum[j] * exp_nat(mx[j] - ref);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a += exp_nat(s[j][i] - ref);
-            sum[j] = a;
-            mx[j] = top;
-        }
+        for (int j = 0; j < NTK; ++j) ref[j] = fmaxf(ref[j], fmaxf(fmaxf(s[j][0], s[j][1]), fmaxf(s[j][2], s[j][3])));
     }
     f32x4 y[NTK][DT];
 #pragma unroll
     for (int j = 0; j < NTK; ++j) {
-        const float top = group_max(mx[j]), ref = safe_ref(top);
-        lse[j] = ref + __logf(group_sum(sum[j] * exp_nat(mx[j] - ref)));
+        ref[j] = safe_ref(group_max(ref[j]));
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) y[j][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -138,7 +131,8 @@ __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restri
 #pragma unroll
         for (int j = 0; j < NTK; ++j) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) s[j][i] = exp_nat(s[j][i] - lse[j]);      // 0 past the bank
+            for (int i = 0; i < 4; ++i) s[j][i] = exp_nat(s[j][i] - ref[j]);          // 0 past the bank
+            sum[j] += (s[j][0] + s[j][1]) + (s[j][2] + s[j][3]);
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -148,6 +142,7 @@ __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restri
 #pragma unroll
     for (int j = 0; j < NTK; ++j) {
         const int t = t0 + TT * j + c;
+        const float all = group_sum(sum[j]), norm = 1.0f / all;
         const size_t row = (((size_t)b * N + t) * H + h) * D;
 #pragma unroll
         for (int pc = 0, dt = 0; pc < pieces<DT>(); dt = piece_start<DT>(++pc))
@@ -156,13 +151,13 @@ __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restri
                 float o[4];
                 const int P = piece_of<DT>(dt);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = e < P ? y[j][dt + e < DT ? dt + e : 0][i] : 0.0f;
+                for (int e = 0; e < 4; ++e) o[e] = e < P ? y[j][dt + e < DT ? dt + e : 0][i] * norm : 0.0f;
                 const size_t at = row + col_of<DT>(dt, 4 * g + i);
                 if (P == 4) store_cols<4>(Y, at, o, out_dtype);
                 else if (P == 2) store_cols<2>(Y, at, o, out_dtype);
                 else store_cols<1>(Y, at, o, out_dtype);
             }
-        if (lse_out != nullptr && g == 0) lse_out[(size_t)bh * N + t] = lse[j];
+        if (lse_out != nullptr && g == 0) lse_out[(size_t)bh * N + t] = ref[j] + __logf(all);
     }
 }
 
