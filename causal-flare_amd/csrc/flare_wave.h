@@ -46,7 +46,6 @@ typedef u32 u32x2 __attribute__((ext_vector_type(2), may_alias));
 typedef u32 u32x4 __attribute__((ext_vector_type(4), may_alias));
 typedef unsigned short u16_a __attribute__((may_alias));
 typedef float f32x4_a __attribute__((ext_vector_type(4), may_alias));
-typedef mfma::bf16 bf16x8_a __attribute__((ext_vector_type(8), may_alias));
 
 constexpr int TT = 16;              // tokens per tile
 
@@ -94,18 +93,6 @@ template <typename T, int D>
 struct RowOp {   // 16-bit: steps of 32 columns, 8 a lane group; a last step of 16 fills two groups
     static constexpr int S = (D + 31) / 32;
     bf16x8 a[S];
-    __device__ __forceinline__ void load(const T* row, int g) {
-        const mfma::bf16* p = reinterpret_cast<const mfma::bf16*>(row);
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            if (32 * s + 32 <= D) {
-                a[s] = *reinterpret_cast<const bf16x8_a*>(p + 32 * s + 8 * g);
-            } else {
-                const bf16x8 x = *reinterpret_cast<const bf16x8_a*>(p + 32 * s + 8 * (g & 1));
-                a[s] = g < 2 ? x : bf16x8{};
-            }
-        }
-    }
     // byte offset of this lane within a row, and the load from it
     static __device__ __forceinline__ unsigned lane(int g) { return 16 * g; }
     __device__ __forceinline__ void load(const Bytes& b, unsigned row, int g) {
@@ -123,10 +110,6 @@ struct RowOp {   // 16-bit: steps of 32 columns, 8 a lane group; a last step of 
 template <int D>
 struct RowOp<float, D> {   // lane group g holds columns [g D/4, (g+1) D/4)
     f32x4 a[D / 16];
-    __device__ __forceinline__ void load(const float* row, int g) {
-#pragma unroll
-        for (int s = 0; s < D / 16; ++s) a[s] = *reinterpret_cast<const f32x4_a*>(row + g * (D / 4) + 4 * s);
-    }
     static __device__ __forceinline__ unsigned lane(int g) { return g * D; }
     __device__ __forceinline__ void load(const Bytes& b, unsigned row, int) {
 #pragma unroll

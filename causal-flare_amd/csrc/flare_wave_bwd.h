@@ -1074,7 +1074,8 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_gz_kernel(BwdPtrs a, int 
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
                     for (int k = 0; k < 4; ++k)
-                        if (k < walk_piece<DT, FLAT>(dt)) row[walk_col<DT, FLAT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
+                        if (k < walk_piece<DT, FLAT>(dt))
+                            row[walk_col<DT, FLAT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
         }
     }
 }
@@ -1348,7 +1349,9 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
         // dv and X += W^T g, a piece of value columns at a time.  Token by token the other tokens' g, which may not be finite, are taken as
         // zero.  (A select each time and no branch: after a branch around it the compiler reads
         // the product above too early on the skipped side.)
-        const bool on[4] = {j < 0 || 4 * g == j, j < 0 || 4 * g + 1 == j, j < 0 || 4 * g + 2 == j, j < 0 || 4 * g + 3 == j};
+        bool on[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) on[i] = j < 0 || 4 * g + i == j;
 #pragma unroll
         for (int st = 0, d1 = 0; st < steps<T, DT>(); d1 = step_start<T, DT>(++st)) {
             stage<DT>();

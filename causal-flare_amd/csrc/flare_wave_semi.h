@@ -361,7 +361,8 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_semi_gz_kernel(BwdPtrs a,
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
                     for (int k = 0; k < 4; ++k)
-                        if (k < walk_piece<DT, FLAT>(dt)) row[walk_col<DT, FLAT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
+                        if (k < walk_piece<DT, FLAT>(dt))
+                            row[walk_col<DT, FLAT>(dt, 4 * g + i) + k] = x[mt][dt + k < DT ? dt + k : 0][i];
         }
     }
 }
