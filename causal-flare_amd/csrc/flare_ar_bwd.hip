@@ -1221,7 +1221,7 @@ static int launch_contract(const T* q, const T* k, const T* qd, const T* kd, boo
     // Where rows can be read 16 bytes at a time: the wave kernels.  Against the 16-bit MFMA
     // kernels below, dQ 74 -> 33 us and dK 41 -> 43 at bf16 B 4, N 4096, H 16, M 128, D 64, dQ
     // 162 -> 126 and dK 127 -> 94 at N 16384, H 16, M 256, D 128; against the scalar ones, dQ
-    // 296 -> 10 and dK 89 -> 10 at B 4, N 2011, H 16, M 64, D 32.
+    // 296 -> 11 and dK 89 -> 10 at B 4, N 2011, H 16, M 64, D 32.
     const bool wave = (mfma_phase_mask() & 3) == 3 && wave_shape(M, Dk, Dk) && M % 16 == 0 && wave_reach(N, M) &&
                       wave_aligned({q, k, qd, kd, dK, dQd, DS, AL, C});
     const wave::ContractPtrs cp{DS, C, AL, gy, cgz};

@@ -244,7 +244,7 @@ static int semi_forward_impl(const void* Q, const void* K, const void* V, const 
     const void* qd = Qdec ? Qdec : K;
     const void* kd = Kdec ? Kdec : Q;
     // Banks the wave kernels have an instance for, on matrix products: bf16 B 4, N 640, blocks of
-    // 32, M 192, D 64 takes 307 us a training step so, 3,578 on the kernel below
+    // 32, M 192, D 64 takes 333 us a training step so, 3,600 with the kernel below
     if ((mfma_phase_mask() & 2) && wave_shape(M, Dk, Dv) && wave_aligned({qd, kd, bnum, Y})) {
         const WaveArgs a{Q, K, V, qd, kd, B, N, H, M, Dk, scale, block, nullptr};
         return dtype == FLARE_BF16  ? wave::semi_output_bf16(a, block, bnum, Y, out_dtype, lse_dec, s)

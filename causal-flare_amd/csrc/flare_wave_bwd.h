@@ -44,13 +44,14 @@
 // 60% of the issue slots are used, 12% of the matrix pipe's).  What is read the other way round
 // (V, g, X and the e / w tiles of 16-bit kernels) comes through transposing LDS reads, X, e and w
 // already split into bf16 hi + lo: splitting after the read took a third more instructions
-// (1,691 against 1,114 in the backward walk at D = 128; 677 -> 515 us at N 16384, M 256).
+// (1,691 against 1,114 in the backward walk at D = 128; 677 -> 515 us at N 16384, M 256, the hi
+// parts cut off).
 // Measured, forward and backward, against per-token statistics and one state per 32 tokens in
 // memory (MI355X):
-//   bf16 B 4, N 4096, H 16, M 128, D 64    1521 -> 520 us (wave_gz 121, wave_ds 161 of it)
-//   bf16 N 16384, H 16, M 256, D 128       3774 -> 1403 us (wave_gz 411, wave_ds 515)
-//   bf16 B 4, N 2011, H 16, M 64, D 32     2947 -> 196 us
-//   fp32 B 2, N 1024, H 8, M 64, D 64, decoder weights of its own   1170 -> 207 us
+//   bf16 B 4, N 4096, H 16, M 128, D 64    1525 -> 529 us (wave_gz 124, wave_ds 166 of it)
+//   bf16 N 16384, H 16, M 256, D 128       3807 -> 1445 us (wave_gz 405, wave_ds 517)
+//   bf16 B 4, N 2011, H 16, M 64, D 32     2946 -> 213 us (wave_gz 37, wave_ds 48)
+//   fp32 B 2, N 1024, H 8, M 64, D 64, decoder weights of its own   1171 -> 216 us
 #pragma once
 
 #include <type_traits>

@@ -12,7 +12,7 @@ namespace wave {
 
 // Latent tiles per wave of the walks: 32 latents.  With 16, four waves a SIMD fit up to D = 64,
 // but each tile's rows, g v^T products and sums over latents serve half as many: B 4, N 4096,
-// H 16, M 128, D 64 takes 122 + 228 us so and 121 + 161 us with 32; fp32 B 2, N 1024, H 8, M 64,
+// H 16, M 128, D 64 takes 122 + 228 us so and 124 + 166 us with 32; fp32 B 2, N 1024, H 8, M 64,
 // D 64 takes 43 + 36 and 33 + 30 us.  At D = 128 a wave of 16 spills as well.
 constexpr int kWalkTiles = 2;
 

@@ -15,8 +15,8 @@
 //
 // Bound by the latency of a step's chain (load, scores, exponentials, products, barrier) at two
 // to four waves a SIMD.  Measured, forward and backward, against one state per block in memory:
-// bf16 B 2, N 8192, blocks of 64, H 16, M 128, D 64: 1448 -> 482 us (wave_semi_gz 101,
-// wave_semi_ds 146 of it).
+// bf16 B 2, N 8192, blocks of 64, H 16, M 128, D 64: 1449 -> 485 us (wave_semi_gz 101,
+// wave_semi_ds 143 of it).
 #pragma once
 
 #include "flare_wave_bwd.h"
@@ -77,8 +77,7 @@ struct StepRows {
 // with z as they are.  (A running log-sum-exp and weights taken from it: lse up to 3.5% and y 60%
 // further from 64 bits in fp32, in the same time.)  Bound by
 // the latency of z's and the latents' rows from cache (a block's z serves its few waves).
-// Measured: forward and backward of bf16 B 4, N 640, blocks of 32, H 16, M 192, D 64 take 307 us,
-// 3,578 with the readout as scalar products in LDS.
+// Measured: forward and backward of bf16 B 4, N 640, blocks of 32, H 16, M 192, D 64 take 333 us.
 // ---------------------------------------------------------------------------
 template <typename T, int DT, int NTK>
 __global__ __launch_bounds__(256) void wave_semi_output_kernel(const T* __restrict__ Qd, const T* __restrict__ Kd,
