@@ -33,7 +33,7 @@
 // 2^-18.  Two parts serve the banks whose states always met the matrix units as two parts (M
 // 128 and 256, D 64 and 128), three the banks whose kernels were all fp32 (three_parts).  Share
 // of dV entries that are not the rounded 64-bit value, against those kernels, fp16, N 1531: M 64,
-// D 32 0.16 -> 0.13% (0.7% with two parts), M 128, D 64 0.73 -> 0.57% (1.1% with two of which
+// D 32 0.16 -> 0.13% (0.7% with two parts), M 128, D 64 0.73 -> 0.52% (1.1% with two of which
 // the first is cut off and not rounded); dK of separate decoder weights at M 64, D 32 1.75 -> 0.18%.
 //
 // Numerics.  Weights inside a tile are relative to the latents' max after the tile, X and Y
@@ -1345,11 +1345,14 @@ __global__ __launch_bounds__(64 * (16 / MT)) void wave_ds_kernel(BwdPtrs a, int 
             }
         }
         wave_lds_sync();
-        const F gf = factor<F>(4 * g >= c ? G[0] : 0.0f, 4 * g + 1 >= c ? G[1] : 0.0f, 4 * g + 2 >= c ? G[2] : 0.0f,
-                               4 * g + 3 >= c ? G[3] : 0.0f);
-        // dv and X += W^T g, a piece of value columns at a time.  Token by token the other tokens' g, which may not be finite, are taken as
-        // zero.  (A select each time and no branch: after a branch around it the compiler reads
-        // the product above too early on the skipped side.)
+        // (whole in every 16-bit instance: rounded to two parts it alone put dV of short sequences 5
+        // to 40% further off where the states are two parts)
+        typedef typename ProdOf<T, 3>::F Whole;
+        const Whole gf = factor<Whole>(4 * g >= c ? G[0] : 0.0f, 4 * g + 1 >= c ? G[1] : 0.0f, 4 * g + 2 >= c ? G[2] : 0.0f,
+                                       4 * g + 3 >= c ? G[3] : 0.0f);
+        // dv and X += W^T g, a piece of value columns at a time.  Token by token the other tokens' g,
+        // which may not be finite, are taken as zero.  (A select each time and no branch: after a
+        // branch around it the compiler reads the product above too early on the skipped side.)
         bool on[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) on[i] = j < 0 || 4 * g + i == j;

@@ -161,18 +161,19 @@ def test_wave_backward(M, D, N, dtype, sep):
 # dV is a sum without cancellation of fp32 factors, so a share of about 2 |error| / ulp of its
 # entries does not come out as the rounded exact value.  fp32 sums here end within some 2^-22 of the
 # value: 0.1% of fp16's ulp of 2^-10, an eighth of that in bf16; factors of 16 to 17 bits 0.8 to
-# 1.5%.  The 16-bit kernels' own banks, whose states were two bf16 parts before the walks, had 0.75%.
+# 1.5%.  The 16-bit kernels' own banks, whose states were two bf16 parts before the walks, had 0.75%
+# (0.5% in 33 tokens, where the sums inside a tile, then in fp32, count for more).
 @pytest.mark.parametrize("M,D,dtype,share", [(64, 32, torch.float16, 4e-3), (48, 48, torch.float16, 4e-3),
                                              (96, 64, torch.float16, 4e-3), (208, 96, torch.float16, 4e-3),
                                              (192, 128, torch.float16, 4e-3), (64, 32, torch.bfloat16, 1e-3),
-                                             (128, 64, torch.float16, 7.5e-3), (256, 128, torch.float16, 7.5e-3)])
-@pytest.mark.parametrize("block", [0, 64])
-def test_wave_backward_keeps_fp32_factors(M, D, dtype, share, block):
+                                             (128, 64, torch.float16, 6.5e-3), (256, 128, torch.float16, 6.5e-3)])
+@pytest.mark.parametrize("block,N,H", [(0, 512, 2), (64, 512, 2), (0, 40, 16)])
+def test_wave_backward_keeps_fp32_factors(M, D, dtype, share, block, N, H):
     """What the walks hold in fp32 enters their products whole: dV is the rounded exact value up to
     fp32 sums (one wave to a full workgroup, one X tile in LDS and two, both layers)."""
     from causal_flare import flare_semi_autoregressive_trition
-    print("CASE wave_fp32_factors", M, D, dtype, block, flush=True)
-    B, N, H = 1, 512, 2
+    print("CASE wave_fp32_factors", M, D, dtype, block, N, flush=True)
+    B = 1
     q, k, v = seeded(3 * M + D, B, N, H, M, D, D, dtype)
     g = torch.randn(B, N, H, D, generator=torch.Generator().manual_seed(M)).to(dtype)
     if block:
@@ -183,7 +184,7 @@ def test_wave_backward_keeps_fp32_factors(M, D, dtype, share, block):
     else:
         dv, ref = _grads(q, k, v, g)["v"], O.ar_grads(q, k, v, g)[2]
     wrong = float((dv.cpu() != torch.from_numpy(np.asarray(ref)).to(dtype)).double().mean())
-    assert wrong <= share, f"{wrong:.4f} of dV is not the rounded value"
+    assert wrong <= min(share, 5.5e-3 if N < 64 else share), f"{wrong:.4f} of dV is not the rounded value"
 
 
 @pytest.mark.parametrize("M,D,dtype", [(64, 32, torch.float32), (128, 64, torch.float32), (128, 64, torch.bfloat16)])
